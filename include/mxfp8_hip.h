@@ -408,6 +408,36 @@ int mx_grouped_wgrad_nt(const uint8_t *aq, const uint8_t *as, int64_t lda, int64
                         int64_t M, void *dw, int dw_dtype, int64_t stride_dwe, int64_t lddw, int64_t N,
                         int64_t Kout, void *workspace, int64_t workspace_bytes, void *stream);
 
+/* ---- top-k router ------------------------------------------------------------------------ */
+
+/*
+ * Sigmoid top-k routing of x (T, D) over E experts with the router matrix w (E, D, contiguous):
+ *   scores = sigmoid(x w^T), evaluated in fp32;  choose by scores + bias (bias (E,) or NULL), the top_k largest in
+ *   descending order, ties to the lower expert;
+ *   idx (T, top_k) = the experts;  weight (T, top_k), in x's type, = factor * score, the scores of a token divided by
+ *   max(their sum, 1e-9) first when norm != 0;  scores (T, top_k) fp32 = the selected scores (what the backward takes;
+ *   may be NULL);  counts (E,) int32 = rows per expert (overwritten).
+ * x and w share a 16-bit type or w is fp32; fp32 x takes fp32 w.  D % 8 == 0, 16-byte aligned rows, E <= 256,
+ * top_k <= 64.
+ * Replaces TopKRouter.route (src/kohakuwullm/models/components/moe.py:97-199) without groups and auxiliary losses, and
+ * expert_counts (:38-46) behind it.
+ */
+int mx_router_topk(const void *x, int x_dtype, int64_t ldx, const void *w, int w_dtype, const void *bias, int bias_dtype,
+                   int64_t T, int64_t D, int64_t E, int64_t top_k, int norm, float factor, int64_t *idx, void *weight,
+                   float *scores, int32_t *counts, void *stream);
+
+/*
+ * The gradient of mx_router_topk's gate weights: grad_weight (T, top_k) into dx (T, D), in x's type, and dw (E, D), in
+ * w's type; either may be NULL.  idx and scores as the forward wrote them.  fp32 arithmetic, one writer per element, the
+ * partial sums of dw added in a fixed order.  top_k <= 16.  workspace (for dw): fp32 scratch of
+ * mx_router_backward_workspace(T, D, E) elements.
+ */
+int64_t mx_router_backward_workspace(int64_t T, int64_t D, int64_t E);
+int mx_router_topk_backward(const void *grad_weight, int gw_dtype, const int64_t *idx, const float *scores, const void *x,
+                            int x_dtype, int64_t ldx, const void *w, int w_dtype, int64_t T, int64_t D, int64_t E,
+                            int64_t top_k, int norm, float factor, void *dx, int64_t lddx, void *dw, float *workspace,
+                            int64_t workspace_len, void *stream);
+
 /* ---- expert dispatch either side of the routed-expert GEMMs ------------------------------ */
 
 /*

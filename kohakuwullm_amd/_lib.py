@@ -21,7 +21,7 @@ MX_OK, MX_EINVAL, MX_EUNSUPPORTED, MX_ELAUNCH, MX_ENODEV, MX_ECAPTURE, MX_ETOOBI
 MX_ABI_VERSION = 2
 MX_DTYPE = {torch.bfloat16: 0, torch.float16: 1, torch.float32: 2}
 
-_i64, _p, _ci = ctypes.c_int64, ctypes.c_void_p, ctypes.c_int
+_i64, _p, _ci, _f = ctypes.c_int64, ctypes.c_void_p, ctypes.c_int, ctypes.c_float
 
 # name -> (restype, argtypes); mirrors include/mxfp8_hip.h declaration by declaration.
 SIGNATURES = {
@@ -59,6 +59,11 @@ SIGNATURES = {
         _ci, [_p, _ci, _i64, _i64, _i64, _p, _ci, ctypes.c_float, _p, _p, _i64, _p, _i64, _p, _i64, _p, _i64, _p]),
     "mx_rmsnorm_backward": (
         _ci, [_p, _ci, _i64, _i64, _i64, _p, _ci, _p, _i64, _p, _p, _i64, _p, _i64, _p]),
+    "mx_router_topk": (
+        _ci, [_p, _ci, _i64, _p, _ci, _p, _ci, _i64, _i64, _i64, _i64, _ci, _f, _p, _p, _p, _p, _p]),
+    "mx_router_backward_workspace": (_i64, [_i64, _i64, _i64]),
+    "mx_router_topk_backward": (
+        _ci, [_p, _ci, _p, _p, _p, _ci, _i64, _p, _ci, _i64, _i64, _i64, _i64, _ci, _f, _p, _i64, _p, _p, _i64, _p]),
     "mx_expert_counts": (_ci, [_p, _ci, _i64, _i64, _p, _p]),
     "mx_expert_sort_workspace": (_i64, [_i64, _i64]),
     "mx_expert_sort": (_ci, [_p, _ci, _i64, _p, _i64, _i64, _p, _p, _p, _p, _p, _i64, _p]),

@@ -4,6 +4,8 @@
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
+#include <atomic>
+
 #include "mxfp8_hip.h"
 
 #define MX_BLOCK 32
@@ -13,10 +15,14 @@ namespace mx {
 // Whether work on `st` is being recorded into a graph (mx_gemm.hip).  Every entry point asks before it
 // launches and returns MX_ECAPTURE: recording this library's launches is switched off.
 bool stream_is_capturing(hipStream_t st);
+int num_cus();  // CUs of the current device (cached per device ordinal)
+// hipFuncSetAttribute(MaxDynamicSharedMemorySize) once per device; `done` has one bit per device ordinal.
+bool allow_dynamic_lds(const void *kernel, int bytes, std::atomic<uint64_t> &done);
 
 typedef int v8i __attribute__((ext_vector_type(8)));
 typedef int v4i __attribute__((ext_vector_type(4)));
 typedef int v2i __attribute__((ext_vector_type(2)));
+typedef float v2f __attribute__((ext_vector_type(2)));
 typedef float v4f __attribute__((ext_vector_type(4)));
 typedef unsigned short v8us __attribute__((ext_vector_type(8)));
 

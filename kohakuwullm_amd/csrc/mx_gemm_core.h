@@ -852,12 +852,6 @@ __device__ __forceinline__ void tile_of(int id, int tiles_m, int tiles_n, int &t
     if (stagger) tn = (tn + (group * xcds / groups) * tiles_n / xcds) % tiles_n;
 }
 
-// Host-side launch helpers shared by the GEMM translation units (defined in mx_gemm.hip).
-int num_cus();                            // CUs of the current device (cached per device ordinal)
-bool stream_is_capturing(hipStream_t st);  // true also when the capture status cannot be read
-// hipFuncSetAttribute(MaxDynamicSharedMemorySize) once per device; `done` has one bit per device ordinal.
-bool allow_dynamic_lds(const void *kernel, int bytes, std::atomic<uint64_t> &done);
-
 // Launch of a kernel that needs more than 64 KiB of dynamic LDS.  The "attribute already set" word is a
 // function-local static of this instantiation, i.e. one per kernel: no table shared between kernels, no lock.
 template <auto Kern, typename Args>

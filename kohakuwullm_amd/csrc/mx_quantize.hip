@@ -8,7 +8,6 @@
 #include "mx_common.h"
 
 namespace mx {
-int num_cus();  // CUs of the current device (mx_gemm.hip)
 }
 
 namespace mx {

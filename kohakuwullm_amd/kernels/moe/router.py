@@ -1,0 +1,76 @@
+"""Sigmoid top-k routing on the HIP kernels: scores, selection, gate weights and histogram in one pass, with its backward.
+
+Counterpart of ``TopKRouter.route`` (``src/kohakuwullm/models/components/moe.py:97-199``) for a router without groups and
+auxiliary losses; :class:`kohakuwullm_amd.models.moe.TopKRouter` uses it where :func:`can_route` allows and its PyTorch
+composition elsewhere.
+"""
+
+from __future__ import annotations
+
+import torch
+
+from kohakuwullm_amd import _lib
+
+MAX_EXPERTS, MAX_TOP_K = 256, 16
+
+
+def can_route(x: torch.Tensor, weight: torch.Tensor, top_k: int) -> bool:
+    """Whether the kernels take these operands (types, alignment, limits); autocast changes the arithmetic and is not covered."""
+    e, d = weight.shape
+    return (x.is_cuda and x.dim() == 2 and x.shape[0] > 0 and x.dtype in _lib.MX_DTYPE and weight.dtype in (x.dtype, torch.float32)
+            and d % 8 == 0 and e <= MAX_EXPERTS and top_k <= min(MAX_TOP_K, e) and weight.is_contiguous()
+            and weight.device == x.device and weight.data_ptr() % 16 == 0 and not torch.is_autocast_enabled("cuda"))
+
+
+class _RouteTopK(torch.autograd.Function):
+    @staticmethod
+    def forward(ctx, x, weight, bias, top_k, norm, factor):
+        if x.stride(1) != 1 or x.stride(0) * x.element_size() % 16 or x.data_ptr() % 16:
+            x = x.contiguous()
+        (t, d), e, dev = x.shape, weight.shape[0], x.device
+        need = ctx.needs_input_grad[0] or ctx.needs_input_grad[1]
+        idx = torch.empty(t, top_k, device=dev, dtype=torch.int64)
+        gate = torch.empty(t, top_k, device=dev, dtype=x.dtype)
+        scores = torch.empty(t, top_k, device=dev, dtype=torch.float32) if need else None
+        counts = torch.empty(e, device=dev, dtype=torch.int32)
+        _lib.invoke(
+            "mx_router_topk", 2.0 * t * d * e, x, x.data_ptr(), _lib.MX_DTYPE[x.dtype], x.stride(0), weight.data_ptr(),
+            _lib.MX_DTYPE[weight.dtype], 0 if bias is None else bias.data_ptr(), 0 if bias is None else _lib.MX_DTYPE[bias.dtype],
+            t, d, e, top_k, int(norm), float(factor), idx.data_ptr(), gate.data_ptr(), 0 if scores is None else scores.data_ptr(),
+            counts.data_ptr(),
+        )
+        if need:
+            ctx.save_for_backward(x, weight, idx, scores)
+            ctx.norm, ctx.factor = norm, factor
+        ctx.mark_non_differentiable(idx, counts)
+        ctx.set_materialize_grads(False)
+        return idx, gate, counts
+
+    @staticmethod
+    def backward(ctx, _idx, grad, _counts):
+        if grad is None:
+            return (None,) * 6
+        x, weight, idx, scores = ctx.saved_tensors
+        (t, d), e, lib = x.shape, weight.shape[0], _lib.load()
+        grad = grad.contiguous()
+        dx = torch.empty(t, d, device=x.device, dtype=x.dtype) if ctx.needs_input_grad[0] else None
+        dw = torch.empty_like(weight) if ctx.needs_input_grad[1] else None
+        words = lib.mx_router_backward_workspace(t, d, e) if dw is not None else 0
+        scratch = torch.empty(words, device=x.device, dtype=torch.float32)
+        _lib.invoke(
+            "mx_router_topk_backward", 4.0 * t * d * e, x, grad.data_ptr(), _lib.MX_DTYPE[grad.dtype], idx.data_ptr(),
+            scores.data_ptr(), x.data_ptr(), _lib.MX_DTYPE[x.dtype], x.stride(0), weight.data_ptr(), _lib.MX_DTYPE[weight.dtype],
+            t, d, e, idx.shape[1], int(ctx.norm), float(ctx.factor), 0 if dx is None else dx.data_ptr(), d,
+            0 if dw is None else dw.data_ptr(), scratch.data_ptr() if words else 0, words,
+        )
+        return dx, dw, None, None, None, None
+
+
+def route_topk(x: torch.Tensor, weight: torch.Tensor, bias: torch.Tensor | None, top_k: int, norm: bool, factor: float):
+    """``(idx (T, k) int64, gate (T, k) in x's type, counts (E,) int32)`` of sigmoid scores ``x @ weight.T``.
+
+    The ``top_k`` experts with the largest ``score + bias``, best first (ties to the lower expert); ``gate`` is ``factor``
+    times their scores, normalized over the token's picks when ``norm``.  Differentiable in ``x`` and ``weight`` through
+    ``gate``.  See :func:`can_route` for what it takes.
+    """
+    return _RouteTopK.apply(x, weight, bias, top_k, norm, factor)

@@ -11,8 +11,9 @@ the cache drop on ``_apply``, ``forward(x, route_on=None)``, ``router_losses`` a
 reference's keywords (``components/moe.py:49-248``).
 
 What runs where.  The MXFP8 routed paths (``mxfp8_expert_path`` ``"fused"`` | ``"unfused"``), the
-dispatch (``expert_counts``, ``expert_sort``) and the combine run on this package's HIP kernels.
-The router's scores and top-k, and the 16-bit routed path a layer uses before ``enable_mxfp8``
+router (sigmoid scores without groups and auxiliary losses, outside autocast: ``kernels/moe/router.py``), the dispatch
+(``expert_counts``, ``expert_sort``) and the combine run on this package's HIP kernels.
+Other routers' scores and top-k, and the 16-bit routed path a layer uses before ``enable_mxfp8``
 (the reference's bf16 Triton kernels, which are not part of the MXFP8 path), are plain PyTorch
 here: ``expert_path`` ``"fused"`` and ``"eager"`` name the same PyTorch composition.
 """
@@ -24,6 +25,7 @@ import torch.nn as nn
 import torch.nn.functional as F
 
 from kohakuwullm_amd.kernels.moe.moe_dispatch import combine_routed, expert_counts, expert_sort
+from kohakuwullm_amd.kernels.moe.router import can_route, route_topk
 from kohakuwullm_amd.kernels.mxfp8.linear import compute_dtype
 from kohakuwullm_amd.kernels.mxfp8.moe import (
     MXFP8ExpertWeights,
@@ -52,7 +54,7 @@ def _histogram(flat_idx: torch.Tensor, num_buckets: int) -> torch.Tensor:
 
 @ROUTER.register("topk")
 class TopKRouter(nn.Module):
-    """Token -> expert assignment (``components/moe.py:49-248``), evaluated in fp32 with PyTorch ops.
+    """Token -> expert assignment (``components/moe.py:49-248``), evaluated in fp32.
 
     Scores are ``score_func(x W^T)``; selection adds the balancing bias (a buffer moved by
     :meth:`update_bias`, never by a gradient) and may be limited to the strongest ``topk_groups``
@@ -92,8 +94,20 @@ class TopKRouter(nn.Module):
         """``x (T, D)`` -> ``(topk_idx, topk_weight)``."""
         return self.route(x)[:2]
 
+    def _on_kernels(self, x: torch.Tensor) -> bool:
+        """Whether the fused kernels evaluate this call: sigmoid scores, one group, no auxiliary loss, shapes they take."""
+        return (self.score_func == "sigmoid" and self.n_groups == 1 and self.aux_loss_weight <= 0 and self.z_loss_weight <= 0
+                and can_route(x, self.weight, self.top_k))
+
     def route(self, x: torch.Tensor):
         """``(topk_idx (T, k), topk_weight (T, k) in x.dtype, counts (E,) int32)``."""
+        if self._on_kernels(x):
+            self.aux_loss = self.z_loss = None
+            topk_idx, topk_weight, counts = route_topk(x, self.weight, self.expert_bias, self.top_k,
+                                                       self.norm_topk_prob and self.top_k > 1, self.routed_scaling_factor)
+            if self.training and self.load_accum is not None:
+                self.load_accum += counts
+            return topk_idx, topk_weight, counts
         logits = F.linear(x.float(), self.weight.float())
         scores = SCORE_FUNCS[self.score_func](logits)
         choose_by = scores if self.expert_bias is None else scores + self.expert_bias

@@ -1,0 +1,80 @@
+"""The fused top-k router against fp64 on the CPU: selection, gate weights, histogram and both gradients, at the edges of
+its tiles (tokens per workgroup 16, 32 or 64 by their number, experts per MFMA tile 16 and per lane 64, K steps of 32 over eight waves, chunks of
+tokens and 128 columns in the backward)."""
+
+import pytest
+import torch
+
+from conftest import SEED
+
+pytestmark = pytest.mark.gpu
+DEV = "cuda:0"
+BF, HF, F32 = torch.bfloat16, torch.float16, torch.float32
+
+
+@pytest.mark.parametrize("tokens,dim,experts,top_k,xdt,wdt,norm,biased", [
+    (1, 8, 1, 1, BF, BF, False, False),
+    (16, 256, 64, 6, BF, BF, True, True),
+    (17, 72, 16, 4, BF, F32, True, True),
+    (50, 1024, 33, 8, HF, HF, True, False),
+    (300, 520, 100, 16, F32, F32, False, True),
+    (130, 136, 256, 5, HF, F32, True, True),
+    (5003, 1024, 64, 6, BF, BF, True, True),
+    (12301, 136, 48, 4, HF, HF, True, True),
+])
+def test_route_topk(tokens, dim, experts, top_k, xdt, wdt, norm, biased):
+    from kohakuwullm_amd.kernels.moe.router import can_route, route_topk
+
+    g = torch.Generator().manual_seed(SEED)
+    x = torch.randn(tokens, dim, generator=g).to(xdt)
+    w = (torch.randn(experts, dim, generator=g) * dim**-0.5).to(wdt)
+    bias = (torch.randn(experts, generator=g) * 0.05).to(BF) if biased else None
+    up = torch.randn(tokens, top_k, generator=g).to(xdt)
+    xd, wd = x.to(DEV).requires_grad_(True), w.to(DEV).requires_grad_(True)
+    assert can_route(xd, wd, top_k)
+    idx, gate, counts = route_topk(xd, wd, None if bias is None else bias.to(DEV), top_k, norm, 1.5)
+    assert idx.dtype == torch.int64 and gate.dtype == xdt and counts.dtype == torch.int32
+
+    x64, w64 = x.double().requires_grad_(True), w.double().requires_grad_(True)
+    scores = (x64 @ w64.T).sigmoid()
+    choose = scores.detach() + (0.0 if bias is None else bias.double())
+    want = choose.topk(top_k, dim=-1).indices
+    got = idx.cpu()
+    # a different pick is a near tie: an fp32 sum of `dim` products of size ~1/sqrt(dim) and the sigmoid are off by less
+    # than 2^-24 (sqrt(dim) + 8) here, and the two picks' scores differ by no more than twice that
+    bound = 2.0 ** -23 * (dim**0.5 + 8)
+    gap = (choose.gather(1, got) - choose.gather(1, want)).abs()
+    assert (gap[got != want] < bound).all()
+    assert torch.equal(counts.cpu().long(), torch.bincount(got.reshape(-1), minlength=experts))
+    picked = scores.gather(1, got)
+    ref = 1.5 * (picked / picked.sum(-1, keepdim=True) if norm else picked)
+    # half a unit in the last place, relative: 2^-p for a significand of p bits (8, 11, 24), plus the fp32 error of the logit
+    half_ulp = {BF: 2.0**-8, HF: 2.0**-11, F32: 2.0**-24}
+    assert ((gate.detach().cpu().double() - ref.detach()).abs() <= ref.detach() * half_ulp[xdt] * 1.01 + bound).all()
+
+    gate.backward(up.to(DEV))
+    ref.backward(up.double())
+    for mine, theirs, dtype in ((xd.grad, x64.grad, xdt), (wd.grad, w64.grad, wdt)):
+        assert mine.dtype == dtype
+        err = (mine.cpu().double() - theirs).norm() / theirs.norm().clamp_min(1e-30)
+        # rounding to the output type, and fp32 sums whose terms carry a few relative roundings each
+        assert err <= half_ulp[dtype] + 2.0**-24 * (tokens**0.5 + 64), (err, dtype)
+
+
+def test_router_module_on_kernels_matches_its_composition():
+    """TopKRouter with the kernels and with its PyTorch composition (the same call under a group count it composes)."""
+    from kohakuwullm_amd.models.moe import TopKRouter
+
+    torch.manual_seed(SEED)
+    router = TopKRouter(256, 32, top_k=4).to(DEV)
+    router.expert_bias.normal_(std=0.02)
+    x = torch.randn(700, 256, device=DEV)
+    idx, gate, counts = router.route(x)
+    router.z_loss_weight = 1e-6  # an auxiliary term: the composition
+    ref_idx, ref_gate, ref_counts = router.route(x)
+    router.z_loss_weight = 0.0
+    assert torch.equal(idx, ref_idx) and torch.equal(counts, ref_counts)
+    assert torch.allclose(gate, ref_gate, rtol=1e-5, atol=0)
+    assert torch.equal(router.load_accum, 2.0 * counts)
+    with torch.no_grad():
+        assert torch.equal(router.route(x)[1], gate)
