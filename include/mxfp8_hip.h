@@ -165,6 +165,30 @@ int mx_swiglu_bwd_quantize_dual(const void *dh, int64_t lddh, const void *gu, in
                                 uint8_t *qT, int64_t ldqT, uint8_t *sT, int64_t ldsT, void *stream);
 
 /*
+ * The activation quantizers of a training step, for any number of rows.  x (M, KV), of any type, is taken as (MT, K) with
+ * zeros past its rows and columns: (q, s) (M, K) codes and scales along K for the M rows that exist; (qT, sT) along the
+ * tokens, MT of them -- a multiple of 128 chosen by the caller -- with qT always stage-major (MT/128, K, 128).
+ * mx_quantize_dual on a matrix padded with zero rows and columns gives the same bytes.  cast_dtype: x's own type, or for
+ * fp32 x a 16-bit type the values are rounded to first (the cast a mixed-precision caller would have made).
+ * KV % 8 == 0, K % 32 == 0, 16-byte aligned rows of x.
+ */
+int mx_quantize_tokens(const void *x, int x_dtype, int cast_dtype, int64_t M, int64_t KV, int64_t ldx, int64_t MT, int64_t K,
+                       uint8_t *q, int64_t ldq, uint8_t *s, int64_t lds, uint8_t *qT, uint8_t *sT, int64_t ldsT, void *stream);
+
+/*
+ * mx_swiglu_quantize_dual and mx_swiglu_bwd_quantize_dual in the same form: M rows of gu (and dh), token-axis operands of MT
+ * tokens stage-major, (q, s) for the M rows (the backward's q stage-major when ldq == 128 and H % 128 == 0).
+ * rounded != 0: the arithmetic of the unfused 16-bit activation and its gradient -- silu(g), h, dh u, dh silu(g) and dgate
+ * are rounded to the input type one by one (mlp.py:68-73 of the reference, where nn.functional.silu and a product stand
+ * between the two projections) -- otherwise everything up to the cast is fp32.
+ */
+int mx_swiglu_quantize_tokens(const void *gu, int dtype, int rounded, int64_t M, int64_t H, int64_t ldgu, int64_t MT, uint8_t *q,
+                              int64_t ldq, uint8_t *s, int64_t lds, uint8_t *qT, uint8_t *sT, int64_t ldsT, void *stream);
+int mx_swiglu_bwd_quantize_tokens(const void *dh, int64_t lddh, const void *gu, int64_t ldgu, int dtype, int rounded, int64_t M,
+                                  int64_t H, int64_t MT, uint8_t *q, int64_t ldq, uint8_t *s, int64_t lds, uint8_t *qT,
+                                  uint8_t *sT, int64_t ldsT, void *stream);
+
+/*
  * RMSNorm as a producer of MXFP8 operands: rstd[m] = 1 / sqrt(mean_k(x[m,k]^2) + eps),
  * y = x * rstd * weight (fp32; weight NULL: 1).  Any of three results, from one pass over x:
  * out (M,K) in x_dtype (NULL: not written), rstd (M) fp32 for the backward (NULL: not

@@ -37,6 +37,10 @@ SIGNATURES = {
     "mx_swiglu_quantize_dual": (_ci, [_p, _ci, _i64, _i64, _i64, _p, _i64, _p, _i64, _p, _i64, _p, _i64, _p]),
     "mx_swiglu_bwd_quantize_dual": (
         _ci, [_p, _i64, _p, _i64, _ci, _i64, _i64, _p, _i64, _p, _i64, _p, _i64, _p, _i64, _p]),
+    "mx_quantize_tokens": (_ci, [_p, _ci, _ci, _i64, _i64, _i64, _i64, _i64, _p, _i64, _p, _i64, _p, _p, _i64, _p]),
+    "mx_swiglu_quantize_tokens": (_ci, [_p, _ci, _ci, _i64, _i64, _i64, _i64, _p, _i64, _p, _i64, _p, _p, _i64, _p]),
+    "mx_swiglu_bwd_quantize_tokens": (
+        _ci, [_p, _i64, _p, _i64, _ci, _ci, _i64, _i64, _i64, _p, _i64, _p, _i64, _p, _p, _i64, _p]),
     "mx_grouped_gemm_nt": (
         _ci, [_p, _p, _i64, _i64, _i64, _p, _p, _p, _i64, _i64, _i64, _i64, _p, _i64, _p, _ci, _i64, _i64, _i64, _i64, _p]),
     "mx_experts_gemm1": (

@@ -207,7 +207,9 @@ struct QuantTileOut {
 
 // Quantizes the 128 x TK tile (TK = 16 R columns) held as v[R][8] per thread (rows m0 + rg*R + i,
 // columns kc0 + cg*8 + c of the OUTPUT matrix, which has K columns and M rows) along the column
-// axis, and along the row axis too when ROWS.  `tile`/`tscale` are the workgroup's LDS
+// axis, and along the row axis too when ROWS.  The token axis is MT long, M rounded up by the
+// caller to whole blocks or more: the tile holds zeros for rows past M, they are quantized along
+// the columns like any other, and have no row-axis output.  `tile`/`tscale` are the workgroup's LDS
 // staging buffers; the caller must not touch them until the function's trailing barrier.
 template <int R>
 struct TileGeom {
@@ -220,7 +222,7 @@ struct TileGeom {
 };
 
 template <bool ROWS, int R = 8, bool NTS = false>  // NTS: the code stores carry the non-temporal hint
-__device__ __forceinline__ void quant_tile(float (&v)[R][8], const QuantTileOut &o, int64_t M, int64_t K, int64_t m0,
+__device__ __forceinline__ void quant_tile(float (&v)[R][8], const QuantTileOut &o, int64_t M, int64_t MT, int64_t K, int64_t m0,
                                            int64_t kc0, uint8_t *tile, uint8_t *tscale) {
     typedef TileGeom<R> G;
     const int t = threadIdx.x;
@@ -229,7 +231,7 @@ __device__ __forceinline__ void quant_tile(float (&v)[R][8], const QuantTileOut 
     const int64_t col = kc0 + cg * 8;
     const int64_t row0 = m0 + rg * R;
     const bool col_ok = col < K;
-    const bool blk_ok = m0 + wave * 32 < M;
+    const bool whole = m0 + QC_TILE <= M;  // uniform: every row of the tile exists
 
     if (ROWS) {
         // Row-axis outputs: the 4 lanes of a quad hold 32 consecutive columns of a row.
@@ -248,7 +250,7 @@ __device__ __forceinline__ void quant_tile(float (&v)[R][8], const QuantTileOut 
                 // row gets block 1's byte from lane 4 (12)
                 packed |= (uint32_t)__builtin_amdgcn_mov_dpp((int)packed, 0x12C, 0xF, 0xF, true);
             }
-            if (col_ok && blk_ok) {
+            if (col_ok && (whole || row0 + i < M)) {
                 v2i codes;
                 codes[0] = (int)pack4_e4m3(v[i][0] * inv, v[i][1] * inv, v[i][2] * inv, v[i][3] * inv);
                 codes[1] = (int)pack4_e4m3(v[i][4] * inv, v[i][5] * inv, v[i][6] * inv, v[i][7] * inv);
@@ -306,7 +308,7 @@ __device__ __forceinline__ void quant_tile(float (&v)[R][8], const QuantTileOut 
 #pragma unroll
     for (int j = 0; j < G::TK / 32; j++) {
         int kr = j * 32 + (t >> 3), ch = t & 7;
-        if (kc0 + kr < K && m0 + ch * 16 < M) {
+        if (kc0 + kr < K && m0 + ch * 16 < MT) {
             const v2i *src = (const v2i *)(tile + kr * QC_PITCH + ch * 16);
             v4i w;
             v2i a = src[0], b = src[1];
@@ -319,7 +321,7 @@ __device__ __forceinline__ void quant_tile(float (&v)[R][8], const QuantTileOut 
     }
     if (t < G::TK && kc0 + t < K) {
         uint8_t *sp = o.sT + (kc0 + t) * o.ldsT + (m0 >> 5);
-        int64_t nb = (M - m0) >> 5;
+        int64_t nb = (MT - m0) >> 5;
         if (o.pack_col_scales && nb >= 4) {
             *(uint32_t *)sp = *(const uint32_t *)(tscale + t * 4);
         } else {
@@ -335,7 +337,7 @@ __device__ __forceinline__ void quant_tile(float (&v)[R][8], const QuantTileOut 
 // tile in fp32), so that the 1536 tiles of a 16384 x 1536 activation are resident at once instead of in 1.2 rounds.
 // Same arithmetic on the same values: bit-identical outputs.
 template <int DT, bool ROWS, bool NTS>
-__device__ __forceinline__ void quant_tile_raw(typename Elem<DT>::raw (&r)[8], bool ok, const QuantTileOut &o, int64_t M,
+__device__ __forceinline__ void quant_tile_raw(typename Elem<DT>::raw (&r)[8], const QuantTileOut &o, int64_t M, int64_t MT,
                                                int64_t K, int64_t m0, int64_t kc0, uint8_t *tile, uint8_t *tscale) {
     typedef TileGeom<8> G;
     typedef Elem<DT> E;
@@ -344,19 +346,19 @@ __device__ __forceinline__ void quant_tile_raw(typename Elem<DT>::raw (&r)[8], b
     const int cg = G::cg(t), rg = G::rg(t);
     const int64_t col = kc0 + cg * 8;
     const int64_t row0 = m0 + rg * 8;
-    auto val = [&](int i, int c) { return ok ? E::elem(r[i], c) : 0.0f; };
+    const bool col_ok = col < K, whole = m0 + QC_TILE <= M;
 
     if (ROWS) {
 #pragma unroll
         for (int i = 0; i < 8; i++) {
             float v[8];
 #pragma unroll
-            for (int c = 0; c < 8; c++) v[c] = val(i, c);
+            for (int c = 0; c < 8; c++) v[c] = E::elem(r[i], c);
             const float amax = quad_max(amax8(v));
             const uint32_t byte = scale_byte(amax);
             const float inv = inv_scale(byte);
             const uint32_t packed = gather_row_scales(byte, lane);
-            if (ok) {
+            if (col_ok && (whole || row0 + i < M)) {
                 v2i codes;
                 codes[0] = (int)pack4_e4m3(v[0] * inv, v[1] * inv, v[2] * inv, v[3] * inv);
                 codes[1] = (int)pack4_e4m3(v[4] * inv, v[5] * inv, v[6] * inv, v[7] * inv);
@@ -379,7 +381,7 @@ __device__ __forceinline__ void quant_tile_raw(typename Elem<DT>::raw (&r)[8], b
     for (int c = 0; c < 8; c++) {
         float v[8];
 #pragma unroll
-        for (int i = 0; i < 8; i++) v[i] = val(i, c);
+        for (int i = 0; i < 8; i++) v[i] = E::elem(r[i], c);
         float cm = amax8(v);
         cm = fmaxf(cm, __shfl_xor(cm, 16, 64));
         cm = fmaxf(cm, __shfl_xor(cm, 32, 64));
@@ -395,7 +397,7 @@ __device__ __forceinline__ void quant_tile_raw(typename Elem<DT>::raw (&r)[8], b
 #pragma unroll
     for (int j = 0; j < G::TK / 32; j++) {
         const int kr = j * 32 + (t >> 3), ch = t & 7;
-        if (kc0 + kr < K && m0 + ch * 16 < M) {
+        if (kc0 + kr < K && m0 + ch * 16 < MT) {
             const v2i *src = (const v2i *)(tile + kr * QC_PITCH + ch * 16);
             const v2i a = src[0], b = src[1];
             stream_store<NTS>((v4i *)(o.qT + (o.qT_ks ? (m0 >> 7) * o.qT_ks + (kc0 + kr) * 128 : (kc0 + kr) * o.ldqT + m0) + ch * 16),
@@ -404,7 +406,7 @@ __device__ __forceinline__ void quant_tile_raw(typename Elem<DT>::raw (&r)[8], b
     }
     if (t < G::TK && kc0 + t < K) {
         uint8_t *sp = o.sT + (kc0 + t) * o.ldsT + (m0 >> 5);
-        const int64_t nb = (M - m0) >> 5;
+        const int64_t nb = (MT - m0) >> 5;
         if (o.pack_col_scales && nb >= 4) {
             *(uint32_t *)sp = *(const uint32_t *)(tscale + t * 4);
         } else {
@@ -422,10 +424,60 @@ __device__ __forceinline__ void load_rows(const void *x, int64_t first, int64_t 
     for (int i = 0; i < R; i++) r[i] = Elem<DT>::template load_raw<NT>((const T *)x + first + i * ld);
 }
 
+// The same for a tile that the matrix may end in: `rows` of the thread's R rows exist (all of them when it is R or more,
+// none when it is not positive), the others come back as zeros.  Straight-line code on purpose: rows that do not exist
+// read the last one that does (or the matrix's first element) and are zeroed by selects.  With branches around the loads
+// the compiler converted the tile in every branch and held it twice (the SwiGLU' kernel: 256 registers instead of 162).
+// EDGE = false: a launch whose matrix ends in no tile (rows and columns multiples of 128, nothing padded) needs none of it;
+// the selects cost the SwiGLU kernels 2 % of their time there.
+template <int DT, int R, bool NT, bool EDGE>
+__device__ __forceinline__ void load_rows_or_last(const void *x, int64_t first, int64_t ld, int64_t rows, typename Elem<DT>::raw (&r)[R]) {
+    typedef typename Elem<DT>::type T;
+    if constexpr (!EDGE) {
+        load_rows<DT, R, NT>(x, first, ld, r);
+        return;
+    }
+    const int n = rows < R ? (int)(rows > 0 ? rows : 0) : R;
+    const T *const base = (const T *)x + (n ? first : 0);
+#pragma unroll
+    for (int i = 0; i < R; i++) r[i] = Elem<DT>::template load_raw<NT>(base + (i < n ? i : n ? n - 1 : 0) * ld);
+}
+template <int DT, int R, bool NT, bool EDGE>
+__device__ __forceinline__ void load_rows_or_zero(const void *x, int64_t first, int64_t ld, int64_t rows, typename Elem<DT>::raw (&r)[R]) {
+    load_rows_or_last<DT, R, NT, EDGE>(x, first, ld, rows, r);
+    if constexpr (!EDGE) return;
+#pragma unroll
+    for (int i = 0; i < R; i++) {
+        typedef int bits_t __attribute__((ext_vector_type(sizeof(r[i]) / 4)));
+        const bits_t bits = __builtin_bit_cast(bits_t, r[i]);
+        bits_t kept;
+#pragma unroll
+        for (int e = 0; e < (int)sizeof(r[i]) / 4; e++) kept[e] = i < rows ? bits[e] : 0;
+        r[i] = __builtin_bit_cast(typename Elem<DT>::raw, kept);
+    }
+}
+
+// fp32 values rounded to a 16-bit type and widened again: what a cast in front of the quantizer would have left.
+template <int CDT>
+__device__ __forceinline__ void round_values(float (&v)[8]) {
+    if constexpr (CDT == MX_BF16) {
+#pragma unroll
+        for (int c = 0; c < 8; c += 2) {
+            const uint32_t w = pack2_bf16(v[c], v[c + 1]);
+            v[c] = bits2f(w << 16), v[c + 1] = bits2f(w & 0xFFFF0000u);
+        }
+    } else if constexpr (CDT == MX_FP16) {
+#pragma unroll
+        for (int c = 0; c < 8; c++) v[c] = (float)(_Float16)v[c];
+    }
+}
+
 // RAW (16-bit inputs, R = 8): the tile stays packed as loaded (quant_tile_raw): 64 registers, eight waves per SIMD.
-template <int DT, bool DUAL, int R, bool RAW = false>
-__global__ __launch_bounds__(256) void quant_cols_kernel(const void *__restrict__ x, int64_t M, int64_t K, int64_t ldx,
-                                                          QuantTileOut o) {
+// x has M rows and KV columns, the outputs MT and K (both rounded up by the caller): what lies past x is zero.
+// CDT: the type fp32 values are rounded to before they are quantized (MX_FP32: none).
+template <int DT, bool DUAL, int R, bool EDGE, bool RAW = false, int CDT = MX_FP32>
+__global__ __launch_bounds__(256) void quant_cols_kernel(const void *__restrict__ x, int64_t M, int64_t MT, int64_t KV, int64_t K,
+                                                          int64_t ldx, QuantTileOut o) {
     typedef TileGeom<R> G;
     __shared__ __attribute__((aligned(16))) uint8_t tile[G::TK * QC_PITCH];
     __shared__ __attribute__((aligned(4))) uint8_t tscale[G::TK * 4];
@@ -433,28 +485,23 @@ __global__ __launch_bounds__(256) void quant_cols_kernel(const void *__restrict_
     const int64_t m0 = (int64_t)blockIdx.y * QC_TILE, k0 = (int64_t)blockIdx.x * G::TK;
     const int64_t col = k0 + G::cg(t) * 8;
     const int64_t row0 = m0 + G::rg(t) * R;
-    const bool ok = col < K && m0 + (t >> 6) * 32 < M;  // K % 8 == 0 and M % 32 == 0
     // the thread's loads go out together (row by row, each waited for the one before it)
     typename Elem<DT>::raw r[R];
     // both axes at once is the activation path of a training step, where the 16-bit input is not read again soon: its
     // loads carry the non-temporal hint; the codes are read by the next GEMM and are stored plainly
-    if (ok) load_rows<DT, R, DUAL>(x, row0 * ldx + col, ldx, r);
+    load_rows_or_zero<DT, R, DUAL, EDGE>(x, row0 * ldx + col, ldx, col < KV ? M - row0 : 0, r);
     if constexpr (RAW) {
         static_assert(DT != MX_FP32 && R == 8, "a packed tile of 16-bit values");
-        quant_tile_raw<DT, DUAL, false>(r, ok, o, M, K, m0, k0, tile, tscale);
+        quant_tile_raw<DT, DUAL, false>(r, o, M, MT, K, m0, k0, tile, tscale);
         return;
     }
     float v[R][8];
 #pragma unroll
     for (int i = 0; i < R; i++) {
-        if (ok) {
-            Elem<DT>::unpack(r[i], v[i]);
-        } else {
-#pragma unroll
-            for (int c = 0; c < 8; c++) v[i][c] = 0.0f;
-        }
+        Elem<DT>::unpack(r[i], v[i]);
+        round_values<CDT>(v[i]);
     }
-    quant_tile<DUAL, R>(v, o, M, K, m0, k0, tile, tscale);
+    quant_tile<DUAL, R>(v, o, M, MT, K, m0, k0, tile, tscale);
 }
 
 // RMSNorm in front of both quantizers: y = (x * rstd[row]) * w[col] in fp32 -- the two products in the order
@@ -501,7 +548,7 @@ __global__ __launch_bounds__(256) void rmsnorm_quant_dual_kernel(const void *__r
             for (int c = 0; c < 8; c++) v[i][c] = 0.0f;
         }
     }
-    quant_tile<true, 8>(v, o, M, K, m0, k0, tile, tscale);
+    quant_tile<true, 8>(v, o, M, M, K, m0, k0, tile, tscale);
 }
 
 // Several matrices behind one launch: workgroup `id` finds its matrix in the running tile
@@ -548,15 +595,17 @@ __global__ __launch_bounds__(256) void quant_dual_batch_kernel(QuantBatchArgs b)
             for (int c = 0; c < 8; c++) v[i][c] = 0.0f;
         }
     }
-    quant_tile<true>(v, b.o[j], M, K, m0, k0, tile, tscale);
+    quant_tile<true>(v, b.o[j], M, M, K, m0, k0, tile, tscale);
 }
 
 __device__ __forceinline__ float sigmoid_fast(float x) { return sigmoid_f32(x); }
 
 // h = silu(g) * u from the fused projection output gu (M, 2H) (gate half first), quantized
-// along both axes: (q,s) (M,H) for the down projection's forward, (qT,sT) (H,M) for its wgrad.
-template <int DT, int R>
-__global__ __launch_bounds__(256) void swiglu_quant_dual_kernel(const void *__restrict__ gu, int64_t M, int64_t H,
+// along both axes: (q,s) (M,H) for the down projection's forward, (qT,sT) (H,MT) for its wgrad.
+// ROUNDED: silu(g) and the product are rounded to the input type one after the other, as the two
+// 16-bit operators of an unfused activation leave them; otherwise h stays in fp32 up to the cast.
+template <int DT, int R, bool ROUNDED, bool EDGE>
+__global__ __launch_bounds__(256) void swiglu_quant_dual_kernel(const void *__restrict__ gu, int64_t M, int64_t MT, int64_t H,
                                                                  int64_t ldgu, QuantTileOut o) {
     typedef TileGeom<R> G;
     __shared__ __attribute__((aligned(16))) uint8_t tile[G::TK * QC_PITCH];
@@ -565,40 +614,43 @@ __global__ __launch_bounds__(256) void swiglu_quant_dual_kernel(const void *__re
     const int64_t m0 = (int64_t)blockIdx.y * QC_TILE, k0 = (int64_t)blockIdx.x * G::TK;
     const int64_t col = k0 + G::cg(t) * 8;
     const int64_t row0 = m0 + G::rg(t) * R;
-    const bool ok = col < H && m0 + (t >> 6) * 32 < M;
+    const int64_t rows = col < H ? M - row0 : 0;
     float v[R][8];
     typename Elem<DT>::raw rg[R], ru[R];  // all loads in flight before the first conversion
-    if (ok) {
-        load_rows<DT, R, true>(gu, row0 * ldgu + col, ldgu, rg);
-        load_rows<DT, R, true>(gu, row0 * ldgu + H + col, ldgu, ru);
-    }
+    load_rows_or_zero<DT, R, true, EDGE>(gu, row0 * ldgu + col, ldgu, rows, rg);
+    load_rows_or_zero<DT, R, true, EDGE>(gu, row0 * ldgu + H + col, ldgu, rows, ru);
 #pragma unroll
-    for (int i = 0; i < R; i++) {
-        if (ok) {
-            float g[8], u[8];
-            Elem<DT>::unpack(rg[i], g);
-            Elem<DT>::unpack(ru[i], u);
+    for (int i = 0; i < R; i++) {  // zeros give zeros
+        float g[8], u[8];
+        Elem<DT>::unpack(rg[i], g);
+        Elem<DT>::unpack(ru[i], u);
+        if constexpr (ROUNDED) {
 #pragma unroll
-            for (int c = 0; c < 8; c++) v[i][c] = g[c] * sigmoid_fast(g[c]) * u[c];
+            for (int c = 0; c < 8; c++) v[i][c] = g[c] * sigmoid_fast(g[c]);
+            round_values<DT>(v[i]);
+#pragma unroll
+            for (int c = 0; c < 8; c++) v[i][c] *= u[c];
+            round_values<DT>(v[i]);
         } else {
 #pragma unroll
-            for (int c = 0; c < 8; c++) v[i][c] = 0.0f;
+            for (int c = 0; c < 8; c++) v[i][c] = g[c] * sigmoid_fast(g[c]) * u[c];
         }
     }
     // hundreds of MB in, hundreds out, nothing of it small enough to be found in a cache by its consumer: all hinted
-    quant_tile<true, R, true>(v, o, M, H, m0, k0, tile, tscale);
+    quant_tile<true, R, true>(v, o, M, MT, H, m0, k0, tile, tscale);
 }
 
 // SwiGLU backward fused with both quantizers.  Reads dh (M,H) and the saved projection
 // output gu (M,2H); forms dgate = dh * u * s * (1 + g (1 - s)) and dup = dh * g * s with
 // s = sigmoid(g) in fp32 (elementwise/swiglu.py:108-119, experts_bwd.py:145-148 of the
 // reference); writes dpre = [dgate | dup] quantized along 2H ((q,s): (M,2H)) for the input
-// projection's dgrad and along M ((qT,sT): (2H,M)) for its wgrad.  o.q/o.qT address the
-// full (M,2H) / (2H,M) outputs.
-template <int DT, int R>
+// projection's dgrad and along the tokens ((qT,sT): (2H,MT)) for its wgrad.  o.q/o.qT address the
+// full (M,2H) / (2H,MT) outputs.  ROUNDED: the gradients of the unfused activation, whose 16-bit
+// operators round silu(g), dh * u, dgate and dup to the input type.
+template <int DT, int R, bool ROUNDED, bool EDGE>
 __global__ __launch_bounds__(256) void swiglu_bwd_quant_dual_kernel(const void *__restrict__ dh, int64_t lddh,
                                                                      const void *__restrict__ gu, int64_t ldgu,
-                                                                     int64_t M, int64_t H, QuantTileOut o) {
+                                                                     int64_t M, int64_t MT, int64_t H, QuantTileOut o) {
     typedef TileGeom<R> G;
     __shared__ __attribute__((aligned(16))) uint8_t tile[G::TK * QC_PITCH];
     __shared__ __attribute__((aligned(4))) uint8_t tscale[G::TK * 4];
@@ -606,29 +658,48 @@ __global__ __launch_bounds__(256) void swiglu_bwd_quant_dual_kernel(const void *
     const int64_t m0 = (int64_t)blockIdx.y * QC_TILE, k0 = (int64_t)blockIdx.x * G::TK;
     const int64_t col = k0 + G::cg(t) * 8;
     const int64_t row0 = m0 + G::rg(t) * R;
-    const bool ok = col < H && m0 + (t >> 6) * 32 < M;
+    const int64_t rows = col < H ? M - row0 : 0;
     float v[R][8], w[R][8];
     // All loads of the thread go out before the first conversion.  Written row by row (load three,
     // convert, next row) the compiler kept that order and every thread had 48 bytes in flight at a time,
-    // with a memory latency in front of each of its rows.
+    // with a memory latency in front of each of its rows.  Rows past the end of the matrix repeat the
+    // last one and are left out below.
     typename Elem<DT>::raw rg[R], ru[R], rd[R];
-    if (ok) {
-        load_rows<DT, R, true>(gu, row0 * ldgu + col, ldgu, rg);
-        load_rows<DT, R, true>(gu, row0 * ldgu + H + col, ldgu, ru);
-        load_rows<DT, R, true>(dh, row0 * lddh + col, lddh, rd);
-    }
+    load_rows_or_last<DT, R, true, EDGE>(gu, row0 * ldgu + col, ldgu, rows, rg);
+    load_rows_or_last<DT, R, true, EDGE>(gu, row0 * ldgu + H + col, ldgu, rows, ru);
+    load_rows_or_last<DT, R, true, EDGE>(dh, row0 * lddh + col, lddh, rows, rd);
 #pragma unroll
     for (int i = 0; i < R; i++) {
-        if (ok) {
+        if (i < rows) {  // (always so without EDGE: a block per row all the same, or the compiler takes 256 registers for them)
             float g[8], u[8], d[8];
             Elem<DT>::unpack(rg[i], g);
             Elem<DT>::unpack(ru[i], u);
             Elem<DT>::unpack(rd[i], d);
+            if constexpr (ROUNDED) {
+                float slope[8];
 #pragma unroll
-            for (int c = 0; c < 8; c++) {
-                float sg = sigmoid_fast(g[c]);
-                v[i][c] = d[c] * u[c] * sg * (1.0f + g[c] * (1.0f - sg));
-                w[i][c] = d[c] * g[c] * sg;
+                for (int c = 0; c < 8; c++) {
+                    const float sg = sigmoid_fast(g[c]);
+                    slope[c] = sg * (1.0f + g[c] * (1.0f - sg));
+                    w[i][c] = g[c] * sg;
+                    v[i][c] = d[c] * u[c];
+                }
+                round_values<DT>(w[i]);
+                round_values<DT>(v[i]);
+#pragma unroll
+                for (int c = 0; c < 8; c++) {
+                    w[i][c] *= d[c];
+                    v[i][c] *= slope[c];
+                }
+                round_values<DT>(w[i]);
+                round_values<DT>(v[i]);
+            } else {
+#pragma unroll
+                for (int c = 0; c < 8; c++) {
+                    float sg = sigmoid_fast(g[c]);
+                    v[i][c] = d[c] * u[c] * sg * (1.0f + g[c] * (1.0f - sg));
+                    w[i][c] = d[c] * g[c] * sg;
+                }
             }
         } else {
 #pragma unroll
@@ -637,13 +708,13 @@ __global__ __launch_bounds__(256) void swiglu_bwd_quant_dual_kernel(const void *
     }
     // The gate half occupies output columns [0,H), the up half [H,2H): same tile, shifted.
     // Columns at or beyond H inside the gate-half tile are masked by passing K = H.
-    quant_tile<true, R, true>(v, o, M, H, m0, k0, tile, tscale);
+    quant_tile<true, R, true>(v, o, M, MT, H, m0, k0, tile, tscale);
     QuantTileOut o2 = o;
     o2.q += o.q_ks ? (H >> 7) * o.q_ks : H;
     o2.s += H / MX_BLOCK;
     o2.qT += o.qT_ks ? H * 128 : H * o.ldqT;
     o2.sT += H * o.ldsT;
-    quant_tile<true, R, true>(w, o2, M, H, m0, k0, tile, tscale);
+    quant_tile<true, R, true>(w, o2, M, MT, H, m0, k0, tile, tscale);
 }
 
 // ------------------------------------------------------------------------------------
@@ -794,7 +865,7 @@ __global__ __launch_bounds__(256) void quant_cols_grouped_kernel(GroupedQuantArg
             for (int c = 0; c < 8; c++) v[i][c] = 0.0f;
         }
     }
-    quant_tile<false>(v, o, mpad, a.C, (int64_t)rt * QC_TILE, k0, tile, tscale);
+    quant_tile<false>(v, o, mpad, mpad, a.C, (int64_t)rt * QC_TILE, k0, tile, tscale);
 }
 
 // The same quantizer for wide inputs: a workgroup keeps its 128 rows and walks `span` column tiles.
@@ -888,7 +959,7 @@ __global__ __launch_bounds__(256) void quant_cols_grouped_walk_kernel(GroupedQua
                 for (int c = 0; c < 8; c++) v[i][c] = 0.0f;
             }
         }
-        quant_tile<false>(v, o, mpad, a.C, (int64_t)rt * QC_TILE, k0, tile, tscale);
+        quant_tile<false>(v, o, mpad, mpad, a.C, (int64_t)rt * QC_TILE, k0, tile, tscale);
     }
 }
 
@@ -962,21 +1033,34 @@ static bool tile_grid(int64_t M, int64_t K, dim3 &grid) {
     return grid.y <= 65535u;
 }
 
+// x has M rows and KV columns; the outputs span MT (token axis) and K.  cast: the 16-bit type fp32 values are rounded to
+// first, MX_FP32 for none.
 template <int DT, bool DUAL>
-static int launch_cols(const void *x, int64_t M, int64_t K, int64_t ldx, uint8_t *qT, int64_t ldqT, uint8_t *sT,
-                       int64_t ldsT, uint8_t *q, int64_t ldq, uint8_t *s, int64_t lds, hipStream_t st, int64_t qT_ks = 0) {
+static int launch_cols(const void *x, int64_t M, int64_t MT, int64_t KV, int64_t K, int64_t ldx, uint8_t *qT, int64_t ldqT,
+                       uint8_t *sT, int64_t ldsT, uint8_t *q, int64_t ldq, uint8_t *s, int64_t lds, hipStream_t st,
+                       int64_t qT_ks = 0, int cast = MX_FP32) {
     dim3 grid;
-    if (!tile_grid<MX_QR_COLS>(M, K, grid)) return MX_EUNSUPPORTED;
+    if (!tile_grid<MX_QR_COLS>(MT, K, grid)) return MX_EUNSUPPORTED;
     const QuantTileOut o = tile_out(qT, ldqT, sT, ldsT, q, ldq, s, lds, 0, qT_ks);
     // Both axes of a 16-bit matrix whose tiles are all resident at once with eight waves per SIMD, but not with the five
     // the fp32 tile allows, go to the packed-tile kernel: 16384 x 1536 (1536 tiles on 256 CUs) 27.0 -> 24.9 us.  Larger
     // matrices run several rounds either way and are faster with fewer, fatter waves (16384 x 4096: 54.4 against 58.9 us).
-    bool raw = false;
-    if constexpr (DT != MX_FP32 && DUAL) raw = (int64_t)grid.x * grid.y <= 8 * (int64_t)num_cus();
+    const dim3 block(256);
+    const bool edge = M % QC_TILE || K % QC_TILE || MT != M || KV != K;
+#define MX_LAUNCH_COLS(...)                                                                                                   \
+    (edge ? quant_cols_kernel<DT, DUAL, MX_QR_COLS, true, __VA_ARGS__><<<grid, block, 0, st>>>(x, M, MT, KV, K, ldx, o)       \
+          : quant_cols_kernel<DT, DUAL, MX_QR_COLS, false, __VA_ARGS__><<<grid, block, 0, st>>>(x, M, MT, KV, K, ldx, o))
     if constexpr (DT != MX_FP32 && DUAL) {
-        if (raw) quant_cols_kernel<DT, DUAL, MX_QR_COLS, true><<<grid, dim3(256), 0, st>>>(x, M, K, ldx, o);
+        if ((int64_t)grid.x * grid.y <= 8 * (int64_t)num_cus()) MX_LAUNCH_COLS(true);
+        else MX_LAUNCH_COLS(false);
+    } else if constexpr (DUAL) {
+        if (cast == MX_BF16) MX_LAUNCH_COLS(false, MX_BF16);
+        else if (cast == MX_FP16) MX_LAUNCH_COLS(false, MX_FP16);
+        else MX_LAUNCH_COLS(false);
+    } else {
+        MX_LAUNCH_COLS(false);
     }
-    if (!raw) quant_cols_kernel<DT, DUAL, MX_QR_COLS><<<grid, dim3(256), 0, st>>>(x, M, K, ldx, o);
+#undef MX_LAUNCH_COLS
     MX_LAUNCH_CHECK();
     return MX_OK;
 }
@@ -1040,9 +1124,9 @@ extern "C" int mx_quantize_cols(const void *x, int x_dtype, int64_t M, int64_t K
         }
     }
     switch (x_dtype) {
-    case MX_BF16: return launch_cols<MX_BF16, false>(x, M, K, ldx, qT, ldqT, sT, ldsT, nullptr, 0, nullptr, 0, st);
-    case MX_FP16: return launch_cols<MX_FP16, false>(x, M, K, ldx, qT, ldqT, sT, ldsT, nullptr, 0, nullptr, 0, st);
-    case MX_FP32: return launch_cols<MX_FP32, false>(x, M, K, ldx, qT, ldqT, sT, ldsT, nullptr, 0, nullptr, 0, st);
+    case MX_BF16: return launch_cols<MX_BF16, false>(x, M, M, K, K, ldx, qT, ldqT, sT, ldsT, nullptr, 0, nullptr, 0, st);
+    case MX_FP16: return launch_cols<MX_FP16, false>(x, M, M, K, K, ldx, qT, ldqT, sT, ldsT, nullptr, 0, nullptr, 0, st);
+    case MX_FP32: return launch_cols<MX_FP32, false>(x, M, M, K, K, ldx, qT, ldqT, sT, ldsT, nullptr, 0, nullptr, 0, st);
     default: return MX_EINVAL;
     }
 }
@@ -1116,9 +1200,9 @@ extern "C" int mx_quantize_dual(const void *x, int x_dtype, int64_t M, int64_t K
     }
     const int64_t ks = panels ? K * 128 : 0;
     switch (x_dtype) {
-    case MX_BF16: return launch_cols<MX_BF16, true>(x, M, K, ldx, qT, ldqT, sT, ldsT, q, ldq, s, lds, st, ks);
-    case MX_FP16: return launch_cols<MX_FP16, true>(x, M, K, ldx, qT, ldqT, sT, ldsT, q, ldq, s, lds, st, ks);
-    case MX_FP32: return launch_cols<MX_FP32, true>(x, M, K, ldx, qT, ldqT, sT, ldsT, q, ldq, s, lds, st, ks);
+    case MX_BF16: return launch_cols<MX_BF16, true>(x, M, M, K, K, ldx, qT, ldqT, sT, ldsT, q, ldq, s, lds, st, ks);
+    case MX_FP16: return launch_cols<MX_FP16, true>(x, M, M, K, K, ldx, qT, ldqT, sT, ldsT, q, ldq, s, lds, st, ks);
+    case MX_FP32: return launch_cols<MX_FP32, true>(x, M, M, K, K, ldx, qT, ldqT, sT, ldsT, q, ldq, s, lds, st, ks);
     default: return MX_EINVAL;
     }
 }
@@ -1203,6 +1287,42 @@ extern "C" int mx_swiglu_quantize_rows(const void *gate, const void *up, int dty
                             : launch_swiglu<MX_FP16>(gate, up, M, K, ldg, ldu, q, ldq, s, lds, st);
 }
 
+template <int DT, bool ROUNDED>
+static int launch_swiglu_dual(const void *gu, int64_t M, int64_t MT, int64_t H, int64_t ldgu, dim3 grid, const QuantTileOut &o, hipStream_t st) {
+    constexpr int R = MX_QR_SWIGLU;
+    if (M % QC_TILE || H % QC_TILE || MT != M) swiglu_quant_dual_kernel<DT, R, ROUNDED, true><<<grid, dim3(256), 0, st>>>(gu, M, MT, H, ldgu, o);
+    else swiglu_quant_dual_kernel<DT, R, ROUNDED, false><<<grid, dim3(256), 0, st>>>(gu, M, MT, H, ldgu, o);
+    MX_LAUNCH_CHECK();
+    return MX_OK;
+}
+
+static int launch_swiglu_dual(const void *gu, int dtype, int64_t M, int64_t MT, int64_t H, int64_t ldgu, int rounded, dim3 grid,
+                              const QuantTileOut &o, hipStream_t st) {
+    if (dtype == MX_BF16)
+        return rounded ? launch_swiglu_dual<MX_BF16, true>(gu, M, MT, H, ldgu, grid, o, st) : launch_swiglu_dual<MX_BF16, false>(gu, M, MT, H, ldgu, grid, o, st);
+    return rounded ? launch_swiglu_dual<MX_FP16, true>(gu, M, MT, H, ldgu, grid, o, st) : launch_swiglu_dual<MX_FP16, false>(gu, M, MT, H, ldgu, grid, o, st);
+}
+
+template <int DT, bool ROUNDED>
+static int launch_swiglu_bwd_dual(const void *dh, int64_t lddh, const void *gu, int64_t ldgu, int64_t M, int64_t MT, int64_t H, dim3 grid,
+                                  const QuantTileOut &o, hipStream_t st) {
+    constexpr int R = MX_QR_SWIGLU_BWD;
+    if (M % QC_TILE || H % QC_TILE || MT != M)
+        swiglu_bwd_quant_dual_kernel<DT, R, ROUNDED, true><<<grid, dim3(256), 0, st>>>(dh, lddh, gu, ldgu, M, MT, H, o);
+    else swiglu_bwd_quant_dual_kernel<DT, R, ROUNDED, false><<<grid, dim3(256), 0, st>>>(dh, lddh, gu, ldgu, M, MT, H, o);
+    MX_LAUNCH_CHECK();
+    return MX_OK;
+}
+
+static int launch_swiglu_bwd_dual(const void *dh, int64_t lddh, const void *gu, int64_t ldgu, int dtype, int64_t M, int64_t MT,
+                                  int64_t H, int rounded, dim3 grid, const QuantTileOut &o, hipStream_t st) {
+    if (dtype == MX_BF16)
+        return rounded ? launch_swiglu_bwd_dual<MX_BF16, true>(dh, lddh, gu, ldgu, M, MT, H, grid, o, st)
+                       : launch_swiglu_bwd_dual<MX_BF16, false>(dh, lddh, gu, ldgu, M, MT, H, grid, o, st);
+    return rounded ? launch_swiglu_bwd_dual<MX_FP16, true>(dh, lddh, gu, ldgu, M, MT, H, grid, o, st)
+                   : launch_swiglu_bwd_dual<MX_FP16, false>(dh, lddh, gu, ldgu, M, MT, H, grid, o, st);
+}
+
 extern "C" int mx_swiglu_quantize_dual(const void *gu, int dtype, int64_t M, int64_t H, int64_t ldgu, uint8_t *q,
                                        int64_t ldq, uint8_t *s, int64_t lds, uint8_t *qT, int64_t ldqT, uint8_t *sT,
                                        int64_t ldsT, void *stream) {
@@ -1219,10 +1339,7 @@ extern "C" int mx_swiglu_quantize_dual(const void *gu, int dtype, int64_t M, int
     hipStream_t st = (hipStream_t)stream;
     if (mx::stream_is_capturing(st)) return MX_ECAPTURE;
     QuantTileOut o = tile_out(qT, ldqT, sT, ldsT, q, ldq, s, lds, 0, panels ? H * 128 : 0);
-    if (dtype == MX_BF16) swiglu_quant_dual_kernel<MX_BF16, MX_QR_SWIGLU><<<grid, dim3(256), 0, st>>>(gu, M, H, ldgu, o);
-    else swiglu_quant_dual_kernel<MX_FP16, MX_QR_SWIGLU><<<grid, dim3(256), 0, st>>>(gu, M, H, ldgu, o);
-    MX_LAUNCH_CHECK();
-    return MX_OK;
+    return launch_swiglu_dual(gu, dtype, M, M, H, ldgu, 0, grid, o, st);
 }
 
 extern "C" int mx_swiglu_bwd_quantize_dual(const void *dh, int64_t lddh, const void *gu, int64_t ldgu, int dtype,
@@ -1244,11 +1361,65 @@ extern "C" int mx_swiglu_bwd_quantize_dual(const void *dh, int64_t lddh, const v
     if (mx::stream_is_capturing(st)) return MX_ECAPTURE;
     QuantTileOut o = tile_out(qT, ldqT, sT, ldsT, q, ldq, s, lds, q_panels ? M * 128 : 0, qt_panels ? 2 * H * 128 : 0);
     if (H % 128) o.pack_row_scales = 0;  // the up half's scale columns start at H/32: keep the packed stores aligned
-    if (dtype == MX_BF16)
-        swiglu_bwd_quant_dual_kernel<MX_BF16, MX_QR_SWIGLU_BWD><<<grid, dim3(256), 0, st>>>(dh, lddh, gu, ldgu, M, H, o);
-    else swiglu_bwd_quant_dual_kernel<MX_FP16, MX_QR_SWIGLU_BWD><<<grid, dim3(256), 0, st>>>(dh, lddh, gu, ldgu, M, H, o);
-    MX_LAUNCH_CHECK();
-    return MX_OK;
+    return launch_swiglu_bwd_dual(dh, lddh, gu, ldgu, dtype, M, M, H, 0, grid, o, st);
+}
+
+// ------------------------------------------------------------------------------------
+// The activation quantizers of a training step: any row count, token-axis operand in whole 128-token panels.
+// ------------------------------------------------------------------------------------
+
+static bool token_extent_ok(int64_t M, int64_t MT) { return M > 0 && MT >= M && MT % QC_TILE == 0; }
+
+extern "C" int mx_quantize_tokens(const void *x, int x_dtype, int cast_dtype, int64_t M, int64_t KV, int64_t ldx, int64_t MT,
+                                  int64_t K, uint8_t *q, int64_t ldq, uint8_t *s, int64_t lds, uint8_t *qT, uint8_t *sT,
+                                  int64_t ldsT, void *stream) {
+    if (!token_extent_ok(M, MT) || KV <= 0 || KV > K || K % MX_BLOCK || !x || !q || !s || !qT || !sT || ldx < KV || ldq < K ||
+        lds < K / MX_BLOCK || ldsT < MT / MX_BLOCK || (cast_dtype != x_dtype && x_dtype != MX_FP32))
+        return MX_EINVAL;
+    if (KV % 8 || !cols_vec_ok(x, x_dtype, K, ldx, qT, 128) || !aligned(q, 8) || ldq % 8) return MX_EUNSUPPORTED;
+    hipStream_t st = (hipStream_t)stream;
+    if (mx::stream_is_capturing(st)) return MX_ECAPTURE;
+    const int64_t ks = K * 128;
+    switch (x_dtype) {
+    case MX_BF16: return launch_cols<MX_BF16, true>(x, M, MT, KV, K, ldx, qT, 128, sT, ldsT, q, ldq, s, lds, st, ks);
+    case MX_FP16: return launch_cols<MX_FP16, true>(x, M, MT, KV, K, ldx, qT, 128, sT, ldsT, q, ldq, s, lds, st, ks);
+    case MX_FP32: return launch_cols<MX_FP32, true>(x, M, MT, KV, K, ldx, qT, 128, sT, ldsT, q, ldq, s, lds, st, ks, cast_dtype);
+    default: return MX_EINVAL;
+    }
+}
+
+extern "C" int mx_swiglu_quantize_tokens(const void *gu, int dtype, int rounded, int64_t M, int64_t H, int64_t ldgu, int64_t MT,
+                                         uint8_t *q, int64_t ldq, uint8_t *s, int64_t lds, uint8_t *qT, uint8_t *sT,
+                                         int64_t ldsT, void *stream) {
+    if (!token_extent_ok(M, MT) || H <= 0 || H % MX_BLOCK || !gu || !q || !s || !qT || !sT || ldgu < 2 * H || ldq < H ||
+        lds < H / MX_BLOCK || ldsT < MT / MX_BLOCK)
+        return MX_EINVAL;
+    if ((dtype != MX_BF16 && dtype != MX_FP16) || !aligned(gu, 16) || (ldgu * 2) % 16 || !aligned(q, 8) || ldq % 8 || !aligned(qT, 16))
+        return MX_EUNSUPPORTED;
+    dim3 grid;
+    if (!tile_grid<MX_QR_SWIGLU>(MT, H, grid)) return MX_EUNSUPPORTED;
+    hipStream_t st = (hipStream_t)stream;
+    if (mx::stream_is_capturing(st)) return MX_ECAPTURE;
+    return launch_swiglu_dual(gu, dtype, M, MT, H, ldgu, rounded, grid, tile_out(qT, 128, sT, ldsT, q, ldq, s, lds, 0, H * 128), st);
+}
+
+extern "C" int mx_swiglu_bwd_quantize_tokens(const void *dh, int64_t lddh, const void *gu, int64_t ldgu, int dtype, int rounded,
+                                             int64_t M, int64_t H, int64_t MT, uint8_t *q, int64_t ldq, uint8_t *s, int64_t lds,
+                                             uint8_t *qT, uint8_t *sT, int64_t ldsT, void *stream) {
+    const bool q_panels = stage_major(ldq, 2 * H);
+    if (!token_extent_ok(M, MT) || H <= 0 || H % MX_BLOCK || !dh || !gu || !q || !s || !qT || !sT || lddh < H || ldgu < 2 * H ||
+        (ldq < 2 * H && !q_panels) || (q_panels && H % 128) || lds < 2 * H / MX_BLOCK || ldsT < MT / MX_BLOCK)
+        return MX_EINVAL;
+    if ((dtype != MX_BF16 && dtype != MX_FP16) || !aligned(gu, 16) || (ldgu * 2) % 16 || !aligned(dh, 16) || (lddh * 2) % 16 ||
+        !aligned(q, 8) || ldq % 8 || !aligned(qT, 16))
+        return MX_EUNSUPPORTED;
+    dim3 grid;
+    if (!tile_grid<MX_QR_SWIGLU_BWD>(MT, H, grid)) return MX_EUNSUPPORTED;
+    hipStream_t st = (hipStream_t)stream;
+    if (mx::stream_is_capturing(st)) return MX_ECAPTURE;
+    QuantTileOut o = tile_out(qT, 128, sT, ldsT, q, ldq, s, lds, q_panels ? M * 128 : 0, 2 * H * 128);
+    if (H % 128) o.pack_row_scales = 0;  // the up half's scale columns start at H/32: keep the packed stores aligned
+    return launch_swiglu_bwd_dual(dh, lddh, gu, ldgu, dtype, M, MT, H, rounded, grid, o, st);
 }
 
 extern "C" int mx_quantize_cols_grouped(const void *x, int dtype, int64_t ldx, int64_t C, int source,

@@ -16,16 +16,20 @@ emit the row-blocked operand for the next GEMM and the token-blocked operand for
 from __future__ import annotations
 
 import torch
+import torch.nn.functional as F
 
 from kohakuwullm_amd import _lib
-from kohakuwullm_amd.kernels.mxfp8.linear import compute_dtype, pad_tokens
+from kohakuwullm_amd.kernels.mxfp8.linear import compute_dtype, gradient_dtype
 from kohakuwullm_amd.kernels.mxfp8.quantize import (
     BLOCK_SCALE,
     PANEL,
+    activation_matrix,
     mxfp8_matmul_pq,
-    mxfp8_matmul_pq_batch,
+    products_by_dtype,
     quantize_mx_dual,
+    quantize_tokens,
     stage_major_ok,
+    token_extent,
 )
 
 _FP8 = torch.float8_e4m3fn
@@ -65,27 +69,34 @@ def swiglu_mx_dual(gu: torch.Tensor, stage_major_t: bool = False):
 def swiglu_bwd_mx_dual(dh: torch.Tensor, gu: torch.Tensor, stage_major: bool = False):
     """SwiGLU backward emitted straight in MXFP8: ``dpre = [dgate | dup]`` as ``(q, s, qT, sT)``.
 
-    ``stage_major``: ``q`` as ``(2H // 128, tokens, 128)`` and ``qT`` as ``(tokens // 128, 2H, 128)``
-    (tokens and H multiples of 128; see :func:`quantize_mx_dual`).
+    ``stage_major``: ``q`` as ``(2H // 128, tokens, 128)`` and ``qT`` as ``(MT // 128, 2H, 128)`` with ``MT =
+    token_extent(tokens)`` (H a multiple of 128, any token count; see :func:`quantize_tokens`).
     """
     m, two_h = gu.shape
     h = two_h // 2
-    if dh.shape != (m, h) or h % BLOCK_SCALE or m % BLOCK_SCALE:
+    if dh.shape != (m, h) or h % BLOCK_SCALE or (m % BLOCK_SCALE and not stage_major):
         raise ValueError(f"dh {tuple(dh.shape)} does not match gu {tuple(gu.shape)}")
-    if stage_major and not (stage_major_ok(m) and stage_major_ok(h)):
-        raise ValueError(f"stage_major needs tokens={m} and H={h} to be positive multiples of {PANEL}")
+    if stage_major and not stage_major_ok(h):
+        raise ValueError(f"stage_major needs H={h} to be a positive multiple of {PANEL}")
     _lib.require_gpu(gu, "gu")
-    q = torch.empty((two_h // PANEL, m, PANEL) if stage_major else (m, two_h), device=gu.device, dtype=_FP8)
+    if stage_major:
+        return swiglu_bwd_tokens(dh, gu)
+    q = torch.empty(m, two_h, device=gu.device, dtype=_FP8)
     s = torch.empty(m, two_h // BLOCK_SCALE, device=gu.device, dtype=torch.uint8)
-    qt = torch.empty((m // PANEL, two_h, PANEL) if stage_major else (two_h, m), device=gu.device, dtype=_FP8)
+    qt = torch.empty(two_h, m, device=gu.device, dtype=_FP8)
     st = torch.empty(two_h, m // BLOCK_SCALE, device=gu.device, dtype=torch.uint8)
     _lib.invoke(
         "mx_swiglu_bwd_quantize_dual", m * h * (3 * gu.element_size() + 4 * (1 + 1 / BLOCK_SCALE)), gu,
         dh.data_ptr(), dh.stride(0), gu.data_ptr(), gu.stride(0), _lib.MX_DTYPE[gu.dtype], m, h,
-        q.data_ptr(), PANEL if stage_major else two_h, s.data_ptr(), two_h // BLOCK_SCALE,
-        qt.data_ptr(), PANEL if stage_major else m, st.data_ptr(), m // BLOCK_SCALE,
+        q.data_ptr(), two_h, s.data_ptr(), two_h // BLOCK_SCALE, qt.data_ptr(), m, st.data_ptr(), m // BLOCK_SCALE,
     )
     return q, s, qt, st
+
+
+def pad_tokens(x2d: torch.Tensor) -> torch.Tensor:
+    """``x2d`` with zero rows appended up to the next multiple of 32 tokens (itself when it already is one)."""
+    extra = -x2d.shape[0] % BLOCK_SCALE
+    return F.pad(x2d, (0, 0, 0, extra)) if extra else x2d
 
 
 _WHOLE_RANGE: dict = {}
@@ -122,30 +133,64 @@ def fused_swiglu_projection(xq, xs, wq, ws, out_dtype):
     return gu, hq, hs, htq, hts
 
 
+def swiglu_tokens(gu: torch.Tensor, rounded: bool = False):
+    """``h = silu(gu[:, :H]) * gu[:, H:]`` as ``(q, s, qT, sT)`` for any token count (see :func:`quantize_tokens`).
+
+    ``rounded``: ``silu`` and the product each rounded to the type of ``gu``, the arithmetic of the unfused activation.
+    """
+    m, h, dev = gu.shape[0], gu.shape[1] // 2, gu.device
+    mt = token_extent(m)
+    q = torch.empty(m, h, device=dev, dtype=_FP8)
+    s = torch.empty(m, h // BLOCK_SCALE, device=dev, dtype=torch.uint8)
+    qt = torch.empty(mt // PANEL, h, PANEL, device=dev, dtype=_FP8)
+    st = torch.empty(h, mt // BLOCK_SCALE, device=dev, dtype=torch.uint8)
+    _lib.invoke(
+        "mx_swiglu_quantize_tokens", m * h * (2 * gu.element_size() + 2 * (1 + 1 / BLOCK_SCALE)), gu,
+        gu.data_ptr(), _lib.MX_DTYPE[gu.dtype], int(rounded), m, h, gu.stride(0), mt, q.data_ptr(), h, s.data_ptr(),
+        h // BLOCK_SCALE, qt.data_ptr(), st.data_ptr(), mt // BLOCK_SCALE,
+    )
+    return q, s, qt, st
+
+
+def swiglu_bwd_tokens(dh: torch.Tensor, gu: torch.Tensor, rounded: bool = False):
+    """``dpre = [dgate | dup]`` as ``(q, s, qT, sT)``, both code matrices stage-major, for any token count (``H % 128 == 0``)."""
+    m, two_h = gu.shape
+    h, dev, mt = two_h // 2, gu.device, token_extent(m)
+    q = torch.empty(two_h // PANEL, m, PANEL, device=dev, dtype=_FP8)
+    s = torch.empty(m, two_h // BLOCK_SCALE, device=dev, dtype=torch.uint8)
+    qt = torch.empty(mt // PANEL, two_h, PANEL, device=dev, dtype=_FP8)
+    st = torch.empty(two_h, mt // BLOCK_SCALE, device=dev, dtype=torch.uint8)
+    _lib.invoke(
+        "mx_swiglu_bwd_quantize_tokens", m * h * (3 * gu.element_size() + 4 * (1 + 1 / BLOCK_SCALE)), gu,
+        dh.data_ptr(), dh.stride(0), gu.data_ptr(), gu.stride(0), _lib.MX_DTYPE[gu.dtype], int(rounded), m, h, mt,
+        q.data_ptr(), PANEL, s.data_ptr(), two_h // BLOCK_SCALE, qt.data_ptr(), st.data_ptr(), mt // BLOCK_SCALE,
+    )
+    return q, s, qt, st
+
+
 class _MXFP8SwiGLUMLP(torch.autograd.Function):
     @staticmethod
     def forward(ctx, x, w_in, w_out, in_f, in_d, out_f, out_d):
         compute = compute_dtype(x)
         shape = x.shape
-        x2d = x.reshape(-1, shape[-1]).to(compute)
-        if x2d.stride(-1) != 1:
-            x2d = x2d.contiguous()
+        x2d = activation_matrix(x, compute)
         tokens = x2d.shape[0]
-        x2d = pad_tokens(x2d)  # whole 32-token blocks for WGRAD; zero rows change no gradient
-        # The operands of the three backward products that go down in one launch (contractions of
-        # 8192 and 16384) are written stage-major: each K stage of a tile is then one contiguous run.
-        sm = x.dtype == compute and stage_major_ok(tokens) and stage_major_ok(w_out.shape[1])
-        xq, xs, xtq, xts = quantize_mx_dual(x2d, stage_major_t=sm)
+        # The token-axis operands (and dpre below) are written stage-major: each K stage of a tile of the three backward
+        # products, which contract over thousands of tokens, is then one contiguous run.  A hidden width that is not
+        # whole panels keeps the row-major kernels, which take whole 32-token blocks: zero rows change no gradient.
+        sm = stage_major_ok(w_out.shape[1]) and tokens > 0
+        xq, xs, xtq, xts = quantize_tokens(x2d, compute) if sm else quantize_mx_dual(pad_tokens(x2d.to(compute)))
         # GEMM, then one bandwidth-bound pass for SwiGLU and both casts: measured faster at the
         # benchmark shape (220 + 89 us) than the same work in the GEMM's epilogue
         # (fused_swiglu_projection: 329 us), whose vector ALU work cannot overlap the MFMAs.
         gu = mxfp8_matmul_pq(xq, xs, *in_f, compute, out_pad=_PITCH_PAD)
-        hq, hs, htq, hts = swiglu_mx_dual(gu, stage_major_t=sm)
+        hq, hs, htq, hts = swiglu_tokens(gu) if sm else swiglu_mx_dual(gu)
         y = mxfp8_matmul_pq(hq, hs, *out_f, compute)
         if any(ctx.needs_input_grad):
             ctx.save_for_backward(xtq, xts, gu, htq, hts, *in_d, *out_d)
             ctx.compute = compute
             ctx.x_dtype = x.dtype
+            ctx.dw_dtypes = gradient_dtype(w_in, compute), gradient_dtype(w_out, compute)
             ctx.stage_major = sm
         return y[:tokens].reshape(*shape[:-1], y.shape[-1])
 
@@ -153,30 +198,21 @@ class _MXFP8SwiGLUMLP(torch.autograd.Function):
     def backward(ctx, dout):
         xtq, xts, gu, htq, hts, win_dq, win_ds, wout_dq, wout_ds = ctx.saved_tensors
         shape = dout.shape
-        d2d = dout.reshape(-1, shape[-1]).to(ctx.compute).contiguous()
+        d2d = activation_matrix(dout, ctx.compute)
         tokens = d2d.shape[0]
-        dq, ds, dtq, dts = quantize_mx_dual(pad_tokens(d2d), stage_major_t=ctx.stage_major)
+        if ctx.stage_major:
+            dq, ds, dtq, dts = quantize_tokens(d2d, ctx.compute)
+        else:
+            dq, ds, dtq, dts = quantize_mx_dual(pad_tokens(d2d.to(ctx.compute)))
         dh = mxfp8_matmul_pq(dq, ds, wout_dq, wout_ds, ctx.compute, out_pad=_PITCH_PAD)
         pq, ps, ptq, pts = swiglu_bwd_mx_dual(dh, gu, stage_major=ctx.stage_major)
         # The last three products are independent and none fills the GPU alone (dW has few
-        # tiles with a long K): they go down together and share the GPU by work.
-        wanted = [
-            (pq, ps, win_dq, win_ds) if ctx.needs_input_grad[0] else None,
-            (ptq, pts, xtq, xts) if ctx.needs_input_grad[1] else None,
-            (dtq, dts, htq, hts) if ctx.needs_input_grad[2] else None,
-        ]
-        grads = [None, None, None]
-        if ctx.x_dtype == ctx.compute:
-            live = [i for i, w in enumerate(wanted) if w is not None]
-            for i, g in zip(live, mxfp8_matmul_pq_batch([wanted[i] for i in live], ctx.compute)):
-                grads[i] = g
-        else:
-            for i, w in enumerate(wanted):
-                if w is not None:
-                    grads[i] = mxfp8_matmul_pq(*w, ctx.x_dtype if i == 0 else ctx.compute)
-        dx, dw_in, dw_out = grads
+        # tiles with a long K): those of one output type go down together and share the GPU by work.
+        wanted = [((pq, ps, win_dq, win_ds), ctx.x_dtype), ((ptq, pts, xtq, xts), ctx.dw_dtypes[0]),
+                  ((dtq, dts, htq, hts), ctx.dw_dtypes[1])]
+        dx, dw_in, dw_out = products_by_dtype(wanted, ctx.needs_input_grad)
         if dx is not None:
-            dx = dx[:tokens].reshape(*shape[:-1], -1)
+            dx = dx[:tokens].reshape(*shape[:-1], dx.shape[-1])
         return dx, dw_in, dw_out, None, None, None, None
 
 
@@ -186,8 +222,7 @@ def mxfp8_swiglu_mlp(x, w_in, w_out, packed) -> torch.Tensor:
     ``packed`` is ``(in_fwd, in_dgrad, out_fwd, out_dgrad)``, each a ``(codes, scales)`` pair:
     the weights blocked along their contraction axis for FPROP and along the other axis for
     DGRAD.  ``w_in``/``w_out`` are passed so autograd routes ``dW`` to the master parameters.
-    ``dim`` and ``H`` must be multiples of 32; any token count is taken (it is padded with zero
-    rows to whole 32-token blocks, which changes no result).
+    ``dim`` and ``H`` must be multiples of 32; any token count is taken.
     """
     if w_in.shape[0] != 2 * w_out.shape[1] or w_in.shape[1] != x.shape[-1] or w_out.shape[0] != x.shape[-1]:
         raise ValueError(f"shape mismatch: x {tuple(x.shape)}, w_in {tuple(w_in.shape)}, w_out {tuple(w_out.shape)}")

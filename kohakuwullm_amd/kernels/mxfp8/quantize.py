@@ -124,6 +124,53 @@ def quantize_mx_dual(x: torch.Tensor, stage_major_t: bool = False):
     return q, s, qt, st
 
 
+def token_extent(tokens: int) -> int:
+    """Length of the token axis of a WGRAD operand: whole 128-token panels, whole groups of four where that is nearly free.
+
+    A contraction of a multiple of 512 runs the GEMM's two-stage look-ahead with its scale bytes 16 at a time, one of whole
+    32-token blocks fetches them byte by byte: dW of 8192 x 1536 over 5024 tokens takes 138 us, over 5120 75 us.  Whole
+    panels that are not groups of four are in between (2176 tokens 40.2 us, 2560 40.9; 2048 x 2048: 31.6 and 35.3 us), so
+    up to a sixteenth more zeros are taken for the groups.
+    """
+    panels = -(-tokens // PANEL) * PANEL
+    groups = -(-tokens // (4 * PANEL)) * 4 * PANEL
+    return groups if 16 * (groups - panels) <= panels else panels
+
+
+def activation_matrix(x: torch.Tensor, compute: torch.dtype) -> torch.Tensor:
+    """``x`` flattened to two dimensions as the activation quantizer takes it: in ``compute`` or, to be rounded there, in fp32."""
+    x2d = x.reshape(-1, x.shape[-1])
+    if x2d.dtype != compute and not (x2d.dtype == torch.float32 and compute in (torch.bfloat16, torch.float16)):
+        x2d = x2d.to(compute)
+    if x2d.stride(1) != 1 or x2d.stride(0) * x2d.element_size() % 16 or x2d.data_ptr() % 16:
+        x2d = x2d.contiguous()
+    return x2d
+
+
+def quantize_tokens(x: torch.Tensor, compute: torch.dtype, cols: int | None = None):
+    """Both operands an activation ``x (M, KV)`` of any row count gives a training step, in one pass over it.
+
+    Returns ``(q, s, qT, sT)``: ``q (M, K)``, ``s (M, K//32)`` along the columns and, along the tokens,
+    ``qT (MT//128, K, 128)`` (stage-major), ``sT (K, MT//32)`` with ``MT = token_extent(M)``.  ``K = cols`` or the width of
+    ``x``; rows and columns past ``x`` are zero, which adds nothing to a product.  fp32 values are rounded to ``compute``
+    first.  Same bytes as casting, padding with zeros and :func:`quantize_mx_dual`.  ``x`` as :func:`activation_matrix`
+    returns it, its width a multiple of 8, ``K`` a multiple of 32.
+    """
+    _check_2d(x, "x")
+    m, kv = x.shape
+    k, mt = cols or kv, token_extent(m)
+    q = torch.empty(m, k, device=x.device, dtype=_FP8)
+    s = torch.empty(m, k // BLOCK_SCALE, device=x.device, dtype=torch.uint8)
+    qt = torch.empty(mt // PANEL, k, PANEL, device=x.device, dtype=_FP8)
+    st = torch.empty(k, mt // BLOCK_SCALE, device=x.device, dtype=torch.uint8)
+    _lib.invoke(
+        "mx_quantize_tokens", m * kv * (x.element_size() + 2 * (1 + 1 / BLOCK_SCALE)), x,
+        x.data_ptr(), _lib.MX_DTYPE[x.dtype], _lib.MX_DTYPE[compute], m, kv, x.stride(0), mt, k,
+        q.data_ptr(), k, s.data_ptr(), k // BLOCK_SCALE, qt.data_ptr(), st.data_ptr(), mt // BLOCK_SCALE,
+    )
+    return q, s, qt, st
+
+
 def quantize_mx_dual_batch(xs: list[torch.Tensor]) -> list[tuple[torch.Tensor, torch.Tensor, torch.Tensor, torch.Tensor]]:
     """``quantize_mx_dual`` of every matrix of ``xs`` behind one launch per 24 matrices.
 
@@ -272,6 +319,17 @@ def mxfp8_matmul_pq_batch(problems, out_dtype: torch.dtype = torch.bfloat16) -> 
     _lib.invoke("mx_gemm_nt_batch", flops, outs[0], ctypes.addressof(descs), len(problems), _lib.MX_DTYPE[out_dtype],
                 ws.data_ptr(), ws.numel())
     return outs
+
+
+def products_by_dtype(wanted, needed) -> list:
+    """The products ``(operands, out_dtype)`` of ``wanted`` that ``needed`` asks for, one batched launch per output type."""
+    results = [None] * len(wanted)
+    live = [i for i in range(len(wanted)) if needed[i]]
+    for dtype in dict.fromkeys(wanted[i][1] for i in live):
+        group = [i for i in live if wanted[i][1] == dtype]
+        for i, out in zip(group, mxfp8_matmul_pq_batch([wanted[i][0] for i in group], dtype)):
+            results[i] = out
+    return results
 
 
 def mxfp8_matmul(a: torch.Tensor, b: torch.Tensor, out_dtype: torch.dtype | None = None) -> torch.Tensor:
