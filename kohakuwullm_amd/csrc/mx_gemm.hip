@@ -6,9 +6,12 @@
 #include <atomic>
 
 #include "mx_gemm_core.h"
+#include "mx_gemm_ring.h"
 #ifdef MX_BENCH_VARIANTS
 #include "mx_gemm_variants.h"
 #endif
+
+#define MX_BATCH_MAX 4
 
 namespace mx {
 
@@ -272,7 +275,6 @@ __global__ __launch_bounds__(S::NTHR) __attribute__((amdgpu_waves_per_eu(2, 2)))
 // Several independent products in one launch.  The XCDs are partitioned among the problems
 // (x_lo[j] .. x_lo[j+1]) in proportion to their work, so a product with too few
 // tiles to fill the GPU runs beside the others instead of leaving most of it idle.
-#define MX_BATCH_MAX 4
 // Problem j owns XCDs [x_lo[j], x_lo[j + 1]) whole: all 32 CUs of an XCD then work on one product
 // and share its panels in that XCD's L2.  (Dealing every problem a few CUs of every XCD instead
 // was measured: the three backward products of the feed-forward block pulled 1957 MiB through
@@ -335,8 +337,8 @@ __global__ __launch_bounds__(S::NTHR) void split_reduce_kernel(DenseArgs p) {
 
 // Adds the split_k fp32 slices of every tile, in slice order, and stores C.  One block per (tile, i).
 template <typename S, int CDT>
-__global__ __launch_bounds__(S::NTHR) void slice_reduce_kernel(DenseArgs p) {
-    const int index = blockIdx.x / S::MT, i = blockIdx.x % S::MT;
+__device__ __forceinline__ void slice_reduce(const DenseArgs &p, int block) {
+    const int index = block / S::MT, i = block % S::MT;
     const int tid = threadIdx.x;
     v4f sum[S::NT];
 #pragma unroll
@@ -350,16 +352,47 @@ __global__ __launch_bounds__(S::NTHR) void slice_reduce_kernel(DenseArgs p) {
     tile_of(index, p.tiles_m, p.tiles_n, tm, tn, stagger_columns(p.K), p.xcds);
     const int wave = tid >> 6, lane = tid & 63;
     const int wm = p.phased ? wave & 3 : wave / S::WGN, wn = p.phased ? wave >> 2 : wave % S::WGN;
-    const int n = tn * S::BN + wn * S::WTN + 8 * (lane & 15);
+    const int n = tn * S::BN + wn * S::WTN + S::NT * (lane & 15);
 #pragma unroll
     for (int v = 0; v < 4; v++) {
         const int m = tm * S::BM + wm * S::WTM + 16 * i + 4 * (lane >> 4) + v;
         if (m < p.M && n < p.N) {
-            const v4f lo = {sum[0][v], sum[1][v], sum[2][v], sum[3][v]};
-            const v4f hi = {sum[4][v], sum[5][v], sum[6][v], sum[7][v]};
-            store8<CDT>(p.c, (int64_t)m * p.ldc + n, lo, hi, p.N - n < 8 ? p.N - n : 8, p.c_vec != 0);
+            float run[S::NT];
+#pragma unroll
+            for (int j = 0; j < S::NT; j++) run[j] = sum[j][v];
+            store_run<CDT, S::NT>(p.c, (int64_t)m * p.ldc + n, run, p.N - n < S::NT ? p.N - n : S::NT, p.c_vec != 0);
         }
     }
+}
+
+template <typename S, int CDT>
+__global__ __launch_bounds__(S::NTHR) void slice_reduce_kernel(DenseArgs p) {
+    slice_reduce<S, CDT>(p, (int)blockIdx.x);
+}
+
+// Up to MX_BATCH_MAX products on the ring kernel's tiles behind one launch: workgroup `id` belongs to the problem whose
+// range [end[j - 1], end[j]) it falls into, and computes one tile or one K slice of a tile of it.
+struct RingArgs {
+    DenseArgs prob[MX_BATCH_MAX];
+    int end[MX_BATCH_MAX];
+    int count;
+};
+
+template <int CDT>
+__global__ __launch_bounds__(RingShape::NTHR, 2) void gemm_nt_ring_kernel(RingArgs b) {
+    extern __shared__ __attribute__((aligned(1024))) uint8_t smem[];
+    int j = 0;
+    while (j + 1 < b.count && (int)blockIdx.x >= b.end[j]) j++;
+    DenseProblem<RingShape, CDT> prob(b.prob[j], (int)blockIdx.x - (j ? b.end[j - 1] : 0), 0x40000000);
+    ring_gemm(prob, smem);
+}
+
+// slice_reduce for every problem of such a launch that was cut along K (`end` counts blocks of those).
+template <int CDT>
+__global__ __launch_bounds__(RingShape::NTHR) void ring_reduce_kernel(RingArgs b) {
+    int j = 0;
+    while (j + 1 < b.count && (int)blockIdx.x >= b.end[j]) j++;
+    slice_reduce<RingShape, CDT>(b.prob[j], (int)blockIdx.x - (j ? b.end[j - 1] : 0));
 }
 
 // Any K % 32 == 0, any alignment: one thread per output element.  The slow path.
@@ -470,6 +503,47 @@ static int scale_mode(const DenseArgs &a) {
     return SCALES_BYTES;
 }
 
+// Whether a product can go to the ring kernel: whole groups of four stages, no accumulation, scale rows the copy engine takes.
+static bool ring_ok(const DenseArgs &a) {
+    return a.K % 512 == 0 && a.split_k == 1 && !a.accumulate && aligned(a.as, 4) && aligned(a.bs, 4) && a.ldas % 4 == 0 && a.ldbs % 4 == 0 &&
+           (int64_t)a.M * a.ldas < ((int64_t)1 << 32) && (int64_t)a.N * a.ldbs < ((int64_t)1 << 32);
+}
+
+static int64_t tiles_of(const DenseArgs &a, int edge) { return (int64_t)((a.M + edge - 1) / edge) * ((a.N + edge - 1) / edge); }
+
+// K slices of a ring product: a long contraction (64 stages and more) of few tiles is cut so that the chip has a workgroup per
+// CU, into slices of at least 16 stages.  512 x 512 x 8192 (16 tiles): 27.2 us whole, 18.2 in four slices; 512 x 1536 x 16384:
+// 76.2 and 31.9 us; 1536 x 512 x 4096 (32 stages) 16.8 whole, 16.7 and 18.4 in two and four: not worth it.
+static int ring_slices(const DenseArgs &a, int free_tiles) {
+    const int KT = a.K >> 7;
+    const int64_t tiles = tiles_of(a, RingShape::BM);
+    if (KT < 64) return 1;
+    int best = 1;
+    for (int s = 2; s <= 8; s *= 2) {
+        const int per = ((KT + s - 1) / s + 3) & ~3;
+        if (tiles * s <= num_cus() && tiles * s <= free_tiles && per >= 16 && (s - 1) * per < KT) best = s;
+    }
+    return best;
+}
+
+// ... and whether it should.  Both kernels are priced in us from what they were measured to take (operands cold): a ring
+// workgroup 0.52 per stage and 1.5 per tile on top of 6, the persistent kernel 1.4 per stage of a 256 x 256 tile (1.6 with
+// more than half of the CUs busy), four stages per tile and 3, or, the last round's K stages dealt out evenly, its share of
+// the work and about 35 for the fp32 pieces.  us persistent / ring where the line lies: 1500 x 1536 x 4096 50.1 / 20.0, 2048 x 2048
+// x 3072 41.1 / 18.7, 3001 x 2048 x 2048 29.6 / 22.2, 5003 x 1536 x 4096 54.3 / 43.4, 16384 x 512 x 2048 32.3 / 29.0, 3000 x 3072 x 2048
+// 30.6 / 30.3, 4096 x 3072 x 2048 32.0 / 32.4, 2048 x 2048 x 16384 82.4 / 79.4, 5003 x 8192 x 1536 73 / 85, 1536 x 4096 x 16384 105 / 140.
+static bool ring_pays(const DenseArgs &a) {
+    if (!ring_ok(a)) return false;
+    const int64_t small = tiles_of(a, 128), large = tiles_of(a, 256), cus = num_cus();
+    if (small > 4 * cus) return false;
+    const double KT = a.K >> 7;
+    const int slices = ring_slices(a, 0x7FFFFFFF);
+    const double ring = slices > 1 ? 0.52 * KT / slices + 13.5 : (double)((small + cus - 1) / cus) * (0.52 * KT + 1.5) + 6;
+    const double stage = 2 * large > cus ? 1.6 : 1.4;
+    const double whole = (double)((large + cus - 1) / cus) * (KT + 4) * stage + 3, dealt = (double)large * KT / cus * 1.65 + 35;
+    return ring < (whole < dealt ? whole : dealt);
+}
+
 template <typename S, int CDT>
 static int launch_tiled(DenseArgs a, float *ws, int ws_slots, hipStream_t st, bool phased = false) {
     a.tiles_m = (a.M + S::BM - 1) / S::BM;
@@ -488,7 +562,11 @@ static int launch_tiled(DenseArgs a, float *ws, int ws_slots, hipStream_t st, bo
     // tile, so no tile is cut into more than 9 pieces.
     const int rest = (int)(work % cus);
     const int KT = ((a.K + 127) >> 7), KT4 = (KT + 3) & ~3;
-    if (a.split_k == 1 && !a.accumulate && rest > 0 && KT4 >= 8) {
+    bool deal = a.split_k == 1 && !a.accumulate && rest > 0 && KT4 >= 8;
+#ifdef MX_BENCH_VARIANTS
+    deal = deal && !ring_pays(a);  // an alternative kernel splits K where the default would, and there the default is the ring
+#endif
+    if (deal) {
         int64_t q = ((int64_t)rest * KT4 + cus - 1) / cus;
         if (q < KT4 / 8) q = KT4 / 8;
         q = (q + 3) & ~(int64_t)3;
@@ -561,6 +639,43 @@ static bool tiled_ok(const DenseArgs &a) {
            ((M + 255) / 256) * ((N + 255) / 256) * a.split_k < 0x7FFFFFFF;
 }
 
+// `count` products on the ring kernel's tiles behind one launch.  `ws`: fp32 tile slots of 256 x 256, four ring tiles each.
+template <int CDT>
+static int launch_ring(DenseArgs *probs, int count, float *ws, int ws_slots, hipStream_t st) {
+    typedef RingShape S;
+    RingArgs b, red;
+    b.count = count, red.count = 0;
+    int blocks = 0, rblocks = 0, free_tiles = ws_slots >= 2 * num_cus() ? 8 * num_cus() : 0;  // a short workspace is left alone
+    int64_t slot = 0;
+    for (int j = 0; j < count; j++) {
+        DenseArgs &a = probs[j];
+        a.tiles_m = (a.M + S::BM - 1) / S::BM;
+        a.tiles_n = (a.N + S::BN - 1) / S::BN;
+        a.c_vec = aligned(a.c, 16) && (a.ldc * (CDT == MX_FP32 ? 4 : 2)) % 16 == 0;
+        const int tiles = a.tiles_m * a.tiles_n;
+        a.dp_tiles = tiles, a.sk_tiles = 0, a.sk_q = 0, a.sk_ws = nullptr;
+        a.xcds = 8, a.phased = 0;
+        a.split_k = ring_slices(a, free_tiles);
+        a.slice_ws = nullptr;
+        if (a.split_k > 1) {
+            a.slice_ws = ws + slot * (S::BM * S::BN);
+            slot += (int64_t)tiles * a.split_k;
+            free_tiles -= tiles * a.split_k;
+            red.prob[red.count] = a;
+            rblocks += tiles * S::MT;
+            red.end[red.count++] = rblocks;
+        }
+        blocks += tiles * a.split_k;
+        b.prob[j] = a;
+        b.end[j] = blocks;
+    }
+    const dim3 grid((unsigned)blocks), block(S::NTHR);
+    const int rc = launch_with_lds<gemm_nt_ring_kernel<CDT>>(grid, block, RING_LDS_BYTES, st, b);
+    if (rc != MX_OK) return rc;
+    if (red.count) ring_reduce_kernel<CDT><<<dim3((unsigned)rblocks), block, 0, st>>>(red);
+    return hipGetLastError() == hipSuccess ? MX_OK : MX_ELAUNCH;
+}
+
 template <int CDT>
 static int gemm_dispatch(DenseArgs a, float *ws, int ws_slots, hipStream_t st, bool pair = false, bool phased = false,
                          bool wide = false) {
@@ -579,6 +694,7 @@ static int gemm_dispatch(DenseArgs a, float *ws, int ws_slots, hipStream_t st, b
                                                                                   a.lda, a.ldas, a.ldb, a.ldbs, a.ldc);
         return hipGetLastError() == hipSuccess ? MX_OK : MX_ELAUNCH;
     }
+    if (!phased && ring_pays(a)) return launch_ring<CDT>(&a, 1, ws, ws_slots, st);
     return launch_tiled<DenseShape, CDT>(a, ws, ws_slots, st, phased);
 }
 
@@ -594,6 +710,12 @@ template <int CDT>
 static int batch_dispatch(DenseArgs *probs, int count, float *ws, int ws_slots, hipStream_t st) {
     typedef DenseShape S;
     const int cus = num_cus();
+    // All of them on the ring kernel: its tiles side by side fill the chip, whoever they belong to (4096 x 512 x 1536 beside
+    // 1536 x 512 x 4096: 39 -> 20 us; 3001 x 2048 x 2048 beside 2048 x 2048 x 3072: 45 -> 41).  A mixed batch shares the XCDs
+    // below instead: one launch for each kind won 7 % on one such batch and lost up to 25 % on the others.
+    bool ring = true;
+    for (int j = 0; j < count; j++) ring = ring && tiled_ok(probs[j]) && ring_pays(probs[j]);
+    if (ring && count) return launch_ring<CDT>(probs, count, ws, ws_slots, st);
     bool fuse = count > 1 && count <= MX_BATCH_MAX;
     DenseBatchArgs b;
     int64_t tiles[MX_BATCH_MAX], alone = 0;

@@ -1,0 +1,59 @@
+"""The small-tile GEMM (csrc/mx_gemm_ring.h) against dequantize-then-matmul in fp64 at the edges of what it takes: single
+groups of four K stages, ragged and single rows, K slices, padded rows, stage-major operands, several products in a launch.
+
+Tolerances are those of the other GEMM tests: 1e-4 in fp32 (the block-scaled MFMA's own adder), 4e-3 in bf16 (its rounding)."""
+
+import pytest
+import torch
+
+from conftest import SEED
+
+pytestmark = pytest.mark.gpu
+DEV = "cuda:0"
+F8 = torch.float8_e4m3fn
+TOL = {torch.float32: 1e-4, torch.bfloat16: 4e-3, torch.float16: 6e-4}
+
+
+def _operands(oracle, m, n, k):
+    g = torch.Generator().manual_seed(SEED + m)
+    a = (torch.randn(m, k, generator=g)).bfloat16()
+    b = (torch.randn(n, k, generator=g) * 0.02).bfloat16()
+    return *oracle.quantize_rows(a), *oracle.quantize_rows(b)
+
+
+def _dev(ops, panels=False):
+    aq, a_s, bq, b_s = (t.to(DEV) for t in ops)
+    if panels:
+        aq, bq = (t.view(t.shape[0], t.shape[1] // 128, 128).permute(1, 0, 2).contiguous() for t in (aq, bq))
+    return aq.view(F8), a_s, bq.view(F8), b_s
+
+
+@pytest.mark.parametrize("m,n,k", [
+    (1, 1, 512), (1, 3072, 2048), (127, 129, 512), (128, 128, 1024), (129, 257, 1536), (700, 260, 4096),
+    (300, 520, 8192),  # 15 tiles, cut into eight K slices
+    (16, 40, 16384), (130, 1000, 10240),  # slices of unequal length
+])
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16, torch.float16])
+def test_ring_gemm(oracle, m, n, k, dtype):
+    from kohakuwullm_amd.kernels.mxfp8 import mxfp8_matmul_pq
+
+    ops = _operands(oracle, m, n, k)
+    ref = oracle.gemm_nt(*ops)
+    out = mxfp8_matmul_pq(*_dev(ops), dtype)
+    assert oracle.rel_error(out.cpu(), ref) < TOL[dtype]
+    padded = mxfp8_matmul_pq(*_dev(ops), dtype, out_pad=24)
+    assert padded.stride(0) == n + 24 and torch.equal(padded, out)
+    assert torch.equal(mxfp8_matmul_pq(*_dev(ops, panels=True), dtype), out)
+
+
+def test_ring_gemm_several_products_in_one_launch(oracle):
+    from kohakuwullm_amd.kernels.mxfp8 import mxfp8_matmul_pq, mxfp8_matmul_pq_batch
+
+    shapes = [(515, 256, 512), (64, 384, 8192), (1, 129, 1024), (256, 512, 8192), (300, 40, 2048)]
+    ops = [_operands(oracle, *s) for s in shapes]
+    problems = [_dev(o, panels=i % 2 == 1) for i, o in enumerate(ops)]
+    outs = mxfp8_matmul_pq_batch(problems, torch.float32)
+    for o, p, out in zip(ops, problems, outs):
+        assert oracle.rel_error(out.cpu(), oracle.gemm_nt(*o)) < 1e-4
+        alone = mxfp8_matmul_pq(*p, torch.float32)
+        assert oracle.rel_error(out.cpu(), alone.double().cpu()) < 1e-5  # the same sums, K slices apart
