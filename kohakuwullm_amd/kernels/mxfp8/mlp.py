@@ -19,7 +19,7 @@ import torch
 import torch.nn.functional as F
 
 from kohakuwullm_amd import _lib
-from kohakuwullm_amd.kernels.mxfp8.linear import compute_dtype, gradient_dtype
+from kohakuwullm_amd.kernels.mxfp8.linear import compute_dtype, gradient_dtype, unobserved
 from kohakuwullm_amd.kernels.mxfp8.quantize import (
     BLOCK_SCALE,
     PANEL,
@@ -33,6 +33,7 @@ from kohakuwullm_amd.kernels.mxfp8.quantize import (
 )
 
 _FP8 = torch.float8_e4m3fn
+_TENSORS = (torch.Tensor, torch.nn.Parameter)  # a subclass dispatches each operator itself
 
 # The two projection outputs that only the SwiGLU quantizers read (`gu`, `dh`) are allocated with 128 spare
 # elements per row.  Their natural pitches (16 KiB and 8 KiB at the benchmark shape) put the 128 rows a quantizer
@@ -170,7 +171,7 @@ def swiglu_bwd_tokens(dh: torch.Tensor, gu: torch.Tensor, rounded: bool = False)
 
 class _MXFP8SwiGLUMLP(torch.autograd.Function):
     @staticmethod
-    def forward(ctx, x, w_in, w_out, in_f, in_d, out_f, out_d):
+    def forward(ctx, x, w_in, w_out, in_f, in_d, out_f, out_d, rounded):
         compute = compute_dtype(x)
         shape = x.shape
         x2d = activation_matrix(x, compute)
@@ -184,14 +185,14 @@ class _MXFP8SwiGLUMLP(torch.autograd.Function):
         # benchmark shape (220 + 89 us) than the same work in the GEMM's epilogue
         # (fused_swiglu_projection: 329 us), whose vector ALU work cannot overlap the MFMAs.
         gu = mxfp8_matmul_pq(xq, xs, *in_f, compute, out_pad=_PITCH_PAD)
-        hq, hs, htq, hts = swiglu_tokens(gu) if sm else swiglu_mx_dual(gu)
+        hq, hs, htq, hts = swiglu_tokens(gu, rounded) if sm else swiglu_mx_dual(gu)
         y = mxfp8_matmul_pq(hq, hs, *out_f, compute)
         if any(ctx.needs_input_grad):
             ctx.save_for_backward(xtq, xts, gu, htq, hts, *in_d, *out_d)
             ctx.compute = compute
             ctx.x_dtype = x.dtype
             ctx.dw_dtypes = gradient_dtype(w_in, compute), gradient_dtype(w_out, compute)
-            ctx.stage_major = sm
+            ctx.stage_major, ctx.rounded = sm, rounded
         return y[:tokens].reshape(*shape[:-1], y.shape[-1])
 
     @staticmethod
@@ -205,7 +206,7 @@ class _MXFP8SwiGLUMLP(torch.autograd.Function):
         else:
             dq, ds, dtq, dts = quantize_mx_dual(pad_tokens(d2d.to(ctx.compute)))
         dh = mxfp8_matmul_pq(dq, ds, wout_dq, wout_ds, ctx.compute, out_pad=_PITCH_PAD)
-        pq, ps, ptq, pts = swiglu_bwd_mx_dual(dh, gu, stage_major=ctx.stage_major)
+        pq, ps, ptq, pts = swiglu_bwd_tokens(dh, gu, ctx.rounded) if ctx.stage_major else swiglu_bwd_mx_dual(dh, gu)
         # The last three products are independent and none fills the GPU alone (dW has few
         # tiles with a long K): those of one output type go down together and share the GPU by work.
         wanted = [((pq, ps, win_dq, win_ds), ctx.x_dtype), ((ptq, pts, xtq, xts), ctx.dw_dtypes[0]),
@@ -213,7 +214,7 @@ class _MXFP8SwiGLUMLP(torch.autograd.Function):
         dx, dw_in, dw_out = products_by_dtype(wanted, ctx.needs_input_grad)
         if dx is not None:
             dx = dx[:tokens].reshape(*shape[:-1], dx.shape[-1])
-        return dx, dw_in, dw_out, None, None, None, None
+        return dx, dw_in, dw_out, None, None, None, None, None
 
 
 def mxfp8_swiglu_mlp(x, w_in, w_out, packed) -> torch.Tensor:
@@ -226,4 +227,26 @@ def mxfp8_swiglu_mlp(x, w_in, w_out, packed) -> torch.Tensor:
     """
     if w_in.shape[0] != 2 * w_out.shape[1] or w_in.shape[1] != x.shape[-1] or w_out.shape[0] != x.shape[-1]:
         raise ValueError(f"shape mismatch: x {tuple(x.shape)}, w_in {tuple(w_in.shape)}, w_out {tuple(w_out.shape)}")
-    return _MXFP8SwiGLUMLP.apply(x, w_in, w_out, *packed)
+    return _MXFP8SwiGLUMLP.apply(x, w_in, w_out, *packed, False)
+
+
+def mxfp8_swiglu_pair(x, w_in, w_out) -> torch.Tensor | None:
+    """``w_out(silu(gate) * value)`` of two :class:`MXFP8Linear` around the 16-bit activation, as one graph.
+
+    The activation's two operators and their gradients ran as six library passes over ``(tokens, H)`` or ``(tokens, 2H)``
+    matrices, between quantizers that read each result back: 174 us of a 600 us step over 5003 tokens x 1536 x 4096.  Here
+    the SwiGLU quantizers do them on the way, with every intermediate rounded as those operators round it.  ``None`` for
+    what this graph does not stand for: a layer someone watches (hooks), padded widths, a type other than bf16 / fp16.
+    """
+    if not (unobserved(w_in) and unobserved(w_out)) or not x.is_cuda or not x.numel() or type(x) not in _TENSORS:
+        return None
+    compute = compute_dtype(x)
+    if compute not in (torch.bfloat16, torch.float16) or x.dtype not in _lib.MX_DTYPE or x.shape[-1] != w_in.in_features:
+        return None
+    if w_in.out_features != 2 * w_out.in_features or w_out.out_features % PANEL:
+        return None
+    for lin in (w_in, w_out):
+        if lin._cache is None:
+            lin.refresh_quantized_weight()
+    (in_f, in_d), (out_f, out_d) = ((lin._cache[:2], lin._cache[2:]) for lin in (w_in, w_out))
+    return _MXFP8SwiGLUMLP.apply(x, w_in.weight, w_out.weight, in_f, in_d, out_f, out_d, True)

@@ -14,7 +14,7 @@ import torch
 import torch.nn as nn
 import torch.nn.functional as F
 
-from kohakuwullm_amd.kernels.mxfp8.mlp import mxfp8_swiglu_mlp
+from kohakuwullm_amd.kernels.mxfp8.mlp import mxfp8_swiglu_mlp, mxfp8_swiglu_pair
 from kohakuwullm_amd.kernels.mxfp8.quantize import quantize_mx, quantize_mx_cols
 from kohakuwullm_amd.models.mxfp8_swap import Matmul
 from kohakuwullm_amd.registry import MLP
@@ -47,6 +47,10 @@ class GLUMLP(nn.Module):
 
     def forward(self, x: torch.Tensor) -> torch.Tensor:
         if self.fused_gate:
+            if self.act is F.silu:
+                out = mxfp8_swiglu_pair(x, self.w_in, self.w_out)
+                if out is not None:
+                    return out
             gate, value = self.w_in(x).chunk(2, dim=-1)
         else:
             gate, value = self.gate_proj(x), self.up_proj(x)
