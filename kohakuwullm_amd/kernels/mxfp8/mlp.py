@@ -206,7 +206,7 @@ class _MXFP8SwiGLUMLP(torch.autograd.Function):
         else:
             dq, ds, dtq, dts = quantize_mx_dual(pad_tokens(d2d.to(ctx.compute)))
         dh = mxfp8_matmul_pq(dq, ds, wout_dq, wout_ds, ctx.compute, out_pad=_PITCH_PAD)
-        pq, ps, ptq, pts = swiglu_bwd_tokens(dh, gu, ctx.rounded) if ctx.stage_major else swiglu_bwd_mx_dual(dh, gu)
+        pq, ps, ptq, pts = swiglu_bwd_tokens(dh, gu, True) if ctx.rounded else swiglu_bwd_mx_dual(dh, gu, stage_major=ctx.stage_major)
         # The last three products are independent and none fills the GPU alone (dW has few
         # tiles with a long K): those of one output type go down together and share the GPU by work.
         wanted = [((pq, ps, win_dq, win_ds), ctx.x_dtype), ((ptq, pts, xtq, xts), ctx.dw_dtypes[0]),
