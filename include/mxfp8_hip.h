@@ -170,7 +170,7 @@ int mx_swiglu_bwd_quantize_dual(const void *dh, int64_t lddh, const void *gu, in
  * tokens, MT of them -- a multiple of 128 chosen by the caller -- with qT always stage-major (MT/128, K, 128).
  * mx_quantize_dual on a matrix padded with zero rows and columns gives the same bytes.  cast_dtype: x's own type, or for
  * fp32 x a 16-bit type the values are rounded to first (the cast a mixed-precision caller would have made).
- * KV % 8 == 0, K % 32 == 0, 16-byte aligned rows of x.
+ * KV % 8 == 0, K % 32 == 0, 16-byte aligned rows of x.  qT and sT NULL: the token-axis operand is not wanted (KV == K).
  */
 int mx_quantize_tokens(const void *x, int x_dtype, int cast_dtype, int64_t M, int64_t KV, int64_t ldx, int64_t MT, int64_t K,
                        uint8_t *q, int64_t ldq, uint8_t *s, int64_t lds, uint8_t *qT, uint8_t *sT, int64_t ldsT, void *stream);
@@ -180,7 +180,7 @@ int mx_quantize_tokens(const void *x, int x_dtype, int cast_dtype, int64_t M, in
  * tokens stage-major, (q, s) for the M rows (the backward's q stage-major when ldq == 128 and H % 128 == 0).
  * rounded != 0: the arithmetic of the unfused 16-bit activation and its gradient -- silu(g), h, dh u, dh silu(g) and dgate
  * are rounded to the input type one by one (mlp.py:68-73 of the reference, where nn.functional.silu and a product stand
- * between the two projections) -- otherwise everything up to the cast is fp32.
+ * between the two projections) -- otherwise everything up to the cast is fp32.  The forward takes qT and sT NULL as above.
  */
 int mx_swiglu_quantize_tokens(const void *gu, int dtype, int rounded, int64_t M, int64_t H, int64_t ldgu, int64_t MT, uint8_t *q,
                               int64_t ldq, uint8_t *s, int64_t lds, uint8_t *qT, uint8_t *sT, int64_t ldsT, void *stream);

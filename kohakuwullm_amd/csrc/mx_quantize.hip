@@ -24,7 +24,23 @@ __device__ __forceinline__ uint32_t gather_row_scales(uint32_t byte, int lane) {
     return v;
 }
 
-template <int DT, int U, bool FLAT>
+// fp32 values rounded to a 16-bit type and widened again: what a cast in front of the quantizer would have left.
+template <int CDT>
+__device__ __forceinline__ void round_values(float (&v)[8]) {
+    if constexpr (CDT == MX_BF16) {
+#pragma unroll
+        for (int c = 0; c < 8; c += 2) {
+            const uint32_t w = pack2_bf16(v[c], v[c + 1]);
+            v[c] = bits2f(w << 16), v[c + 1] = bits2f(w & 0xFFFF0000u);
+        }
+    } else if constexpr (CDT == MX_FP16) {
+#pragma unroll
+        for (int c = 0; c < 8; c++) v[c] = (float)(_Float16)v[c];
+    }
+}
+
+// CDT: the type fp32 values are rounded to before they are quantized (MX_FP32: none).
+template <int DT, int U, bool FLAT, int CDT = MX_FP32>
 __global__ __launch_bounds__(256) void quant_rows_kernel(const void *__restrict__ x, uint32_t chunks_per_row,
                                                           int64_t sx_row, uint8_t *__restrict__ q, int64_t ldq,
                                                           uint8_t *__restrict__ s, int64_t lds, uint32_t total_chunks,
@@ -53,6 +69,7 @@ __global__ __launch_bounds__(256) void quant_rows_kernel(const void *__restrict_
         }
         if (ok[u]) {
             Elem<DT>::load8((const T *)x + xoff, v[u]);
+            round_values<CDT>(v[u]);
         } else {
 #pragma unroll
             for (int i = 0; i < 8; i++) v[u][i] = 0.0f;
@@ -457,21 +474,6 @@ __device__ __forceinline__ void load_rows_or_zero(const void *x, int64_t first, 
     }
 }
 
-// fp32 values rounded to a 16-bit type and widened again: what a cast in front of the quantizer would have left.
-template <int CDT>
-__device__ __forceinline__ void round_values(float (&v)[8]) {
-    if constexpr (CDT == MX_BF16) {
-#pragma unroll
-        for (int c = 0; c < 8; c += 2) {
-            const uint32_t w = pack2_bf16(v[c], v[c + 1]);
-            v[c] = bits2f(w << 16), v[c + 1] = bits2f(w & 0xFFFF0000u);
-        }
-    } else if constexpr (CDT == MX_FP16) {
-#pragma unroll
-        for (int c = 0; c < 8; c++) v[c] = (float)(_Float16)v[c];
-    }
-}
-
 // RAW (16-bit inputs, R = 8): the tile stays packed as loaded (quant_tile_raw): 64 registers, eight waves per SIMD.
 // x has M rows and KV columns, the outputs MT and K (both rounded up by the caller): what lies past x is zero.
 // CDT: the type fp32 values are rounded to before they are quantized (MX_FP32: none).
@@ -718,10 +720,10 @@ __global__ __launch_bounds__(256) void swiglu_bwd_quant_dual_kernel(const void *
 }
 
 // ------------------------------------------------------------------------------------
-// silu(gate) * up in fp32 -> row-axis MXFP8 (fused_act.py:37-66 of the reference).
+// silu(gate) * up in fp32 -> row-axis MXFP8 (fused_act.py:37-66 of the reference).  ROUNDED as in swiglu_quant_dual_kernel.
 // ------------------------------------------------------------------------------------
 
-template <int DT, int U>
+template <int DT, int U, bool ROUNDED>
 __global__ __launch_bounds__(256) void swiglu_quant_rows_kernel(const void *__restrict__ g, const void *__restrict__ up,
                                                                  uint32_t chunks_per_row, int64_t ldg, int64_t ldu,
                                                                  uint8_t *__restrict__ q, int64_t ldq,
@@ -755,8 +757,12 @@ __global__ __launch_bounds__(256) void swiglu_quant_rows_kernel(const void *__re
 #pragma unroll
         for (int i = 0; i < 8; i++) {
             float gv = a[u][i];
-            v[i] = gv * sigmoid_f32(gv) * b[u][i];
+            v[i] = gv * sigmoid_f32(gv);
         }
+        if constexpr (ROUNDED) round_values<DT>(v);
+#pragma unroll
+        for (int i = 0; i < 8; i++) v[i] *= b[u][i];
+        if constexpr (ROUNDED) round_values<DT>(v);
         float amax = quad_max(amax8(v));
         uint32_t byte = scale_byte(amax);
         float inv = inv_scale(byte);
@@ -979,13 +985,14 @@ static inline int esize(int dt) { return dt == MX_FP32 ? 4 : 2; }
         if (hipGetLastError() != hipSuccess) return MX_ELAUNCH; \
     } while (0)
 
-template <int DT>
+template <int DT, int CDT = MX_FP32>
 static int launch_rows(const void *x, int64_t M, int64_t K, int64_t sx_row, int64_t sx_col, uint8_t *q, int64_t ldq,
                        uint8_t *s, int64_t lds, hipStream_t st) {
     const int64_t KB = K / MX_BLOCK;
     const bool vec_ok = sx_col == 1 && aligned(x, 16) && (sx_row * esize(DT)) % 16 == 0 && aligned(q, 8) &&
                         ldq % 8 == 0 && M * (K / 8) < (int64_t)0x7FFFFF00;
     if (!vec_ok) {
+        if (CDT != MX_FP32) return MX_EUNSUPPORTED;
         int64_t blocks = M * KB;
         if ((blocks + 255) / 256 > 0x7FFFFFFF) return MX_EUNSUPPORTED;
         quant_rows_generic_kernel<DT><<<dim3((unsigned)((blocks + 255) / 256)), dim3(256), 0, st>>>(
@@ -1001,10 +1008,10 @@ static int launch_rows(const void *x, int64_t M, int64_t K, int64_t sx_row, int6
     const bool flat = sx_row == K && ldq == K && lds == KB;
     if (flat) {
         int pack = aligned(s, 4);
-        quant_rows_kernel<DT, U, true><<<dim3(grid), dim3(256), 0, st>>>(x, cpr, sx_row, q, ldq, s, lds, total, pack);
+        quant_rows_kernel<DT, U, true, CDT><<<dim3(grid), dim3(256), 0, st>>>(x, cpr, sx_row, q, ldq, s, lds, total, pack);
     } else {
         int pack = aligned(s, 4) && lds % 4 == 0 && KB % 4 == 0;
-        quant_rows_kernel<DT, U, false><<<dim3(grid), dim3(256), 0, st>>>(x, cpr, sx_row, q, ldq, s, lds, total, pack);
+        quant_rows_kernel<DT, U, false, CDT><<<dim3(grid), dim3(256), 0, st>>>(x, cpr, sx_row, q, ldq, s, lds, total, pack);
     }
     MX_LAUNCH_CHECK();
     return MX_OK;
@@ -1260,14 +1267,14 @@ extern "C" int mx_quantize_dual_batch(const mx_quant_problem *problems, int coun
     return flush();
 }
 
-template <int DT>
+template <int DT, bool ROUNDED>
 static int launch_swiglu(const void *g, const void *u, int64_t M, int64_t K, int64_t ldg, int64_t ldu, uint8_t *q,
                          int64_t ldq, uint8_t *s, int64_t lds, hipStream_t st) {
     constexpr int U = 2;
     const uint32_t total = (uint32_t)(M * (K / 8));
     const unsigned grid = (total + U * 256 - 1) / (U * 256);
     int pack = aligned(s, 4) && lds % 4 == 0 && (K / MX_BLOCK) % 4 == 0;
-    swiglu_quant_rows_kernel<DT, U><<<dim3(grid), dim3(256), 0, st>>>(g, u, (uint32_t)(K / 8), ldg, ldu, q, ldq, s, lds,
+    swiglu_quant_rows_kernel<DT, U, ROUNDED><<<dim3(grid), dim3(256), 0, st>>>(g, u, (uint32_t)(K / 8), ldg, ldu, q, ldq, s, lds,
                                                                       total, pack);
     MX_LAUNCH_CHECK();
     return MX_OK;
@@ -1283,8 +1290,8 @@ extern "C" int mx_swiglu_quantize_rows(const void *gate, const void *up, int dty
         return MX_EUNSUPPORTED;
     hipStream_t st = (hipStream_t)stream;
     if (mx::stream_is_capturing(st)) return MX_ECAPTURE;
-    return dtype == MX_BF16 ? launch_swiglu<MX_BF16>(gate, up, M, K, ldg, ldu, q, ldq, s, lds, st)
-                            : launch_swiglu<MX_FP16>(gate, up, M, K, ldg, ldu, q, ldq, s, lds, st);
+    return dtype == MX_BF16 ? launch_swiglu<MX_BF16, false>(gate, up, M, K, ldg, ldu, q, ldq, s, lds, st)
+                            : launch_swiglu<MX_FP16, false>(gate, up, M, K, ldg, ldu, q, ldq, s, lds, st);
 }
 
 template <int DT, bool ROUNDED>
@@ -1365,7 +1372,10 @@ extern "C" int mx_swiglu_bwd_quantize_dual(const void *dh, int64_t lddh, const v
 }
 
 // ------------------------------------------------------------------------------------
-// The activation quantizers of a training step: any row count, token-axis operand in whole 128-token panels.
+// The activation quantizers of a training step: any row count, token-axis operand in whole 128-token panels.  Without a
+// token-axis operand (qT and sT null: a forward nobody will differentiate, or frozen weights) they are the row kernels:
+// half the bytes and no transposition.  us both axes / rows: 8 x 2048 6.4 / 2.4, 1500 x 1536 8.4 / 3.6, SwiGLU of 1500 x 4096
+// 11.6 / 6.5.
 // ------------------------------------------------------------------------------------
 
 static bool token_extent_ok(int64_t M, int64_t MT) { return M > 0 && MT >= M && MT % QC_TILE == 0; }
@@ -1373,9 +1383,24 @@ static bool token_extent_ok(int64_t M, int64_t MT) { return M > 0 && MT >= M && 
 extern "C" int mx_quantize_tokens(const void *x, int x_dtype, int cast_dtype, int64_t M, int64_t KV, int64_t ldx, int64_t MT,
                                   int64_t K, uint8_t *q, int64_t ldq, uint8_t *s, int64_t lds, uint8_t *qT, uint8_t *sT,
                                   int64_t ldsT, void *stream) {
-    if (!token_extent_ok(M, MT) || KV <= 0 || KV > K || K % MX_BLOCK || !x || !q || !s || !qT || !sT || ldx < KV || ldq < K ||
-        lds < K / MX_BLOCK || ldsT < MT / MX_BLOCK || (cast_dtype != x_dtype && x_dtype != MX_FP32))
+    const bool rows_only = !qT && !sT;
+    if (!token_extent_ok(M, MT) || KV <= 0 || KV > K || K % MX_BLOCK || !x || !q || !s || (!rows_only && (!qT || !sT)) || ldx < KV ||
+        ldq < K || lds < K / MX_BLOCK || (!rows_only && ldsT < MT / MX_BLOCK) || (cast_dtype != x_dtype && x_dtype != MX_FP32))
         return MX_EINVAL;
+    if (rows_only) {
+        if (KV != K || M * (K / 8) >= (int64_t)0x7FFFFF00) return MX_EUNSUPPORTED;
+        hipStream_t st = (hipStream_t)stream;
+        if (mx::stream_is_capturing(st)) return MX_ECAPTURE;
+        switch (x_dtype) {
+        case MX_BF16: return launch_rows<MX_BF16>(x, M, K, ldx, 1, q, ldq, s, lds, st);
+        case MX_FP16: return launch_rows<MX_FP16>(x, M, K, ldx, 1, q, ldq, s, lds, st);
+        case MX_FP32:
+            return cast_dtype == MX_BF16   ? launch_rows<MX_FP32, MX_BF16>(x, M, K, ldx, 1, q, ldq, s, lds, st)
+                   : cast_dtype == MX_FP16 ? launch_rows<MX_FP32, MX_FP16>(x, M, K, ldx, 1, q, ldq, s, lds, st)
+                                           : launch_rows<MX_FP32>(x, M, K, ldx, 1, q, ldq, s, lds, st);
+        default: return MX_EINVAL;
+        }
+    }
     if (KV % 8 || !cols_vec_ok(x, x_dtype, K, ldx, qT, 128) || !aligned(q, 8) || ldq % 8) return MX_EUNSUPPORTED;
     hipStream_t st = (hipStream_t)stream;
     if (mx::stream_is_capturing(st)) return MX_ECAPTURE;
@@ -1391,9 +1416,23 @@ extern "C" int mx_quantize_tokens(const void *x, int x_dtype, int cast_dtype, in
 extern "C" int mx_swiglu_quantize_tokens(const void *gu, int dtype, int rounded, int64_t M, int64_t H, int64_t ldgu, int64_t MT,
                                          uint8_t *q, int64_t ldq, uint8_t *s, int64_t lds, uint8_t *qT, uint8_t *sT,
                                          int64_t ldsT, void *stream) {
-    if (!token_extent_ok(M, MT) || H <= 0 || H % MX_BLOCK || !gu || !q || !s || !qT || !sT || ldgu < 2 * H || ldq < H ||
-        lds < H / MX_BLOCK || ldsT < MT / MX_BLOCK)
+    const bool rows_only = !qT && !sT;
+    if (!token_extent_ok(M, MT) || H <= 0 || H % MX_BLOCK || !gu || !q || !s || (!rows_only && (!qT || !sT)) || ldgu < 2 * H ||
+        ldq < H || lds < H / MX_BLOCK || (!rows_only && ldsT < MT / MX_BLOCK))
         return MX_EINVAL;
+    if (rows_only) {
+        const uint8_t *const up = (const uint8_t *)gu + H * 2;
+        if ((dtype != MX_BF16 && dtype != MX_FP16) || !aligned(gu, 16) || (ldgu * 2) % 16 || !aligned(q, 8) || ldq % 8 ||
+            M * (H / 8) >= (int64_t)0x7FFFFF00)
+            return MX_EUNSUPPORTED;
+        hipStream_t st = (hipStream_t)stream;
+        if (mx::stream_is_capturing(st)) return MX_ECAPTURE;
+        if (dtype == MX_BF16)
+            return rounded ? launch_swiglu<MX_BF16, true>(gu, up, M, H, ldgu, ldgu, q, ldq, s, lds, st)
+                           : launch_swiglu<MX_BF16, false>(gu, up, M, H, ldgu, ldgu, q, ldq, s, lds, st);
+        return rounded ? launch_swiglu<MX_FP16, true>(gu, up, M, H, ldgu, ldgu, q, ldq, s, lds, st)
+                       : launch_swiglu<MX_FP16, false>(gu, up, M, H, ldgu, ldgu, q, ldq, s, lds, st);
+    }
     if ((dtype != MX_BF16 && dtype != MX_FP16) || !aligned(gu, 16) || (ldgu * 2) % 16 || !aligned(q, 8) || ldq % 8 || !aligned(qT, 16))
         return MX_EUNSUPPORTED;
     dim3 grid;

@@ -29,6 +29,7 @@ from kohakuwullm_amd.kernels.mxfp8.quantize import (
     quantize_mx_dual,
     quantize_tokens,
     stage_major_ok,
+    token_axis_buffers,
     token_extent,
 )
 
@@ -134,21 +135,20 @@ def fused_swiglu_projection(xq, xs, wq, ws, out_dtype):
     return gu, hq, hs, htq, hts
 
 
-def swiglu_tokens(gu: torch.Tensor, rounded: bool = False):
+def swiglu_tokens(gu: torch.Tensor, rounded: bool = False, token_axis: bool = True):
     """``h = silu(gu[:, :H]) * gu[:, H:]`` as ``(q, s, qT, sT)`` for any token count (see :func:`quantize_tokens`).
 
     ``rounded``: ``silu`` and the product each rounded to the type of ``gu``, the arithmetic of the unfused activation.
+    Without ``token_axis`` ``qT`` and ``sT`` are not made and come back as ``None``.
     """
     m, h, dev = gu.shape[0], gu.shape[1] // 2, gu.device
-    mt = token_extent(m)
     q = torch.empty(m, h, device=dev, dtype=_FP8)
     s = torch.empty(m, h // BLOCK_SCALE, device=dev, dtype=torch.uint8)
-    qt = torch.empty(mt // PANEL, h, PANEL, device=dev, dtype=_FP8)
-    st = torch.empty(h, mt // BLOCK_SCALE, device=dev, dtype=torch.uint8)
+    qt, st, out_t = token_axis_buffers(m, h, dev, token_axis)
     _lib.invoke(
-        "mx_swiglu_quantize_tokens", m * h * (2 * gu.element_size() + 2 * (1 + 1 / BLOCK_SCALE)), gu,
-        gu.data_ptr(), _lib.MX_DTYPE[gu.dtype], int(rounded), m, h, gu.stride(0), mt, q.data_ptr(), h, s.data_ptr(),
-        h // BLOCK_SCALE, qt.data_ptr(), st.data_ptr(), mt // BLOCK_SCALE,
+        "mx_swiglu_quantize_tokens", m * h * (2 * gu.element_size() + (1 if qt is None else 2) * (1 + 1 / BLOCK_SCALE)), gu,
+        gu.data_ptr(), _lib.MX_DTYPE[gu.dtype], int(rounded), m, h, gu.stride(0), token_extent(m), q.data_ptr(), h,
+        s.data_ptr(), h // BLOCK_SCALE, *out_t,
     )
     return q, s, qt, st
 
@@ -171,7 +171,7 @@ def swiglu_bwd_tokens(dh: torch.Tensor, gu: torch.Tensor, rounded: bool = False)
 
 class _MXFP8SwiGLUMLP(torch.autograd.Function):
     @staticmethod
-    def forward(ctx, x, w_in, w_out, in_f, in_d, out_f, out_d, rounded):
+    def forward(ctx, x, w_in, w_out, in_f, in_d, out_f, out_d, rounded, differentiable):
         compute = compute_dtype(x)
         shape = x.shape
         x2d = activation_matrix(x, compute)
@@ -180,14 +180,15 @@ class _MXFP8SwiGLUMLP(torch.autograd.Function):
         # products, which contract over thousands of tokens, is then one contiguous run.  A hidden width that is not
         # whole panels keeps the row-major kernels, which take whole 32-token blocks: zero rows change no gradient.
         sm = stage_major_ok(w_out.shape[1]) and tokens > 0
-        xq, xs, xtq, xts = quantize_tokens(x2d, compute) if sm else quantize_mx_dual(pad_tokens(x2d.to(compute)))
+        wgrad_in, wgrad_out = (need and differentiable for need in ctx.needs_input_grad[1:3])
+        xq, xs, xtq, xts = quantize_tokens(x2d, compute, token_axis=wgrad_in) if sm else quantize_mx_dual(pad_tokens(x2d.to(compute)))
         # GEMM, then one bandwidth-bound pass for SwiGLU and both casts: measured faster at the
         # benchmark shape (220 + 89 us) than the same work in the GEMM's epilogue
         # (fused_swiglu_projection: 329 us), whose vector ALU work cannot overlap the MFMAs.
         gu = mxfp8_matmul_pq(xq, xs, *in_f, compute, out_pad=_PITCH_PAD)
-        hq, hs, htq, hts = swiglu_tokens(gu, rounded) if sm else swiglu_mx_dual(gu)
+        hq, hs, htq, hts = swiglu_tokens(gu, rounded, wgrad_out) if sm else swiglu_mx_dual(gu)
         y = mxfp8_matmul_pq(hq, hs, *out_f, compute)
-        if any(ctx.needs_input_grad):
+        if differentiable and any(ctx.needs_input_grad):
             ctx.save_for_backward(xtq, xts, gu, htq, hts, *in_d, *out_d)
             ctx.compute = compute
             ctx.x_dtype = x.dtype
@@ -202,7 +203,7 @@ class _MXFP8SwiGLUMLP(torch.autograd.Function):
         d2d = activation_matrix(dout, ctx.compute)
         tokens = d2d.shape[0]
         if ctx.stage_major:
-            dq, ds, dtq, dts = quantize_tokens(d2d, ctx.compute)
+            dq, ds, dtq, dts = quantize_tokens(d2d, ctx.compute, token_axis=ctx.needs_input_grad[2])
         else:
             dq, ds, dtq, dts = quantize_mx_dual(pad_tokens(d2d.to(ctx.compute)))
         dh = mxfp8_matmul_pq(dq, ds, wout_dq, wout_ds, ctx.compute, out_pad=_PITCH_PAD)
@@ -214,7 +215,7 @@ class _MXFP8SwiGLUMLP(torch.autograd.Function):
         dx, dw_in, dw_out = products_by_dtype(wanted, ctx.needs_input_grad)
         if dx is not None:
             dx = dx[:tokens].reshape(*shape[:-1], dx.shape[-1])
-        return dx, dw_in, dw_out, None, None, None, None, None
+        return dx, dw_in, dw_out, None, None, None, None, None, None
 
 
 def mxfp8_swiglu_mlp(x, w_in, w_out, packed) -> torch.Tensor:
@@ -227,7 +228,7 @@ def mxfp8_swiglu_mlp(x, w_in, w_out, packed) -> torch.Tensor:
     """
     if w_in.shape[0] != 2 * w_out.shape[1] or w_in.shape[1] != x.shape[-1] or w_out.shape[0] != x.shape[-1]:
         raise ValueError(f"shape mismatch: x {tuple(x.shape)}, w_in {tuple(w_in.shape)}, w_out {tuple(w_out.shape)}")
-    return _MXFP8SwiGLUMLP.apply(x, w_in, w_out, *packed, False)
+    return _MXFP8SwiGLUMLP.apply(x, w_in, w_out, *packed, False, torch.is_grad_enabled())
 
 
 def mxfp8_swiglu_pair(x, w_in, w_out) -> torch.Tensor | None:
@@ -249,4 +250,5 @@ def mxfp8_swiglu_pair(x, w_in, w_out) -> torch.Tensor | None:
         if lin._cache is None:
             lin.refresh_quantized_weight()
     (in_f, in_d), (out_f, out_d) = ((lin._cache[:2], lin._cache[2:]) for lin in (w_in, w_out))
-    return _MXFP8SwiGLUMLP.apply(x, w_in.weight, w_out.weight, in_f, in_d, out_f, out_d, True)
+    return _MXFP8SwiGLUMLP.apply(x, w_in.weight, w_out.weight, in_f, in_d, out_f, out_d, True,
+                                 torch.is_grad_enabled())

@@ -147,26 +147,42 @@ def activation_matrix(x: torch.Tensor, compute: torch.dtype) -> torch.Tensor:
     return x2d
 
 
-def quantize_tokens(x: torch.Tensor, compute: torch.dtype, cols: int | None = None):
+ROW_CHUNKS = 0x7FFFFF00  # 8-element chunks one launch of the row quantizers covers
+
+
+def token_axis_buffers(rows: int, cols: int, device, wanted: bool):
+    """``(qT, sT, (pointers and pitch for the library))`` of a token-axis operand over ``rows`` tokens; not ``wanted``: none.
+
+    A matrix past the row quantizers' range gets one all the same: the tile quantizers take any size.
+    """
+    if not wanted and rows * cols // 8 < ROW_CHUNKS:
+        return None, None, (None, None, 0)
+    mt = token_extent(rows)
+    qt = torch.empty(mt // PANEL, cols, PANEL, device=device, dtype=_FP8)
+    st = torch.empty(cols, mt // BLOCK_SCALE, device=device, dtype=torch.uint8)
+    return qt, st, (qt.data_ptr(), st.data_ptr(), mt // BLOCK_SCALE)
+
+
+def quantize_tokens(x: torch.Tensor, compute: torch.dtype, cols: int | None = None, token_axis: bool = True):
     """Both operands an activation ``x (M, KV)`` of any row count gives a training step, in one pass over it.
 
     Returns ``(q, s, qT, sT)``: ``q (M, K)``, ``s (M, K//32)`` along the columns and, along the tokens,
     ``qT (MT//128, K, 128)`` (stage-major), ``sT (K, MT//32)`` with ``MT = token_extent(M)``.  ``K = cols`` or the width of
     ``x``; rows and columns past ``x`` are zero, which adds nothing to a product.  fp32 values are rounded to ``compute``
     first.  Same bytes as casting, padding with zeros and :func:`quantize_mx_dual`.  ``x`` as :func:`activation_matrix`
-    returns it, its width a multiple of 8, ``K`` a multiple of 32.
+    returns it, its width a multiple of 8, ``K`` a multiple of 32.  Without ``token_axis`` (``K`` the width of ``x``)
+    ``qT`` and ``sT`` are not made and come back as ``None``.
     """
     _check_2d(x, "x")
     m, kv = x.shape
-    k, mt = cols or kv, token_extent(m)
+    k = cols or kv
     q = torch.empty(m, k, device=x.device, dtype=_FP8)
     s = torch.empty(m, k // BLOCK_SCALE, device=x.device, dtype=torch.uint8)
-    qt = torch.empty(mt // PANEL, k, PANEL, device=x.device, dtype=_FP8)
-    st = torch.empty(k, mt // BLOCK_SCALE, device=x.device, dtype=torch.uint8)
+    qt, st, out_t = token_axis_buffers(m, k, x.device, token_axis or k != kv)
     _lib.invoke(
-        "mx_quantize_tokens", m * kv * (x.element_size() + 2 * (1 + 1 / BLOCK_SCALE)), x,
-        x.data_ptr(), _lib.MX_DTYPE[x.dtype], _lib.MX_DTYPE[compute], m, kv, x.stride(0), mt, k,
-        q.data_ptr(), k, s.data_ptr(), k // BLOCK_SCALE, qt.data_ptr(), st.data_ptr(), mt // BLOCK_SCALE,
+        "mx_quantize_tokens", m * kv * (x.element_size() + (1 if qt is None else 2) * (1 + 1 / BLOCK_SCALE)), x,
+        x.data_ptr(), _lib.MX_DTYPE[x.dtype], _lib.MX_DTYPE[compute], m, kv, x.stride(0), token_extent(m), k,
+        q.data_ptr(), k, s.data_ptr(), k // BLOCK_SCALE, *out_t,
     )
     return q, s, qt, st
 

@@ -87,3 +87,18 @@ def test_who_runs_layer_by_layer():
     # another activation, a projection of its own kind
     block.act = F.gelu
     assert block(x.bfloat16()).isfinite().all() and not torch.equal(block(x.bfloat16()), pair(x.bfloat16()))
+
+
+def test_forward_alone_is_the_training_forward():
+    """Without gradients only the row-axis operands are made; the result is the training forward's, bit for bit."""
+    from kohakuwullm_amd.kernels.mxfp8.linear import MXFP8Linear
+    from kohakuwullm_amd.models.mlp import MXFP8SwiGLU
+
+    for module in (_block(BF), MXFP8Linear(256, 200).to(DEV), MXFP8SwiGLU(256, hidden=384).to(DEV)):
+        for x, autocast in ((torch.randn(77, 256, device=DEV).to(BF), False), (torch.randn(77, 256, device=DEV), True)):
+            with torch.autocast("cuda", dtype=BF, enabled=autocast):
+                want = module(x.requires_grad_(True)).detach()
+                with torch.no_grad():
+                    assert torch.equal(module(x), want)
+                with torch.inference_mode():
+                    assert torch.equal(module(x), want)

@@ -32,6 +32,10 @@ def test_quantize_tokens(oracle, m, kv, k, dtype, compute):
     q, s, qt, st = quantize_tokens(activation_matrix(x.to(DEV), compute), compute, k)
     mt = token_extent(m)
     assert mt % 128 == 0 and m <= mt < m + 128 + m / 16 + 128 and qt.shape == (mt // 128, k, 128) and st.shape == (k, mt // 32)
+    if k == kv:  # the row axis alone, from a pitched view too
+        for src in (x.to(DEV), F.pad(x, (0, 16)).to(DEV)[:, :kv]):
+            q1, s1, qt1, st1 = quantize_tokens(activation_matrix(src, compute), compute, token_axis=False)
+            assert qt1 is None and st1 is None and torch.equal(_u8(q1), _u8(q)) and torch.equal(s1, s)
     padded = F.pad(x.to(compute), (0, k - kv, 0, mt - m))
     rq, rs = oracle.quantize_rows(padded[:m])
     cq, cs = oracle.quantize_cols(padded)
@@ -53,6 +57,9 @@ def test_swiglu_tokens(oracle, m, h, dtype):
         q = got[0] if got[0].dim() == 2 else rows_of_stage_major(got[0])
         assert torch.equal(_u8(q), _u8(want[0][:m])) and torch.equal(got[1], want[1][:m])
         assert torch.equal(_u8(rows_of_stage_major(got[2])), _u8(want[2])) and torch.equal(got[3], want[3])
+    for rounded in (False, True):
+        both, one = swiglu_tokens(gu.to(DEV), rounded), swiglu_tokens(gu.to(DEV), rounded, token_axis=False)
+        assert torch.equal(_u8(one[0]), _u8(both[0])) and torch.equal(one[1], both[1]) and one[2] is None and one[3] is None
 
     gc = gu.clone().requires_grad_(True)
     gate, up = gc.chunk(2, dim=-1)
