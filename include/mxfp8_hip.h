@@ -176,6 +176,26 @@ int mx_quantize_tokens(const void *x, int x_dtype, int cast_dtype, int64_t M, in
                        uint8_t *q, int64_t ldq, uint8_t *s, int64_t lds, uint8_t *qT, uint8_t *sT, int64_t ldsT, void *stream);
 
 /*
+ * mx_quantize_tokens of the (M, sum of K_j) matrix that 1 to 8 16-bit matrices of M rows form side by side, without putting it
+ * together: (q, s) (M, sum K_j), (qT, sT) (sum K_j, MT) with qT stage-major.  Every K_j % 128 == 0, 16-byte aligned rows.
+ * mx_join_codes copies quantized matrices (rows, K_j) together in the same way: codes (rows, sum K_j), scales alike; 16-byte
+ * aligned code rows, 4-byte aligned scale rows.  For projections that share an input: dX = [dY_0 dY_1 ..] . [W_0; W_1; ..] is
+ * one product, so is the stack of their dW.
+ */
+typedef struct {
+    const void *x;
+    int64_t K, ldx;
+} mx_side_source;
+int mx_quantize_tokens_side(const mx_side_source *sources, int count, int x_dtype, int64_t M, int64_t MT, uint8_t *q, int64_t ldq,
+                            uint8_t *s, int64_t lds, uint8_t *qT, uint8_t *sT, int64_t ldsT, void *stream);
+typedef struct {
+    const uint8_t *codes, *scales;
+    int64_t K, ld, lds;
+} mx_code_source;
+int mx_join_codes(const mx_code_source *sources, int count, int64_t rows, uint8_t *codes, int64_t ld, uint8_t *scales, int64_t lds,
+                  void *stream);
+
+/*
  * mx_swiglu_quantize_dual and mx_swiglu_bwd_quantize_dual in the same form: M rows of gu (and dh), token-axis operands of MT
  * tokens stage-major, (q, s) for the M rows (the backward's q stage-major when ldq == 128 and H % 128 == 0).
  * rounded != 0: the arithmetic of the unfused 16-bit activation and its gradient -- silu(g), h, dh u, dh silu(g) and dgate

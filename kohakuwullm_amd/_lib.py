@@ -38,6 +38,8 @@ SIGNATURES = {
     "mx_swiglu_bwd_quantize_dual": (
         _ci, [_p, _i64, _p, _i64, _ci, _i64, _i64, _p, _i64, _p, _i64, _p, _i64, _p, _i64, _p]),
     "mx_quantize_tokens": (_ci, [_p, _ci, _ci, _i64, _i64, _i64, _i64, _i64, _p, _i64, _p, _i64, _p, _p, _i64, _p]),
+    "mx_quantize_tokens_side": (_ci, [_p, _ci, _ci, _i64, _i64, _p, _i64, _p, _i64, _p, _p, _i64, _p]),
+    "mx_join_codes": (_ci, [_p, _ci, _i64, _p, _i64, _p, _i64, _p]),
     "mx_swiglu_quantize_tokens": (_ci, [_p, _ci, _ci, _i64, _i64, _i64, _i64, _p, _i64, _p, _i64, _p, _p, _i64, _p]),
     "mx_swiglu_bwd_quantize_tokens": (
         _ci, [_p, _i64, _p, _i64, _ci, _ci, _i64, _i64, _i64, _p, _i64, _p, _i64, _p, _p, _i64, _p]),
@@ -102,6 +104,18 @@ class QuantProblem(ctypes.Structure):
     _fields_ = [(n, _p) for n in ("x", "q", "s", "qT", "sT")] + [
         (n, _i64) for n in ("M", "K", "ldx", "ldq", "lds", "ldqT", "ldsT")
     ]
+
+
+class SideSource(ctypes.Structure):
+    """``mx_side_source`` of the C header."""
+
+    _fields_ = [("x", _p), ("K", _i64), ("ldx", _i64)]
+
+
+class CodeSource(ctypes.Structure):
+    """``mx_code_source`` of the C header."""
+
+    _fields_ = [("codes", _p), ("scales", _p), ("K", _i64), ("ld", _i64), ("lds", _i64)]
 
 
 _lib: ctypes.CDLL | None = None

@@ -506,6 +506,66 @@ __global__ __launch_bounds__(256) void quant_cols_kernel(const void *__restrict_
     quant_tile<DUAL, R>(v, o, M, MT, K, m0, k0, tile, tscale);
 }
 
+// Several matrices of the same rows quantized as the column panels of one (M, K) matrix: what the gradients of projections
+// that share an input are to the products of their backward, which contract over (or have rows for) all of them together.
+// HBM-bound like quant_cols_kernel, whose tiles these are (every width is a multiple of 128, so a tile has one source);
+// 32768 x (2048 + 512 + 512): 77 us in one launch against 53 + 18 + 17 in three.
+#define MX_SIDE_MAX 8
+struct SideArgs {
+    const void *x[MX_SIDE_MAX];
+    int64_t ldx[MX_SIDE_MAX];
+    int tile_end[MX_SIDE_MAX];  // column tiles of sources 0..j
+    int count;
+};
+
+template <int DT, bool EDGE, bool RAW>
+__global__ __launch_bounds__(256) void quant_side_kernel(SideArgs a, int64_t M, int64_t MT, int64_t K, QuantTileOut o) {
+    typedef TileGeom<8> G;
+    typedef typename Elem<DT>::type T;
+    __shared__ __attribute__((aligned(16))) uint8_t tile[G::TK * QC_PITCH];
+    __shared__ __attribute__((aligned(4))) uint8_t tscale[G::TK * 4];
+    const int t = threadIdx.x;
+    int j = 0;
+    while (j + 1 < a.count && (int)blockIdx.x >= a.tile_end[j]) j++;
+    const int64_t m0 = (int64_t)blockIdx.y * QC_TILE, k0 = (int64_t)blockIdx.x * G::TK;
+    const int64_t col = k0 - (int64_t)(j ? a.tile_end[j - 1] : 0) * G::TK + G::cg(t) * 8;
+    const int64_t row0 = m0 + G::rg(t) * 8;
+    typename Elem<DT>::raw r[8];
+    load_rows_or_zero<DT, 8, true, EDGE>(a.x[j], row0 * a.ldx[j] + col, a.ldx[j], M - row0, r);
+    if constexpr (RAW) {
+        quant_tile_raw<DT, true, false>(r, o, M, MT, K, m0, k0, tile, tscale);
+        return;
+    }
+    float v[8][8];
+#pragma unroll
+    for (int i = 0; i < 8; i++) Elem<DT>::unpack(r[i], v[i]);
+    quant_tile<true, 8>(v, o, M, MT, K, m0, k0, tile, tscale);
+}
+
+// Column panels of one code matrix (codes (rows, K), scale bytes (rows, K/32)) copied together from several: 16 codes per
+// thread, every eighth one the four scale bytes of 128 codes too.  Latency-bound at the sizes of weights: 2048 x (2048 + 512 +
+// 512) 6.9 us.
+struct JoinArgs {
+    const uint8_t *codes[MX_SIDE_MAX], *scales[MX_SIDE_MAX];
+    int64_t ld[MX_SIDE_MAX], lds[MX_SIDE_MAX];
+    int chunk_end[MX_SIDE_MAX];  // 16-code chunks of a row of sources 0..j
+    int count;
+};
+
+__global__ __launch_bounds__(256) void join_codes_kernel(JoinArgs a, uint32_t total, uint32_t chunks_per_row, uint8_t *__restrict__ codes,
+                                                          int64_t ld, uint8_t *__restrict__ scales, int64_t lds) {
+    const uint32_t id = blockIdx.x * 256u + threadIdx.x;
+    if (id >= total) return;
+    const uint32_t row = id / chunks_per_row;
+    const int chunk = (int)(id - row * chunks_per_row);
+    int j = 0;
+    while (j + 1 < a.count && chunk >= a.chunk_end[j]) j++;
+    const int from = chunk - (j ? a.chunk_end[j - 1] : 0);
+    *(v4i *)(codes + (int64_t)row * ld + (int64_t)chunk * 16) = *(const v4i *)(a.codes[j] + (int64_t)row * a.ld[j] + (int64_t)from * 16);
+    if (!(chunk & 7))
+        *(uint32_t *)(scales + (int64_t)row * lds + chunk / 2) = *(const uint32_t *)(a.scales[j] + (int64_t)row * a.lds[j] + from / 2);
+}
+
 // RMSNorm in front of both quantizers: y = (x * rstd[row]) * w[col] in fp32 -- the two products in the order
 // rmsnorm_quant_kernel forms them, so the row-axis pair equals that kernel's bit for bit -- then the tile quantizer.
 // rstd comes from a first pass over x (mx_rmsnorm_quantize asked for nothing else); the second read of an activation
@@ -1411,6 +1471,73 @@ extern "C" int mx_quantize_tokens(const void *x, int x_dtype, int cast_dtype, in
     case MX_FP32: return launch_cols<MX_FP32, true>(x, M, MT, KV, K, ldx, qT, 128, sT, ldsT, q, ldq, s, lds, st, ks, cast_dtype);
     default: return MX_EINVAL;
     }
+}
+
+template <int DT>
+static int launch_side(const SideArgs &a, int64_t M, int64_t MT, int64_t K, dim3 grid, const QuantTileOut &o, hipStream_t st) {
+    const bool raw = (int64_t)grid.x * grid.y <= 8 * (int64_t)num_cus();  // as launch_cols
+    const dim3 block(256);
+    if (M != MT) {
+        if (raw) quant_side_kernel<DT, true, true><<<grid, block, 0, st>>>(a, M, MT, K, o);
+        else quant_side_kernel<DT, true, false><<<grid, block, 0, st>>>(a, M, MT, K, o);
+    } else {
+        if (raw) quant_side_kernel<DT, false, true><<<grid, block, 0, st>>>(a, M, MT, K, o);
+        else quant_side_kernel<DT, false, false><<<grid, block, 0, st>>>(a, M, MT, K, o);
+    }
+    MX_LAUNCH_CHECK();
+    return MX_OK;
+}
+
+extern "C" int mx_quantize_tokens_side(const mx_side_source *sources, int count, int x_dtype, int64_t M, int64_t MT, uint8_t *q,
+                                       int64_t ldq, uint8_t *s, int64_t lds, uint8_t *qT, uint8_t *sT, int64_t ldsT, void *stream) {
+    if (count < 1 || count > MX_SIDE_MAX || !sources || !token_extent_ok(M, MT) || !q || !s || !qT || !sT || ldsT < MT / MX_BLOCK ||
+        (x_dtype != MX_BF16 && x_dtype != MX_FP16))
+        return MX_EINVAL;
+    SideArgs a;
+    int64_t tiles = 0;
+    bool vec = aligned(q, 16) && ldq % 16 == 0 && aligned(qT, 16);
+    for (int j = 0; j < count; j++) {
+        const mx_side_source &p = sources[j];
+        if (!p.x || p.K <= 0 || p.K % QC_TILE || p.ldx < p.K) return MX_EINVAL;
+        tiles += p.K / QC_TILE;
+        if (tiles > 0x7FFFFF) return MX_EUNSUPPORTED;
+        vec = vec && aligned(p.x, 16) && p.ldx % 8 == 0;
+        a.x[j] = p.x, a.ldx[j] = p.ldx, a.tile_end[j] = (int)tiles;
+    }
+    a.count = count;
+    const int64_t K = tiles * QC_TILE;
+    if (ldq < K || lds < K / MX_BLOCK) return MX_EINVAL;
+    dim3 grid;
+    if (!vec || !tile_grid<8>(MT, K, grid)) return MX_EUNSUPPORTED;
+    hipStream_t st = (hipStream_t)stream;
+    if (mx::stream_is_capturing(st)) return MX_ECAPTURE;
+    const QuantTileOut o = tile_out(qT, 128, sT, ldsT, q, ldq, s, lds, 0, K * 128);
+    return x_dtype == MX_BF16 ? launch_side<MX_BF16>(a, M, MT, K, grid, o, st) : launch_side<MX_FP16>(a, M, MT, K, grid, o, st);
+}
+
+extern "C" int mx_join_codes(const mx_code_source *sources, int count, int64_t rows, uint8_t *codes, int64_t ld, uint8_t *scales,
+                             int64_t lds, void *stream) {
+    if (count < 1 || count > MX_SIDE_MAX || !sources || rows <= 0 || !codes || !scales) return MX_EINVAL;
+    JoinArgs a;
+    int64_t chunks = 0;
+    bool vec = aligned(codes, 16) && ld % 16 == 0 && aligned(scales, 4) && lds % 4 == 0;
+    for (int j = 0; j < count; j++) {
+        const mx_code_source &p = sources[j];
+        if (!p.codes || !p.scales || p.K <= 0 || p.K % 128 || p.ld < p.K || p.lds < p.K / MX_BLOCK) return MX_EINVAL;
+        chunks += p.K / 16;
+        if (chunks * rows >= (int64_t)0x7FFFFF00) return MX_EUNSUPPORTED;
+        vec = vec && aligned(p.codes, 16) && p.ld % 16 == 0 && aligned(p.scales, 4) && p.lds % 4 == 0;
+        a.codes[j] = p.codes, a.scales[j] = p.scales, a.ld[j] = p.ld, a.lds[j] = p.lds, a.chunk_end[j] = (int)chunks;
+    }
+    a.count = count;
+    if (ld < chunks * 16 || lds < chunks / 2) return MX_EINVAL;
+    if (!vec) return MX_EUNSUPPORTED;
+    hipStream_t st = (hipStream_t)stream;
+    if (mx::stream_is_capturing(st)) return MX_ECAPTURE;
+    const uint32_t total = (uint32_t)(chunks * rows);
+    join_codes_kernel<<<dim3((total + 255) / 256), dim3(256), 0, st>>>(a, total, (uint32_t)chunks, codes, ld, scales, lds);
+    MX_LAUNCH_CHECK();
+    return MX_OK;
 }
 
 extern "C" int mx_swiglu_quantize_tokens(const void *gu, int dtype, int rounded, int64_t M, int64_t H, int64_t ldgu, int64_t MT,

@@ -19,7 +19,7 @@ import torch
 import torch.nn.functional as F
 
 from kohakuwullm_amd import _lib
-from kohakuwullm_amd.kernels.mxfp8.linear import compute_dtype, gradient_dtype, unobserved
+from kohakuwullm_amd.kernels.mxfp8.linear import TENSORS, compute_dtype, gradient_dtype, unobserved
 from kohakuwullm_amd.kernels.mxfp8.quantize import (
     BLOCK_SCALE,
     PANEL,
@@ -34,7 +34,6 @@ from kohakuwullm_amd.kernels.mxfp8.quantize import (
 )
 
 _FP8 = torch.float8_e4m3fn
-_TENSORS = (torch.Tensor, torch.nn.Parameter)  # a subclass dispatches each operator itself
 
 # The two projection outputs that only the SwiGLU quantizers read (`gu`, `dh`) are allocated with 128 spare
 # elements per row.  Their natural pitches (16 KiB and 8 KiB at the benchmark shape) put the 128 rows a quantizer
@@ -239,7 +238,7 @@ def mxfp8_swiglu_pair(x, w_in, w_out) -> torch.Tensor | None:
     the SwiGLU quantizers do them on the way, with every intermediate rounded as those operators round it.  ``None`` for
     what this graph does not stand for: a layer someone watches (hooks), padded widths, a type other than bf16 / fp16.
     """
-    if not (unobserved(w_in) and unobserved(w_out)) or not x.is_cuda or not x.numel() or type(x) not in _TENSORS:
+    if not (unobserved(w_in) and unobserved(w_out)) or not x.is_cuda or not x.numel() or type(x) not in TENSORS:
         return None
     compute = compute_dtype(x)
     if compute not in (torch.bfloat16, torch.float16) or x.dtype not in _lib.MX_DTYPE or x.shape[-1] != w_in.in_features:

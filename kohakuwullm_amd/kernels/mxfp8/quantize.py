@@ -187,6 +187,37 @@ def quantize_tokens(x: torch.Tensor, compute: torch.dtype, cols: int | None = No
     return q, s, qt, st
 
 
+SIDE_MAX = 8  # matrices one side-by-side call takes
+
+
+def quantize_side(xs: list[torch.Tensor]):
+    """:func:`quantize_tokens` of ``torch.cat(xs, 1)`` for 16-bit matrices of one type, without the concatenation.
+
+    Every ``x`` as :func:`activation_matrix` returns it, its width a multiple of 128; at most ``SIDE_MAX`` of them.
+    """
+    m, k, device = xs[0].shape[0], sum(x.shape[1] for x in xs), xs[0].device
+    sources = (_lib.SideSource * len(xs))(*[(x.data_ptr(), x.shape[1], x.stride(0)) for x in xs])
+    q = torch.empty(m, k, device=device, dtype=_FP8)
+    s = torch.empty(m, k // BLOCK_SCALE, device=device, dtype=torch.uint8)
+    qt, st, out_t = token_axis_buffers(m, k, device, True)
+    _lib.invoke("mx_quantize_tokens_side", m * k * (2 + 2 * (1 + 1 / BLOCK_SCALE)), xs[0], ctypes.addressof(sources), len(xs),
+                _lib.MX_DTYPE[xs[0].dtype], m, token_extent(m), q.data_ptr(), k, s.data_ptr(), k // BLOCK_SCALE, *out_t)
+    return q, s, qt, st
+
+
+def join_codes(pairs):
+    """``(torch.cat(codes, 1), torch.cat(scales, 1))`` of quantized matrices of one height, widths multiples of 128."""
+    if len(pairs) == 1:
+        return pairs[0]
+    rows, k, device = pairs[0][0].shape[0], sum(c.shape[1] for c, _ in pairs), pairs[0][0].device
+    sources = (_lib.CodeSource * len(pairs))(*[(c.data_ptr(), s.data_ptr(), c.shape[1], c.stride(0), s.stride(0)) for c, s in pairs])
+    codes = torch.empty(rows, k, device=device, dtype=_FP8)
+    scales = torch.empty(rows, k // BLOCK_SCALE, device=device, dtype=torch.uint8)
+    _lib.invoke("mx_join_codes", 2 * rows * k * (1 + 1 / BLOCK_SCALE), codes, ctypes.addressof(sources), len(pairs), rows,
+                codes.data_ptr(), k, scales.data_ptr(), k // BLOCK_SCALE)
+    return codes, scales
+
+
 def quantize_mx_dual_batch(xs: list[torch.Tensor]) -> list[tuple[torch.Tensor, torch.Tensor, torch.Tensor, torch.Tensor]]:
     """``quantize_mx_dual`` of every matrix of ``xs`` behind one launch per 24 matrices.
 

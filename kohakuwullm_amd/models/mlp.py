@@ -14,6 +14,7 @@ import torch
 import torch.nn as nn
 import torch.nn.functional as F
 
+from kohakuwullm_amd.kernels.mxfp8.linear import mxfp8_linear_group
 from kohakuwullm_amd.kernels.mxfp8.mlp import mxfp8_swiglu_mlp, mxfp8_swiglu_pair
 from kohakuwullm_amd.kernels.mxfp8.quantize import quantize_mx, quantize_mx_cols
 from kohakuwullm_amd.models.mxfp8_swap import Matmul
@@ -143,10 +144,10 @@ class AttentionProjections(nn.Module):
 
     def project(self, x: torch.Tensor):
         lead = x.shape[:-1]
-        q = self.q_proj(x).view(*lead, self.num_heads, self.head_dim)
-        k = self.k_proj(x).view(*lead, self.num_kv_heads, self.head_dim)
-        v = self.v_proj(x).view(*lead, self.num_kv_heads, self.head_dim)
-        return q, k, v
+        layers = self.q_proj, self.k_proj, self.v_proj
+        q, k, v = mxfp8_linear_group(x, layers) or [layer(x) for layer in layers]
+        kv_shape = *lead, self.num_kv_heads, self.head_dim
+        return q.view(*lead, self.num_heads, self.head_dim), k.view(kv_shape), v.view(kv_shape)
 
     def merge(self, heads: torch.Tensor) -> torch.Tensor:
         return self.o_proj(heads.reshape(*heads.shape[:-2], self.num_heads * self.head_dim))
