@@ -513,6 +513,10 @@ int64_t mx_expert_sort_workspace(int64_t n, int64_t num_buckets);
 int mx_expert_sort(const void *flat_expert, int idx_bytes, int64_t n, const int32_t *counts, int64_t top_k,
                    int64_t num_buckets, int32_t *offsets, int32_t *order, int32_t *token_of, int32_t *max_rows,
                    int32_t *workspace, int64_t workspace_len, void *stream);
+/* ... and positions (n,), the inverse of order: pair index -> sorted position, -1 for a pair without one.  NULL: not wanted. */
+int mx_expert_sort_positions(const void *flat_expert, int idx_bytes, int64_t n, const int32_t *counts, int64_t top_k,
+                             int64_t num_buckets, int32_t *offsets, int32_t *order, int32_t *token_of, int32_t *max_rows,
+                             int32_t *positions, int32_t *workspace, int64_t workspace_len, void *stream);
 
 /*
  * mx_expert_sort for callers that can bring no workspace and must not allocate one: a tight serving loop

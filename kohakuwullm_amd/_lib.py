@@ -73,6 +73,7 @@ SIGNATURES = {
     "mx_expert_counts": (_ci, [_p, _ci, _i64, _i64, _p, _p]),
     "mx_expert_sort_workspace": (_i64, [_i64, _i64]),
     "mx_expert_sort": (_ci, [_p, _ci, _i64, _p, _i64, _i64, _p, _p, _p, _p, _p, _i64, _p]),
+    "mx_expert_sort_positions": (_ci, [_p, _ci, _i64, _p, _i64, _i64, _p, _p, _p, _p, _p, _p, _i64, _p]),
     "mx_expert_sort_static": (_ci, [_p, _ci, _i64, _p, _i64, _i64, _p, _p, _p, _p, _p]),
     "mx_combine_routed": (_ci, [_p, _ci, _i64, _p, _ci, _p, _p, _p, _i64, _i64, _i64, _i64, _p, _i64, _p]),
     "mx_combine_routed_backward": (

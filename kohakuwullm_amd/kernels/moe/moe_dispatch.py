@@ -58,6 +58,12 @@ def expert_sort(flat_expert: torch.Tensor, counts: torch.Tensor, top_k: int, num
         for the grouped GEMM, ``order`` sorted position -> pair index, ``token_of`` sorted
         position -> token index, ``max_rows`` a one-element diagnostic (largest count).
     """
+    return expert_sort_positions(flat_expert, counts, top_k, num_experts, False)[:4]
+
+
+def expert_sort_positions(flat_expert: torch.Tensor, counts: torch.Tensor, top_k: int, num_experts: int, positions: bool = True):
+    """:func:`expert_sort` with the inverse of ``order`` behind its results: ``positions (n,)``, pair index -> sorted position
+    (-1 for a pair without one).  The combines gather by it; written on the way it saves them a fill and a scatter."""
     flat_expert = _index_tensor(flat_expert, "flat_expert")
     _lib.require_gpu(counts, "counts")
     if counts.dtype != torch.int32 or counts.shape != (num_experts,):
@@ -74,11 +80,12 @@ def expert_sort(flat_expert: torch.Tensor, counts: torch.Tensor, top_k: int, num
     if need < 0:
         raise ValueError(f"expert_sort: {n} pairs in {num_experts} buckets is out of range")
     workspace = torch.empty(need, dtype=torch.int32, device=device)
-    _lib.invoke("mx_expert_sort", n * (flat_expert.element_size() + 8), flat_expert,
+    inverse = torch.empty(n, dtype=torch.int32, device=device) if positions else None
+    _lib.invoke("mx_expert_sort_positions", n * (flat_expert.element_size() + 8), flat_expert,
                 flat_expert.data_ptr(), _INDEX[flat_expert.dtype], n, counts.data_ptr(), top_k, num_experts,
                 offsets.data_ptr(), order.data_ptr(), token_of.data_ptr(), max_rows.data_ptr(),
-                workspace.data_ptr(), need)
-    return offsets, order, token_of, max_rows
+                inverse.data_ptr() if positions else None, workspace.data_ptr(), need)
+    return offsets, order, token_of, max_rows, inverse
 
 
 def expert_sort_into(flat_expert: torch.Tensor, counts: torch.Tensor, top_k: int, num_experts: int,

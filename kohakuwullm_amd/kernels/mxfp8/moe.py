@@ -201,18 +201,18 @@ def launch_gemm2_dgrad(dq, ds, token_of, order, gate, wq, ws, hq, hs, pre, dpre,
 
 class _MXFP8Experts(torch.autograd.Function):
     @staticmethod
-    def forward(ctx, x, w_in, w_out, gate, token_of, order, offsets, packed, hidden):
+    def forward(ctx, x, w_in, w_out, gate, token_of, order, offsets, packed, hidden, positions, differentiable):
         del w_in, w_out  # present so autograd routes dW to the master parameters
         rows, dim = x.shape
         m = token_of.numel()
-        # `ctx.needs_input_grad`, not `torch.is_grad_enabled()`: autograd runs forward under no_grad
-        needs_grad = any(ctx.needs_input_grad)
+        # the grad mode comes from the caller: in here it is always off, and `needs_input_grad` does not know it
+        needs_grad = differentiable and any(ctx.needs_input_grad)
         xq, xs = quantize_mx(x)  # once per token; the gather happens inside GEMM1
         hq = torch.empty(m, hidden, device=x.device, dtype=_FP8)
         hs = torch.empty(m, hidden // BLOCK_SCALE, device=x.device, dtype=torch.uint8)
         pre = torch.empty(m, 2 * hidden, device=x.device, dtype=x.dtype) if needs_grad else None
         htq = hts = None
-        if ctx.needs_input_grad[2]:
+        if differentiable and ctx.needs_input_grad[2]:
             # h along the tokens, for dW_out: written by GEMM1's epilogue instead of a pass over `pre`
             mpad = padded_rows(m, packed.in_fwd[0].shape[0])
             htq, hts = token_axis_buffers(hidden, mpad, x.device, TOKEN_AXIS_STAGE_MAJOR)
@@ -221,7 +221,7 @@ class _MXFP8Experts(torch.autograd.Function):
         top_k = gate.numel() // rows if rows and gate.numel() % rows == 0 else 0
         # the pair -> sorted position table of the combine serves the backward's combine too
         out, positions = _routed_product(hq, hs, *packed.out_fwd, token_of, order, gate, offsets, rows, top_k, x.dtype,
-                                         return_positions=True)
+                                         positions, return_positions=True)
         if needs_grad:
             ctx.positions = positions
             ctx.save_for_backward(x, hq, hs, pre, gate, token_of, order, offsets, htq, hts)
@@ -262,7 +262,7 @@ class _MXFP8Experts(torch.autograd.Function):
             # dW_in[e] = dpre rows of e .T @ x rows of e
             xtq, xts = quantize_mx_cols_grouped(x, offsets, m, index=token_of, stage_major=TOKEN_AXIS_STAGE_MAJOR)
             dw_in = grouped_mxfp8_wgrad(ptq, pts, xtq, xts, offsets, m, dout.dtype)
-        return dx, dw_in, dw_out, dgate.to(gate.dtype), None, None, None, None, None
+        return dx, dw_in, dw_out, dgate.to(gate.dtype), None, None, None, None, None, None, None
 
 
 def _validate_expert_call(x, w_in, w_out, token_of, order) -> int:
@@ -292,7 +292,8 @@ def _validate_expert_call(x, w_in, w_out, token_of, order) -> int:
     return hidden
 
 
-def mxfp8_moe_experts(x, w_in, w_out, gate, token_of, order, offsets, packed: MXFP8ExpertWeights) -> torch.Tensor:
+def mxfp8_moe_experts(x, w_in, w_out, gate, token_of, order, offsets, packed: MXFP8ExpertWeights,
+                      positions: torch.Tensor | None = None) -> torch.Tensor:
     """The whole routed-expert path in MXFP8: gather, SwiGLU MLP, gate, combine.
 
     Args:
@@ -305,9 +306,11 @@ def mxfp8_moe_experts(x, w_in, w_out, gate, token_of, order, offsets, packed: MX
         offsets: ``(E+1,)`` int32 exclusive prefix sum of per-expert row counts, truncated to the
             real experts, so a sentinel bucket's rows fall outside every tile.  Never read on the host.
         packed: the four quantized copies, refreshed after each optimizer step.
+        positions: ``(T*top_k,)`` int32, the inverse of ``order`` (pair index -> sorted position, -1 for none below
+            ``offsets[E]``); made from ``order`` when not given.
     """
     hidden = _validate_expert_call(x, w_in, w_out, token_of, order)
-    return _MXFP8Experts.apply(x, w_in, w_out, gate, token_of, order, offsets, packed, hidden)
+    return _MXFP8Experts.apply(x, w_in, w_out, gate, token_of, order, offsets, packed, hidden, positions, torch.is_grad_enabled())
 
 
 def mxfp8_moe_experts_reference(x, w_in, w_out, gate, token_of, order, offsets) -> torch.Tensor:

@@ -24,7 +24,7 @@ import torch
 import torch.nn as nn
 import torch.nn.functional as F
 
-from kohakuwullm_amd.kernels.moe.moe_dispatch import combine_routed, expert_counts, expert_sort
+from kohakuwullm_amd.kernels.moe.moe_dispatch import combine_routed, expert_counts, expert_sort, expert_sort_positions  # noqa: F401  (expert_sort: importable from here)
 from kohakuwullm_amd.kernels.moe.router import can_route, route_topk
 from kohakuwullm_amd.kernels.mxfp8.linear import compute_dtype
 from kohakuwullm_amd.kernels.mxfp8.moe import (
@@ -271,12 +271,12 @@ class MoEMLP(nn.Module):
         scaled = out_sorted[:real] * weight.index_select(0, order[:real].long()).unsqueeze(-1)
         return x.new_zeros(flat.shape[0], self.dim).index_add_(0, token_of[:real].long(), scaled)
 
-    def _routed_mxfp8(self, flat, topk_weight, order, token_of, offsets):
+    def _routed_mxfp8(self, flat, topk_weight, order, token_of, offsets, positions=None):
         if self._packed is None:
             self._refresh_mxfp8()
         x = flat.to(compute_dtype(flat))  # compute dtype follows autocast; the activation may arrive fp32
         return mxfp8_moe_experts(x, self.w_in, self.w_out, topk_weight.reshape(-1), token_of, order,
-                                 offsets[: self.num_experts + 1], self._packed)
+                                 offsets[: self.num_experts + 1], self._packed, positions)
 
     def _routed_mxfp8_unfused(self, flat, topk_weight, order, token_of, offsets):
         if self._packed is None:
@@ -292,8 +292,11 @@ class MoEMLP(nn.Module):
         seen_by_router = flat if route_on is None else route_on.reshape(-1, route_on.shape[-1])
         topk_idx, topk_weight, counts = self.router.route(seen_by_router)
         # slot width from the tensor, not top_k: a router may pad it
-        offsets, order, token_of, _ = expert_sort(topk_idx.reshape(-1), counts, topk_idx.shape[-1], self.num_buckets)
-        out = self._routed(flat, topk_weight, order, token_of, offsets)
+        # the fused path gathers by the inverse order, which covers the real experts alone: with a sentinel bucket it makes its own
+        inverse = self._routed == self._routed_mxfp8 and not self._has_sentinel
+        offsets, order, token_of, _, *positions = expert_sort_positions(topk_idx.reshape(-1), counts, topk_idx.shape[-1],
+                                                                        self.num_buckets, inverse)
+        out = self._routed(flat, topk_weight, order, token_of, offsets, *positions if inverse else ())
         if self.shared is not None:
             out = out + self.shared(flat)  # dtype by promotion, as the reference's forward (components/moe.py:395-449)
         return out.reshape(shape)

@@ -43,11 +43,12 @@ def test_expert_counts_skips_out_of_range_and_rejects_bad_input():
 
 
 @pytest.mark.parametrize("tokens,top_k,experts", [
-    (1, 1, 1), (7, 2, 3), (43, 3, 5), (96, 6, 64), (16384, 6, 64), (16384, 6, 65), (4096, 8, 1024), (300000, 6, 128),
+    (1, 1, 1), (7, 2, 3), (43, 3, 5), (96, 6, 64), (171, 6, 256), (512, 8, 64), (4097, 1, 64), (100, 4, 257), (16384, 6, 64), (16384, 6, 65), (4096, 8, 1024), (300000, 6, 128),
 ])
 @pytest.mark.parametrize("dtype", [torch.int64, torch.int32])
 def test_expert_sort_is_the_stable_sort(oracle, tokens, top_k, experts, dtype):
     from kohakuwullm_amd.kernels.moe import expert_counts, expert_sort
+    from kohakuwullm_amd.kernels.moe.moe_dispatch import expert_sort_positions
 
     flat = _picks(tokens, min(top_k, experts), experts, dtype=dtype)
     slots = flat.numel() // tokens
@@ -59,12 +60,14 @@ def test_expert_sort_is_the_stable_sort(oracle, tokens, top_k, experts, dtype):
     assert torch.equal(order.cpu(), ref_order)
     assert torch.equal(token_of.cpu(), ref_token)
     assert max_rows.item() == int(counts.max())
-    again = expert_sort(dev, counts, slots, experts)
+    again = expert_sort_positions(dev, counts, slots, experts)
     assert torch.equal(again[1], order) and torch.equal(again[2], token_of)
+    assert torch.equal(again[4].cpu(), torch.argsort(ref_order).to(torch.int32))
 
 
 def test_expert_sort_edge_cases(oracle):
     from kohakuwullm_amd.kernels.moe import expert_sort
+    from kohakuwullm_amd.kernels.moe.moe_dispatch import expert_sort_positions
 
     # no pairs at all
     counts = torch.zeros(4, dtype=torch.int32, device=DEV)
@@ -79,7 +82,11 @@ def test_expert_sort_edge_cases(oracle):
     # a sentinel bucket: picks of the padding slots land past the last real expert
     flat = torch.tensor([3, 0, 3, 1, 0, 3], dtype=torch.int64)
     counts = torch.tensor([2, 1, 0, 3], dtype=torch.int32, device=DEV)
-    offsets, order, token_of, _ = expert_sort(flat.to(DEV), counts, 2, 4)
+    offsets, order, token_of, _, positions = expert_sort_positions(flat.to(DEV), counts, 2, 4)
+    assert positions.tolist() == [3, 0, 4, 2, 1, 5]
+    outside = torch.tensor([3, 9, 3, -1, 0, 3], dtype=torch.int64, device=DEV)  # picks outside the buckets have no position
+    counts_in = torch.tensor([1, 0, 0, 3], dtype=torch.int32, device=DEV)
+    assert expert_sort_positions(outside, counts_in, 2, 4)[4].tolist() == [1, -1, 2, -1, 0, 3]
     assert offsets.tolist() == [0, 2, 3, 3, 6] and order.tolist() == [1, 4, 3, 0, 2, 5] and token_of.tolist() == [0, 2, 1, 0, 1, 2]
     # a histogram that overstates the picks points past the end: those positions are dropped, not written
     flat = _picks(512, 2, 8)
