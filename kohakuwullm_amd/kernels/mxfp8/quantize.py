@@ -196,7 +196,7 @@ def quantize_side(xs: list[torch.Tensor]):
     Every ``x`` as :func:`activation_matrix` returns it, its width a multiple of 128; at most ``SIDE_MAX`` of them.
     """
     m, k, device = xs[0].shape[0], sum(x.shape[1] for x in xs), xs[0].device
-    sources = (_lib.SideSource * len(xs))(*[(x.data_ptr(), x.shape[1], x.stride(0)) for x in xs])
+    sources = _lib.words([(x.data_ptr(), x.shape[1], x.stride(0)) for x in xs])  # mx_side_source each
     q = torch.empty(m, k, device=device, dtype=_FP8)
     s = torch.empty(m, k // BLOCK_SCALE, device=device, dtype=torch.uint8)
     qt, st, out_t = token_axis_buffers(m, k, device, True)
@@ -210,7 +210,8 @@ def join_codes(pairs):
     if len(pairs) == 1:
         return pairs[0]
     rows, k, device = pairs[0][0].shape[0], sum(c.shape[1] for c, _ in pairs), pairs[0][0].device
-    sources = (_lib.CodeSource * len(pairs))(*[(c.data_ptr(), s.data_ptr(), c.shape[1], c.stride(0), s.stride(0)) for c, s in pairs])
+    # mx_code_source each
+    sources = _lib.words([(c.data_ptr(), s.data_ptr(), c.shape[1], c.stride(0), s.stride(0)) for c, s in pairs])
     codes = torch.empty(rows, k, device=device, dtype=_FP8)
     scales = torch.empty(rows, k // BLOCK_SCALE, device=device, dtype=torch.uint8)
     _lib.invoke("mx_join_codes", 2 * rows * k * (1 + 1 / BLOCK_SCALE), codes, ctypes.addressof(sources), len(pairs), rows,
@@ -242,20 +243,19 @@ def quantize_mx_dual_batch(xs: list[torch.Tensor]) -> list[tuple[torch.Tensor, t
     scales = torch.empty(2 * sum(n_scales), device=xs[0].device, dtype=torch.uint8)
     code_views = codes.split_with_sizes([n for n in n_codes for _ in (0, 1)])
     scale_views = scales.split_with_sizes([n for n in n_scales for _ in (0, 1)])
-    problems = (_lib.QuantProblem * len(xs))()
-    out, at_code, at_scale, work = [], codes.data_ptr(), scales.data_ptr(), 0.0
+    problems, out, at_code, at_scale, work = [], [], codes.data_ptr(), scales.data_ptr(), 0.0
     for j, x in enumerate(xs):
         m, k = x.shape
         kb, mb = k // BLOCK_SCALE, m // BLOCK_SCALE
-        problems[j] = _lib.QuantProblem(x.data_ptr(), at_code, at_scale, at_code + n_codes[j], at_scale + n_scales[j],
-                                        m, k, x.stride(0), k, kb, m, mb)
+        problems.append((x.data_ptr(), at_code, at_scale, at_code + n_codes[j], at_scale + n_scales[j],
+                         m, k, x.stride(0), k, kb, m, mb))  # the fields of mx_quant_problem
         out.append((code_views[2 * j].view(m, k), scale_views[2 * j].view(m, kb),
                     code_views[2 * j + 1].view(k, m), scale_views[2 * j + 1].view(k, mb)))
         at_code += 2 * n_codes[j]
         at_scale += 2 * n_scales[j]
         work += n_codes[j] * (x.element_size() + 2 * (1 + 1 / BLOCK_SCALE))
     if codes.numel():
-        _lib.invoke("mx_quantize_dual_batch", work, xs[0], ctypes.byref(problems), len(xs), _lib.MX_DTYPE[xs[0].dtype])
+        _lib.invoke("mx_quantize_dual_batch", work, xs[0], ctypes.byref(_lib.words(problems)), len(xs), _lib.MX_DTYPE[xs[0].dtype])
     return out
 
 
@@ -327,9 +327,8 @@ def mxfp8_matmul_pq_batch(problems, out_dtype: torch.dtype = torch.bfloat16) -> 
         raise ValueError(f"out_dtype={out_dtype} is not one of {tuple(_lib.MX_DTYPE)}")
     if not problems:
         return []
-    descs = (_lib.GemmProblem * len(problems))()
-    outs, keep, flops = [], [], 0.0
-    for d, (aq, a_scale, bq, b_scale) in zip(descs, problems):
+    descs, outs, keep, flops = [], [], [], 0.0
+    for aq, a_scale, bq, b_scale in problems:
         # a 3-D operand (K // 128, rows, 128) is a stage-major code matrix (quantize_mx_dual(..., stage_major_t=True))
         shape_a = (aq.shape[1], aq.shape[0] * PANEL) if aq.dim() == 3 and aq.shape[2] == PANEL else tuple(aq.shape)
         shape_b = (bq.shape[1], bq.shape[0] * PANEL) if bq.dim() == 3 and bq.shape[2] == PANEL else tuple(bq.shape)
@@ -357,13 +356,11 @@ def mxfp8_matmul_pq_batch(problems, out_dtype: torch.dtype = torch.bfloat16) -> 
         keep.append(ts)
         outs.append(out)
         flops += 2.0 * m * n * k
-        d.aq, d.a_scale, d.bq, d.b_scale, d.c = (t.data_ptr() for t in (*ts, out))
-        d.M, d.N, d.K = m, n, k
-        d.lda = PANEL if ts[0].dim() == 3 else ts[0].stride(0)
-        d.ldb = PANEL if ts[2].dim() == 3 else ts[2].stride(0)
-        d.ldas, d.ldbs, d.ldc = ts[1].stride(0), ts[3].stride(0), n
+        descs.append((  # the fields of mx_gemm_problem
+            *[t.data_ptr() for t in ts], out.data_ptr(), m, n, k, PANEL if ts[0].dim() == 3 else ts[0].stride(0), ts[1].stride(0),
+            PANEL if ts[2].dim() == 3 else ts[2].stride(0), ts[3].stride(0), n))
     ws = _lib.gemm_workspace(outs[0])
-    _lib.invoke("mx_gemm_nt_batch", flops, outs[0], ctypes.addressof(descs), len(problems), _lib.MX_DTYPE[out_dtype],
+    _lib.invoke("mx_gemm_nt_batch", flops, outs[0], ctypes.byref(_lib.words(descs)), len(problems), _lib.MX_DTYPE[out_dtype],
                 ws.data_ptr(), ws.numel())
     return outs
 

@@ -108,11 +108,11 @@ class MXFP8SwiGLU(nn.Module):
         """Both matrices as dual (row + column axis) quantizations, for ``refresh_mxfp8_weights``' single launch."""
         if self.dim % 32 or self.hidden % 32 or not self.w_in.is_cuda:
             return None
-        return [self.w_in.detach(), self.w_out.detach()]
+        return [self.w_in, self.w_out]
 
     def mxfp8_install(self, copies) -> None:
         (q1, s1, qt1, st1), (q2, s2, qt2, st2) = copies
-        self._packed = ((q1, s1), (qt1, st1), (q2, s2), (qt2, st2))
+        self.__dict__["_packed"] = ((q1, s1), (qt1, st1), (q2, s2), (qt2, st2))  # as MXFP8Linear.mxfp8_install
 
     def forward(self, x: torch.Tensor) -> torch.Tensor:
         if self._packed is None:
