@@ -352,10 +352,11 @@ __device__ __forceinline__ void quant_tile(float (&v)[R][8], const QuantTileOut 
 // is converted where it is used, three times instead of once, and the thread holds 32 registers of tile instead of 64.
 // The plain row + token axis quantizer then fits 64 registers and eight waves per SIMD (90 registers and five with the
 // tile in fp32), so that the 1536 tiles of a 16384 x 1536 activation are resident at once instead of in 1.2 rounds.
-// Same arithmetic on the same values: bit-identical outputs.
+// Same arithmetic on the same values: bit-identical outputs.  gate (token axis alone): a factor for each of the thread's rows.
 template <int DT, bool ROWS, bool NTS>
 __device__ __forceinline__ void quant_tile_raw(typename Elem<DT>::raw (&r)[8], const QuantTileOut &o, int64_t M, int64_t MT,
-                                               int64_t K, int64_t m0, int64_t kc0, uint8_t *tile, uint8_t *tscale) {
+                                               int64_t K, int64_t m0, int64_t kc0, uint8_t *tile, uint8_t *tscale,
+                                               const float *gate = nullptr) {
     typedef TileGeom<8> G;
     typedef Elem<DT> E;
     const int t = threadIdx.x;
@@ -398,7 +399,7 @@ __device__ __forceinline__ void quant_tile_raw(typename Elem<DT>::raw (&r)[8], c
     for (int c = 0; c < 8; c++) {
         float v[8];
 #pragma unroll
-        for (int i = 0; i < 8; i++) v[i] = E::elem(r[i], c);
+        for (int i = 0; i < 8; i++) v[i] = gate ? E::elem(r[i], c) * gate[i] : E::elem(r[i], c);
         float cm = amax8(v);
         cm = fmaxf(cm, __shfl_xor(cm, 16, 64));
         cm = fmaxf(cm, __shfl_xor(cm, 32, 64));
@@ -865,21 +866,14 @@ struct GroupedQuantArgs {
     int scale_f32;
     const int32_t *offsets;
     int E;
-    int span;  // column tiles per workgroup
 };
 
-template <int DT, int SRC>
-__global__ __launch_bounds__(256) void quant_cols_grouped_kernel(GroupedQuantArgs a, QuantTileOut o, int64_t mpad) {
-    typedef typename Elem<DT>::type T;
-    __shared__ __attribute__((aligned(16))) uint8_t tile[QC_TILE * QC_PITCH];
-    __shared__ __attribute__((aligned(4))) uint8_t tscale[QC_TILE * 4];
+// The expert whose tiles contain row tile `rt`: owner[] = expert, its first tile, its first and its end row; owner[0] < 0 for
+// a tile past the last one.  The first wave looks at 64 experts at a time (one coalesced read of `offsets`, a wave scan of
+// their tile counts) instead of walking the experts with a dependent scalar load each: with hundreds of experts, most of them
+// empty, that walk took longer than the tile itself.
+__device__ __forceinline__ void tile_owner(const GroupedQuantArgs &a, int rt, int (&owner)[4]) {
     const int t = threadIdx.x;
-    const int rt = blockIdx.y;
-    // tile_owner: the expert whose tiles contain rt.  The first wave looks at 64 experts at a time
-    // (one coalesced read of `offsets`, a wave scan of their tile counts) instead of walking the
-    // experts with a dependent scalar load each: with hundreds of experts, most of them empty,
-    // that walk took longer than the tile itself.
-    __shared__ int owner[4];
     if (t < 64) {
         int carry = 0;
         bool done = false;
@@ -899,9 +893,18 @@ __global__ __launch_bounds__(256) void quant_cols_grouped_kernel(GroupedQuantArg
         if (!done && t == 0) owner[0] = -1;
     }
     __syncthreads();
-    if (owner[0] < 0) return;  // beyond the last real tile: that part of the padded space is never read
-    const int before = owner[1], start = owner[2], end = owner[3];
-    const int row_base = start + (rt - before) * QC_TILE;
+}
+
+template <int DT>
+__global__ __launch_bounds__(256) void quant_swiglu_grouped_kernel(GroupedQuantArgs a, QuantTileOut o, int64_t mpad) {
+    typedef typename Elem<DT>::type T;
+    __shared__ __attribute__((aligned(16))) uint8_t tile[QC_TILE * QC_PITCH];
+    __shared__ __attribute__((aligned(4))) uint8_t tscale[QC_TILE * 4];
+    __shared__ int owner[4];
+    const int t = threadIdx.x, rt = blockIdx.y;
+    tile_owner(a, rt, owner);
+    if (owner[0] < 0) return;  // that part of the padded space is never read
+    const int end = owner[3], row_base = owner[2] + (rt - owner[1]) * QC_TILE;
     const int64_t k0 = (int64_t)blockIdx.x * QC_TILE;
     const int64_t col = k0 + (t & 15) * 8;
     const bool col_ok = col < a.C;
@@ -911,21 +914,11 @@ __global__ __launch_bounds__(256) void quant_cols_grouped_kernel(GroupedQuantArg
         const int pos = row_base + (t >> 4) * 8 + i;
         if (col_ok && pos < end) {
             const int64_t src = a.index ? a.index[pos] : pos;
-            if (SRC == SRC_PLAIN) {
-                Elem<DT>::load8((const T *)a.x + src * a.ldx + col, v[i]);
-                if (a.row_scale) {
-                    const int si = a.scale_index ? a.scale_index[pos] : pos;
-                    const float sc = a.scale_f32 ? ((const float *)a.row_scale)[si] : Elem<DT>::load1((const T *)a.row_scale + si);
+            float g[8], u[8];
+            Elem<DT>::load8((const T *)a.x + src * a.ldx + col, g);
+            Elem<DT>::load8((const T *)a.x + src * a.ldx + a.C + col, u);
 #pragma unroll
-                    for (int c = 0; c < 8; c++) v[i][c] *= sc;
-                }
-            } else {
-                float g[8], u[8];
-                Elem<DT>::load8((const T *)a.x + src * a.ldx + col, g);
-                Elem<DT>::load8((const T *)a.x + src * a.ldx + a.C + col, u);
-#pragma unroll
-                for (int c = 0; c < 8; c++) v[i][c] = g[c] * sigmoid_fast(g[c]) * u[c];
-            }
+            for (int c = 0; c < 8; c++) v[i][c] = g[c] * sigmoid_fast(g[c]) * u[c];
         } else {
 #pragma unroll
             for (int c = 0; c < 8; c++) v[i][c] = 0.0f;
@@ -934,99 +927,46 @@ __global__ __launch_bounds__(256) void quant_cols_grouped_kernel(GroupedQuantArg
     quant_tile<false>(v, o, mpad, mpad, a.C, (int64_t)rt * QC_TILE, k0, tile, tscale);
 }
 
-// The same quantizer for wide inputs: a workgroup keeps its 128 rows and walks `span` column tiles.
-// Measured at 98304 routed rows x 1024 columns with a row scale: 72 us one tile per workgroup,
-// 60 us four tiles (one expert search, one read of the row indices and scales, 1 KB runs of every
-// source row); without the row scale 56 and 57 us.  One tile per workgroup stays with the kernel
-// above, which is the faster of the two then.
-template <int DT, int SRC>
-__global__ __launch_bounds__(256) void quant_cols_grouped_walk_kernel(GroupedQuantArgs a, QuantTileOut o, int64_t mpad) {
+// SRC_PLAIN.  Bound by the gathered reads and the code stores; what it lacked was waves in flight.  With the tile in fp32 and
+// four column tiles per workgroup it took 166 registers, three waves per SIMD, and the 1664 workgroups of 98304 rows x 1024 ran in
+// 2.2 rounds of 768.  Packed as loaded (quant_tile_raw, which converts every value once here), one tile per workgroup, it takes 57
+// and eight waves: 98304 rows from 16384 x 1024, us before / now: 96 / 55 with a row scale (GATED), 86 / 53 without; 16662 rows from
+// 2777: 25 / 17 and 20 / 15.5.  Four or two tiles per workgroup: 61 and 58, 61 and 55.  (Left to itself the compiler takes 228
+// registers for the straight-line form.)
+template <int DT, bool GATED>
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(8))) void quant_cols_grouped_kernel(GroupedQuantArgs a, QuantTileOut o, int64_t mpad) {
     typedef typename Elem<DT>::type T;
     __shared__ __attribute__((aligned(16))) uint8_t tile[QC_TILE * QC_PITCH];
     __shared__ __attribute__((aligned(4))) uint8_t tscale[QC_TILE * 4];
-    const int t = threadIdx.x;
-    const int rt = blockIdx.y;
-    // tile_owner: the expert whose tiles contain rt.  The first wave looks at 64 experts at a time
-    // (one coalesced read of `offsets`, a wave scan of their tile counts) instead of walking the
-    // experts with a dependent scalar load each: with hundreds of experts, most of them empty,
-    // that walk took longer than the tile itself.
     __shared__ int owner[4];
-    if (t < 64) {
-        int carry = 0;
-        bool done = false;
-        for (int e0 = 0; e0 < a.E && !done; e0 += 64) {
-            const int e = e0 + t;
-            const int lo = e < a.E ? a.offsets[e] : 0, hi = e < a.E ? a.offsets[e + 1] : 0;
-            const int tiles = (hi - lo + QC_TILE - 1) / QC_TILE;
-            const int incl = wave_incl_scan(tiles, t);
-            const int first = carry + incl - tiles;
-            const bool mine = e < a.E && rt >= first && rt < first + tiles;
-            if (__ballot(mine)) {
-                if (mine) owner[0] = e, owner[1] = first, owner[2] = lo, owner[3] = hi;
-                done = true;
-            }
-            carry += __shfl(incl, 63, 64);
+    const int t = threadIdx.x, rt = blockIdx.y;
+    tile_owner(a, rt, owner);
+    if (owner[0] < 0) return;  // that part of the padded space is never read
+    const int end = owner[3], row_base = owner[2] + (rt - owner[1]) * QC_TILE;
+    // each source row's index and scale factor is read by one thread, not by the 16 that hold the row
+    __shared__ __attribute__((aligned(16))) int src_of[QC_TILE];
+    __shared__ __attribute__((aligned(16))) float gate_of[QC_TILE];
+    if (t < QC_TILE) {
+        const int pos = row_base + t;
+        const bool real = pos < end;
+        src_of[t] = !real ? -1 : a.index ? a.index[pos] : pos;
+        if constexpr (GATED) {
+            const int si = !real ? 0 : a.scale_index ? a.scale_index[pos] : pos;
+            gate_of[t] = !real ? 1.0f : a.scale_f32 ? ((const float *)a.row_scale)[si] : Elem<DT>::load1((const T *)a.row_scale + si);
         }
-        if (!done && t == 0) owner[0] = -1;
     }
     __syncthreads();
-    if (owner[0] < 0) return;  // beyond the last real tile: that part of the padded space is never read
-    const int before = owner[1], start = owner[2], end = owner[3];
-    const int row_base = start + (rt - before) * QC_TILE;
-    // this thread's 8 source rows (and their scale factors) serve every column tile of the workgroup
-    int64_t src[8];
-    float sc[8];
+    const int64_t k0 = (int64_t)blockIdx.x * QC_TILE, col = k0 + (t & 15) * 8;
+    typename Elem<DT>::raw r[8];
+    float gate[8];
 #pragma unroll
     for (int i = 0; i < 8; i++) {
-        const int pos = row_base + (t >> 4) * 8 + i;
-        src[i] = -1;
-        sc[i] = 1.0f;
-        if (pos < end) {
-            src[i] = a.index ? a.index[pos] : pos;
-            if (SRC == SRC_PLAIN && a.row_scale) {
-                const int si = a.scale_index ? a.scale_index[pos] : pos;
-                sc[i] = a.scale_f32 ? ((const float *)a.row_scale)[si] : Elem<DT>::load1((const T *)a.row_scale + si);
-            }
-        }
+        const int src = src_of[(t >> 4) * 8 + i];
+        gate[i] = GATED ? gate_of[(t >> 4) * 8 + i] : 1.0f;
+        r[i] = __builtin_bit_cast(typename Elem<DT>::raw, v4i{0, 0, 0, 0});
+        if (col < a.C && src >= 0) r[i] = Elem<DT>::load_raw((const T *)a.x + (int64_t)src * a.ldx + col);
     }
-    // A workgroup walks `span` neighbouring column tiles of its 128 rows: it reads span x 256
-    // contiguous bytes of every source row instead of 256, and finds its expert once.
-    const int ctiles = (a.C + QC_TILE - 1) / QC_TILE;
-    const int kt_end = (int)(blockIdx.x + 1) * a.span < ctiles ? (int)(blockIdx.x + 1) * a.span : ctiles;
-    for (int kt = (int)blockIdx.x * a.span; kt < kt_end; kt++) {
-        const int64_t k0 = (int64_t)kt * QC_TILE;
-        const int64_t col = k0 + (t & 15) * 8;
-        const bool col_ok = col < a.C;
-        float v[8][8];
-        typename Elem<DT>::raw r[8];  // the eight row loads of this column tile go out together
-        if (SRC == SRC_PLAIN) {
-#pragma unroll
-            for (int i = 0; i < 8; i++)
-                if (col_ok && src[i] >= 0) r[i] = Elem<DT>::load_raw((const T *)a.x + src[i] * a.ldx + col);
-        }
-#pragma unroll
-        for (int i = 0; i < 8; i++) {
-            if (col_ok && src[i] >= 0) {
-                if (SRC == SRC_PLAIN) {
-                    Elem<DT>::unpack(r[i], v[i]);
-                    if (a.row_scale) {
-#pragma unroll
-                        for (int c = 0; c < 8; c++) v[i][c] *= sc[i];
-                    }
-                } else {
-                    float g[8], u[8];
-                    Elem<DT>::load8((const T *)a.x + src[i] * a.ldx + col, g);
-                    Elem<DT>::load8((const T *)a.x + src[i] * a.ldx + a.C + col, u);
-#pragma unroll
-                    for (int c = 0; c < 8; c++) v[i][c] = g[c] * sigmoid_fast(g[c]) * u[c];
-                }
-            } else {
-#pragma unroll
-                for (int c = 0; c < 8; c++) v[i][c] = 0.0f;
-            }
-        }
-        quant_tile<false>(v, o, mpad, mpad, a.C, (int64_t)rt * QC_TILE, k0, tile, tscale);
-    }
+    quant_tile_raw<DT, false, false>(r, o, mpad, mpad, a.C, (int64_t)rt * QC_TILE, k0, tile, tscale, GATED ? gate : nullptr);
 }
 
 }  // namespace mx
@@ -1608,23 +1548,15 @@ extern "C" int mx_quantize_cols_grouped(const void *x, int dtype, int64_t ldx, i
     a.scale_f32 = row_scale_dtype == MX_FP32, a.offsets = offsets, a.E = (int)E;
     QuantTileOut o = tile_out(qT, ldqT, sT, ldsT, nullptr, 0, nullptr, 0, 0, qt_panels ? C * 128 : 0);
     const int ctiles = (int)((C + QC_TILE - 1) / QC_TILE);
-    // four column tiles per workgroup while that still leaves every CU several workgroups
-    a.span = ctiles >= 4 && (int64_t)tiles * (ctiles / 4) >= 2 * (int64_t)mx::num_cus() ? 4 : 1;
-    dim3 grid((unsigned)((ctiles + a.span - 1) / a.span), (unsigned)tiles);
+    const dim3 grid((unsigned)ctiles, (unsigned)tiles);
     hipStream_t st = (hipStream_t)stream;
     if (mx::stream_is_capturing(st)) return MX_ECAPTURE;
-#define MX_QCG_LAUNCH(DT, SRC)                                                                     \
-    do {                                                                                           \
-        if (a.span > 1) quant_cols_grouped_walk_kernel<DT, SRC><<<grid, dim3(256), 0, st>>>(a, o, mpad); \
-        else quant_cols_grouped_kernel<DT, SRC><<<grid, dim3(256), 0, st>>>(a, o, mpad);           \
-    } while (0)
-    if (dtype == MX_BF16) {
-        if (source == SRC_PLAIN) MX_QCG_LAUNCH(MX_BF16, SRC_PLAIN);
-        else MX_QCG_LAUNCH(MX_BF16, SRC_SWIGLU);
-    } else {
-        if (source == SRC_PLAIN) MX_QCG_LAUNCH(MX_FP16, SRC_PLAIN);
-        else MX_QCG_LAUNCH(MX_FP16, SRC_SWIGLU);
-    }
+#define MX_QCG_LAUNCH(DT)                                                                                                      \
+    (source == SRC_SWIGLU ? quant_swiglu_grouped_kernel<DT><<<grid, dim3(256), 0, st>>>(a, o, mpad)                            \
+     : row_scale          ? quant_cols_grouped_kernel<DT, true><<<grid, dim3(256), 0, st>>>(a, o, mpad)                        \
+                          : quant_cols_grouped_kernel<DT, false><<<grid, dim3(256), 0, st>>>(a, o, mpad))
+    if (dtype == MX_BF16) MX_QCG_LAUNCH(MX_BF16);
+    else MX_QCG_LAUNCH(MX_FP16);
 #undef MX_QCG_LAUNCH
     MX_LAUNCH_CHECK();
     return MX_OK;
