@@ -244,13 +244,20 @@ int mx_rmsnorm_quantize_dual(const void *x, int x_dtype, int64_t M, int64_t K, i
  * RMSNorm backward: dx = (dy - xhat * mean_k(dy * xhat)) * rstd with dy = dout * weight and
  * xhat = x * rstd, in dtype (bf16 or fp16); dw_part (parts,K) fp32 (NULL: no weight
  * gradient) receives one partial sum of dout * xhat per workgroup, every row of it written;
- * the caller adds the rows.  1 <= parts <= 65535; K <= 4096.
+ * mx_rmsnorm_weight_grad adds the rows.  1 <= parts <= 65535; K <= 4096.
  * Replaces _rmsnorm_bwd (src/kohakuwullm/kernels/elementwise/rmsnorm.py:87-128, launched
  * from _RMSNorm.backward :196-229 with 512 partial rows).
  */
 int mx_rmsnorm_backward(const void *x, int dtype, int64_t M, int64_t K, int64_t ldx, const void *weight,
                         int w_dtype, const void *dout, int64_t lddo, const float *rstd, void *dx, int64_t lddx,
                         float *dw_part, int64_t parts, void *stream);
+
+/*
+ * The weight gradient from mx_rmsnorm_backward's partial rows: dw (K) in dw_dtype (any of the three) = the sum of the rows
+ * of dw_part (parts,K), in fp64 and in a fixed order, rounded to fp32 and then to dw_dtype.
+ * Replaces the host-side sum of _RMSNorm.backward (src/kohakuwullm/kernels/elementwise/rmsnorm.py:196-229).
+ */
+int mx_rmsnorm_weight_grad(const float *dw_part, int64_t parts, int64_t K, void *dw, int dw_dtype, void *stream);
 
 /*
  * Scale layout interop.  The reference's cuBLAS route keeps UE8M0 scales in the flat

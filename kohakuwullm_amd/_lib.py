@@ -65,6 +65,7 @@ SIGNATURES = {
         _ci, [_p, _ci, _i64, _i64, _i64, _p, _ci, ctypes.c_float, _p, _p, _i64, _p, _i64, _p, _i64, _p, _i64, _p]),
     "mx_rmsnorm_backward": (
         _ci, [_p, _ci, _i64, _i64, _i64, _p, _ci, _p, _i64, _p, _p, _i64, _p, _i64, _p]),
+    "mx_rmsnorm_weight_grad": (_ci, [_p, _i64, _i64, _p, _ci, _p]),
     "mx_router_topk": (
         _ci, [_p, _ci, _i64, _p, _ci, _p, _ci, _i64, _i64, _i64, _i64, _ci, _f, _p, _p, _p, _p, _p]),
     "mx_router_backward_workspace": (_i64, [_i64, _i64, _i64]),

@@ -117,7 +117,10 @@ class _RMSNorm(torch.autograd.Function):
                 dout2d.data_ptr(), dout2d.stride(0), rstd.data_ptr(), dx.data_ptr(), dx.stride(0),
                 0 if dw_part is None else dw_part.data_ptr(), parts,
             )
-        dw = dw_part.sum(0).to(weight.dtype) if has_w else None
+        dw = torch.empty(n_cols, dtype=weight.dtype, device=x2d.device) if has_w else None
+        if has_w and n_cols:
+            _lib.invoke("mx_rmsnorm_weight_grad", dw_part.numel() * 4, x2d, dw_part.data_ptr(), parts, n_cols, dw.data_ptr(),
+                        _lib.MX_DTYPE[weight.dtype])
         return dx.reshape(shape), dw, None, None, None, None
 
 

@@ -178,3 +178,24 @@ def test_rmsnorm_mx_dual_full_width_and_errors(oracle):
         rmsnorm_mx_dual(xd[:128], wd, stage_major_t=True)  # one panel is not a stage-major matrix
     with pytest.raises(Exception):
         rmsnorm_mx_dual(x, w)  # CPU tensors: there is no CPU path
+
+
+@pytest.mark.parametrize("parts,k", [(1, 8), (3, 24), (127, 96), (129, 1000), (768, 2048), (1024, 4096)])
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16, torch.float16])
+def test_weight_grad_adds_the_partial_rows(parts, k, dtype):
+    """Against fp64: one rounding to fp32 and one to the weight's type; nothing outside the k elements is written."""
+    from kohakuwullm_amd import _lib
+
+    g = torch.Generator().manual_seed(SEED + parts + k)
+    part = torch.randn(parts, k, generator=g)
+    out = torch.full((k + 64,), 7.0, dtype=dtype, device=DEV)
+    dev = part.to(DEV)
+    _lib.invoke("mx_rmsnorm_weight_grad", part.numel() * 4, dev, dev.data_ptr(), parts, k, out.data_ptr(), _lib.MX_DTYPE[dtype])
+    # the fp64 sums differ by their order only: up to parts 2^-53 of the sum of magnitudes, which moves few fp32 roundings
+    want = part.double().sum(0).float().to(dtype)
+    got = out[:k].cpu()
+    assert (got == want).float().mean().item() >= 0.99
+    ulp = {torch.float32: 2.0**-23, torch.bfloat16: 2.0**-7, torch.float16: 2.0**-10}[dtype]
+    slack = parts * 2.0**-52 * part.double().abs().sum(0)
+    assert ((got.double() - want.double()).abs() <= want.double().abs() * ulp + slack).all()
+    assert (out[k:] == 7.0).all()
