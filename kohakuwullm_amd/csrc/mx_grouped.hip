@@ -867,7 +867,6 @@ __global__ __launch_bounds__(S::NTHR) void grouped_kernel(GroupedArgs args) {
     grouped_body<S, MODE, CDT, K512, AHEAD>(args, smem);
 }
 
-#ifdef MX_BENCH_VARIANTS
 // The same body on the 128 x 128 tile of four waves (one per SIMD), two workgroups resident per CU, so that one
 // workgroup's epilogue can run while the other one's MFMAs do.  The register budget is the one of two waves per SIMD.
 template <typename S, int MODE, int CDT, int K512>
@@ -875,7 +874,6 @@ __global__ __launch_bounds__(S::NTHR) __attribute__((amdgpu_waves_per_eu(2, 2)))
     extern __shared__ __attribute__((aligned(1024))) uint8_t smem[];
     grouped_body<S, MODE, CDT, K512>(args, smem);
 }
-#endif
 
 // Slow path for shapes the tiled kernel does not take (PLAIN only): one thread per output element.
 template <int CDT>
@@ -1278,19 +1276,40 @@ static bool tiled_ok(const GroupedArgs &a, int64_t a_rows) {
 }
 
 // 128 x 128 x 128 tile, 4 waves as 4 (M) x 1 (N), one per SIMD: a wave owns 32 x 128 -- the same eight consecutive N per
-// lane as under Big, so the fused epilogues' column logic is shared -- and two workgroups fit a CU (2 x 73 KB of LDS,
-// 256 registers per lane each).  Twice the operand bytes per flop of Big: for the fused expert epilogues only, whose
-// vector ALU work dwarfs their short K loops.
+// lane as under Big, so the epilogues' column logic is shared and the outputs are the same bits -- and two workgroups fit a
+// CU (2 x 73 KB of LDS, 256 registers per lane each).  Twice the operand bytes per flop of Big.
 typedef GemmShape<128, 128, 4, 1> Slim;
 
-// Built into the variants library only (-DMX_BENCH_VARIANTS), where it replaces Big for the two fused expert kernels:
-// bit-identical outputs, measured slower at the benchmark's routing (GEMM1 148 -> 185 us, GEMM2-dgrad 192 -> 209 us).
-// The eight waves of a CU issue the same vector ALU work either way, and the K loops of a 128 x 128 tile, whose copies
-// must land within a stage of 512 MFMA clocks, cost more than their overlap with the other workgroup's epilogue returns.
+// Which of the two a launch takes.  The host knows the rows and the experts but not who has how many, so an expert is taken
+// to end half a tile into its last one, and both shapes are counted in rounds: one Big tile or two Slim ones per CU.
+// A Slim round does half the MFMA work of a Big one behind the same operand bytes, so the plain product, whose rounds are
+// K loops, goes to Slim wherever that needs no more of them.  The fused kernels' rounds are epilogues, and in those half
+// the values are half the time less what the two workgroups share: 14 us against 22 (GEMM1), 24 against 44 (GEMM2-dgrad),
+// so three Slim rounds are taken in place of two.  Few rows per expert fill a Big tile to a fraction, and few tiles leave
+// CUs idle; from about 300 rows in 64 experts on, Big is ahead again (1536 rows: GEMM1 189 / 199 us, plain 135 / 189).
+// us Big / Slim, 64 experts of 1024 x 512, top 6, by rows per expert:
+//                       3             48            188           260           384
+//   GEMM1          25.3 / 19.0   25.9 / 20.6   47.1 / 33.2   50.7 / 46.9   49.2 / 55.3
+//   GEMM2-dgrad    33.5 / 22.4   40.8 / 25.6   46.6 / 31.1   48.5 / 47.2   48.0 / 53.7
+//   plain, K 512   12.6 /  9.4   13.5 / 10.9   22.7 / 16.9   23.6 / 21.9   23.8 / 24.8
+//   plain, K 1024  19.0 / 14.8   19.6 / 16.3   32.6 / 24.9   33.5 / 32.8   34.8 / 39.7
+template <int MODE>
+static bool slim_pays(const GroupedArgs &a) {
+    if (a.E > row_table_max<Slim, false>()) return false;  // its table of row tiles, half of Big's, keeps the lookup cheap
+    const double live = a.E < a.M ? a.E : a.M, cus = num_cus();
+    auto rounds = [&](int bm, int npt, double slots) {
+        const double rows = (double)a.M / bm + 0.5 * live;
+        return ceil((rows > live ? rows : live) * ((a.N + npt - 1) / npt) / slots - 0.05);
+    };
+    constexpr int half = MODE == MODE_GEMM1 ? 2 : 1;  // a GEMM1 tile spans half as many hidden units as it has columns
+    const double big = rounds(Big::BM, Big::BN / half, cus), small = rounds(Slim::BM, Slim::BN / half, 2 * cus);
+    return small < 1e6 && (MODE == MODE_PLAIN ? small <= big : 2 * small <= 3 * big);
+}
+// The variants library turns the rule round, so that the other shape can be compared with the shipped one at any size.
 #ifdef MX_BENCH_VARIANTS
-#define MX_EXPERT_SLIM 1
+#define MX_EXPERT_OTHER true
 #else
-#define MX_EXPERT_SLIM 0
+#define MX_EXPERT_OTHER false
 #endif
 
 template <typename S, int MODE, int CDT>
@@ -1306,21 +1325,18 @@ static int launch_grouped_shape(GroupedArgs a, hipStream_t st) {
     const int wgs = num_cus() * (pair ? 2 : 1);
     dim3 grid((unsigned)(work < wgs ? work : wgs)), block(S::NTHR);
     int rc;
-#ifdef MX_BENCH_VARIANTS
-    if constexpr (pair)
+    if constexpr (pair) {
         rc = k512 ? launch_with_lds<grouped_pair_kernel<S, MODE, CDT, SCALES_VEC16>>(grid, block, S::LDS_BYTES, st, a)
                   : launch_with_lds<grouped_pair_kernel<S, MODE, CDT, SCALES_DWORD>>(grid, block, S::LDS_BYTES, st, a);
-    else
-#endif
-    {
+    } else {
         // The plain product on whole 512s of K (every tile then has four stages or more): the A operand two stages ahead
         // and scale bytes through the copy engine (32-bit lane offsets: both scale matrices under 4 GB), as the dense
         // kernels; 90 -> 81 us and 132 -> 120 us on 98304 routed rows at K = 512 and 1024.
         bool ahead = false;
-        if constexpr (MODE == MODE_PLAIN && !pair)
+        if constexpr (MODE == MODE_PLAIN)
             ahead = k512 && a.E <= MX_TABLE_MAX_STAGED && a.x_rows > 0 && a.x_rows * a.ldxs < ((int64_t)1 << 32) &&
                     ((int64_t)a.E - 1) * a.stride_wse + (int64_t)a.N * a.ldws < ((int64_t)1 << 32);
-        if constexpr (MODE == MODE_PLAIN && !pair) {
+        if constexpr (MODE == MODE_PLAIN) {
             if (ahead) rc = launch_with_lds<grouped_kernel<S, MODE, CDT, SCALES_COPY, true>>(grid, block, S::LDS_BYTES_AHEAD, st, a);
         }
         if (!ahead)
@@ -1333,8 +1349,9 @@ static int launch_grouped_shape(GroupedArgs a, hipStream_t st) {
 
 template <int MODE, int CDT>
 static int launch_grouped(const GroupedArgs &a, hipStream_t st) {
-    if constexpr (MX_EXPERT_SLIM && (MODE == MODE_GEMM1 || MODE == MODE_DGRAD2)) return launch_grouped_shape<Slim, MODE, CDT>(a, st);
-    else return launch_grouped_shape<Big, MODE, CDT>(a, st);
+    if constexpr (MODE != MODE_SCATTER)
+        if (slim_pays<MODE>(a) != MX_EXPERT_OTHER) return launch_grouped_shape<Slim, MODE, CDT>(a, st);
+    return launch_grouped_shape<Big, MODE, CDT>(a, st);
 }
 
 template <int MODE>

@@ -677,7 +677,7 @@ def test_gemm2_dgrad_token_axis(oracle):
 
 @pytest.mark.parametrize("counts,hid", [([200, 0, 56, 300], 160), ([1, 700], 544), ([130] * 5, 256)])
 def test_expert_kernels_on_small_tiles_agree(counts, hid):
-    """The variants library runs the two fused expert kernels on 128 x 128 tiles, two workgroups per CU: every element
+    """The variants library runs the expert kernels on the tile shape (128 x 128 or 256 x 256) the shipped rule passes over: every element
     contracts the same K sequence and goes through the same epilogue arithmetic, so every output of GEMM1 and of
     GEMM2-dgrad equals the shipped kernels' bit for bit (dgate, a sum of atomics, by norm)."""
     from kohakuwullm_amd import _lib
@@ -716,6 +716,36 @@ def test_expert_kernels_on_small_tiles_agree(counts, hid):
     for name, a, b in zip("hq hs pre htq hts dpre dpq dps ptq pts".split(), shipped, small):
         assert torch.equal(a, b), name
     assert float((dgate - dgate_small).norm() / dgate.norm()) < 1e-5
+
+
+@pytest.mark.parametrize("counts", [[1], [127, 128, 129], [0, 256, 0, 257, 1], [3] * 40, [700, 2, 0]])
+@pytest.mark.parametrize("n,k,dtype", [(1000, 512, torch.bfloat16), (136, 384, torch.float16), (257, 1024, torch.float32)])
+def test_grouped_product_on_either_tile_shape(counts, n, k, dtype):
+    """The plain product on 128 x 128 and on 256 x 256 tiles (the variants library turns the rule round): the same bits, no row
+    or column outside the experts' written, at tile edges, ragged N, gathered rows and K with and without whole groups."""
+    from kohakuwullm_amd import _lib
+    from kohakuwullm_amd.kernels.mxfp8.grouped import grouped_mxfp8_gemm
+    from kohakuwullm_amd.kernels.mxfp8.quantize import quantize_mx
+
+    g = torch.Generator().manual_seed(SEED + n)
+    e, m = len(counts), sum(counts)
+    offsets = torch.tensor([0] + counts).cumsum(0).int().to(DEV)
+    index = torch.randint(0, m + 5, (m,), generator=g).int().to(DEV)
+    xq, xs = quantize_mx(torch.randn(m + 5, k, generator=g).bfloat16().to(DEV))
+    wq, ws = quantize_mx((torch.randn(e * n, k, generator=g) * 0.1).bfloat16().to(DEV))
+    wq, ws = wq.view(e, n, k), ws.view(e, n, k // 32)
+
+    def run():
+        out = torch.full((m + 3, n), 7.0, device=DEV, dtype=dtype)
+        grouped_mxfp8_gemm(xq, xs, wq, ws, offsets, index=index, out_dtype=dtype, out=out[:m])
+        torch.cuda.synchronize()
+        return out
+
+    shipped = run()
+    with _lib.variants_library():
+        other = run()
+    assert torch.equal(shipped, other)
+    assert (shipped[m:] == 7.0).all() and shipped[:m].isfinite().all()
 
 
 def test_expert_call_contract():
