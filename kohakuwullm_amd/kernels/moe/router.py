@@ -14,12 +14,19 @@ from kohakuwullm_amd import _lib
 MAX_EXPERTS, MAX_TOP_K = 256, 16
 
 
-def can_route(x: torch.Tensor, weight: torch.Tensor, top_k: int) -> bool:
-    """Whether the kernels take these operands (types, alignment, limits); autocast changes the arithmetic and is not covered."""
+def operands_fit(x: torch.Tensor, weight: torch.Tensor, top_k: int) -> bool:
+    """Whether shapes, types and layouts are what the kernels assume; the library sees pointers and cannot check a width."""
+    if x.dim() != 2 or weight.dim() != 2:
+        return False
     e, d = weight.shape
-    return (x.is_cuda and x.dim() == 2 and x.shape[0] > 0 and x.dtype in _lib.MX_DTYPE and weight.dtype in (x.dtype, torch.float32)
-            and d % 8 == 0 and e <= MAX_EXPERTS and top_k <= min(MAX_TOP_K, e) and weight.is_contiguous()
-            and weight.device == x.device and weight.data_ptr() % 16 == 0 and not torch.is_autocast_enabled("cuda"))
+    return (x.shape[0] > 0 and x.shape[1] == d and x.dtype in _lib.MX_DTYPE and weight.dtype in (x.dtype, torch.float32)
+            and d % 8 == 0 and e <= MAX_EXPERTS and 0 < top_k <= min(MAX_TOP_K, e) and weight.is_contiguous()
+            and weight.device == x.device and weight.data_ptr() % 16 == 0)
+
+
+def can_route(x: torch.Tensor, weight: torch.Tensor, top_k: int) -> bool:
+    """Whether the kernels take this call; autocast changes the arithmetic and is not covered."""
+    return x.is_cuda and operands_fit(x, weight, top_k) and not torch.is_autocast_enabled("cuda")
 
 
 class _RouteTopK(torch.autograd.Function):
@@ -71,6 +78,8 @@ def route_topk(x: torch.Tensor, weight: torch.Tensor, bias: torch.Tensor | None,
 
     The ``top_k`` experts with the largest ``score + bias``, best first (ties to the lower expert); ``gate`` is ``factor``
     times their scores, normalized over the token's picks when ``norm``.  Differentiable in ``x`` and ``weight`` through
-    ``gate``.  See :func:`can_route` for what it takes.
+    ``gate``.  See :func:`can_route` for what it takes; other operands are refused here.
     """
+    if not operands_fit(x, weight, top_k):
+        raise ValueError(f"route_topk: x {tuple(x.shape)} {x.dtype}, weight {tuple(weight.shape)} {weight.dtype}, top_k {top_k}")
     return _RouteTopK.apply(x, weight, bias, top_k, norm, factor)

@@ -78,3 +78,16 @@ def test_router_module_on_kernels_matches_its_composition():
     assert torch.equal(router.load_accum, 2.0 * counts)
     with torch.no_grad():
         assert torch.equal(router.route(x)[1], gate)
+
+
+def test_router_of_another_width_raises():
+    """A block whose router reads another width than it is given: an error, as the composition's product raises it."""
+    from kohakuwullm_amd.models.moe import MoEMLP
+
+    block = MoEMLP(256, hidden=128, num_experts=16, top_k=4, num_shared=0, router_dim=128).to(DEV).to(BF)
+    x = torch.randn(40, 256, device=DEV).to(BF)
+    with pytest.raises(RuntimeError):
+        block(x)
+    with pytest.raises(RuntimeError):
+        block(x, route_on=x[:, :64])
+    assert block(x, route_on=x[:, :128].contiguous()).shape == x.shape

@@ -1,0 +1,43 @@
+"""Which calls the router's kernels may stand for, decided on the host: what does not fit goes to the PyTorch composition."""
+
+import pytest
+import torch
+
+BF, HF, F32 = torch.bfloat16, torch.float16, torch.float32
+
+
+def _operands(tokens=4, dim=64, experts=16, xdt=BF, wdt=BF):
+    return torch.zeros(tokens, dim, dtype=xdt), torch.zeros(experts, dim, dtype=wdt)
+
+
+def test_operands_that_fit():
+    from kohakuwullm_amd.kernels.moe.router import can_route, operands_fit
+
+    for xdt, wdt in ((BF, BF), (HF, HF), (F32, F32), (BF, F32), (HF, F32)):
+        x, w = _operands(xdt=xdt, wdt=wdt)
+        assert operands_fit(x, w, 4)
+        assert not can_route(x, w, 4)  # on the CPU
+
+
+@pytest.mark.parametrize("width", [8, 56, 72, 128])
+def test_input_of_another_width_is_refused(width):
+    """The kernels index the router matrix by the input's width: a wider input read past the matrix, and the backward wrote
+    past its gradient."""
+    from kohakuwullm_amd.kernels.moe.router import operands_fit, route_topk
+
+    x, w = torch.zeros(4, width, dtype=BF), _operands()[1]
+    assert not operands_fit(x, w, 4)
+    with pytest.raises(ValueError):
+        route_topk(x, w, None, 4, True, 1.0)
+
+
+def test_other_operands_are_refused():
+    from kohakuwullm_amd.kernels.moe.router import operands_fit
+
+    x, w = _operands()
+    assert not operands_fit(x[0], w, 4) and not operands_fit(x[:0], w, 4) and not operands_fit(x, w.view(16, 8, 8), 4)
+    assert not operands_fit(x, w, 0) and not operands_fit(x, w, 17)
+    assert not operands_fit(x.double(), w, 4) and not operands_fit(x.float(), w, 4) and not operands_fit(x, w.half(), 4)
+    assert not operands_fit(*_operands(dim=60), 4) and not operands_fit(*_operands(experts=257), 4)
+    assert not operands_fit(x, torch.zeros(64, 16, dtype=BF).t(), 4)
+    assert not operands_fit(x, torch.zeros(16 * 64 + 1, dtype=BF)[1:].view(16, 64), 4)
