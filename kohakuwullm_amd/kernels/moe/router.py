@@ -14,19 +14,21 @@ from kohakuwullm_amd import _lib
 MAX_EXPERTS, MAX_TOP_K = 256, 16
 
 
-def operands_fit(x: torch.Tensor, weight: torch.Tensor, top_k: int) -> bool:
+def operands_fit(x: torch.Tensor, weight: torch.Tensor, top_k: int, bias: torch.Tensor | None = None) -> bool:
     """Whether shapes, types and layouts are what the kernels assume; the library sees pointers and cannot check a width."""
     if x.dim() != 2 or weight.dim() != 2:
         return False
     e, d = weight.shape
+    if bias is not None and not (bias.shape == (e,) and bias.dtype in _lib.MX_DTYPE and bias.is_contiguous() and bias.device == x.device):
+        return False
     return (x.shape[0] > 0 and x.shape[1] == d and x.dtype in _lib.MX_DTYPE and weight.dtype in (x.dtype, torch.float32)
             and d % 8 == 0 and e <= MAX_EXPERTS and 0 < top_k <= min(MAX_TOP_K, e) and weight.is_contiguous()
             and weight.device == x.device and weight.data_ptr() % 16 == 0)
 
 
-def can_route(x: torch.Tensor, weight: torch.Tensor, top_k: int) -> bool:
+def can_route(x: torch.Tensor, weight: torch.Tensor, top_k: int, bias: torch.Tensor | None = None) -> bool:
     """Whether the kernels take this call; autocast changes the arithmetic and is not covered."""
-    return x.is_cuda and operands_fit(x, weight, top_k) and not torch.is_autocast_enabled("cuda")
+    return x.is_cuda and operands_fit(x, weight, top_k, bias) and not torch.is_autocast_enabled("cuda")
 
 
 class _RouteTopK(torch.autograd.Function):
@@ -80,6 +82,7 @@ def route_topk(x: torch.Tensor, weight: torch.Tensor, bias: torch.Tensor | None,
     times their scores, normalized over the token's picks when ``norm``.  Differentiable in ``x`` and ``weight`` through
     ``gate``.  See :func:`can_route` for what it takes; other operands are refused here.
     """
-    if not operands_fit(x, weight, top_k):
-        raise ValueError(f"route_topk: x {tuple(x.shape)} {x.dtype}, weight {tuple(weight.shape)} {weight.dtype}, top_k {top_k}")
+    if not operands_fit(x, weight, top_k, bias):
+        raise ValueError(f"route_topk: x {tuple(x.shape)} {x.dtype}, weight {tuple(weight.shape)} {weight.dtype}, top_k {top_k}, "
+                         f"bias {None if bias is None else (tuple(bias.shape), bias.dtype, bias.device)}")
     return _RouteTopK.apply(x, weight, bias, top_k, norm, factor)

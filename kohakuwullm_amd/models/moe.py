@@ -97,7 +97,7 @@ class TopKRouter(nn.Module):
     def _on_kernels(self, x: torch.Tensor) -> bool:
         """Whether the fused kernels evaluate this call: sigmoid scores, one group, no auxiliary loss, shapes they take."""
         return (self.score_func == "sigmoid" and self.n_groups == 1 and self.aux_loss_weight <= 0 and self.z_loss_weight <= 0
-                and can_route(x, self.weight, self.top_k))
+                and can_route(x, self.weight, self.top_k, self.expert_bias))
 
     def route(self, x: torch.Tensor):
         """``(topk_idx (T, k), topk_weight (T, k) in x.dtype, counts (E,) int32)``."""

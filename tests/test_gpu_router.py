@@ -80,6 +80,20 @@ def test_router_module_on_kernels_matches_its_composition():
         assert torch.equal(router.route(x)[1], gate)
 
 
+def test_router_bias_of_another_type_is_composed():
+    """An fp64 bias was accepted by the composition and is again (the kernels know 16-bit and fp32 ones)."""
+    from kohakuwullm_amd.models.moe import TopKRouter
+
+    torch.manual_seed(SEED)
+    router = TopKRouter(128, 16, top_k=4).to(DEV)
+    router.expert_bias.normal_(std=0.02)
+    x = torch.randn(50, 128, device=DEV)
+    idx, gate, counts = router.route(x)
+    router.expert_bias = router.expert_bias.double()
+    again = router.route(x)
+    assert torch.equal(again[0], idx) and torch.equal(again[2], counts) and torch.allclose(again[1], gate, rtol=1e-5, atol=0)
+
+
 def test_router_of_another_width_raises():
     """A block whose router reads another width than it is given: an error, as the composition's product raises it."""
     from kohakuwullm_amd.models.moe import MoEMLP

@@ -41,3 +41,17 @@ def test_other_operands_are_refused():
     assert not operands_fit(*_operands(dim=60), 4) and not operands_fit(*_operands(experts=257), 4)
     assert not operands_fit(x, torch.zeros(64, 16, dtype=BF).t(), 4)
     assert not operands_fit(x, torch.zeros(16 * 64 + 1, dtype=BF)[1:].view(16, 64), 4)
+
+
+def test_bias_that_is_not_the_kernels_is_refused():
+    """The selection bias reaches the kernels as a pointer: its length, type, layout and device are checked on the host."""
+    from kohakuwullm_amd.kernels.moe.router import operands_fit, route_topk
+
+    x, w = _operands()
+    for dtype in (BF, HF, F32):
+        assert operands_fit(x, w, 4, torch.zeros(16, dtype=dtype))
+    for bias in (torch.zeros(16, dtype=torch.float64), torch.zeros(15), torch.zeros(1, 16), torch.zeros(1), torch.zeros(32)[::2],
+                 torch.zeros(1).expand(16), torch.zeros(16, device="meta")):
+        assert not operands_fit(x, w, 4, bias)
+        with pytest.raises(ValueError):
+            route_topk(x, w, bias, 4, True, 1.0)
