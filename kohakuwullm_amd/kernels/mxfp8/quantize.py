@@ -137,14 +137,24 @@ def token_extent(tokens: int) -> int:
     return groups if 16 * (groups - panels) <= panels else panels
 
 
+def aligned_rows(x2d: torch.Tensor) -> torch.Tensor:
+    """``x2d`` if its rows are fetched 16 bytes at a time as they lie, else a copy that is.
+
+    The kernels that have no slower form take nothing else: unit column stride, rows that do not overlap and start on 16-byte
+    boundaries.  A copy and not ``contiguous()``, which returns a contiguous view at an odd offset of its buffer, and a single
+    row of any pitch, as it is.
+    """
+    if (x2d.stride(1) != 1 or x2d.stride(0) < x2d.shape[1] or x2d.stride(0) * x2d.element_size() % 16 or x2d.data_ptr() % 16):
+        return x2d.clone(memory_format=torch.contiguous_format)
+    return x2d
+
+
 def activation_matrix(x: torch.Tensor, compute: torch.dtype) -> torch.Tensor:
     """``x`` flattened to two dimensions as the activation quantizer takes it: in ``compute`` or, to be rounded there, in fp32."""
     x2d = x.reshape(-1, x.shape[-1])
     if x2d.dtype != compute and not (x2d.dtype == torch.float32 and compute in (torch.bfloat16, torch.float16)):
         x2d = x2d.to(compute)
-    if x2d.stride(1) != 1 or x2d.stride(0) * x2d.element_size() % 16 or x2d.data_ptr() % 16:
-        x2d = x2d.contiguous()
-    return x2d
+    return aligned_rows(x2d)
 
 
 ROW_CHUNKS = 0x7FFFFF00  # 8-element chunks one launch of the row quantizers covers

@@ -1,0 +1,85 @@
+"""Activations as programs hold them -- views at odd offsets of flat buffers, slices, broadcast rows -- through the entry points
+whose quantizers fetch 16 bytes at a time: the host's repair on the CPU, the modules on the GPU."""
+
+import pytest
+import torch
+
+from conftest import SEED
+
+DEV = "cuda:0"
+BF, HF, F32 = torch.bfloat16, torch.float16, torch.float32
+
+
+def _views(m, k, dtype, device="cpu"):
+    """Tensors of shape (m, k) and one content each, in layouts the kernels do not take as they are."""
+    g = torch.Generator().manual_seed(SEED)
+    flat = torch.randn(m * k + 8, generator=g).to(dtype).to(device)
+    wide = torch.randn(m, k + 4, generator=g).to(dtype).to(device)
+    return {
+        "offset": flat[4 : 4 + m * k].view(m, k), "odd offset": flat[1 : 1 + m * k].view(m, k), "pitch": wide[:, :k],
+        "broadcast": flat[:k].expand(m, k), "transposed": flat[: m * k].view(k, m).t(), "one row": wide[:1, :k],
+    }
+
+
+@pytest.mark.parametrize("compute,dtype", [(BF, BF), (HF, HF), (BF, F32), (F32, F32)])
+@pytest.mark.parametrize("m", [1, 3, 128])
+def test_activation_matrix_is_what_the_kernels_take(m, compute, dtype):
+    from kohakuwullm_amd.kernels.mxfp8.quantize import activation_matrix
+
+    for name, x in _views(m, 64, dtype).items():
+        got = activation_matrix(x, compute)
+        assert torch.equal(got, x), name
+        assert got.stride(1) == 1 and got.stride(0) >= 64 and got.stride(0) * got.element_size() % 16 == 0 and got.data_ptr() % 16 == 0, name
+    fine = torch.zeros(m, 80, dtype=compute)[:, :64]
+    assert activation_matrix(fine, compute).data_ptr() == fine.data_ptr()  # and is not copied
+
+
+def _modules(dtype):
+    from kohakuwullm_amd.kernels.mxfp8.linear import MXFP8Linear, mxfp8_linear_group
+    from kohakuwullm_amd.models.mlp import MXFP8SwiGLU, SwiGLU
+    from kohakuwullm_amd.models.mxfp8_swap import swap_mxfp8
+
+    torch.manual_seed(SEED)
+    swapped = SwiGLU(256, hidden=384).to(DEV).to(dtype)
+    swap_mxfp8(swapped)
+    layers = torch.nn.ModuleList(MXFP8Linear(256, w) for w in (256, 128)).to(DEV).to(dtype)
+    group = torch.nn.Module()
+    group.layers = layers
+    group.forward = lambda x: torch.cat(mxfp8_linear_group(x, layers), -1)
+    return {"linear": MXFP8Linear(256, 384).to(DEV).to(dtype), "linear, width % 8": MXFP8Linear(256, 100).to(DEV).to(dtype), "group": group,
+            "swapped": swapped, "fused": MXFP8SwiGLU(256, hidden=384).to(DEV).to(dtype)}
+
+
+def _step(module, x, dy, autocast):
+    for p in module.parameters():
+        p.grad = None
+    x = x.detach().requires_grad_(True)
+    with torch.autocast("cuda", dtype=BF, enabled=autocast):
+        y = module(x)
+        with torch.no_grad():
+            alone = module(x)
+    y.backward(dy.to(y.dtype))
+    return [y.detach(), alone, x.grad, *(p.grad for p in module.parameters())]
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("dtype,autocast", [(BF, False), (HF, False), (F32, True)])
+@pytest.mark.parametrize("m", [1, 129, 256])
+def test_modules_take_any_layout(m, dtype, autocast):
+    for label, module in _modules(dtype).items():
+        for name, x in _views(m, 256, dtype, DEV).items():
+            if name == "one row" and m > 1:
+                continue
+            with torch.no_grad(), torch.autocast("cuda", dtype=BF, enabled=autocast):
+                width = module(x).shape[1]
+            plain = (torch.randn(m, width, device=DEV) * 1e-2).to(BF if autocast else dtype)
+            flat = torch.cat((plain.new_zeros(4), plain.reshape(-1)))
+            want = _step(module, x.contiguous().clone(), plain, autocast)
+            for dy in (plain, flat[4:].view(m, width)):  # (autograd leaves a gradient's layout alone)
+                for a, b in zip(_step(module, x, dy, autocast), want):
+                    assert a.dtype == b.dtype and torch.equal(a, b), (label, name)
+        # a gradient that is one row for every token, as a sum over the tokens gives it
+        x = torch.randn(m, 256, device=DEV).to(dtype)
+        row = plain[:1].expand(m, width)
+        for a, b in zip(_step(module, x, row, autocast), _step(module, x, row.clone(memory_format=torch.contiguous_format), autocast)):
+            assert torch.equal(a, b), label
