@@ -10,6 +10,7 @@ from __future__ import annotations
 import torch
 
 from kohakuwullm_amd import _lib
+from kohakuwullm_amd.kernels.mxfp8.quantize import aligned_rows
 
 MAX_EXPERTS, MAX_TOP_K = 256, 16
 
@@ -34,8 +35,6 @@ def can_route(x: torch.Tensor, weight: torch.Tensor, top_k: int, bias: torch.Ten
 class _RouteTopK(torch.autograd.Function):
     @staticmethod
     def forward(ctx, x, weight, bias, top_k, norm, factor):
-        if x.stride(1) != 1 or x.stride(0) * x.element_size() % 16 or x.data_ptr() % 16:
-            x = x.contiguous()
         (t, d), e, dev = x.shape, weight.shape[0], x.device
         need = ctx.needs_input_grad[0] or ctx.needs_input_grad[1]
         idx = torch.empty(t, top_k, device=dev, dtype=torch.int64)
@@ -85,4 +84,5 @@ def route_topk(x: torch.Tensor, weight: torch.Tensor, bias: torch.Tensor | None,
     if not operands_fit(x, weight, top_k, bias):
         raise ValueError(f"route_topk: x {tuple(x.shape)} {x.dtype}, weight {tuple(weight.shape)} {weight.dtype}, top_k {top_k}, "
                          f"bias {None if bias is None else (tuple(bias.shape), bias.dtype, bias.device)}")
-    return _RouteTopK.apply(x, weight, bias, top_k, norm, factor)
+    # a copied input is copied in front of the graph's node, which then keeps the tensor it differentiates
+    return _RouteTopK.apply(aligned_rows(x), weight, bias, top_k, norm, factor)

@@ -80,6 +80,27 @@ def test_router_module_on_kernels_matches_its_composition():
         assert torch.equal(router.route(x)[1], gate)
 
 
+@pytest.mark.parametrize("dtype", [BF, HF, F32])
+@pytest.mark.parametrize("tokens", [1, 37])
+def test_route_takes_any_layout(tokens, dtype):
+    """Views at odd offsets, pitched and broadcast rows: the result and gradients of an aligned copy."""
+    from kohakuwullm_amd.kernels.moe.router import route_topk
+
+    torch.manual_seed(SEED)
+    w = torch.randn(16, 64, device=DEV).to(dtype).requires_grad_(True)
+    flat, wide = torch.randn(tokens * 64 + 1, device=DEV).to(dtype), torch.randn(tokens, 68, device=DEV).to(dtype)
+    up = torch.randn(tokens, 4, device=DEV).to(dtype)
+
+    def step(x):
+        x = x.detach().requires_grad_(True)
+        idx, gate, counts = route_topk(x, w, None, 4, True, 1.0)
+        return [idx, gate.detach(), counts, *torch.autograd.grad(gate, [x, w], up)]
+
+    for x in (flat[1:].view(tokens, 64), wide[:, :64], flat[:64].expand(tokens, 64), flat[: tokens * 64].view(64, tokens).t()):
+        for a, b in zip(step(x), step(x.clone(memory_format=torch.contiguous_format))):
+            assert torch.equal(a, b)
+
+
 def test_router_bias_of_another_type_is_composed():
     """An fp64 bias was accepted by the composition and is again (the kernels know 16-bit and fp32 ones)."""
     from kohakuwullm_amd.models.moe import TopKRouter
