@@ -8,6 +8,8 @@ composition elsewhere.
 from __future__ import annotations
 
 import torch
+import torch.nn.functional as F
+from torch.autograd import forward_ad
 
 from kohakuwullm_amd import _lib
 from kohakuwullm_amd.kernels.mxfp8.quantize import aligned_rows
@@ -27,9 +29,32 @@ def operands_fit(x: torch.Tensor, weight: torch.Tensor, top_k: int, bias: torch.
             and weight.device == x.device and weight.data_ptr() % 16 == 0)
 
 
+def plain_call(*tensors: torch.Tensor) -> bool:
+    """Whether an autograd function may stand for the operators it replaces: nobody traces them (torch.compile, torch.jit, dispatch
+    modes), transforms them (vmap, torch.func, forward mode) or dispatches them itself (tensor subclasses).  A gradient mapped by
+    ``is_grads_batched`` shows by its missing storage alone: its backward runs on a thread that knows of no transform."""
+    return not (torch.compiler.is_compiling() or torch.jit.is_tracing() or torch._C._are_functorch_transforms_active()
+                or forward_ad._current_level >= 0 or torch._C._len_torch_dispatch_stack()
+                or any(type(t) not in (torch.Tensor, torch.nn.Parameter) or not torch._C._has_storage(t) for t in tensors))
+
+
 def can_route(x: torch.Tensor, weight: torch.Tensor, top_k: int, bias: torch.Tensor | None = None) -> bool:
     """Whether the kernels take this call; autocast changes the arithmetic and is not covered."""
-    return x.is_cuda and operands_fit(x, weight, top_k, bias) and not torch.is_autocast_enabled("cuda")
+    return (plain_call(x, weight) and x.is_cuda and operands_fit(x, weight, top_k, bias)
+            and not torch.is_autocast_enabled("cuda"))
+
+
+def composed_gradients(grad, x, weight, idx, norm: bool, factor: float):
+    """``(dx, dweight)`` of the gate weights by PyTorch operators, for backwards that are themselves differentiated or mapped."""
+    scores = F.linear(x.float(), weight.float()).sigmoid()
+    picked, g = scores.gather(1, idx), grad.float() * factor
+    if norm:
+        total = picked.sum(-1, keepdim=True)
+        unit = total.clamp_min(1e-9)
+        along = (g * picked).sum(-1, keepdim=True) / unit
+        g = (g - torch.where(total < 1e-9, torch.zeros_like(along), along)) / unit
+    dlogit = torch.zeros_like(scores).scatter(1, idx, g * picked * (1.0 - picked))
+    return (dlogit @ weight.float()).to(x.dtype), (dlogit.transpose(0, 1) @ x.float()).to(weight.dtype)
 
 
 class _RouteTopK(torch.autograd.Function):
@@ -59,6 +84,10 @@ class _RouteTopK(torch.autograd.Function):
         if grad is None:
             return (None,) * 6
         x, weight, idx, scores = ctx.saved_tensors
+        if torch.is_grad_enabled() or not plain_call(grad):  # create_graph; a vmap over upstream gradients
+            dx, dw = composed_gradients(grad, x, weight, idx, ctx.norm, ctx.factor)
+            return dx if ctx.needs_input_grad[0] else None, dw if ctx.needs_input_grad[1] else None, None, None, None, None
+        x, weight = aligned_rows(x), weight.contiguous()  # as they were saved, unless a saved-tensor hook laid them out anew
         (t, d), e, lib = x.shape, weight.shape[0], _lib.load()
         grad = grad.contiguous()
         dx = torch.empty(t, d, device=x.device, dtype=x.dtype) if ctx.needs_input_grad[0] else None

@@ -101,6 +101,40 @@ def test_route_takes_any_layout(tokens, dtype):
             assert torch.equal(a, b)
 
 
+@pytest.mark.parametrize("norm", [False, True])
+def test_route_differentiated_twice_batched_and_forward(norm):
+    """create_graph, batched upstream gradients and forward mode give what the composition gives."""
+    from torch.autograd import forward_ad
+
+    from kohakuwullm_amd.models.moe import TopKRouter
+
+    torch.manual_seed(SEED)
+    router = TopKRouter(64, 16, top_k=4, norm_topk_prob=norm).to(DEV)
+    x = torch.randn(20, 64, device=DEV).requires_grad_(True)
+    up, ups = torch.randn(20, 4, device=DEV), torch.randn(3, 20, 4, device=DEV)
+    leaves = [x, router.weight]
+
+    def results():
+        gate = router.route(x)[1]
+        first = torch.autograd.grad(gate, leaves, up, create_graph=True)
+        second = torch.autograd.grad(sum(t.pow(2).sum() for t in first), leaves, retain_graph=True)
+        mapped = torch.autograd.grad(gate, leaves, ups, is_grads_batched=True)
+        return [gate, *first, *second, *mapped]
+
+    got, kernel_name = results(), type(router.route(x)[1].grad_fn).__name__
+    with torch.no_grad(), forward_ad.dual_level():
+        tangent = forward_ad.unpack_dual(router.route(forward_ad.make_dual(x.detach(), torch.ones_like(x)))[1]).tangent
+    router.z_loss_weight = 1e-6  # an auxiliary term: the composition throughout
+    want = results()
+    assert kernel_name == "_RouteTopKBackward"
+    # fp32 sums of 64 products of size 1 in another order, two derivatives deep
+    for a, b in zip(got, want):
+        assert torch.allclose(a, b, rtol=1e-4, atol=1e-5)
+    with torch.no_grad(), forward_ad.dual_level():
+        ref = forward_ad.unpack_dual(router.route(forward_ad.make_dual(x.detach(), torch.ones_like(x)))[1]).tangent
+    assert torch.equal(tangent, ref)
+
+
 def test_router_bias_of_another_type_is_composed():
     """An fp64 bias was accepted by the composition and is again (the kernels know 16-bit and fp32 ones)."""
     from kohakuwullm_amd.models.moe import TopKRouter

@@ -3,6 +3,8 @@
 import pytest
 import torch
 
+from conftest import SEED
+
 BF, HF, F32 = torch.bfloat16, torch.float16, torch.float32
 
 
@@ -55,3 +57,52 @@ def test_bias_that_is_not_the_kernels_is_refused():
         assert not operands_fit(x, w, 4, bias)
         with pytest.raises(ValueError):
             route_topk(x, w, bias, 4, True, 1.0)
+
+
+def test_traced_and_transformed_calls_are_composed():
+    """Calls that someone traces, maps or differentiates forward are left to operators those can see."""
+    from torch.autograd import forward_ad
+    from torch.utils._python_dispatch import TorchDispatchMode
+
+    from kohakuwullm_amd.kernels.moe.router import plain_call
+
+    class Seen(TorchDispatchMode):
+        def __torch_dispatch__(self, func, types, args=(), kwargs=None):
+            return func(*args, **(kwargs or {}))
+
+    class Sub(torch.Tensor):
+        pass
+
+    x, seen = torch.zeros(2, 3), []
+    note = lambda t: (seen.append(plain_call(t)), t * 1.0)[1]  # noqa: E731
+    assert plain_call(x, torch.nn.Parameter(x))
+    torch.func.vmap(note)(x)
+    torch.func.jvp(note, (x,), (x,))
+    torch.func.grad(lambda t: note(t).sum())(x)
+    torch.jit.trace(note, x, check_trace=False)
+    with forward_ad.dual_level():
+        note(forward_ad.make_dual(x, x))
+    with Seen():
+        note(x)
+    assert seen == [False] * 6
+    assert not plain_call(x.as_subclass(Sub)) and plain_call(x)
+
+
+@pytest.mark.parametrize("norm", [False, True])
+def test_composed_gradients(norm):
+    """The backward's operators against autograd's of the forward, once and twice differentiated."""
+    from kohakuwullm_amd.kernels.moe.router import composed_gradients
+
+    torch.manual_seed(SEED)
+    x, w, up = (torch.randn(*s).requires_grad_(True) for s in ((5, 8), (6, 8), (5, 3)))
+    scores = (x @ w.T).sigmoid()
+    idx = scores.topk(3, dim=-1).indices
+    gate = scores.gather(1, idx)
+    gate = 1.5 * (gate / gate.sum(-1, keepdim=True).clamp_min(1e-9) if norm else gate)
+    want = torch.autograd.grad(gate, [x, w], up, create_graph=True)
+    got = composed_gradients(up, x, w, idx, norm, 1.5)
+    # fp32 sums of at most 8 terms of size 1, a few roundings each: 64 units of 2^-24 bound both orders
+    close = lambda a, b: torch.allclose(a, b, rtol=64 * 2.0**-24, atol=64 * 2.0**-24)  # noqa: E731
+    assert all(close(a, b) for a, b in zip(got, want))
+    twice = [torch.autograd.grad(sum(t.pow(2).sum() for t in ts), [x, w, up], retain_graph=True) for ts in (got, want)]
+    assert all(torch.allclose(a, b, rtol=1e-4, atol=1e-5) for a, b in zip(*twice))  # a second derivative: ten such sums deep
