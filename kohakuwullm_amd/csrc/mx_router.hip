@@ -17,6 +17,9 @@ namespace mx {
 // so they are kept as exact as fp32 gives them (unlike SwiGLU's sigmoid_f32).
 __device__ __forceinline__ float router_sigmoid(float l) { return 1.0f / (1.0f + expf(-l)); }
 
+// clamp(total, 1e-9) that keeps a NaN (fmaxf drops it: a token with one NaN score would get gates of 1e9 for its other picks)
+__device__ __forceinline__ float clamp_total(float total) { return total < 1e-9f ? 1e-9f : total; }
+
 // Unsigned integers in the order of the floats; NaN above everything, as torch.topk has it.
 __device__ __forceinline__ uint32_t ordered_key(float f) {
     const uint32_t u = f2bits(f);
@@ -216,7 +219,7 @@ __global__ __launch_bounds__(ROUTER_WAVES * 64, MT > 1 ? 2 : NT <= 8 ? 4 : 2) vo
                     open = false;
                 }
             }
-            total = fmaxf(total, 1e-9f);
+            total = clamp_total(total);
             if (lane < p.top_k) {
                 const int64_t at = (int64_t)t * p.top_k + lane;
                 p.idx[at] = mine_e;
@@ -275,8 +278,8 @@ __device__ __forceinline__ void form_picks(const RouterBwdArgs &p, int64_t lo, i
                 sum += other[1];
                 dot += other[0] * other[1];
             }
-            const float S = fmaxf(sum, 1e-9f);
-            ds = (g - (sum >= 1e-9f ? dot / S : 0.0f)) / S;
+            const float S = clamp_total(sum);
+            ds = (g - (sum < 1e-9f ? 0.0f : dot / S)) / S;
         }
         sink(i, ds * s * (1.0f - s), e);
     }

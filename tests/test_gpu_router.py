@@ -81,6 +81,36 @@ def test_router_module_on_kernels_matches_its_composition():
 
 
 @pytest.mark.parametrize("dtype", [BF, HF, F32])
+@pytest.mark.parametrize("what", [float("nan"), float("inf"), -float("inf")])
+def test_scores_that_are_not_finite(what, dtype):
+    """One expert whose scores are NaN or saturated: picks, gates and gradients are not finite where the composition's are not."""
+    from kohakuwullm_amd.models.moe import TopKRouter
+
+    torch.manual_seed(SEED)
+    router = TopKRouter(64, 16, top_k=4).to(DEV).to(dtype)
+    x = torch.randn(40, 64, device=DEV).abs().to(dtype).requires_grad_(True)
+    up = torch.randn(40, 4, device=DEV).to(dtype)
+    with torch.no_grad():
+        router.weight[5, 7] = what
+    results = []
+    for z_loss_weight in (0.0, 1e-6):  # kernels, composition
+        router.z_loss_weight = z_loss_weight
+        idx, gate, counts = router.route(x)
+        results.append([idx, counts, gate.detach(), *torch.autograd.grad(gate, [x, router.weight], up)])
+    for name, a, b in zip(("idx", "counts", "gate", "dx", "dw"), *results):
+        if not a.is_floating_point():
+            assert torch.equal(a, b)
+            continue
+        if name == "dx" and what == -float("inf"):
+            # nobody picks that expert: its gradient of 0 is no term of the kernel's dx, in the dense product it is 0 * inf
+            assert a.isfinite().all()
+            a = torch.where(b.isnan(), b, a)
+        assert torch.equal(a.isnan(), b.isnan()), name
+        # rounding to the type (2^-8 at most), and fp32 sums of 64 products
+        assert torch.allclose(a.float().nan_to_num(), b.float().nan_to_num(), rtol=2.0**-7, atol=2.0**-7), name
+
+
+@pytest.mark.parametrize("dtype", [BF, HF, F32])
 @pytest.mark.parametrize("tokens", [1, 37])
 def test_route_takes_any_layout(tokens, dtype):
     """Views at odd offsets, pitched and broadcast rows: the result and gradients of an aligned copy."""
