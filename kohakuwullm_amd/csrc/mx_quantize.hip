@@ -8,9 +8,6 @@
 #include "mx_common.h"
 
 namespace mx {
-}
-
-namespace mx {
 
 // ------------------------------------------------------------------------------------
 // Row axis.  One lane owns 8 consecutive elements; the 4 lanes of a quad own one block.
@@ -228,6 +225,10 @@ struct QuantTileOut {
 // caller to whole blocks or more: the tile holds zeros for rows past M, they are quantized along
 // the columns like any other, and have no row-axis output.  `tile`/`tscale` are the workgroup's LDS
 // staging buffers; the caller must not touch them until the function's trailing barrier.
+// EDGE = false: no matrix of the launch ends inside a tile (M, MT and K are multiples of the tile), and the stores carry no
+// tests.  us with the tests / without, bf16: both axes of 16384 x 4096 55.4 / 54.6, of 8192 x 2048 15.1 / 14.6, of 4096 x 512
+// 6.9 / 6.4; SwiGLU 4096 x 4096 22.1 / 21.2.
+// COLS: the columns are tested (see the SwiGLU' kernel for the one that keeps the test without EDGE).
 template <int R>
 struct TileGeom {
     static_assert(R == 8 || R == 4, "8 rows x 8 columns or 4 rows x 8 columns per thread");
@@ -238,7 +239,7 @@ struct TileGeom {
     static __device__ __forceinline__ int rg(int t) { return t / CGS; }
 };
 
-template <bool ROWS, int R = 8, bool NTS = false>  // NTS: the code stores carry the non-temporal hint
+template <bool ROWS, int R, bool NTS, bool EDGE, bool COLS = EDGE>  // NTS: the code stores carry the non-temporal hint
 __device__ __forceinline__ void quant_tile(float (&v)[R][8], const QuantTileOut &o, int64_t M, int64_t MT, int64_t K, int64_t m0,
                                            int64_t kc0, uint8_t *tile, uint8_t *tscale) {
     typedef TileGeom<R> G;
@@ -247,8 +248,8 @@ __device__ __forceinline__ void quant_tile(float (&v)[R][8], const QuantTileOut 
     const int cg = G::cg(t), rg = G::rg(t);
     const int64_t col = kc0 + cg * 8;
     const int64_t row0 = m0 + rg * R;
-    const bool col_ok = col < K;
-    const bool whole = m0 + QC_TILE <= M;  // uniform: every row of the tile exists
+    const bool col_ok = !COLS || col < K;
+    const bool whole = !EDGE || m0 + QC_TILE <= M;  // uniform: every row of the tile exists
 
     if (ROWS) {
         // Row-axis outputs: the 4 lanes of a quad hold 32 consecutive columns of a row.
@@ -273,7 +274,7 @@ __device__ __forceinline__ void quant_tile(float (&v)[R][8], const QuantTileOut 
                 codes[1] = (int)pack4_e4m3(v[i][4] * inv, v[i][5] * inv, v[i][6] * inv, v[i][7] * inv);
                 stream_store<NTS>((v2i *)(o.q + (o.q_ks ? (col >> 7) * o.q_ks + (row0 + i) * 128 + (col & 127) : (row0 + i) * o.ldq + col)), codes);
                 uint8_t *sp = o.s + (row0 + i) * o.lds + (col >> 5);
-                bool full = kc0 + G::TK <= K;
+                bool full = !EDGE || kc0 + G::TK <= K;
                 if (o.pack_row_scales && full) {
                     if (cg == 0) {
                         if (R == 8) *(uint32_t *)sp = packed;
@@ -325,7 +326,7 @@ __device__ __forceinline__ void quant_tile(float (&v)[R][8], const QuantTileOut 
 #pragma unroll
     for (int j = 0; j < G::TK / 32; j++) {
         int kr = j * 32 + (t >> 3), ch = t & 7;
-        if (kc0 + kr < K && m0 + ch * 16 < MT) {
+        if (!EDGE || (kc0 + kr < K && m0 + ch * 16 < MT)) {
             const v2i *src = (const v2i *)(tile + kr * QC_PITCH + ch * 16);
             v4i w;
             v2i a = src[0], b = src[1];
@@ -336,9 +337,9 @@ __device__ __forceinline__ void quant_tile(float (&v)[R][8], const QuantTileOut 
             stream_store<NTS>((v4i *)(o.qT + (o.qT_ks ? (m0 >> 7) * o.qT_ks + (kc0 + kr) * 128 : (kc0 + kr) * o.ldqT + m0) + ch * 16), w);
         }
     }
-    if (t < G::TK && kc0 + t < K) {
+    if (t < G::TK && (!EDGE || kc0 + t < K)) {
         uint8_t *sp = o.sT + (kc0 + t) * o.ldsT + (m0 >> 5);
-        int64_t nb = (MT - m0) >> 5;
+        int64_t nb = EDGE ? (MT - m0) >> 5 : 4;
         if (o.pack_col_scales && nb >= 4) {
             *(uint32_t *)sp = *(const uint32_t *)(tscale + t * 4);
         } else {
@@ -348,12 +349,12 @@ __device__ __forceinline__ void quant_tile(float (&v)[R][8], const QuantTileOut 
     __syncthreads();
 }
 
-// quant_tile<ROWS, 8, NTS> for a tile of 16-bit values kept as loaded (r[i]: row i's eight values, packed): every value
+// quant_tile<ROWS, 8, NTS, EDGE> for a tile of 16-bit values kept as loaded (r[i]: row i's eight values, packed): every value
 // is converted where it is used, three times instead of once, and the thread holds 32 registers of tile instead of 64.
 // The plain row + token axis quantizer then fits 64 registers and eight waves per SIMD (90 registers and five with the
 // tile in fp32), so that the 1536 tiles of a 16384 x 1536 activation are resident at once instead of in 1.2 rounds.
 // Same arithmetic on the same values: bit-identical outputs.  gate (token axis alone): a factor for each of the thread's rows.
-template <int DT, bool ROWS, bool NTS>
+template <int DT, bool ROWS, bool NTS, bool EDGE>
 __device__ __forceinline__ void quant_tile_raw(typename Elem<DT>::raw (&r)[8], const QuantTileOut &o, int64_t M, int64_t MT,
                                                int64_t K, int64_t m0, int64_t kc0, uint8_t *tile, uint8_t *tscale,
                                                const float *gate = nullptr) {
@@ -364,7 +365,7 @@ __device__ __forceinline__ void quant_tile_raw(typename Elem<DT>::raw (&r)[8], c
     const int cg = G::cg(t), rg = G::rg(t);
     const int64_t col = kc0 + cg * 8;
     const int64_t row0 = m0 + rg * 8;
-    const bool col_ok = col < K, whole = m0 + QC_TILE <= M;
+    const bool col_ok = !EDGE || col < K, whole = !EDGE || m0 + QC_TILE <= M;
 
     if (ROWS) {
 #pragma unroll
@@ -382,7 +383,7 @@ __device__ __forceinline__ void quant_tile_raw(typename Elem<DT>::raw (&r)[8], c
                 codes[1] = (int)pack4_e4m3(v[4] * inv, v[5] * inv, v[6] * inv, v[7] * inv);
                 stream_store<NTS>((v2i *)(o.q + (o.q_ks ? (col >> 7) * o.q_ks + (row0 + i) * 128 + (col & 127) : (row0 + i) * o.ldq + col)), codes);
                 uint8_t *sp = o.s + (row0 + i) * o.lds + (col >> 5);
-                const bool full = kc0 + G::TK <= K;
+                const bool full = !EDGE || kc0 + G::TK <= K;
                 if (o.pack_row_scales && full) {
                     if (cg == 0) *(uint32_t *)sp = packed;
                 } else if ((cg & 3) == 0) {
@@ -415,16 +416,16 @@ __device__ __forceinline__ void quant_tile_raw(typename Elem<DT>::raw (&r)[8], c
 #pragma unroll
     for (int j = 0; j < G::TK / 32; j++) {
         const int kr = j * 32 + (t >> 3), ch = t & 7;
-        if (kc0 + kr < K && m0 + ch * 16 < MT) {
+        if (!EDGE || (kc0 + kr < K && m0 + ch * 16 < MT)) {
             const v2i *src = (const v2i *)(tile + kr * QC_PITCH + ch * 16);
             const v2i a = src[0], b = src[1];
             stream_store<NTS>((v4i *)(o.qT + (o.qT_ks ? (m0 >> 7) * o.qT_ks + (kc0 + kr) * 128 : (kc0 + kr) * o.ldqT + m0) + ch * 16),
                               v4i{a[0], a[1], b[0], b[1]});
         }
     }
-    if (t < G::TK && kc0 + t < K) {
+    if (t < G::TK && (!EDGE || kc0 + t < K)) {
         uint8_t *sp = o.sT + (kc0 + t) * o.ldsT + (m0 >> 5);
-        const int64_t nb = (MT - m0) >> 5;
+        const int64_t nb = EDGE ? (MT - m0) >> 5 : 4;
         if (o.pack_col_scales && nb >= 4) {
             *(uint32_t *)sp = *(const uint32_t *)(tscale + t * 4);
         } else {
@@ -495,7 +496,7 @@ __global__ __launch_bounds__(256) void quant_cols_kernel(const void *__restrict_
     load_rows_or_zero<DT, R, DUAL, EDGE>(x, row0 * ldx + col, ldx, col < KV ? M - row0 : 0, r);
     if constexpr (RAW) {
         static_assert(DT != MX_FP32 && R == 8, "a packed tile of 16-bit values");
-        quant_tile_raw<DT, DUAL, false>(r, o, M, MT, K, m0, k0, tile, tscale);
+        quant_tile_raw<DT, DUAL, false, EDGE>(r, o, M, MT, K, m0, k0, tile, tscale);
         return;
     }
     float v[R][8];
@@ -504,7 +505,7 @@ __global__ __launch_bounds__(256) void quant_cols_kernel(const void *__restrict_
         Elem<DT>::unpack(r[i], v[i]);
         round_values<CDT>(v[i]);
     }
-    quant_tile<DUAL, R>(v, o, M, MT, K, m0, k0, tile, tscale);
+    quant_tile<DUAL, R, false, EDGE>(v, o, M, MT, K, m0, k0, tile, tscale);
 }
 
 // Several matrices of the same rows quantized as the column panels of one (M, K) matrix: what the gradients of projections
@@ -534,13 +535,13 @@ __global__ __launch_bounds__(256) void quant_side_kernel(SideArgs a, int64_t M, 
     typename Elem<DT>::raw r[8];
     load_rows_or_zero<DT, 8, true, EDGE>(a.x[j], row0 * a.ldx[j] + col, a.ldx[j], M - row0, r);
     if constexpr (RAW) {
-        quant_tile_raw<DT, true, false>(r, o, M, MT, K, m0, k0, tile, tscale);
+        quant_tile_raw<DT, true, false, EDGE>(r, o, M, MT, K, m0, k0, tile, tscale);
         return;
     }
     float v[8][8];
 #pragma unroll
     for (int i = 0; i < 8; i++) Elem<DT>::unpack(r[i], v[i]);
-    quant_tile<true, 8>(v, o, M, MT, K, m0, k0, tile, tscale);
+    quant_tile<true, 8, false, EDGE>(v, o, M, MT, K, m0, k0, tile, tscale);
 }
 
 // Column panels of one code matrix (codes (rows, K), scale bytes (rows, K/32)) copied together from several: 16 codes per
@@ -611,7 +612,7 @@ __global__ __launch_bounds__(256) void rmsnorm_quant_dual_kernel(const void *__r
             for (int c = 0; c < 8; c++) v[i][c] = 0.0f;
         }
     }
-    quant_tile<true, 8>(v, o, M, M, K, m0, k0, tile, tscale);
+    quant_tile<true, 8, false, true>(v, o, M, M, K, m0, k0, tile, tscale);
 }
 
 // Several matrices behind one launch: workgroup `id` finds its matrix in the running tile
@@ -658,7 +659,7 @@ __global__ __launch_bounds__(256) void quant_dual_batch_kernel(QuantBatchArgs b)
             for (int c = 0; c < 8; c++) v[i][c] = 0.0f;
         }
     }
-    quant_tile<true>(v, b.o[j], M, M, K, m0, k0, tile, tscale);
+    quant_tile<true, 8, false, true>(v, b.o[j], M, M, K, m0, k0, tile, tscale);
 }
 
 __device__ __forceinline__ float sigmoid_fast(float x) { return sigmoid_f32(x); }
@@ -700,7 +701,7 @@ __global__ __launch_bounds__(256) void swiglu_quant_dual_kernel(const void *__re
         }
     }
     // hundreds of MB in, hundreds out, nothing of it small enough to be found in a cache by its consumer: all hinted
-    quant_tile<true, R, true>(v, o, M, MT, H, m0, k0, tile, tscale);
+    quant_tile<true, R, true, EDGE>(v, o, M, MT, H, m0, k0, tile, tscale);
 }
 
 // SwiGLU backward fused with both quantizers.  Reads dh (M,H) and the saved projection
@@ -731,6 +732,12 @@ __global__ __launch_bounds__(256) void swiglu_bwd_quant_dual_kernel(const void *
     load_rows_or_last<DT, R, true, EDGE>(gu, row0 * ldgu + col, ldgu, rows, rg);
     load_rows_or_last<DT, R, true, EDGE>(gu, row0 * ldgu + H + col, ldgu, rows, ru);
     load_rows_or_last<DT, R, true, EDGE>(dh, row0 * lddh + col, lddh, rows, rd);
+    // waited for here and not row by row, where the stores of the rows before are waited for too (they count alike)
+    // (16384 x 4096: 126.1 -> 124.9 us with the tests gone; a matrix that ends in a tile gains nothing: 44.5 and 44.9 us at 5003 x 4096)
+    if constexpr (!EDGE) {
+#pragma unroll
+        for (int i = 0; i < R; i++) asm volatile("" : "+v"(rg[i]), "+v"(ru[i]), "+v"(rd[i]));
+    }
 #pragma unroll
     for (int i = 0; i < R; i++) {
         if (i < rows) {  // (always so without EDGE: a block per row all the same, or the compiler takes 256 registers for them)
@@ -770,14 +777,16 @@ __global__ __launch_bounds__(256) void swiglu_bwd_quant_dual_kernel(const void *
         }
     }
     // The gate half occupies output columns [0,H), the up half [H,2H): same tile, shifted.
-    // Columns at or beyond H inside the gate-half tile are masked by passing K = H.
-    quant_tile<true, R, true>(v, o, M, MT, H, m0, k0, tile, tscale);
+    // Columns at or beyond H inside the gate-half tile are masked by passing K = H.  The column test stays without EDGE: as
+    // straight-line code the rows' stores overlap in 175 registers, two waves per SIMD instead of three (16384 x 4096: 134.4 us
+    // without it, 124.9 with it).
+    quant_tile<true, R, true, EDGE, true>(v, o, M, MT, H, m0, k0, tile, tscale);
     QuantTileOut o2 = o;
     o2.q += o.q_ks ? (H >> 7) * o.q_ks : H;
     o2.s += H / MX_BLOCK;
     o2.qT += o.qT_ks ? H * 128 : H * o.ldqT;
     o2.sT += H * o.ldsT;
-    quant_tile<true, R, true>(w, o2, M, MT, H, m0, k0, tile, tscale);
+    quant_tile<true, R, true, EDGE, true>(w, o2, M, MT, H, m0, k0, tile, tscale);
 }
 
 // ------------------------------------------------------------------------------------
@@ -924,7 +933,7 @@ __global__ __launch_bounds__(256) void quant_swiglu_grouped_kernel(GroupedQuantA
             for (int c = 0; c < 8; c++) v[i][c] = 0.0f;
         }
     }
-    quant_tile<false>(v, o, mpad, mpad, a.C, (int64_t)rt * QC_TILE, k0, tile, tscale);
+    quant_tile<false, 8, false, true>(v, o, mpad, mpad, a.C, (int64_t)rt * QC_TILE, k0, tile, tscale);
 }
 
 // SRC_PLAIN.  Bound by the gathered reads and the code stores; what it lacked was waves in flight.  With the tile in fp32 and
@@ -966,7 +975,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(8))) void q
         r[i] = __builtin_bit_cast(typename Elem<DT>::raw, v4i{0, 0, 0, 0});
         if (col < a.C && src >= 0) r[i] = Elem<DT>::load_raw((const T *)a.x + (int64_t)src * a.ldx + col);
     }
-    quant_tile_raw<DT, false, false>(r, o, mpad, mpad, a.C, (int64_t)rt * QC_TILE, k0, tile, tscale, GATED ? gate : nullptr);
+    quant_tile_raw<DT, false, false, true>(r, o, mpad, mpad, a.C, (int64_t)rt * QC_TILE, k0, tile, tscale, GATED ? gate : nullptr);
 }
 
 }  // namespace mx
