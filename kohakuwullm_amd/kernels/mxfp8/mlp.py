@@ -16,10 +16,9 @@ emit the row-blocked operand for the next GEMM and the token-blocked operand for
 from __future__ import annotations
 
 import torch
-import torch.nn.functional as F
 
 from kohakuwullm_amd import _lib
-from kohakuwullm_amd.kernels.mxfp8.linear import TENSORS, compute_dtype, gradient_dtype, unobserved
+from kohakuwullm_amd.kernels.mxfp8.linear import TENSORS, compute_dtype, gradient_dtype, pad_tokens, unobserved
 from kohakuwullm_amd.kernels.mxfp8.quantize import (
     BLOCK_SCALE,
     PANEL,
@@ -92,12 +91,6 @@ def swiglu_bwd_mx_dual(dh: torch.Tensor, gu: torch.Tensor, stage_major: bool = F
         q.data_ptr(), two_h, s.data_ptr(), two_h // BLOCK_SCALE, qt.data_ptr(), m, st.data_ptr(), m // BLOCK_SCALE,
     )
     return q, s, qt, st
-
-
-def pad_tokens(x2d: torch.Tensor) -> torch.Tensor:
-    """``x2d`` with zero rows appended up to the next multiple of 32 tokens (itself when it already is one)."""
-    extra = -x2d.shape[0] % BLOCK_SCALE
-    return F.pad(x2d, (0, 0, 0, extra)) if extra else x2d
 
 
 _WHOLE_RANGE: dict = {}

@@ -241,3 +241,12 @@ def test_moe_block_builds_from_a_reference_spec():
         build({"name": "moe", "score_func": "relu"}, MLP, dim=128)
     loop = build({"name": "moe", "hidden": 128, "num_experts": 4, "top_k": 2, "dense_fallback": True}, MLP, dim=128)
     assert "dense_fallback" in loop.mxfp8_matmul()["w_in"].refusal
+
+
+def test_pad_tokens_stays_importable_from_the_linear_module():
+    from kohakuwullm_amd.kernels.mxfp8.linear import pad_tokens
+
+    x = torch.randn(33, 8)
+    padded = pad_tokens(x)
+    assert padded.shape == (64, 8) and torch.equal(padded[:33], x) and not padded[33:].any()
+    assert pad_tokens(padded) is padded
