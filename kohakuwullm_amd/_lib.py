@@ -91,25 +91,24 @@ SIGNATURES = {
 }
 
 
-def words(rows) -> ctypes.Array:
-    """An array of structures whose fields are all 8 bytes wide (pointers, int64), filled in one call instead of field by field."""
-    return (_i64 * sum(map(len, rows)))(*[v for row in rows for v in row])
+def _record(name: str, doc: str, pointers: str, ints: str) -> type[ctypes.Structure]:
+    fields = [(n, _p) for n in pointers.split()] + [(n, _i64) for n in ints.split()]
+    return type(name, (ctypes.Structure,), {"__doc__": doc, "_fields_": fields})
 
 
-class GemmProblem(ctypes.Structure):
-    """``mx_gemm_problem`` of the C header."""
+# the records of the C header, field by field; all fields are 8 bytes wide
+GemmProblem = _record("GemmProblem", "``mx_gemm_problem``", "aq a_scale bq b_scale c", "M N K lda ldas ldb ldbs ldc")
+QuantProblem = _record("QuantProblem", "``mx_quant_problem``", "x q s qT sT", "M K ldx ldq lds ldqT ldsT")
+SideSource = _record("SideSource", "``mx_side_source``", "x", "K ldx")
+CodeSource = _record("CodeSource", "``mx_code_source``", "codes scales", "K ld lds")
 
-    _fields_ = [(n, _p) for n in ("aq", "a_scale", "bq", "b_scale", "c")] + [
-        (n, _i64) for n in ("M", "N", "K", "lda", "ldas", "ldb", "ldbs", "ldc")
-    ]
 
-
-class QuantProblem(ctypes.Structure):
-    """``mx_quant_problem`` of the C header."""
-
-    _fields_ = [(n, _p) for n in ("x", "q", "s", "qT", "sT")] + [
-        (n, _i64) for n in ("M", "K", "ldx", "ldq", "lds", "ldqT", "ldsT")
-    ]
+def words(record: type[ctypes.Structure], rows) -> ctypes.Array:
+    """An array of ``record``, a tuple of all its fields in order for each, filled in one call instead of field by field."""
+    flat = [v for row in rows for v in row]
+    if any(len(row) != len(record._fields_) for row in rows):
+        raise ValueError(f"{record.__name__} has the fields {[n for n, _ in record._fields_]}")
+    return (_i64 * len(flat))(*flat)
 
 
 _lib: ctypes.CDLL | None = None

@@ -206,7 +206,7 @@ def quantize_side(xs: list[torch.Tensor]):
     Every ``x`` as :func:`activation_matrix` returns it, its width a multiple of 128; at most ``SIDE_MAX`` of them.
     """
     m, k, device = xs[0].shape[0], sum(x.shape[1] for x in xs), xs[0].device
-    sources = _lib.words([(x.data_ptr(), x.shape[1], x.stride(0)) for x in xs])  # mx_side_source each
+    sources = _lib.words(_lib.SideSource, [(x.data_ptr(), x.shape[1], x.stride(0)) for x in xs])
     q = torch.empty(m, k, device=device, dtype=_FP8)
     s = torch.empty(m, k // BLOCK_SCALE, device=device, dtype=torch.uint8)
     qt, st, out_t = token_axis_buffers(m, k, device, True)
@@ -220,8 +220,7 @@ def join_codes(pairs):
     if len(pairs) == 1:
         return pairs[0]
     rows, k, device = pairs[0][0].shape[0], sum(c.shape[1] for c, _ in pairs), pairs[0][0].device
-    # mx_code_source each
-    sources = _lib.words([(c.data_ptr(), s.data_ptr(), c.shape[1], c.stride(0), s.stride(0)) for c, s in pairs])
+    sources = _lib.words(_lib.CodeSource, [(c.data_ptr(), s.data_ptr(), c.shape[1], c.stride(0), s.stride(0)) for c, s in pairs])
     codes = torch.empty(rows, k, device=device, dtype=_FP8)
     scales = torch.empty(rows, k // BLOCK_SCALE, device=device, dtype=torch.uint8)
     _lib.invoke("mx_join_codes", 2 * rows * k * (1 + 1 / BLOCK_SCALE), codes, ctypes.addressof(sources), len(pairs), rows,
@@ -265,7 +264,7 @@ def quantize_mx_dual_batch(xs: list[torch.Tensor]) -> list[tuple[torch.Tensor, t
         at_scale += 2 * n_scales[j]
         work += n_codes[j] * (x.element_size() + 2 * (1 + 1 / BLOCK_SCALE))
     if codes.numel():
-        _lib.invoke("mx_quantize_dual_batch", work, xs[0], ctypes.byref(_lib.words(problems)), len(xs), _lib.MX_DTYPE[xs[0].dtype])
+        _lib.invoke("mx_quantize_dual_batch", work, xs[0], ctypes.byref(_lib.words(_lib.QuantProblem, problems)), len(xs), _lib.MX_DTYPE[xs[0].dtype])
     return out
 
 
@@ -370,7 +369,7 @@ def mxfp8_matmul_pq_batch(problems, out_dtype: torch.dtype = torch.bfloat16) -> 
             *[t.data_ptr() for t in ts], out.data_ptr(), m, n, k, PANEL if ts[0].dim() == 3 else ts[0].stride(0), ts[1].stride(0),
             PANEL if ts[2].dim() == 3 else ts[2].stride(0), ts[3].stride(0), n))
     ws = _lib.gemm_workspace(outs[0])
-    _lib.invoke("mx_gemm_nt_batch", flops, outs[0], ctypes.byref(_lib.words(descs)), len(problems), _lib.MX_DTYPE[out_dtype],
+    _lib.invoke("mx_gemm_nt_batch", flops, outs[0], ctypes.byref(_lib.words(_lib.GemmProblem, descs)), len(problems), _lib.MX_DTYPE[out_dtype],
                 ws.data_ptr(), ws.numel())
     return outs
 

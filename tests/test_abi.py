@@ -101,3 +101,29 @@ def test_entry_points_validate_before_launch():
     assert lib.mx_gemm_nt(None, None, None, None, None, 0, 4, 4, 256, 64, 8, 256, 8, 4, 0, None, 0, None) == _lib.MX_EINVAL  # lda < K, not 128
     assert lib.mx_quantize_dual(None, 0, 0, 64, 64, None, 64, None, 2, None, 128, None, 0, None) == _lib.MX_OK
     assert lib.mx_quantize_dual(None, 0, 160, 64, 64, None, 64, None, 2, None, 128, None, 5, None) == _lib.MX_EINVAL  # panels need M % 128
+
+
+def test_records_match_header():
+    """Every record the binding fills is the header's, field by field; rows of another length are refused."""
+    from kohakuwullm_amd import _lib
+
+    text = re.sub(r"/\*.*?\*/", "", open(os.path.join(ROOT, "include", "mxfp8_hip.h")).read(), flags=re.S)
+    declared = {}
+    for body, name in re.findall(r"typedef struct(?: \w+)? \{(.*?)\}\s*(\w+);", text, flags=re.S):
+        fields = declared[name] = []
+        for base, names in re.findall(r"((?:const )?\w+)\s+([^;]*);", body):
+            for n in names.split(","):
+                assert "*" in n or base == "int64_t", (name, n)
+                fields.append((n.strip(" *\n"), ctypes.c_void_p if "*" in n else ctypes.c_int64))
+    records = {"mx_gemm_problem": _lib.GemmProblem, "mx_quant_problem": _lib.QuantProblem, "mx_side_source": _lib.SideSource,
+               "mx_code_source": _lib.CodeSource}
+    assert set(declared) == set(records)
+    for name, record in records.items():
+        assert record._fields_ == declared[name]
+        n = len(record._fields_)
+        rows = [tuple(range(1 + i * n, 1 + (i + 1) * n)) for i in range(2)]
+        array = ctypes.cast(_lib.words(record, rows), ctypes.POINTER(record))
+        assert [tuple(getattr(array[i], f) for f, _ in record._fields_) for i in range(2)] == rows
+        for wrong in (rows[0][:-1], rows[0] + (0,)):
+            with pytest.raises(ValueError):
+                _lib.words(record, [rows[1], wrong])
