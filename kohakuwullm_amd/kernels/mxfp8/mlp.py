@@ -22,6 +22,7 @@ from kohakuwullm_amd.kernels.mxfp8.linear import TENSORS, compute_dtype, gradien
 from kohakuwullm_amd.kernels.mxfp8.quantize import (
     BLOCK_SCALE,
     PANEL,
+    TILE_ROWS,
     activation_matrix,
     mxfp8_matmul_pq,
     products_by_dtype,
@@ -229,9 +230,12 @@ def mxfp8_swiglu_pair(x, w_in, w_out) -> torch.Tensor | None:
     The activation's two operators and their gradients ran as six library passes over ``(tokens, H)`` or ``(tokens, 2H)``
     matrices, between quantizers that read each result back: 174 us of a 600 us step over 5003 tokens x 1536 x 4096.  Here
     the SwiGLU quantizers do them on the way, with every intermediate rounded as those operators round it.  ``None`` for
-    what this graph does not stand for: a layer someone watches (hooks), padded widths, a type other than bf16 / fp16.
+    what this graph does not stand for: a layer someone watches (hooks), padded widths, a type other than bf16 / fp16, more
+    tokens than its quantizers cover.
     """
     if not (unobserved(w_in) and unobserved(w_out)) or not x.is_cuda or not x.numel() or type(x) not in TENSORS:
+        return None
+    if x.numel() // x.shape[-1] > TILE_ROWS:
         return None
     compute = compute_dtype(x)
     if compute not in (torch.bfloat16, torch.float16) or x.dtype not in _lib.MX_DTYPE or x.shape[-1] != w_in.in_features:

@@ -124,6 +124,9 @@ def quantize_mx_dual(x: torch.Tensor, stage_major_t: bool = False):
     return q, s, qt, st
 
 
+TILE_ROWS = 65535 * PANEL  # rows one launch of the tile quantizers covers (a panel per workgroup along the grid's second axis)
+
+
 def token_extent(tokens: int) -> int:
     """Length of the token axis of a WGRAD operand: whole 128-token panels, whole groups of four where that is nearly free.
 
@@ -134,7 +137,7 @@ def token_extent(tokens: int) -> int:
     """
     panels = -(-tokens // PANEL) * PANEL
     groups = -(-tokens // (4 * PANEL)) * 4 * PANEL
-    return groups if 16 * (groups - panels) <= panels else panels
+    return groups if 16 * (groups - panels) <= panels and groups <= TILE_ROWS else panels
 
 
 def aligned_rows(x2d: torch.Tensor) -> torch.Tensor:
@@ -163,7 +166,7 @@ ROW_CHUNKS = 0x7FFFFF00  # 8-element chunks one launch of the row quantizers cov
 def token_axis_buffers(rows: int, cols: int, device, wanted: bool):
     """``(qT, sT, (pointers and pitch for the library))`` of a token-axis operand over ``rows`` tokens; not ``wanted``: none.
 
-    A matrix past the row quantizers' range gets one all the same: the tile quantizers take any size.
+    A matrix past the row quantizers' range gets one all the same: the tile quantizers take any width.
     """
     if not wanted and rows * cols // 8 < ROW_CHUNKS:
         return None, None, (None, None, 0)
@@ -186,6 +189,8 @@ def quantize_tokens(x: torch.Tensor, compute: torch.dtype, cols: int | None = No
     _check_2d(x, "x")
     m, kv = x.shape
     k = cols or kv
+    if not token_axis and k == kv and m > TILE_ROWS and m * k // 8 >= ROW_CHUNKS:  # past both kernels: the general one
+        return *quantize_mx(x.to(compute)), None, None
     q = torch.empty(m, k, device=x.device, dtype=_FP8)
     s = torch.empty(m, k // BLOCK_SCALE, device=x.device, dtype=torch.uint8)
     qt, st, out_t = token_axis_buffers(m, k, x.device, token_axis or k != kv)

@@ -83,3 +83,48 @@ def test_modules_take_any_layout(m, dtype, autocast):
         row = plain[:1].expand(m, width)
         for a, b in zip(_step(module, x, row, autocast), _step(module, x, row.clone(memory_format=torch.contiguous_format), autocast)):
             assert torch.equal(a, b), label
+
+
+@pytest.mark.parametrize("m,k,entry", [
+    (65535 * 128, 2048, "mx_quantize_tokens"), (65535 * 128 + 1, 1024, "mx_quantize_tokens"),
+    (65535 * 128 + 1, 2080, "mx_quantize_rows"), (2**25, 512, "mx_quantize_rows"),
+])
+def test_forwards_past_the_tile_and_row_kernels_take_the_general_one(monkeypatch, m, k, entry):
+    from kohakuwullm_amd.kernels.mxfp8 import quantize
+
+    calls = []
+    monkeypatch.setattr(quantize._lib, "require_gpu", lambda *a: None)
+    monkeypatch.setattr(quantize._lib, "invoke", lambda name, work, x, *a: calls.append((name, x.dtype)))
+    x = torch.empty(m, k, dtype=F32, device="meta")
+    q, s, qt, st = quantize.quantize_tokens(x, BF, token_axis=False)
+    assert calls == [(entry, BF if entry == "mx_quantize_rows" else F32)]  # rounded in front of it, as a cast would
+    assert q.shape == (m, k) and s.shape == (m, k // 32) and (qt is None) == (st is None)
+
+
+def test_token_extent_stays_within_the_tile_kernels_grid():
+    from kohakuwullm_amd.kernels.mxfp8.quantize import TILE_ROWS, token_extent
+
+    assert token_extent(TILE_ROWS) == TILE_ROWS and token_extent(TILE_ROWS - 128) <= TILE_ROWS
+    assert token_extent(5024) == 5120 and token_extent(2176) == 2176
+
+
+@pytest.mark.gpu
+def test_swapped_block_past_the_tile_kernels(tokens=65535 * 128 + 1):
+    """Frozen weights, more tokens than a token-axis quantizer covers: forward and dX, row by row as in a short batch."""
+    from kohakuwullm_amd.models.mlp import SwiGLU
+    from kohakuwullm_amd.models.mxfp8_swap import swap_mxfp8
+
+    torch.manual_seed(SEED)
+    block = SwiGLU(128, hidden=128).to(DEV).to(BF)
+    swap_mxfp8(block)
+    block.requires_grad_(False)
+    tail = torch.randn(256, 128, device=DEV).to(BF)
+    x = tail.repeat(-(-tokens // 256) + 1, 1)[-tokens:]
+    out = []
+    for part in (x, tail):
+        part = part.detach().requires_grad_(True)
+        y = block(part)
+        y.backward(y.detach())
+        out.append((y.detach()[-256:].clone(), part.grad[-256:].clone()))
+    for a, b in zip(*out):
+        assert torch.equal(a, b)
