@@ -15,6 +15,7 @@ from kohakuwullm_amd import _lib
 from kohakuwullm_amd.kernels.mxfp8.quantize import aligned_rows
 
 MAX_EXPERTS, MAX_TOP_K = 256, 16
+MAX_TOKENS, MAX_WIDTH = 65535 * 256, (1 << 24) - 1  # the backward's grid has 65535 chunks of 256 tokens at most
 
 
 def operands_fit(x: torch.Tensor, weight: torch.Tensor, top_k: int, bias: torch.Tensor | None = None) -> bool:
@@ -24,7 +25,7 @@ def operands_fit(x: torch.Tensor, weight: torch.Tensor, top_k: int, bias: torch.
     e, d = weight.shape
     if bias is not None and not (bias.shape == (e,) and bias.dtype in _lib.MX_DTYPE and bias.is_contiguous() and bias.device == x.device):
         return False
-    return (x.shape[0] > 0 and x.shape[1] == d and x.dtype in _lib.MX_DTYPE and weight.dtype in (x.dtype, torch.float32)
+    return (0 < x.shape[0] <= MAX_TOKENS and x.shape[1] == d <= MAX_WIDTH and x.dtype in _lib.MX_DTYPE and weight.dtype in (x.dtype, torch.float32)
             and d % 8 == 0 and e <= MAX_EXPERTS and 0 < top_k <= min(MAX_TOP_K, e) and weight.is_contiguous()
             and weight.device == x.device and weight.data_ptr() % 16 == 0)
 

@@ -45,6 +45,17 @@ def test_other_operands_are_refused():
     assert not operands_fit(x, torch.zeros(16 * 64 + 1, dtype=BF)[1:].view(16, 64), 4)
 
 
+def test_operands_past_the_grid_are_refused():
+    """Token counts and widths that the backward, or either direction, has no launch for; the composition takes them."""
+    from kohakuwullm_amd.kernels.moe.router import operands_fit
+
+    def fits(tokens, dim):
+        return operands_fit(torch.empty(tokens, dim, dtype=BF, device="meta"), torch.empty(8, dim, dtype=BF, device="meta"), 2)
+
+    assert fits(65535 * 256, 64) and not fits(65535 * 256 + 1, 64)
+    assert fits(4, (1 << 24) - 8) and not fits(4, 1 << 24)
+
+
 def test_bias_that_is_not_the_kernels_is_refused():
     """The selection bias reaches the kernels as a pointer: its length, type, layout and device are checked on the host."""
     from kohakuwullm_amd.kernels.moe.router import operands_fit, route_topk
