@@ -148,7 +148,8 @@ def combine_sorted_rows(y, order, offsets, num_experts, gate, tokens: int, top_k
     m, n = y.shape
     out = torch.empty(tokens, n, device=y.device, dtype=y.dtype)
     reuse = positions is not None
-    if reuse and (positions.numel() != tokens * top_k or positions.dtype != torch.int32 or positions.device != y.device):
+    if reuse and (positions.numel() != tokens * top_k or positions.dtype != torch.int32 or positions.device != y.device
+                  or not positions.is_contiguous()):
         raise ValueError(f"positions {tuple(positions.shape)} {positions.dtype} does not fit {tokens} tokens x top_k {top_k}")
     inv = positions if reuse else torch.empty(tokens * top_k, device=y.device, dtype=torch.int32)
     _lib.invoke(

@@ -250,3 +250,14 @@ def test_pad_tokens_stays_importable_from_the_linear_module():
     padded = pad_tokens(x)
     assert padded.shape == (64, 8) and torch.equal(padded[:33], x) and not padded[33:].any()
     assert pad_tokens(padded) is padded
+
+
+def test_positions_of_another_layout_are_refused():
+    """The combine reads the inverse order through a pointer; a caller's strided or broadcast table would be read out of range."""
+    from kohakuwullm_amd.kernels.mxfp8.moe import combine_sorted_rows
+
+    y, offsets = torch.zeros(8, 16), torch.tensor([0, 8], dtype=torch.int32)
+    table = torch.zeros(16, dtype=torch.int32)
+    for positions in (table[::2], table[:1].expand(8), table[:7], table[:8].long()):
+        with pytest.raises(ValueError, match="positions"):
+            combine_sorted_rows(y, None, offsets, 1, None, 4, 2, positions)
