@@ -88,7 +88,8 @@ class _RouteTopK(torch.autograd.Function):
         if torch.is_grad_enabled() or not plain_call(grad):  # create_graph; a vmap over upstream gradients
             dx, dw = composed_gradients(grad, x, weight, idx, ctx.norm, ctx.factor)
             return dx if ctx.needs_input_grad[0] else None, dw if ctx.needs_input_grad[1] else None, None, None, None, None
-        x, weight = aligned_rows(x), weight.contiguous()  # as they were saved, unless a saved-tensor hook laid them out anew
+        # as they were saved, unless a saved-tensor hook laid them out anew
+        x, weight, idx, scores = aligned_rows(x), aligned_rows(weight.contiguous()), idx.contiguous(), scores.contiguous()
         (t, d), e, lib = x.shape, weight.shape[0], _lib.load()
         grad = grad.contiguous()
         dx = torch.empty(t, d, device=x.device, dtype=x.dtype) if ctx.needs_input_grad[0] else None

@@ -117,3 +117,44 @@ def test_composed_gradients(norm):
     assert all(close(a, b) for a, b in zip(got, want))
     twice = [torch.autograd.grad(sum(t.pow(2).sum() for t in ts), [x, w, up], retain_graph=True) for ts in (got, want)]
     assert all(torch.allclose(a, b, rtol=1e-4, atol=1e-5) for a, b in zip(*twice))  # a second derivative: ten such sums deep
+
+
+@pytest.mark.parametrize("layout", ["offset", "strides"])
+def test_backward_of_operands_that_a_hook_laid_out_anew(monkeypatch, layout):
+    """Saved-tensor hooks may give the operands back at an odd offset or in another order of strides; the kernels get pointers."""
+    import ctypes
+    from types import SimpleNamespace
+
+    from kohakuwullm_amd.kernels.moe import router
+
+    seen = {}
+
+    def invoke(name, work, like, *args):
+        if name == "mx_router_topk_backward":
+            for key, at, size in (("idx", 2, 5 * 3 * 8), ("scores", 3, 5 * 3 * 4), ("x", 4, 5 * 8 * 4), ("weight", 7, 6 * 8 * 4)):
+                seen[key] = args[at] % 16, ctypes.string_at(args[at], size)
+
+    monkeypatch.setattr(router, "_lib", SimpleNamespace(
+        MX_DTYPE=router._lib.MX_DTYPE, invoke=invoke, load=lambda: SimpleNamespace(mx_router_backward_workspace=lambda *a: 1)))
+    kept = []
+
+    def pack(t):
+        kept.append(t.detach())
+        return t
+
+    def unpack(t):
+        t = t.detach()
+        if layout == "strides":
+            return t.t().contiguous().t()
+        return t.new_empty(t.numel() + 1)[1:].view(t.shape).copy_(t)
+
+    torch.manual_seed(SEED)
+    x, w = torch.randn(5, 8).requires_grad_(True), torch.randn(6, 8).requires_grad_(True)
+    with torch.autograd.graph.saved_tensors_hooks(pack, unpack):
+        gate = router.route_topk(x, w, None, 3, True, 1.0)[1]
+    kept[2].copy_(torch.arange(15).view(5, 3) % 6)  # nobody wrote them: no kernel ran
+    kept[3].copy_(torch.arange(15.0).view(5, 3))
+    gate.backward(torch.ones(5, 3))
+    for key, t in zip(("x", "weight", "idx", "scores"), kept):
+        assert seen[key][1] == t.contiguous().numpy().tobytes(), key
+    assert seen["x"][0] == 0 and seen["weight"][0] == 0
