@@ -24,6 +24,7 @@ from kohakuwullm_amd.kernels.mxfp8.quantize import (
     PANEL,
     TILE_ROWS,
     activation_matrix,
+    aligned_rows,
     mxfp8_matmul_pq,
     products_by_dtype,
     quantize_mx_dual,
@@ -148,6 +149,7 @@ def swiglu_tokens(gu: torch.Tensor, rounded: bool = False, token_axis: bool = Tr
 
 def swiglu_bwd_tokens(dh: torch.Tensor, gu: torch.Tensor, rounded: bool = False):
     """``dpre = [dgate | dup]`` as ``(q, s, qT, sT)``, both code matrices stage-major, for any token count (``H % 128 == 0``)."""
+    gu = aligned_rows(gu)  # as the product wrote it, unless a saved-tensor hook laid it out anew
     m, two_h = gu.shape
     h, dev, mt = two_h // 2, gu.device, token_extent(m)
     q = torch.empty(two_h // PANEL, m, PANEL, device=dev, dtype=_FP8)

@@ -152,6 +152,11 @@ def aligned_rows(x2d: torch.Tensor) -> torch.Tensor:
     return x2d
 
 
+def packed(t: torch.Tensor, alignment: int) -> torch.Tensor:
+    """``t`` if it is contiguous at a multiple of ``alignment`` bytes, as what the quantizers made is, else a copy that is."""
+    return t if t.is_contiguous() and t.data_ptr() % alignment == 0 else t.clone(memory_format=torch.contiguous_format)
+
+
 def activation_matrix(x: torch.Tensor, compute: torch.dtype) -> torch.Tensor:
     """``x`` flattened to two dimensions as the activation quantizer takes it: in ``compute`` or, to be rounded there, in fp32."""
     x2d = x.reshape(-1, x.shape[-1])
@@ -224,6 +229,7 @@ def join_codes(pairs):
     """``(torch.cat(codes, 1), torch.cat(scales, 1))`` of quantized matrices of one height, widths multiples of 128."""
     if len(pairs) == 1:
         return pairs[0]
+    pairs = [(packed(c, 16), packed(s, 4)) for c, s in pairs]
     rows, k, device = pairs[0][0].shape[0], sum(c.shape[1] for c, _ in pairs), pairs[0][0].device
     sources = _lib.words(_lib.CodeSource, [(c.data_ptr(), s.data_ptr(), c.shape[1], c.stride(0), s.stride(0)) for c, s in pairs])
     codes = torch.empty(rows, k, device=device, dtype=_FP8)
@@ -359,13 +365,12 @@ def mxfp8_matmul_pq_batch(problems, out_dtype: torch.dtype = torch.bfloat16) -> 
             )
         _lib.require_gpu(aq, "aq")
         ts = []
+        if aq.dim() == 3 or bq.dim() == 3:  # no slower kernel reads these, so neither operand may need one
+            aq, bq = (packed(t, 16) if t.dim() == 3 else aligned_rows(t) for t in (aq, bq))
         for t in (aq, a_scale, bq, b_scale):
             if t.element_size() != 1:
                 raise ValueError(f"codes and scales must be 1-byte tensors, got {t.dtype}")
-            if t.dim() == 3:
-                ts.append(t.contiguous())
-            else:
-                ts.append(t if t.stride(1) == 1 else t.contiguous())
+            ts.append(t if t.dim() == 3 or t.stride(1) == 1 else t.contiguous())
         out = torch.empty(m, n, device=aq.device, dtype=out_dtype)
         keep.append(ts)
         outs.append(out)

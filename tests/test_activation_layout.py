@@ -128,3 +128,57 @@ def test_swapped_block_past_the_tile_kernels(tokens=65535 * 128 + 1):
         out.append((y.detach()[-256:].clone(), part.grad[-256:].clone()))
     for a, b in zip(*out):
         assert torch.equal(a, b)
+
+
+def _off(t):
+    """A copy of ``t`` one element past an allocation's start, as an arena of a saved-tensor hook may give it back."""
+    return t.new_empty(t.numel() + 1)[1:].view(t.shape).copy_(t)
+
+
+def test_saved_operands_at_odd_offsets_are_laid_back(monkeypatch):
+    """What reaches the kernels that take aligned operands alone: stage-major codes, joined weights, the saved projection."""
+    import ctypes
+
+    from kohakuwullm_amd import _lib
+    from kohakuwullm_amd.kernels.mxfp8 import mlp, quantize
+
+    seen = {}
+    monkeypatch.setattr(_lib, "require_gpu", lambda *a: None)
+    monkeypatch.setattr(_lib, "gemm_workspace", lambda t: torch.empty(1))
+    monkeypatch.setattr(_lib, "invoke", lambda name, work, like, *args: seen.__setitem__(name, (args, _records(name, args))))
+
+    def _records(name, args):
+        record = {"mx_join_codes": _lib.CodeSource, "mx_gemm_nt_batch": _lib.GemmProblem}.get(name)
+        if record is None:
+            return None
+        at = args[0] if isinstance(args[0], int) else ctypes.addressof(args[0]._obj)
+        return [{n: getattr(r, n) for n, _ in record._fields_} for r in (record * args[1]).from_buffer_copy(ctypes.string_at(at, ctypes.sizeof(record) * args[1]))]
+
+    f8, u8 = torch.float8_e4m3fn, torch.uint8
+    codes, scales = torch.zeros(256, 128).to(f8), torch.zeros(256, 4, dtype=u8)
+    quantize.join_codes([(_off(codes), _off(scales)), (codes, scales)])
+    for r in seen["mx_join_codes"][1]:
+        assert r["codes"] % 16 == 0 and r["ld"] == 128 and r["scales"] % 4 == 0 and r["lds"] == 4
+    panels = codes.view(2, 128, 128)
+    s8 = torch.zeros(128, 8, dtype=u8)
+    quantize.mxfp8_matmul_pq_batch([(_off(panels), s8, _off(panels), s8), (panels, s8, _off(codes.view(128, 256)), s8)])
+    for r in seen["mx_gemm_nt_batch"][1]:
+        assert r["aq"] % 16 == 0 and r["bq"] % 16 == 0
+    mlp.swiglu_bwd_tokens(torch.zeros(5, 128, dtype=BF), _off(torch.zeros(5, 256, dtype=BF)))
+    assert seen["mx_swiglu_bwd_quantize_tokens"][0][2] % 16 == 0
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("dtype,autocast", [(BF, False), (F32, True)])
+def test_modules_under_a_saved_tensor_hook(dtype, autocast):
+    for label, module in _modules(dtype).items():
+        x = torch.randn(129, 256, device=DEV).to(dtype)
+        with torch.no_grad(), torch.autocast("cuda", dtype=BF, enabled=autocast):
+            dy = torch.randn_like(module(x)) * 1e-2
+        want = _step(module, x, dy, autocast)
+        with torch.autograd.graph.saved_tensors_hooks(_off, lambda t: t):
+            got = _step(module, x, dy, autocast)
+        for a, b in zip(got, want):
+            # products of row-major weights at odd offsets run on the element-wise kernel: fp32 sums in another order, and a
+            # 16-bit result rounded the other way is off by 2^-8 of itself at most
+            assert a.dtype == b.dtype and float((a - b).float().norm()) <= 4e-3 * float(b.float().norm()), label
