@@ -526,12 +526,16 @@ static int ring_slices(const DenseArgs &a, int free_tiles) {
     return best;
 }
 
-// ... and whether it should.  Both kernels are priced in us from what they were measured to take (operands cold): a ring
-// workgroup 0.52 per stage and 1.5 per tile on top of 6, the persistent kernel 1.4 per stage of a 256 x 256 tile (1.6 with
+// ... and whether it should.  Both kernels are priced in us from what they were measured to take: a ring
+// workgroup 0.52 per stage and 1.5 per tile on top of 6 (K = 2048 against 4096 gives per stage, operands in cache / from HBM,
+// 0.37 / 0.63 on 16 tiles, 0.38 / 0.67 on 48 and 0.48 / 0.73 on 256), the persistent kernel 1.4 per stage of a 256 x 256 tile (1.6 with
 // more than half of the CUs busy), four stages per tile and 3, or, the last round's K stages dealt out evenly, its share of
 // the work and about 35 for the fp32 pieces.  us persistent / ring where the line lies: 1500 x 1536 x 4096 50.1 / 20.0, 2048 x 2048
 // x 3072 41.1 / 18.7, 3001 x 2048 x 2048 29.6 / 22.2, 5003 x 1536 x 4096 54.3 / 43.4, 16384 x 512 x 2048 32.3 / 29.0, 3000 x 3072 x 2048
 // 30.6 / 30.3, 4096 x 3072 x 2048 32.0 / 32.4, 2048 x 2048 x 16384 82.4 / 79.4, 5003 x 8192 x 1536 73 / 85, 1536 x 4096 x 16384 105 / 140.
+// A caller without a workspace gets neither K slices nor dealt stages.  The choice holds there too where slices were priced:
+// such a product has at most one tile per CU, and one round of whole ring tiles (0.52 per stage) is under one of whole large
+// ones (1.4).
 static bool ring_pays(const DenseArgs &a) {
     if (!ring_ok(a)) return false;
     const int64_t small = tiles_of(a, 128), large = tiles_of(a, 256), cus = num_cus();

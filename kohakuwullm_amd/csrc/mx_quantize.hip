@@ -354,7 +354,8 @@ __device__ __forceinline__ void quant_tile(float (&v)[R][8], const QuantTileOut 
 // The plain row + token axis quantizer then fits 64 registers and eight waves per SIMD (90 registers and five with the
 // tile in fp32), so that the 1536 tiles of a 16384 x 1536 activation are resident at once instead of in 1.2 rounds.
 // Same arithmetic on the same values: bit-identical outputs.  gate (token axis alone): a factor for each of the thread's rows.
-template <int DT, bool ROWS, bool NTS, bool EDGE>
+// COLS: the columns are tested in front of the row stores (see quant_cols_kernel for who keeps the test without EDGE).
+template <int DT, bool ROWS, bool NTS, bool EDGE, bool COLS = EDGE>
 __device__ __forceinline__ void quant_tile_raw(typename Elem<DT>::raw (&r)[8], const QuantTileOut &o, int64_t M, int64_t MT,
                                                int64_t K, int64_t m0, int64_t kc0, uint8_t *tile, uint8_t *tscale,
                                                const float *gate = nullptr) {
@@ -365,7 +366,7 @@ __device__ __forceinline__ void quant_tile_raw(typename Elem<DT>::raw (&r)[8], c
     const int cg = G::cg(t), rg = G::rg(t);
     const int64_t col = kc0 + cg * 8;
     const int64_t row0 = m0 + rg * 8;
-    const bool col_ok = !EDGE || col < K, whole = !EDGE || m0 + QC_TILE <= M;
+    const bool col_ok = !COLS || col < K, whole = !EDGE || m0 + QC_TILE <= M;
 
     if (ROWS) {
 #pragma unroll
@@ -479,7 +480,8 @@ __device__ __forceinline__ void load_rows_or_zero(const void *x, int64_t first, 
 // RAW (16-bit inputs, R = 8): the tile stays packed as loaded (quant_tile_raw): 64 registers, eight waves per SIMD.
 // x has M rows and KV columns, the outputs MT and K (both rounded up by the caller): what lies past x is zero.
 // CDT: the type fp32 values are rounded to before they are quantized (MX_FP32: none).
-template <int DT, bool DUAL, int R, bool EDGE, bool RAW = false, int CDT = MX_FP32>
+// COLS: the thread's loads and row stores stand behind a test of its tile, also where every tile is whole (see launch_cols).
+template <int DT, bool DUAL, int R, bool EDGE, bool RAW = false, int CDT = MX_FP32, bool COLS = EDGE>
 __global__ __launch_bounds__(256) void quant_cols_kernel(const void *__restrict__ x, int64_t M, int64_t MT, int64_t KV, int64_t K,
                                                           int64_t ldx, QuantTileOut o) {
     typedef TileGeom<R> G;
@@ -493,10 +495,14 @@ __global__ __launch_bounds__(256) void quant_cols_kernel(const void *__restrict_
     typename Elem<DT>::raw r[R];
     // both axes at once is the activation path of a training step, where the 16-bit input is not read again soon: its
     // loads carry the non-temporal hint; the codes are read by the next GEMM and are stored plainly
-    load_rows_or_zero<DT, R, DUAL, EDGE>(x, row0 * ldx + col, ldx, col < KV ? M - row0 : 0, r);
+    if constexpr (COLS && !EDGE) {
+        if (col < KV && row0 < M) load_rows<DT, R, DUAL>(x, row0 * ldx + col, ldx, r);  // always so
+    } else {
+        load_rows_or_zero<DT, R, DUAL, EDGE>(x, row0 * ldx + col, ldx, col < KV ? M - row0 : 0, r);
+    }
     if constexpr (RAW) {
         static_assert(DT != MX_FP32 && R == 8, "a packed tile of 16-bit values");
-        quant_tile_raw<DT, DUAL, false, EDGE>(r, o, M, MT, K, m0, k0, tile, tscale);
+        quant_tile_raw<DT, DUAL, false, EDGE, COLS>(r, o, M, MT, K, m0, k0, tile, tscale);
         return;
     }
     float v[R][8];
@@ -520,7 +526,7 @@ struct SideArgs {
     int count;
 };
 
-template <int DT, bool EDGE, bool RAW>
+template <int DT, bool EDGE, bool RAW, bool COLS = EDGE>  // COLS as in quant_cols_kernel
 __global__ __launch_bounds__(256) void quant_side_kernel(SideArgs a, int64_t M, int64_t MT, int64_t K, QuantTileOut o) {
     typedef TileGeom<8> G;
     typedef typename Elem<DT>::type T;
@@ -533,9 +539,13 @@ __global__ __launch_bounds__(256) void quant_side_kernel(SideArgs a, int64_t M, 
     const int64_t col = k0 - (int64_t)(j ? a.tile_end[j - 1] : 0) * G::TK + G::cg(t) * 8;
     const int64_t row0 = m0 + G::rg(t) * 8;
     typename Elem<DT>::raw r[8];
-    load_rows_or_zero<DT, 8, true, EDGE>(a.x[j], row0 * a.ldx[j] + col, a.ldx[j], M - row0, r);
+    if constexpr (COLS && !EDGE) {
+        if (row0 < M) load_rows<DT, 8, true>(a.x[j], row0 * a.ldx[j] + col, a.ldx[j], r);  // always so
+    } else {
+        load_rows_or_zero<DT, 8, true, EDGE>(a.x[j], row0 * a.ldx[j] + col, a.ldx[j], M - row0, r);
+    }
     if constexpr (RAW) {
-        quant_tile_raw<DT, true, false, EDGE>(r, o, M, MT, K, m0, k0, tile, tscale);
+        quant_tile_raw<DT, true, false, EDGE, COLS>(r, o, M, MT, K, m0, k0, tile, tscale);
         return;
     }
     float v[8][8];
@@ -1061,13 +1071,20 @@ static int launch_cols(const void *x, int64_t M, int64_t MT, int64_t KV, int64_t
     // Both axes of a 16-bit matrix whose tiles are all resident at once with eight waves per SIMD, but not with the five
     // the fp32 tile allows, go to the packed-tile kernel: 16384 x 1536 (1536 tiles on 256 CUs) 27.0 -> 24.9 us.  Larger
     // matrices run several rounds either way and are faster with fewer, fatter waves (16384 x 4096: 54.4 against 58.9 us).
+    // Launches of whole tiles carry no tests, but for those of more than four and up to six tiles per CU, which are faster
+    // with a test around a thread's loads and row stores.  us without / with, bf16: 8192 x 2048 (1024 tiles) 15.1 / 16.0,
+    // 9216 x 2048 19.5 / 17.6, 4096 x 5120 (1280) 20.5 / 17.6, 16384 x 1536 24.0 / 23.1, 14336 x 2048 (1792) 26.2 / 26.6,
+    // 16384 x 2048 29.3 / 30.6.
     const dim3 block(256);
     const bool edge = M % QC_TILE || K % QC_TILE || MT != M || KV != K;
 #define MX_LAUNCH_COLS(...)                                                                                                   \
     (edge ? quant_cols_kernel<DT, DUAL, MX_QR_COLS, true, __VA_ARGS__><<<grid, block, 0, st>>>(x, M, MT, KV, K, ldx, o)       \
           : quant_cols_kernel<DT, DUAL, MX_QR_COLS, false, __VA_ARGS__><<<grid, block, 0, st>>>(x, M, MT, KV, K, ldx, o))
     if constexpr (DT != MX_FP32 && DUAL) {
-        if ((int64_t)grid.x * grid.y <= 8 * (int64_t)num_cus()) MX_LAUNCH_COLS(true);
+        const int64_t tiles = (int64_t)grid.x * grid.y, cus = num_cus();
+        if (tiles > 4 * cus && tiles <= 6 * cus && !edge)
+            quant_cols_kernel<DT, true, MX_QR_COLS, false, true, MX_FP32, true><<<grid, block, 0, st>>>(x, M, MT, KV, K, ldx, o);
+        else if (tiles <= 8 * cus) MX_LAUNCH_COLS(true);
         else MX_LAUNCH_COLS(false);
     } else if constexpr (DUAL) {
         if (cast == MX_BF16) MX_LAUNCH_COLS(false, MX_BF16);
@@ -1424,13 +1441,16 @@ extern "C" int mx_quantize_tokens(const void *x, int x_dtype, int cast_dtype, in
 
 template <int DT>
 static int launch_side(const SideArgs &a, int64_t M, int64_t MT, int64_t K, dim3 grid, const QuantTileOut &o, hipStream_t st) {
-    const bool raw = (int64_t)grid.x * grid.y <= 8 * (int64_t)num_cus();  // as launch_cols
+    const int64_t tiles = (int64_t)grid.x * grid.y, cus = num_cus();
+    // as launch_cols; without / with the tests, K = 3072: 6144 rows (1152 tiles) 20.1 / 17.9 us, 8192 24.2 / 23.3, 9216 26.3 / 27.5
+    const bool raw = tiles <= 8 * cus, tested = tiles > 4 * cus && tiles <= 6 * cus;
     const dim3 block(256);
     if (M != MT) {
         if (raw) quant_side_kernel<DT, true, true><<<grid, block, 0, st>>>(a, M, MT, K, o);
         else quant_side_kernel<DT, true, false><<<grid, block, 0, st>>>(a, M, MT, K, o);
     } else {
-        if (raw) quant_side_kernel<DT, false, true><<<grid, block, 0, st>>>(a, M, MT, K, o);
+        if (raw && tested) quant_side_kernel<DT, false, true, true><<<grid, block, 0, st>>>(a, M, MT, K, o);
+        else if (raw) quant_side_kernel<DT, false, true><<<grid, block, 0, st>>>(a, M, MT, K, o);
         else quant_side_kernel<DT, false, false><<<grid, block, 0, st>>>(a, M, MT, K, o);
     }
     MX_LAUNCH_CHECK();

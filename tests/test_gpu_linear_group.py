@@ -22,7 +22,7 @@ def _randn(*shape, scale=1.0):
 
 
 @pytest.mark.parametrize("m,widths,dtype", [(1, (128,), BF), (129, (256, 128), HF), (5003, (512, 128, 128), BF), (70000, (384, 128, 256), BF),
-                                            (256, (128,) * 8, BF)])
+                                            (256, (128,) * 8, BF), (6144, (2048, 512, 512), BF)])
 def test_quantize_side_and_join(m, widths, dtype):
     from kohakuwullm_amd.kernels.mxfp8.quantize import activation_matrix, join_codes, quantize_side, quantize_tokens
 

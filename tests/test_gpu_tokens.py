@@ -24,8 +24,9 @@ def _draw(*shape, dtype=BF, scale=1.0):
 @pytest.mark.parametrize("m,kv,k,dtype,compute", [
     (1, 32, 32, BF, BF), (31, 128, 128, HF, HF), (33, 104, 128, BF, BF), (128, 256, 256, F32, F32), (129, 1000, 1024, BF, BF),
     (700, 160, 160, F32, BF), (1535, 256, 256, F32, HF), (5003, 512, 512, BF, BF), (70000, 1536, 1536, HF, HF),
-    # whole tiles, whose kernels test nothing: a few of them (kept as loaded) and more than eight per CU
-    (512, 384, 384, HF, HF), (16384, 2176, 2176, BF, BF),
+    # whole tiles, whose kernels test nothing: a few of them (kept as loaded) and more than eight per CU; four and a half
+    # per CU, which are tested all the same
+    (512, 384, 384, HF, HF), (16384, 2176, 2176, BF, BF), (9216, 2048, 2048, HF, HF), (6144, 3072, 3072, BF, BF),
 ])
 def test_quantize_tokens(oracle, m, kv, k, dtype, compute):
     from kohakuwullm_amd.kernels.mxfp8.quantize import activation_matrix, quantize_tokens, rows_of_stage_major, token_extent
