@@ -115,5 +115,10 @@ def route_topk(x: torch.Tensor, weight: torch.Tensor, bias: torch.Tensor | None,
     if not operands_fit(x, weight, top_k, bias):
         raise ValueError(f"route_topk: x {tuple(x.shape)} {x.dtype}, weight {tuple(weight.shape)} {weight.dtype}, top_k {top_k}, "
                          f"bias {None if bias is None else (tuple(bias.shape), bias.dtype, bias.device)}")
+    return route_fitting(x, weight, bias, top_k, norm, factor)
+
+
+def route_fitting(x, weight, bias, top_k: int, norm: bool, factor: float):
+    """:func:`route_topk` of operands that :func:`can_route` has just looked at (a second look takes 2.6 us)."""
     # a copied input is copied in front of the graph's node, which then keeps the tensor it differentiates
     return _RouteTopK.apply(aligned_rows(x), weight, bias, top_k, norm, factor)

@@ -147,7 +147,8 @@ def aligned_rows(x2d: torch.Tensor) -> torch.Tensor:
     boundaries.  A copy and not ``contiguous()``, which returns a contiguous view at an odd offset of its buffer, and a single
     row of any pitch, as it is.
     """
-    if (x2d.stride(1) != 1 or x2d.stride(0) < x2d.shape[1] or x2d.stride(0) * x2d.element_size() % 16 or x2d.data_ptr() % 16):
+    pitch, unit = x2d.stride()
+    if unit != 1 or pitch < x2d.shape[1] or pitch * x2d.element_size() % 16 or x2d.data_ptr() % 16:
         return x2d.clone(memory_format=torch.contiguous_format)
     return x2d
 

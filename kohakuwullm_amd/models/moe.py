@@ -25,7 +25,7 @@ import torch.nn as nn
 import torch.nn.functional as F
 
 from kohakuwullm_amd.kernels.moe.moe_dispatch import combine_routed, expert_counts, expert_sort, expert_sort_positions  # noqa: F401  (expert_sort: importable from here)
-from kohakuwullm_amd.kernels.moe.router import can_route, route_topk
+from kohakuwullm_amd.kernels.moe.router import can_route, route_fitting, route_topk  # noqa: F401  (route_topk: importable from here)
 from kohakuwullm_amd.kernels.mxfp8.linear import compute_dtype
 from kohakuwullm_amd.kernels.mxfp8.moe import (
     MXFP8ExpertWeights,
@@ -103,8 +103,8 @@ class TopKRouter(nn.Module):
         """``(topk_idx (T, k), topk_weight (T, k) in x.dtype, counts (E,) int32)``."""
         if self._on_kernels(x):
             self.aux_loss = self.z_loss = None
-            topk_idx, topk_weight, counts = route_topk(x, self.weight, self.expert_bias, self.top_k,
-                                                       self.norm_topk_prob and self.top_k > 1, self.routed_scaling_factor)
+            topk_idx, topk_weight, counts = route_fitting(x, self.weight, self.expert_bias, self.top_k,
+                                                          self.norm_topk_prob and self.top_k > 1, self.routed_scaling_factor)
             if self.training and self.load_accum is not None:
                 self.load_accum += counts
             return topk_idx, topk_weight, counts
