@@ -384,7 +384,8 @@ __global__ __launch_bounds__(RingShape::NTHR, 2) void gemm_nt_ring_kernel(RingAr
     int j = 0;
     while (j + 1 < b.count && (int)blockIdx.x >= b.end[j]) j++;
     DenseProblem<RingShape, CDT> prob(b.prob[j], (int)blockIdx.x - (j ? b.end[j - 1] : 0), 0x40000000);
-    ring_gemm(prob, smem);
+    if (b.prob[j].K < 512) ring_gemm_short(prob, smem);
+    else ring_gemm(prob, smem);
 }
 
 // slice_reduce for every problem of such a launch that was cut along K (`end` counts blocks of those).
@@ -503,9 +504,9 @@ static int scale_mode(const DenseArgs &a) {
     return SCALES_BYTES;
 }
 
-// Whether a product can go to the ring kernel: whole groups of four stages, no accumulation, scale rows the copy engine takes.
+// Whether a product can go to the ring kernel: whole stages, no accumulation, scale rows the copy engine takes.
 static bool ring_ok(const DenseArgs &a) {
-    return a.K % 512 == 0 && a.split_k == 1 && !a.accumulate && aligned(a.as, 4) && aligned(a.bs, 4) && a.ldas % 4 == 0 && a.ldbs % 4 == 0 &&
+    return a.K % 128 == 0 && a.split_k == 1 && !a.accumulate && aligned(a.as, 4) && aligned(a.bs, 4) && a.ldas % 4 == 0 && a.ldbs % 4 == 0 &&
            (int64_t)a.M * a.ldas < ((int64_t)1 << 32) && (int64_t)a.N * a.ldbs < ((int64_t)1 << 32);
 }
 
@@ -533,6 +534,8 @@ static int ring_slices(const DenseArgs &a, int free_tiles) {
 // the work and about 35 for the fp32 pieces.  us persistent / ring where the line lies: 1500 x 1536 x 4096 50.1 / 20.0, 2048 x 2048
 // x 3072 41.1 / 18.7, 3001 x 2048 x 2048 29.6 / 22.2, 5003 x 1536 x 4096 54.3 / 43.4, 16384 x 512 x 2048 32.3 / 29.0, 3000 x 3072 x 2048
 // 30.6 / 30.3, 4096 x 3072 x 2048 32.0 / 32.4, 2048 x 2048 x 16384 82.4 / 79.4, 5003 x 8192 x 1536 73 / 85, 1536 x 4096 x 16384 105 / 140.
+// K needs no whole groups of four stages (the token axis of a batch of odd length): both gradients of 512 -> 1536 over 2304 tokens
+// 29.2 / 11.8, of 1536 -> 1536 over 640 22.2 / 10.2, 4352 x 1024 x 2816 36.5 / 26.8.
 // A caller without a workspace gets neither K slices nor dealt stages.  The choice holds there too where slices were priced:
 // such a product has at most one tile per CU, and one round of whole ring tiles (0.52 per stage) is under one of whole large
 // ones (1.4).

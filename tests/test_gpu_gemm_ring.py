@@ -46,6 +46,22 @@ def test_ring_gemm(oracle, m, n, k, dtype):
     assert torch.equal(mxfp8_matmul_pq(*_dev(ops, panels=True), dtype), out)
 
 
+@pytest.mark.parametrize("m,n,k", [
+    (1, 1, 128), (130, 300, 128), (257, 129, 256), (128, 264, 384), (3, 2048, 384),  # without a whole group
+    (1, 1, 640), (129, 130, 768), (5, 257, 896), (128, 128, 1152), (300, 40, 1408), (513, 260, 2176),
+    (16, 40, 8320), (130, 200, 16384 + 384),  # K slices whose last one ends inside a group
+])
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+def test_ring_gemm_ends_inside_a_group(oracle, m, n, k, dtype):
+    """One to three stages in the last group, or in all; the matrices end where their allocations do."""
+    from kohakuwullm_amd.kernels.mxfp8 import mxfp8_matmul_pq
+
+    ops = _operands(oracle, m, n, k)
+    out = mxfp8_matmul_pq(*_dev(ops), dtype)
+    assert oracle.rel_error(out.cpu(), oracle.gemm_nt(*ops)) < TOL[dtype]
+    assert torch.equal(mxfp8_matmul_pq(*_dev(ops, panels=True), dtype), out)
+
+
 def test_ring_gemm_several_products_in_one_launch(oracle):
     from kohakuwullm_amd.kernels.mxfp8 import mxfp8_matmul_pq, mxfp8_matmul_pq_batch
 
@@ -57,3 +73,12 @@ def test_ring_gemm_several_products_in_one_launch(oracle):
         assert oracle.rel_error(out.cpu(), oracle.gemm_nt(*o)) < 1e-4
         alone = mxfp8_matmul_pq(*p, torch.float32)
         assert oracle.rel_error(out.cpu(), alone.double().cpu()) < 1e-5  # the same sums, K slices apart
+
+
+def test_ring_gemm_short_and_long_products_in_one_launch(oracle):
+    """The gradients of a layer over few tokens: dX over the outputs beside dW over one to three panels."""
+    from kohakuwullm_amd.kernels.mxfp8 import mxfp8_matmul_pq_batch
+
+    ops = [_operands(oracle, *s) for s in [(200, 512, 1536), (1536, 512, 256), (130, 60, 640), (264, 129, 384)]]
+    for o, out in zip(ops, mxfp8_matmul_pq_batch([_dev(o, panels=i == 1) for i, o in enumerate(ops)], torch.bfloat16)):
+        assert oracle.rel_error(out.cpu(), oracle.gemm_nt(*o)) < TOL[torch.bfloat16]
