@@ -19,7 +19,7 @@ from __future__ import annotations
 
 import torch
 
-from kohakuwullm_amd import _lib
+from kohakuwullm_amd import _lib, host
 
 _INDEX = {torch.int32: 4, torch.int64: 8}
 _ROWS = (torch.bfloat16, torch.float16, torch.float32)
@@ -64,6 +64,9 @@ def expert_sort(flat_expert: torch.Tensor, counts: torch.Tensor, top_k: int, num
 def expert_sort_positions(flat_expert: torch.Tensor, counts: torch.Tensor, top_k: int, num_experts: int, positions: bool = True):
     """:func:`expert_sort` with the inverse of ``order`` behind its results: ``positions (n,)``, pair index -> sorted position
     (-1 for a pair without one).  The combines gather by it; written on the way it saves them a fill and a scatter."""
+    made = host.expert_sort(flat_expert, counts, top_k, num_experts, positions)
+    if made is not None:
+        return made
     flat_expert = _index_tensor(flat_expert, "flat_expert")
     _lib.require_gpu(counts, "counts")
     if counts.dtype != torch.int32 or counts.shape != (num_experts,):

@@ -11,7 +11,7 @@ import torch
 import torch.nn.functional as F
 from torch.autograd import forward_ad
 
-from kohakuwullm_amd import _lib
+from kohakuwullm_amd import _lib, host
 from kohakuwullm_amd.kernels.mxfp8.quantize import aligned_rows
 
 MAX_EXPERTS, MAX_TOP_K = 256, 16
@@ -63,16 +63,20 @@ class _RouteTopK(torch.autograd.Function):
     def forward(ctx, x, weight, bias, top_k, norm, factor):
         (t, d), e, dev = x.shape, weight.shape[0], x.device
         need = ctx.needs_input_grad[0] or ctx.needs_input_grad[1]
-        idx = torch.empty(t, top_k, device=dev, dtype=torch.int64)
-        gate = torch.empty(t, top_k, device=dev, dtype=x.dtype)
-        scores = torch.empty(t, top_k, device=dev, dtype=torch.float32) if need else None
-        counts = torch.empty(e, device=dev, dtype=torch.int32)
-        _lib.invoke(
-            "mx_router_topk", 2.0 * t * d * e, x, x.data_ptr(), _lib.MX_DTYPE[x.dtype], x.stride(0), weight.data_ptr(),
-            _lib.MX_DTYPE[weight.dtype], 0 if bias is None else bias.data_ptr(), 0 if bias is None else _lib.MX_DTYPE[bias.dtype],
-            t, d, e, top_k, int(norm), float(factor), idx.data_ptr(), gate.data_ptr(), 0 if scores is None else scores.data_ptr(),
-            counts.data_ptr(),
-        )
+        made = host.route_forward(x, weight, bias, top_k, norm, factor, need)
+        if made is None:
+            idx = torch.empty(t, top_k, device=dev, dtype=torch.int64)
+            gate = torch.empty(t, top_k, device=dev, dtype=x.dtype)
+            scores = torch.empty(t, top_k, device=dev, dtype=torch.float32) if need else None
+            counts = torch.empty(e, device=dev, dtype=torch.int32)
+            _lib.invoke(
+                "mx_router_topk", 2.0 * t * d * e, x, x.data_ptr(), _lib.MX_DTYPE[x.dtype], x.stride(0), weight.data_ptr(),
+                _lib.MX_DTYPE[weight.dtype], 0 if bias is None else bias.data_ptr(), 0 if bias is None else _lib.MX_DTYPE[bias.dtype],
+                t, d, e, top_k, int(norm), float(factor), idx.data_ptr(), gate.data_ptr(), 0 if scores is None else scores.data_ptr(),
+                counts.data_ptr(),
+            )
+        else:
+            idx, gate, scores, counts = made
         if need:
             ctx.save_for_backward(x, weight, idx, scores)
             ctx.norm, ctx.factor = norm, factor
@@ -88,6 +92,9 @@ class _RouteTopK(torch.autograd.Function):
         if torch.is_grad_enabled() or not plain_call(grad):  # create_graph; a vmap over upstream gradients
             dx, dw = composed_gradients(grad, x, weight, idx, ctx.norm, ctx.factor)
             return dx if ctx.needs_input_grad[0] else None, dw if ctx.needs_input_grad[1] else None, None, None, None, None
+        made = host.route_backward(grad, x, weight, idx, scores, ctx.norm, ctx.factor, *ctx.needs_input_grad[:2])
+        if made is not None:
+            return *made, None, None, None, None
         # as they were saved, unless a saved-tensor hook laid them out anew
         x, weight, idx, scores = aligned_rows(x), aligned_rows(weight.contiguous()), idx.contiguous(), scores.contiguous()
         (t, d), e, lib = x.shape, weight.shape[0], _lib.load()
@@ -121,4 +128,9 @@ def route_topk(x: torch.Tensor, weight: torch.Tensor, bias: torch.Tensor | None,
 def route_fitting(x, weight, bias, top_k: int, norm: bool, factor: float):
     """:func:`route_topk` of operands that :func:`can_route` has just looked at (a second look takes 2.6 us)."""
     # a copied input is copied in front of the graph's node, which then keeps the tensor it differentiates
-    return _RouteTopK.apply(aligned_rows(x), weight, bias, top_k, norm, factor)
+    x = aligned_rows(x)
+    if host.unrecorded(x, weight):
+        made = host.route_forward(x, weight, bias, top_k, norm, factor, False)
+        if made is not None:
+            return made[0], made[1], made[3]
+    return _RouteTopK.apply(x, weight, bias, top_k, norm, factor)

@@ -17,7 +17,7 @@ from __future__ import annotations
 
 import torch
 
-from kohakuwullm_amd import _lib
+from kohakuwullm_amd import _lib, host
 from kohakuwullm_amd.kernels.mxfp8.linear import TENSORS, compute_dtype, gradient_dtype, pad_tokens, unobserved
 from kohakuwullm_amd.kernels.mxfp8.quantize import (
     BLOCK_SCALE,
@@ -135,6 +135,9 @@ def swiglu_tokens(gu: torch.Tensor, rounded: bool = False, token_axis: bool = Tr
     ``rounded``: ``silu`` and the product each rounded to the type of ``gu``, the arithmetic of the unfused activation.
     Without ``token_axis`` ``qT`` and ``sT`` are not made and come back as ``None``.
     """
+    made = host.swiglu_tokens(gu, rounded, token_axis)
+    if made is not None:
+        return made
     m, h, dev = gu.shape[0], gu.shape[1] // 2, gu.device
     q = torch.empty(m, h, device=dev, dtype=_FP8)
     s = torch.empty(m, h // BLOCK_SCALE, device=dev, dtype=torch.uint8)
@@ -149,6 +152,9 @@ def swiglu_tokens(gu: torch.Tensor, rounded: bool = False, token_axis: bool = Tr
 
 def swiglu_bwd_tokens(dh: torch.Tensor, gu: torch.Tensor, rounded: bool = False):
     """``dpre = [dgate | dup]`` as ``(q, s, qT, sT)``, both code matrices stage-major, for any token count (``H % 128 == 0``)."""
+    made = host.swiglu_bwd_tokens(dh, gu, rounded)
+    if made is not None:
+        return made
     gu = aligned_rows(gu)  # as the product wrote it, unless a saved-tensor hook laid it out anew
     m, two_h = gu.shape
     h, dev, mt = two_h // 2, gu.device, token_extent(m)
@@ -164,32 +170,45 @@ def swiglu_bwd_tokens(dh: torch.Tensor, gu: torch.Tensor, rounded: bool = False)
     return q, s, qt, st
 
 
+def _forward_products(x, compute, in_f, out_f, rounded, wgrad_in, wgrad_out, stage_major):
+    """``(y, xtq, xts, gu, htq, hts)`` of the forward, ``y`` with the rows of whole blocks where the operands are row-major."""
+    x2d = activation_matrix(x, compute)
+    if stage_major:
+        xq, xs, xtq, xts = quantize_tokens(x2d, compute, token_axis=wgrad_in)
+    else:
+        xq, xs, xtq, xts = quantize_mx_dual(pad_tokens(x2d.to(compute)))
+    # GEMM, then one bandwidth-bound pass for SwiGLU and both casts: measured faster at the
+    # benchmark shape (220 + 89 us) than the same work in the GEMM's epilogue
+    # (fused_swiglu_projection: 329 us), whose vector ALU work cannot overlap the MFMAs.
+    gu = mxfp8_matmul_pq(xq, xs, *in_f, compute, out_pad=_PITCH_PAD)
+    hq, hs, htq, hts = swiglu_tokens(gu, rounded, wgrad_out) if stage_major else swiglu_mx_dual(gu)
+    return mxfp8_matmul_pq(hq, hs, *out_f, compute), xtq, xts, gu, htq, hts
+
+
 class _MXFP8SwiGLUMLP(torch.autograd.Function):
     @staticmethod
     def forward(ctx, x, w_in, w_out, in_f, in_d, out_f, out_d, rounded, differentiable):
         compute = compute_dtype(x)
         shape = x.shape
-        x2d = activation_matrix(x, compute)
-        tokens = x2d.shape[0]
+        tokens = x.numel() // shape[-1] if shape[-1] else 0
         # The token-axis operands (and dpre below) are written stage-major: each K stage of a tile of the three backward
         # products, which contract over thousands of tokens, is then one contiguous run.  A hidden width that is not
         # whole panels keeps the row-major kernels, which take whole 32-token blocks: zero rows change no gradient.
         sm = stage_major_ok(w_out.shape[1]) and tokens > 0
         wgrad_in, wgrad_out = (need and differentiable for need in ctx.needs_input_grad[1:3])
-        xq, xs, xtq, xts = quantize_tokens(x2d, compute, token_axis=wgrad_in) if sm else quantize_mx_dual(pad_tokens(x2d.to(compute)))
-        # GEMM, then one bandwidth-bound pass for SwiGLU and both casts: measured faster at the
-        # benchmark shape (220 + 89 us) than the same work in the GEMM's epilogue
-        # (fused_swiglu_projection: 329 us), whose vector ALU work cannot overlap the MFMAs.
-        gu = mxfp8_matmul_pq(xq, xs, *in_f, compute, out_pad=_PITCH_PAD)
-        hq, hs, htq, hts = swiglu_tokens(gu, rounded, wgrad_out) if sm else swiglu_mx_dual(gu)
-        y = mxfp8_matmul_pq(hq, hs, *out_f, compute)
+        made = host.swiglu_mlp_forward(x, compute, in_f, out_f, rounded, wgrad_in, wgrad_out, _PITCH_PAD) if sm else None
+        if made is None:
+            y, *kept = _forward_products(x, compute, in_f, out_f, rounded, wgrad_in, wgrad_out, sm)
+            y = y[:tokens].reshape(*shape[:-1], y.shape[-1])
+        else:
+            y, *kept = made
         if differentiable and any(ctx.needs_input_grad):
-            ctx.save_for_backward(xtq, xts, gu, htq, hts, *in_d, *out_d)
+            ctx.save_for_backward(*kept, *in_d, *out_d)
             ctx.compute = compute
             ctx.x_dtype = x.dtype
             ctx.dw_dtypes = gradient_dtype(w_in, compute), gradient_dtype(w_out, compute)
             ctx.stage_major, ctx.rounded = sm, rounded
-        return y[:tokens].reshape(*shape[:-1], y.shape[-1])
+        return y
 
     @staticmethod
     def backward(ctx, dout):
@@ -213,6 +232,14 @@ class _MXFP8SwiGLUMLP(torch.autograd.Function):
         return dx, dw_in, dw_out, None, None, None, None, None, None
 
 
+def _evaluated(x, w_in, w_out, in_f, out_f, rounded) -> torch.Tensor | None:
+    """The block's output where no gradient is recorded, without an autograd function around it (``None``: not such a call)."""
+    if not stage_major_ok(out_f[0].shape[1]) or not host.unrecorded(x, w_in, w_out):
+        return None
+    made = host.swiglu_mlp_forward(x, compute_dtype(x), in_f, out_f, rounded, False, False, _PITCH_PAD)
+    return None if made is None else made[0]
+
+
 def mxfp8_swiglu_mlp(x, w_in, w_out, packed) -> torch.Tensor:
     """``(silu(x W_g^T) * (x W_u^T)) W_out^T`` with ``w_in = [W_g; W_u]`` ``(2H, dim)``, ``w_out`` ``(dim, H)``.
 
@@ -223,7 +250,8 @@ def mxfp8_swiglu_mlp(x, w_in, w_out, packed) -> torch.Tensor:
     """
     if w_in.shape[0] != 2 * w_out.shape[1] or w_in.shape[1] != x.shape[-1] or w_out.shape[0] != x.shape[-1]:
         raise ValueError(f"shape mismatch: x {tuple(x.shape)}, w_in {tuple(w_in.shape)}, w_out {tuple(w_out.shape)}")
-    return _MXFP8SwiGLUMLP.apply(x, w_in, w_out, *packed, False, torch.is_grad_enabled())
+    y = _evaluated(x, w_in, w_out, packed[0], packed[2], False)
+    return _MXFP8SwiGLUMLP.apply(x, w_in, w_out, *packed, False, torch.is_grad_enabled()) if y is None else y
 
 
 def mxfp8_swiglu_pair(x, w_in, w_out) -> torch.Tensor | None:
@@ -248,5 +276,8 @@ def mxfp8_swiglu_pair(x, w_in, w_out) -> torch.Tensor | None:
         if lin._cache is None:
             lin.refresh_quantized_weight()
     (in_f, in_d), (out_f, out_d) = ((lin._cache[:2], lin._cache[2:]) for lin in (w_in, w_out))
+    y = _evaluated(x, w_in.weight, w_out.weight, in_f, out_f, True)
+    if y is not None:
+        return y
     return _MXFP8SwiGLUMLP.apply(x, w_in.weight, w_out.weight, in_f, in_d, out_f, out_d, True,
                                  torch.is_grad_enabled())

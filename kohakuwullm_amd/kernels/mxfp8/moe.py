@@ -15,7 +15,7 @@ from __future__ import annotations
 
 import torch
 
-from kohakuwullm_amd import _lib
+from kohakuwullm_amd import _lib, host
 from kohakuwullm_amd.kernels.moe.moe_dispatch import combine_routed
 from kohakuwullm_amd.kernels.mxfp8.grouped import (
     grouped_mxfp8_gemm,
@@ -208,6 +208,17 @@ class _MXFP8Experts(torch.autograd.Function):
         m = token_of.numel()
         # the grad mode comes from the caller: in here it is always off, and `needs_input_grad` does not know it
         needs_grad = differentiable and any(ctx.needs_input_grad)
+        if TOKEN_AXIS_STAGE_MAJOR:
+            made = host.experts_forward(x, gate, token_of, order, offsets, positions, packed.in_fwd, packed.out_fwd, hidden, needs_grad,
+                                        differentiable and ctx.needs_input_grad[2])
+            if made is not None:
+                out, hq, hs, pre, htq, hts, positions = made
+                if needs_grad:
+                    ctx.positions = positions
+                    ctx.save_for_backward(x, hq, hs, pre, gate, token_of, order, offsets, htq, hts)
+                    ctx.packed = packed
+                    ctx.shapes = (hidden, dim, m, rows, gate.numel() // rows)
+                return out
         xq, xs = quantize_mx(x)  # once per token; the gather happens inside GEMM1
         hq = torch.empty(m, hidden, device=x.device, dtype=_FP8)
         hs = torch.empty(m, hidden // BLOCK_SCALE, device=x.device, dtype=torch.uint8)
@@ -235,6 +246,11 @@ class _MXFP8Experts(torch.autograd.Function):
         x, hq, hs, pre, gate, token_of, order, offsets, htq, hts = ctx.saved_tensors
         packed = ctx.packed
         hidden, dim, m, rows, top_k = ctx.shapes
+        if TOKEN_AXIS_STAGE_MAJOR:
+            made = host.experts_backward(dout, x, hq, hs, pre, gate, token_of, order, offsets, ctx.positions, htq, hts, packed.in_dgrad,
+                                         packed.out_dgrad, hidden, *ctx.needs_input_grad[1:3])
+            if made is not None:
+                return *made, None, None, None, None, None, None, None
         dev = dout.device
         dout = dout.contiguous()
         dq, ds = quantize_mx(dout)
@@ -311,6 +327,10 @@ def mxfp8_moe_experts(x, w_in, w_out, gate, token_of, order, offsets, packed: MX
             ``offsets[E]``); made from ``order`` when not given.
     """
     hidden = _validate_expert_call(x, w_in, w_out, token_of, order)
+    if TOKEN_AXIS_STAGE_MAJOR and host.unrecorded(x, gate, w_in, w_out):
+        made = host.experts_forward(x, gate, token_of, order, offsets, positions, packed.in_fwd, packed.out_fwd, hidden, False, False)
+        if made is not None:
+            return made[0]
     return _MXFP8Experts.apply(x, w_in, w_out, gate, token_of, order, offsets, packed, hidden, positions, torch.is_grad_enabled())
 
 

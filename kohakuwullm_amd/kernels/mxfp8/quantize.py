@@ -16,7 +16,7 @@ import ctypes
 
 import torch
 
-from kohakuwullm_amd import _lib
+from kohakuwullm_amd import _lib, host
 
 E4M3_MAX = 448.0
 BLOCK_SCALE = 32
@@ -39,6 +39,9 @@ def quantize_mx(x: torch.Tensor) -> tuple[torch.Tensor, torch.Tensor]:
     transposed view is quantized in place of a copy (the column-axis kernel runs on
     the matrix underneath it).
     """
+    made = host.quantize_rows(x)
+    if made is not None:
+        return made
     if x.shape[-1] % BLOCK_SCALE:
         raise ValueError(f"K={x.shape[-1]} must be a multiple of {BLOCK_SCALE}")
     _check_2d(x, "x")
@@ -192,6 +195,9 @@ def quantize_tokens(x: torch.Tensor, compute: torch.dtype, cols: int | None = No
     returns it, its width a multiple of 8, ``K`` a multiple of 32.  Without ``token_axis`` (``K`` the width of ``x``)
     ``qT`` and ``sT`` are not made and come back as ``None``.
     """
+    made = host.quantize_tokens(x, compute, cols or 0, token_axis)
+    if made is not None:
+        return made
     _check_2d(x, "x")
     m, kv = x.shape
     k = cols or kv
@@ -216,6 +222,9 @@ def quantize_side(xs: list[torch.Tensor]):
 
     Every ``x`` as :func:`activation_matrix` returns it, its width a multiple of 128; at most ``SIDE_MAX`` of them.
     """
+    made = host.quantize_side(xs)
+    if made is not None:
+        return made
     m, k, device = xs[0].shape[0], sum(x.shape[1] for x in xs), xs[0].device
     sources = _lib.words(_lib.SideSource, [(x.data_ptr(), x.shape[1], x.stride(0)) for x in xs])
     q = torch.empty(m, k, device=device, dtype=_FP8)
@@ -230,6 +239,9 @@ def join_codes(pairs):
     """``(torch.cat(codes, 1), torch.cat(scales, 1))`` of quantized matrices of one height, widths multiples of 128."""
     if len(pairs) == 1:
         return pairs[0]
+    made = host.join_codes(pairs)
+    if made is not None:
+        return made
     pairs = [(packed(c, 16), packed(s, 4)) for c, s in pairs]
     rows, k, device = pairs[0][0].shape[0], sum(c.shape[1] for c, _ in pairs), pairs[0][0].device
     sources = _lib.words(_lib.CodeSource, [(c.data_ptr(), s.data_ptr(), c.shape[1], c.stride(0), s.stride(0)) for c, s in pairs])
@@ -250,6 +262,9 @@ def quantize_mx_dual_batch(xs: list[torch.Tensor]) -> list[tuple[torch.Tensor, t
     """
     if not xs:
         return []
+    made = host.quantize_dual_batch(xs)
+    if made is not None:
+        return made
     for x in xs:
         _check_2d(x, "x")
         if x.shape[0] % BLOCK_SCALE or x.shape[1] % BLOCK_SCALE:
@@ -308,6 +323,9 @@ def mxfp8_matmul_pq(
     ``out_pad``: the result is a view of an allocation with that many spare elements per row (a row
     pitch of ``N + out_pad``), for callers that know what pitch suits the kernel reading it next.
     """
+    made = host.matmul(aq, a_scale, bq, b_scale, out_dtype, out_pad)
+    if made is not None:
+        return made
     if out_pad < 0:
         raise ValueError(f"out_pad={out_pad} must not be negative")
     if aq.dim() == 3 or bq.dim() == 3:
@@ -344,6 +362,9 @@ def mxfp8_matmul_pq_batch(problems, out_dtype: torch.dtype = torch.bfloat16) -> 
     of one layer): the library divides the GPU among them instead of running them in turn.
     Same operand contract and same results as :func:`mxfp8_matmul_pq`.
     """
+    made = host.matmul_batch(problems, out_dtype)
+    if made is not None:
+        return made
     if out_dtype not in _lib.MX_DTYPE:
         raise ValueError(f"out_dtype={out_dtype} is not one of {tuple(_lib.MX_DTYPE)}")
     if not problems:

@@ -1,0 +1,213 @@
+"""The C++ host path (csrc/mx_host.cpp) against the Python one it stands for: the same launches, so the same bits, for every
+layout, type and option a call may have; and what it leaves to Python, told by a None with nothing launched."""
+
+import contextlib
+
+import pytest
+import torch
+
+from conftest import SEED
+
+DEV = "cuda:0"
+BF, F16, F32 = torch.bfloat16, torch.float16, torch.float32
+
+
+class _Own(torch.Tensor):
+    pass
+
+
+def test_calls_that_are_not_plain_are_declined():
+    from torch.utils._python_dispatch import TorchDispatchMode
+
+    from kohakuwullm_amd import host
+
+    x, w = torch.zeros(32, 128, dtype=BF), torch.zeros(64, 128, dtype=torch.uint8)
+    s = torch.zeros(64, 4, dtype=torch.uint8)
+    calls = [
+        lambda t: host.quantize_rows(t), lambda t: host.quantize_tokens(t, BF, 0, True), lambda t: host.quantize_side([t, t]),
+        lambda t: host.join_codes([(w, s), (w, s)]), lambda t: host.quantize_dual_batch([t]), lambda t: host.matmul(w, s, w, s, BF, 0),
+        lambda t: host.matmul_batch([(w, s, w, s)], BF), lambda t: host.linear_eval(t, t, w, s), lambda t: host.linear_forward(t, BF, w, s, True),
+        lambda t: host.group_forward(t, BF, [(w, s, w, s)] * 2, True), lambda t: host.rmsnorm_forward(t, None, 1e-6),
+        lambda t: host.route_forward(t, t, None, 2, True, 1.0, True), lambda t: host.quantize_rows(None), lambda t: host.quantize_rows(3),
+        lambda t: host.matmul(w, s, w, s, "bf16", 0),
+    ]
+    for t in (x, x.as_subclass(_Own), torch.nn.Parameter(x), x.to("meta"), torch.zeros(0, 128, dtype=BF)):
+        for i, call in enumerate(calls):
+            assert call(t) is None, (i, type(t), t.device)
+    with torch.no_grad():
+        assert not host.unrecorded(x) and not host.unrecorded(3)
+
+    class Mode(TorchDispatchMode):
+        def __torch_dispatch__(self, func, types, args=(), kwargs=None):
+            return func(*args, **(kwargs or {}))
+
+    with Mode():
+        assert calls[0](x) is None
+
+
+@contextlib.contextmanager
+def _python():
+    """Calls inside go the Python way: a timer is installed."""
+    from kohakuwullm_amd import _lib
+
+    _lib.TIMER = []
+    try:
+        yield
+    finally:
+        _lib.TIMER = None
+
+
+def _bits(t):
+    return t.contiguous().flatten().view(torch.uint8)
+
+
+def _both(run):
+    got = run()
+    with _python():
+        want = run()
+    assert len(got) == len(want)
+    for i, (a, b) in enumerate(zip(got, want)):
+        assert (a is None) == (b is None), i
+        if a is not None:
+            assert a.shape == b.shape and a.dtype == b.dtype and a.stride() == b.stride() and torch.equal(_bits(a), _bits(b)), i
+
+
+def _layouts(tokens, width, dtype):
+    """The same values as they may lie: flat, batched, pitched, transposed, at an odd offset, broadcast over the batch."""
+    g = torch.Generator(device=DEV).manual_seed(SEED)
+    base = torch.randn(tokens, width, device=DEV, generator=g).to(dtype)
+    odd = torch.empty(tokens * width + 1, device=DEV, dtype=dtype)[1:].view(tokens, width).copy_(base)
+    pitched = torch.empty(tokens, width + 8, device=DEV, dtype=dtype)[:, :width].copy_(base)
+    return {"flat": base, "batched": base.view(1, tokens, width), "odd": odd, "pitched": pitched, "transposed": base.t().contiguous().t(),
+            "broadcast": base[:1].expand(3, tokens, width), "empty": base[:0]}
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("layout", ["flat", "batched", "odd", "pitched", "transposed", "broadcast", "empty"])
+@pytest.mark.parametrize("dtype,master,autocast", [(BF, BF, False), (F16, F16, False), (F32, F32, True), (BF, F32, False)])
+@pytest.mark.parametrize("tokens,inp,out", [(1, 128, 1000), (33, 256, 384)])
+def test_linear(layout, dtype, master, autocast, tokens, inp, out):
+    from kohakuwullm_amd.kernels.mxfp8.linear import MXFP8Linear
+
+    torch.manual_seed(SEED)
+    lin = MXFP8Linear(inp, out).to(DEV).to(master)
+    x0 = _layouts(tokens, inp, dtype)[layout]
+
+    def run(train=True, weight=True):
+        lin.weight.requires_grad_(weight)
+        lin.weight.grad = None
+        x = x0.detach().requires_grad_(train)
+        with torch.autocast("cuda", dtype=BF, enabled=autocast), torch.set_grad_enabled(train):
+            y = lin(x)
+        if not train:
+            assert y.grad_fn is None
+            return [y]
+        y.backward(torch.ones_like(y).mul_(1e-2))
+        return [y.detach(), x.grad, lin.weight.grad]
+
+    _both(run)
+    _both(lambda: run(True, False))
+    _both(lambda: run(False))
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("layout", ["flat", "batched", "pitched", "transposed"])
+@pytest.mark.parametrize("dtype", [BF, F16])
+def test_attention_and_norm(layout, dtype):
+    from kohakuwullm_amd.kernels.elementwise.rmsnorm import rms_norm
+    from kohakuwullm_amd.models.mlp import AttentionProjections
+    from kohakuwullm_amd.models.mxfp8_swap import swap_mxfp8
+
+    torch.manual_seed(SEED)
+    block = AttentionProjections(256, 2, 1, 128).to(DEV).to(dtype)
+    swap_mxfp8(block)
+    x0, weight = _layouts(70, 256, dtype)[layout], torch.ones(256, device=DEV, dtype=dtype).requires_grad_()
+
+    def run(train=True):
+        x = x0.detach().requires_grad_(train)
+        weight.grad = None
+        block.zero_grad()
+        with torch.set_grad_enabled(train):
+            outs = [*block.project(rms_norm(x, weight))]
+            outs.append(block.merge(outs[0]))
+        if not train:
+            return outs
+        torch.autograd.backward(outs, [torch.ones_like(o).mul_(1e-2) for o in outs])
+        return [o.detach() for o in outs] + [x.grad, weight.grad] + [p.grad for p in block.parameters()]
+
+    _both(run)
+    _both(lambda: run(False))
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("fused", [True, False])
+@pytest.mark.parametrize("dtype,autocast", [(BF, False), (F32, True)])
+@pytest.mark.parametrize("tokens,hidden", [(1, 128), (97, 384), (64, 160)])
+def test_feed_forward(fused, dtype, autocast, tokens, hidden):
+    from kohakuwullm_amd.models.mlp import MXFP8SwiGLU, SwiGLU
+    from kohakuwullm_amd.models.mxfp8_swap import swap_mxfp8
+
+    if hidden % 128 and not fused:
+        pytest.skip("a projection of this width is not swapped")
+    torch.manual_seed(SEED)
+    block = (MXFP8SwiGLU if fused else SwiGLU)(256, hidden=hidden).to(DEV).to(dtype)
+    if not fused:
+        swap_mxfp8(block)
+    x0 = torch.randn(tokens, 256, device=DEV).to(dtype)
+
+    def run(train=True):
+        x = x0.detach().requires_grad_(train)
+        block.zero_grad()
+        with torch.autocast("cuda", dtype=BF, enabled=autocast), torch.set_grad_enabled(train):
+            y = block(x)
+        if not train:
+            return [y]
+        y.backward(torch.ones_like(y).mul_(1e-2))
+        return [y.detach(), x.grad] + [p.grad for p in block.parameters()]
+
+    _both(run)
+    _both(lambda: run(False))
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("tokens,shared,dtype", [(3, 0, BF), (130, 1, BF), (64, 0, F16)])
+def test_mixture_of_experts(tokens, shared, dtype):
+    from kohakuwullm_amd.models.moe import MoEMLP
+    from kohakuwullm_amd.models.mxfp8_swap import swap_mxfp8
+
+    torch.manual_seed(SEED)
+    block = MoEMLP(256, hidden=128, num_experts=8, top_k=2, num_shared=shared).to(DEV).to(dtype)
+    swap_mxfp8(block)
+    x0 = torch.randn(tokens, 256, device=DEV).to(dtype)
+
+    def run(train=True):
+        x = x0.detach().requires_grad_(train)
+        block.zero_grad()
+        with torch.set_grad_enabled(train):
+            y = block(x)
+        if not train:
+            return [y]
+        y.backward(torch.ones_like(y).mul_(1e-2))
+        # the gate's gradient is added with atomics in any order: what it reaches is compared below
+        return [y.detach(), block.w_in.grad, block.w_out.grad], x.grad, block.router.weight.grad
+
+    got, dx, dr = run()
+    with _python():
+        want, dx2, dr2 = run()
+    for a, b in zip(got, want):
+        assert torch.equal(a, b)
+    for a, b in ((dx, dx2), (dr, dr2)):  # fp32 sums of four terms in another order, rounded to 16 bits behind
+        assert (a.float() - b.float()).norm() <= 4e-3 * b.float().norm()
+    _both(lambda: run(False))
+
+
+@pytest.mark.gpu
+def test_refresh_and_pitched_products():
+    from kohakuwullm_amd.kernels.mxfp8 import mxfp8_matmul_pq, quantize_mx
+    from kohakuwullm_amd.kernels.mxfp8.quantize import quantize_mx_dual_batch
+
+    g = torch.Generator(device=DEV).manual_seed(SEED)
+    ws = [torch.randn(m, k, device=DEV, generator=g).to(BF) for m, k in ((32, 32), (96, 256), (384, 128))] * 9  # two launches
+    _both(lambda: [t for four in quantize_mx_dual_batch(ws) for t in four])
+    q, s = quantize_mx(ws[1])
+    _both(lambda: [mxfp8_matmul_pq(q, s, q, s, F32, out_pad=24)])
