@@ -7,6 +7,7 @@
 
 #include "mx_gemm_core.h"
 #include "mx_gemm_ring.h"
+#include "mx_gemm_skinny.h"
 #ifdef MX_BENCH_VARIANTS
 #include "mx_gemm_variants.h"
 #endif
@@ -388,6 +389,15 @@ __global__ __launch_bounds__(RingShape::NTHR, 2) void gemm_nt_ring_kernel(RingAr
     else ring_gemm(prob, smem);
 }
 
+// Up to MX_BATCH_MAX products with few rows behind one launch, a workgroup per 16 columns of one of them.
+template <int CDT, int MT, int U>
+__global__ __launch_bounds__(SKINNY_WAVES * 64) void gemm_nt_skinny_kernel(RingArgs b) {
+    extern __shared__ __attribute__((aligned(1024))) uint8_t smem[];
+    int j = 0;
+    while (j + 1 < b.count && (int)blockIdx.x >= b.end[j]) j++;
+    skinny_gemm<CDT, MT, U>(b.prob[j], (int)blockIdx.x - (j ? b.end[j - 1] : 0), smem);
+}
+
 // slice_reduce for every problem of such a launch that was cut along K (`end` counts blocks of those).
 template <int CDT>
 __global__ __launch_bounds__(RingShape::NTHR) void ring_reduce_kernel(RingArgs b) {
@@ -551,6 +561,45 @@ static bool ring_pays(const DenseArgs &a) {
     return ring < (whole < dealt ? whole : dealt);
 }
 
+// Whether a product goes to the kernel for few rows: up to 64, and up to 128 where a CU has no second 16 columns to do.  us on
+// ring tiles / there, weights from HBM:
+//            512 -> 1536   2048 -> 3072   4096 -> 1536   1536 -> 8192   1024 -> 5632   256 -> 1000
+//   M = 1     6.1 / 3.1     10.8 / 4.1     17.0 / 5.1      9.6 / 4.9      7.4 / 4.4     5.3 / 2.8
+//   16        6.0 / 3.3     11.0 / 4.5     17.8 / 5.9      9.7 / 5.2      7.5 / 4.7     5.3 / 2.9
+//   64        6.3 / 3.9     12.0 / 6.6     19.1 / 10.0    10.3 / 8.3      7.9 / 6.0     5.5 / 3.6
+//   128       6.1 / 4.7     13.1 / 9.1     22.0 / 16.1    10.8 / 13.2     7.6 / 10.0    5.5 / 4.2
+static bool skinny_pays(const DenseArgs &a) {
+    return a.K % 128 == 0 && a.split_k == 1 && !a.accumulate && aligned(a.as, 4) && aligned(a.bs, 4) && a.ldas % 4 == 0 && a.ldbs % 4 == 0 &&
+           (a.M <= 64 || (a.M <= 128 && a.N <= SKINNY_N * num_cus()));
+}
+
+template <int CDT, int MT, int U>
+static int launch_skinny_tiles(const RingArgs &b, int blocks, hipStream_t st) {
+    return launch_with_lds<gemm_nt_skinny_kernel<CDT, MT, U>>(dim3((unsigned)blocks), dim3(SKINNY_WAVES * 64), SKINNY_WAVES * U * skinny_stage_bytes(MT), st, b);
+}
+
+template <int CDT>
+static int launch_skinny(const DenseArgs *probs, int count, hipStream_t st) {
+    RingArgs b;
+    b.count = count;
+    int blocks = 0, rows = 0, per = 0;
+    for (int j = 0; j < count; j++) {
+        b.prob[j] = probs[j];
+        b.end[j] = blocks += (probs[j].N + SKINNY_N - 1) / SKINNY_N;
+        rows = probs[j].M > rows ? probs[j].M : rows;
+        const int stages = ((probs[j].K >> 7) + SKINNY_WAVES - 1) / SKINNY_WAVES;
+        per = stages > per ? stages : per;
+    }
+    const bool one = per == 1 || blocks > num_cus();  // a stage in flight per wave leaves LDS for a second workgroup per CU
+    int rc;
+    if (rows <= 16) rc = per > 2 ? launch_skinny_tiles<CDT, 1, 4>(b, blocks, st) : launch_skinny_tiles<CDT, 1, 2>(b, blocks, st);
+    else if (rows <= 32) rc = one ? launch_skinny_tiles<CDT, 2, 1>(b, blocks, st) : launch_skinny_tiles<CDT, 2, 2>(b, blocks, st);
+    else if (rows <= 64) rc = one ? launch_skinny_tiles<CDT, 4, 1>(b, blocks, st) : launch_skinny_tiles<CDT, 4, 2>(b, blocks, st);
+    else rc = launch_skinny_tiles<CDT, 8, 1>(b, blocks, st);
+    if (rc != MX_OK) return rc;
+    return hipGetLastError() == hipSuccess ? MX_OK : MX_ELAUNCH;
+}
+
 template <typename S, int CDT>
 static int launch_tiled(DenseArgs a, float *ws, int ws_slots, hipStream_t st, bool phased = false) {
     a.tiles_m = (a.M + S::BM - 1) / S::BM;
@@ -701,6 +750,7 @@ static int gemm_dispatch(DenseArgs a, float *ws, int ws_slots, hipStream_t st, b
                                                                                   a.lda, a.ldas, a.ldb, a.ldbs, a.ldc);
         return hipGetLastError() == hipSuccess ? MX_OK : MX_ELAUNCH;
     }
+    if (!phased && skinny_pays(a)) return launch_skinny<CDT>(&a, 1, st);
     if (!phased && ring_pays(a)) return launch_ring<CDT>(&a, 1, ws, ws_slots, st);
     return launch_tiled<DenseShape, CDT>(a, ws, ws_slots, st, phased);
 }
@@ -720,7 +770,9 @@ static int batch_dispatch(DenseArgs *probs, int count, float *ws, int ws_slots, 
     // All of them on the ring kernel: its tiles side by side fill the chip, whoever they belong to (4096 x 512 x 1536 beside
     // 1536 x 512 x 4096: 39 -> 20 us; 3001 x 2048 x 2048 beside 2048 x 2048 x 3072: 45 -> 41).  A mixed batch shares the XCDs
     // below instead: one launch for each kind won 7 % on one such batch and lost up to 25 % on the others.
-    bool ring = true;
+    bool ring = true, skinny = true;
+    for (int j = 0; j < count; j++) skinny = skinny && tiled_ok(probs[j]) && skinny_pays(probs[j]);
+    if (skinny && count) return launch_skinny<CDT>(probs, count, st);
     for (int j = 0; j < count; j++) ring = ring && tiled_ok(probs[j]) && ring_pays(probs[j]);
     if (ring && count) return launch_ring<CDT>(probs, count, ws, ws_slots, st);
     bool fuse = count > 1 && count <= MX_BATCH_MAX;

@@ -47,9 +47,28 @@ def test_ring_gemm(oracle, m, n, k, dtype):
 
 
 @pytest.mark.parametrize("m,n,k", [
-    (1, 1, 128), (130, 300, 128), (257, 129, 256), (128, 264, 384), (3, 2048, 384),  # without a whole group
-    (1, 1, 640), (129, 130, 768), (5, 257, 896), (128, 128, 1152), (300, 40, 1408), (513, 260, 2176),
-    (16, 40, 8320), (130, 200, 16384 + 384),  # K slices whose last one ends inside a group
+    (1, 1, 128), (1, 17, 384), (15, 16, 640), (16, 4100, 1024), (17, 48, 1152), (32, 4112, 2048), (33, 200, 896), (64, 520, 4224), (64, 4128, 256),
+    (65, 72, 1280), (128, 129, 2176),  # the last group of 16 rows and of 16 columns, one K stage per wave, none, several
+])
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16, torch.float16])
+def test_gemm_of_few_rows(oracle, m, n, k, dtype):
+    from kohakuwullm_amd.kernels.mxfp8 import mxfp8_matmul_pq, mxfp8_matmul_pq_batch
+
+    ops = _operands(oracle, m, n, k)
+    out = mxfp8_matmul_pq(*_dev(ops), dtype)
+    assert oracle.rel_error(out.cpu(), oracle.gemm_nt(*ops)) < TOL[dtype]
+    padded = mxfp8_matmul_pq(*_dev(ops), dtype, out_pad=3)
+    assert padded.stride(0) == n + 3 and torch.equal(padded, out)
+    assert torch.equal(mxfp8_matmul_pq(*_dev(ops, panels=True), dtype), out)
+    other = _operands(oracle, 9, 50, 512)  # beside a product with fewer rows and another K: the same sums
+    both = mxfp8_matmul_pq_batch([_dev(ops), _dev(other)], dtype)
+    assert torch.equal(both[0], out) and oracle.rel_error(both[1].cpu(), oracle.gemm_nt(*other)) < TOL[dtype]
+
+
+@pytest.mark.parametrize("m,n,k", [
+    (130, 300, 128), (257, 129, 256), (200, 264, 384),  # without a whole group
+    (129, 1, 640), (129, 130, 768), (300, 40, 1408), (513, 260, 2176), (300, 257, 896), (256, 128, 1152),
+    (129, 40, 8320), (130, 200, 16384 + 384),  # K slices whose last one ends inside a group
 ])
 @pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
 def test_ring_gemm_ends_inside_a_group(oracle, m, n, k, dtype):
