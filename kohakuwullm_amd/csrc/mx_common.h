@@ -192,6 +192,21 @@ __device__ __forceinline__ uint32_t pack2_bf16(float lo, float hi) {
     return __builtin_bit_cast(uint32_t, __builtin_convertvector(v, b2));
 }
 
+// fp32 values rounded to a 16-bit type and widened again: what a cast in front of the quantizer would have left.
+template <int CDT>
+__device__ __forceinline__ void round_values(float (&v)[8]) {
+    if constexpr (CDT == MX_BF16) {
+#pragma unroll
+        for (int c = 0; c < 8; c += 2) {
+            const uint32_t w = pack2_bf16(v[c], v[c + 1]);
+            v[c] = bits2f(w << 16), v[c + 1] = bits2f(w & 0xFFFF0000u);
+        }
+    } else if constexpr (CDT == MX_FP16) {
+#pragma unroll
+        for (int c = 0; c < 8; c++) v[c] = (float)(_Float16)v[c];
+    }
+}
+
 // Inclusive prefix sum over the 64 lanes of a wave.
 __device__ __forceinline__ int wave_incl_scan(int v, int lane) {
 #pragma unroll

@@ -390,12 +390,12 @@ __global__ __launch_bounds__(RingShape::NTHR, 2) void gemm_nt_ring_kernel(RingAr
 }
 
 // Up to MX_BATCH_MAX products with few rows behind one launch, a workgroup per 16 columns of one of them.
-template <int CDT, int MT, int U>
+template <int CDT, int MT, int U, int SRC>
 __global__ __launch_bounds__(SKINNY_WAVES * 64) void gemm_nt_skinny_kernel(RingArgs b) {
     extern __shared__ __attribute__((aligned(1024))) uint8_t smem[];
     int j = 0;
     while (j + 1 < b.count && (int)blockIdx.x >= b.end[j]) j++;
-    skinny_gemm<CDT, MT, U>(b.prob[j], (int)blockIdx.x - (j ? b.end[j - 1] : 0), smem);
+    skinny_gemm<CDT, MT, U, SRC, CDT>(b.prob[j], (int)blockIdx.x - (j ? b.end[j - 1] : 0), smem);
 }
 
 // slice_reduce for every problem of such a launch that was cut along K (`end` counts blocks of those).
@@ -573,12 +573,14 @@ static bool skinny_pays(const DenseArgs &a) {
            (a.M <= 64 || (a.M <= 128 && a.N <= SKINNY_N * num_cus()));
 }
 
-template <int CDT, int MT, int U>
+template <int CDT, int MT, int U, int SRC>
 static int launch_skinny_tiles(const RingArgs &b, int blocks, hipStream_t st) {
-    return launch_with_lds<gemm_nt_skinny_kernel<CDT, MT, U>>(dim3((unsigned)blocks), dim3(SKINNY_WAVES * 64), SKINNY_WAVES * U * skinny_stage_bytes(MT), st, b);
+    const int rc = launch_with_lds<gemm_nt_skinny_kernel<CDT, MT, U, SRC>>(dim3((unsigned)blocks), dim3(SKINNY_WAVES * 64), skinny_lds_bytes(SRC, MT, U), st, b);
+    if (rc != MX_OK) return rc;
+    return hipGetLastError() == hipSuccess ? MX_OK : MX_ELAUNCH;
 }
 
-template <int CDT>
+template <int CDT, int SRC = SRC_CODES>
 static int launch_skinny(const DenseArgs *probs, int count, hipStream_t st) {
     RingArgs b;
     b.count = count;
@@ -591,13 +593,11 @@ static int launch_skinny(const DenseArgs *probs, int count, hipStream_t st) {
         per = stages > per ? stages : per;
     }
     const bool one = per == 1 || blocks > num_cus();  // a stage in flight per wave leaves LDS for a second workgroup per CU
-    int rc;
-    if (rows <= 16) rc = per > 2 ? launch_skinny_tiles<CDT, 1, 4>(b, blocks, st) : launch_skinny_tiles<CDT, 1, 2>(b, blocks, st);
-    else if (rows <= 32) rc = one ? launch_skinny_tiles<CDT, 2, 1>(b, blocks, st) : launch_skinny_tiles<CDT, 2, 2>(b, blocks, st);
-    else if (rows <= 64) rc = one ? launch_skinny_tiles<CDT, 4, 1>(b, blocks, st) : launch_skinny_tiles<CDT, 4, 2>(b, blocks, st);
-    else rc = launch_skinny_tiles<CDT, 8, 1>(b, blocks, st);
-    if (rc != MX_OK) return rc;
-    return hipGetLastError() == hipSuccess ? MX_OK : MX_ELAUNCH;
+    if (rows <= 16) return per > 2 ? launch_skinny_tiles<CDT, 1, 4, SRC>(b, blocks, st) : launch_skinny_tiles<CDT, 1, 2, SRC>(b, blocks, st);
+    if (rows <= 32) return one ? launch_skinny_tiles<CDT, 2, 1, SRC>(b, blocks, st) : launch_skinny_tiles<CDT, 2, 2, SRC>(b, blocks, st);
+    if constexpr (SRC != SRC_CODES) return MX_EUNSUPPORTED;
+    else if (rows <= 64) return one ? launch_skinny_tiles<CDT, 4, 1, SRC>(b, blocks, st) : launch_skinny_tiles<CDT, 4, 2, SRC>(b, blocks, st);
+    else return launch_skinny_tiles<CDT, 8, 1, SRC>(b, blocks, st);
 }
 
 template <typename S, int CDT>
@@ -980,6 +980,42 @@ extern "C" int mx_gemm_nt_batch(const mx_gemm_problem *problems, int count, int 
         }
     }
     return flush();
+}
+
+// Which activations are quantized inside the product: every workgroup does it again, which costs as much as the launch it saves
+// at 16 rows of a K of 4096 or at 32 of 2048.  us in two launches / in one, weights from HBM:
+//            512 -> 1536   2048 -> 3072   4096 -> 1536   1536 -> 8192
+//   M = 1     5.2 / 3.3      6.3 / 4.7      7.6 / 6.2      7.1 / 5.5
+//   8         5.4 / 3.8      6.6 / 5.1      7.7 / 6.7      7.3 / 6.0
+//   16        5.4 / 4.4      7.0 / 5.8      8.2 / 8.0      7.6 / 7.2
+//   32        5.6 / 4.4      7.8 / 7.7      9.5 / 11.0     8.9 / 10.2
+static bool activation_rows_ok(int64_t M, int64_t K, int64_t columns) {
+    return M <= 16 ? K <= 4096 : M <= 32 && K <= 2048 && columns <= SKINNY_N * num_cus();
+}
+
+extern "C" int mx_activation_gemm_nt(const void *x, int x_dtype, int64_t ldx, const mx_gemm_problem *problems, int count, int c_dtype,
+                                     void *stream) {
+    if (count <= 0 || !problems || !x) return MX_EINVAL;
+    if (count > MX_BATCH_MAX || (c_dtype != MX_BF16 && c_dtype != MX_FP16) || (x_dtype != c_dtype && x_dtype != MX_FP32)) return MX_EUNSUPPORTED;
+    DenseArgs a[MX_BATCH_MAX];
+    int64_t columns = 0;
+    for (int j = 0; j < count; j++) {
+        const mx_gemm_problem &q = problems[j];
+        columns += q.N;
+        if (q.M != problems[0].M || q.K != problems[0].K || q.ldb < q.K) return MX_EINVAL;
+        const int rc = fill_args(a[j], (const uint8_t *)x, nullptr, q.bq, q.b_scale, q.c, q.M, q.N, q.K, q.K, q.K / MX_BLOCK, q.ldb, q.ldbs, q.ldc);
+        if (rc != MX_OK) return rc;
+        if (q.M < 1 || q.N < 1 || q.K < 128 || q.K % 128 || ldx < q.K || !aligned(x, 16) ||
+            ldx * (x_dtype == MX_FP32 ? 4 : 2) % 16 || !aligned(q.bq, 16) || q.ldb % 16 || 256 * q.ldb >= (int64_t)0x7FFFFFFF ||
+            !aligned(q.b_scale, 4) || q.ldbs % 4 || (q.ldb == 128 && q.K > 128))
+            return MX_EUNSUPPORTED;
+        a[j].lda = ldx, a[j].a_ks = 0;
+    }
+    if (!activation_rows_ok(problems[0].M, problems[0].K, columns)) return MX_EUNSUPPORTED;
+    hipStream_t st = (hipStream_t)stream;
+    if (stream_is_capturing(st)) return MX_ECAPTURE;
+    if (x_dtype == MX_FP32) return c_dtype == MX_BF16 ? launch_skinny<MX_BF16, MX_FP32>(a, count, st) : launch_skinny<MX_FP16, MX_FP32>(a, count, st);
+    return c_dtype == MX_BF16 ? launch_skinny<MX_BF16, MX_BF16>(a, count, st) : launch_skinny<MX_FP16, MX_FP16>(a, count, st);
 }
 
 extern "C" int mx_gemm_nt(const uint8_t *aq, const uint8_t *as, const uint8_t *bq, const uint8_t *bs, void *c,

@@ -14,10 +14,17 @@
 namespace mx {
 
 constexpr int SKINNY_WAVES = 8, SKINNY_N = 16;
+constexpr int SRC_CODES = -1;  // A is quantized; else the type of the activations that are quantized on the way
 __host__ __device__ constexpr int skinny_stage_bytes(int mt) { return (mt + 1) * 16 * 128; }
+// ... and, for activations, the scale words of the stage's rows
+__host__ __device__ constexpr int skinny_lds_bytes(int src, int mt, int u) {
+    return SKINNY_WAVES * u * (skinny_stage_bytes(mt) + (src == SRC_CODES ? 0 : 16 * mt * 4));
+}
 
-// MT: sub-tiles of 16 rows; U: K stages a wave has in flight.
-template <int CDT, int MT, int U, typename Args>
+// MT: sub-tiles of 16 rows; U: K stages a wave has in flight.  SRC: where A comes from.  With activations (`p.aq` are they, `p.lda`
+// their pitch in elements) the row quantizer's launch and its round trip through memory go away: every workgroup quantizes the
+// rows again, a K stage of four rows per load, as mx_quantize_rows does -- the same bytes.
+template <int CDT, int MT, int U, int SRC, int CAST, typename Args>
 __device__ __forceinline__ void skinny_gemm(const Args &p, int tile, uint8_t *smem) {
     const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int r16 = lane & 15, g = lane >> 4, n0 = tile * SKINNY_N;
@@ -26,11 +33,12 @@ __device__ __forceinline__ void skinny_gemm(const Args &p, int tile, uint8_t *sm
     const int64_t a_ks = p.a_ks ? p.a_ks : 128, b_ks = p.b_ks ? p.b_ks : 128;
     const int bn = p.N - n0;  // rows past a matrix repeat its last one; never stored
     uint8_t *const mine = smem + wave * (U * skinny_stage_bytes(MT));
+    uint32_t *const my_scales = (uint32_t *)(smem + SKINNY_WAVES * U * skinny_stage_bytes(MT)) + wave * (U * 16 * MT);  // activations
     const uint32_t copy_to = __builtin_amdgcn_readfirstlane(lds_addr(mine));
     uint32_t a_voff[2 * MT], b_voff[2];
     auto chunk_of = [&](int row) { return (uint32_t)(((lane & 7) ^ swz_a(row)) << 4); };
 #pragma unroll
-    for (int q = 0; q < 2 * MT; q++) {
+    for (int q = 0; q < 2 * MT && SRC == SRC_CODES; q++) {
         const int row = 8 * q + (lane >> 3);
         a_voff[q] = (uint32_t)((row < p.M ? row : p.M - 1) * p.lda) + chunk_of(row);
     }
@@ -44,7 +52,7 @@ __device__ __forceinline__ void skinny_gemm(const Args &p, int tile, uint8_t *sm
     constexpr int SW = (MT * 16 + 63) / 64;
     const uint8_t *sa_at[SW];
 #pragma unroll
-    for (int w = 0; w < SW; w++) sa_at[w] = p.as + (int64_t)(64 * w + lane < p.M ? 64 * w + lane : p.M - 1) * p.ldas;
+    for (int w = 0; w < SW && SRC == SRC_CODES; w++) sa_at[w] = p.as + (int64_t)(64 * w + lane < p.M ? 64 * w + lane : p.M - 1) * p.ldas;
     const uint8_t *const sb_at = p.bs + (int64_t)(n0 + (r16 < bn ? r16 : bn - 1)) * p.ldbs;
 
     v4f acc[MT];
@@ -57,7 +65,7 @@ __device__ __forceinline__ void skinny_gemm(const Args &p, int tile, uint8_t *sm
         for (int u = 0; u < U; u++) {
             const int s = s0 + u < end ? s0 + u : s0;  // an absent stage repeats the first one; never multiplied
 #pragma unroll
-            for (int w = 0; w < SW; w++) sa[u][w] = *(const uint32_t *)(sa_at[w] + 4 * s);
+            for (int w = 0; w < SW && SRC == SRC_CODES; w++) sa[u][w] = *(const uint32_t *)(sa_at[w] + 4 * s);
             sb[u] = *(const uint32_t *)(sb_at + 4 * s);
         }
 #pragma unroll
@@ -67,8 +75,38 @@ __device__ __forceinline__ void skinny_gemm(const Args &p, int tile, uint8_t *sm
             const uint32_t to = copy_to + u * skinny_stage_bytes(MT);
 #pragma unroll
             for (int q = 0; q < 2; q++) dma16(gb, b_voff[q], to + (2 * MT + q) * 1024);
+            if constexpr (SRC == SRC_CODES) {
 #pragma unroll
-            for (int q = 0; q < 2 * MT; q++) dma16(ga, a_voff[q], to + q * 1024);
+                for (int q = 0; q < 2 * MT; q++) dma16(ga, a_voff[q], to + q * 1024);
+            }
+        }
+        if constexpr (SRC != SRC_CODES) {
+            typedef Elem<SRC> E;
+            typename E::raw x[U][4 * MT];
+#pragma unroll
+            for (int u = 0; u < U; u++)
+#pragma unroll
+                for (int q = 0; q < 4 * MT; q++) {
+                    const int s = s0 + u < end ? s0 + u : s0, row = 4 * q + g < p.M ? 4 * q + g : p.M - 1;
+                    x[u][q] = E::load_raw((const typename E::type *)p.aq + (int64_t)row * p.lda + 128 * s + 8 * r16);
+                }
+#pragma unroll
+            for (int u = 0; u < U; u++)
+#pragma unroll
+                for (int q = 0; q < 4 * MT; q++) {
+                    if (4 * q >= p.M) break;  // rows past the matrix are multiplied as they lie in LDS and never stored
+                    float v[8];
+                    E::unpack(x[u][q], v);
+                    if constexpr (SRC == MX_FP32) round_values<CAST>(v);
+                    const uint32_t byte = scale_byte(quad_max(amax8(v)));
+                    const float inv = inv_scale(byte);
+                    v2i codes;
+                    codes[0] = (int)pack4_e4m3(v[0] * inv, v[1] * inv, v[2] * inv, v[3] * inv);
+                    codes[1] = (int)pack4_e4m3(v[4] * inv, v[5] * inv, v[6] * inv, v[7] * inv);
+                    const int row = 4 * q + g;
+                    *(v2i *)(mine + u * skinny_stage_bytes(MT) + row * 128 + (((r16 >> 1) ^ swz_a(row)) << 4) + 8 * (r16 & 1)) = codes;
+                    if ((r16 & 3) == 0) ((uint8_t *)(my_scales + u * 16 * MT + row))[r16 >> 2] = (uint8_t)byte;
+                }
         }
         wait_vm_allow_c<0>();
 #pragma unroll
@@ -84,7 +122,8 @@ __device__ __forceinline__ void skinny_gemm(const Args &p, int tile, uint8_t *sm
             const int bs = (int)(sb[u] >> (8 * g));
 #pragma unroll
             for (int i = 0; i < MT; i++) {
-                const int as = (int)((uint32_t)__shfl((int)sa[u][i / 4], 16 * (i % 4) + r16, 64) >> (8 * g));
+                const uint32_t word = SRC == SRC_CODES ? (uint32_t)__shfl((int)sa[u][i / 4], 16 * (i % 4) + r16, 64) : my_scales[u * 16 * MT + 16 * i + r16];
+                const int as = (int)(word >> (8 * g));
                 acc[i] = __builtin_amdgcn_mfma_scale_f32_16x16x128_f8f6f4(fragment(16 * i + r16), b, acc[i], 0, 0, 0, as, 0, bs);
             }
         }

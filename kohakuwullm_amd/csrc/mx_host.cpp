@@ -40,7 +40,7 @@ namespace {
 
 #define MX_ENTRIES(F)                                                                                                       \
     F(mx_quantize_rows) F(mx_quantize_tokens) F(mx_quantize_tokens_side) F(mx_join_codes) F(mx_quantize_dual_batch)         \
-    F(mx_swiglu_quantize_tokens) F(mx_swiglu_bwd_quantize_tokens) F(mx_gemm_nt) F(mx_gemm_nt_batch) F(mx_rmsnorm_quantize)  \
+    F(mx_swiglu_quantize_tokens) F(mx_swiglu_bwd_quantize_tokens) F(mx_gemm_nt) F(mx_gemm_nt_batch) F(mx_activation_gemm_nt) F(mx_rmsnorm_quantize) \
     F(mx_rmsnorm_backward) F(mx_rmsnorm_weight_grad) F(mx_router_topk) F(mx_router_backward_workspace)                      \
     F(mx_router_topk_backward) F(mx_expert_sort_workspace) F(mx_expert_sort_positions) F(mx_experts_gemm1)                  \
     F(mx_grouped_gemm_nt) F(mx_experts_combine) F(mx_experts_gemm2_dgrad) F(mx_quantize_cols_grouped) F(mx_grouped_wgrad_nt)
@@ -352,6 +352,27 @@ std::vector<Tensor> matmul_batch(const std::vector<Product> &ps, ScalarType type
     return outs;
 }
 
+// The products of a few rows with several weights, the rows quantized on the way; false, with nothing launched, for more rows
+// or another layout than that kernel takes.  `outs` are allocated here, x's shape with the weights' widths.
+bool activation_products(const Tensor &x, const Tensor &x2d, ScalarType compute, const std::vector<Quantized> &ws, std::vector<Tensor> &outs) {
+    if (x2d.size(0) > 32 || ws.size() > 4) return false;
+    mx_gemm_problem d[4];
+    for (size_t j = 0; j < ws.size(); j++) {
+        const Tensor &q = ws[j].q, &s = ws[j].s;
+        MX_NEED(plain(q) && plain(s) && q.dim() == 2 && s.dim() == 2 && q.stride(1) == 1 && s.stride(1) == 1 && q.size(1) == x2d.size(1) &&
+                s.size(0) == q.size(0) && s.size(1) * BLOCK == q.size(1) && q.element_size() == 1 && s.element_size() == 1 && q.size(0) > 0);
+        outs.push_back(empty(with_last(x, q.size(0)), compute, x2d));
+        d[j] = {nullptr, nullptr, bytes(q), bytes(s), outs.back().data_ptr(), x2d.size(0), q.size(0), q.size(1), 0, 0, q.stride(0), s.stride(0), q.size(0)};
+    }
+    const int status = lib.mx_activation_gemm_nt(x2d.const_data_ptr(), code_of(x2d.scalar_type()), x2d.stride(0), d, (int)ws.size(), code_of(compute), stream_of(x2d));
+    if (status == MX_EUNSUPPORTED) {
+        outs.clear();
+        return false;
+    }
+    check(status, "mx_activation_gemm_nt");
+    return true;
+}
+
 // ---- arguments and results -------------------------------------------------------------------------------------------------
 
 struct Args {
@@ -530,6 +551,8 @@ PyObject *py_linear_forward(Args &a) {
     const bool token_axis = a.flag();
     MX_NEED(plain(w.q) && w.q.dim() == 2 && x.defined() && x.dim() >= 1 && x.size(-1) == w.q.size(1));
     const Tensor x2d = activation_matrix(x, compute);
+    std::vector<Tensor> few;
+    if (!token_axis && activation_products(x, x2d, compute, {w}, few)) return wrap_all({few[0], Tensor(), Tensor()});
     const Tokens in = quantize_input(x2d, compute, token_axis);
     const Tensor out = matmul({in.row.q, in.row.s, w.q, w.s}, compute, with_last(x, w.q.size(0)), 0);
     return wrap_all({out, in.token.q, in.token.s});
@@ -554,6 +577,8 @@ PyObject *py_linear_eval(Args &a) {
     MX_NEED(x.defined() && unrecorded(x) && unrecorded(weight) && plain(w.q) && w.q.dim() == 2 && x.dim() >= 1 && x.size(-1) == w.q.size(1));
     const ScalarType compute = at::autocast::is_autocast_enabled(at::kCUDA) ? at::autocast::get_autocast_dtype(at::kCUDA) : x.scalar_type();
     const Tensor x2d = activation_matrix(x, compute);
+    std::vector<Tensor> out;
+    if (activation_products(x, x2d, compute, {w}, out)) return wrap(out[0]);
     const Tokens in = quantize_input(x2d, compute, false);
     return wrap(matmul({in.row.q, in.row.s, w.q, w.s}, compute, with_last(x, w.q.size(0)), 0));
 }
@@ -612,9 +637,13 @@ PyObject *py_group_forward(Args &a) {
     }
     MX_NEED(!ws.empty() && ws.size() <= 8);
     const Tensor x2d = activation_matrix(x, compute);
+    std::vector<Tensor> outs;
+    if (!token_axis && activation_products(x, x2d, compute, ws, outs)) {
+        outs.resize(outs.size() + 2);  // no operand along the tokens
+        return wrap_all(outs);
+    }
     const Tokens in = quantize_tokens(x2d, compute, 0, token_axis);
     mx_gemm_problem d[8];
-    std::vector<Tensor> outs;
     for (size_t j = 0; j < ws.size(); j++) {
         d[j] = describe({in.row.q, in.row.s, ws[j].q, ws[j].s});
         outs.push_back(empty(with_last(x, d[j].N), compute, x2d));
@@ -640,8 +669,15 @@ PyObject *py_swiglu_mlp_forward(Args &a) {
     MX_NEED(x.defined() && x.dim() >= 1 && x.size(-1) == in.q.size(1) && in.q.size(0) == 2 * out.q.size(1) && out.q.size(1) % PANEL == 0);
     const Tensor x2d = activation_matrix(x, compute);
     MX_NEED(x2d.size(0) * out.q.size(1) / 8 < ROW_CHUNKS);
-    const Tokens xs = quantize_tokens(x2d, compute, 0, wgrad_in);
-    const Tensor gu = matmul({xs.row.q, xs.row.s, in.q, in.s}, compute, {}, pad);
+    Tokens xs;
+    Tensor gu;
+    std::vector<Tensor> few;
+    if (!wgrad_in && activation_products(x2d, x2d, compute, {in}, few)) {
+        gu = few[0];
+    } else {
+        xs = quantize_tokens(x2d, compute, 0, wgrad_in);
+        gu = matmul({xs.row.q, xs.row.s, in.q, in.s}, compute, {}, pad);
+    }
     const Tokens hs = swiglu_tokens(gu, rounded, wgrad_out);
     const Tensor y = matmul({hs.row.q, hs.row.s, out.q, out.s}, compute, with_last(x, out.q.size(0)), 0);
     return wrap_all({y, xs.token.q, xs.token.s, gu, hs.token.q, hs.token.s});

@@ -21,21 +21,6 @@ __device__ __forceinline__ uint32_t gather_row_scales(uint32_t byte, int lane) {
     return v;
 }
 
-// fp32 values rounded to a 16-bit type and widened again: what a cast in front of the quantizer would have left.
-template <int CDT>
-__device__ __forceinline__ void round_values(float (&v)[8]) {
-    if constexpr (CDT == MX_BF16) {
-#pragma unroll
-        for (int c = 0; c < 8; c += 2) {
-            const uint32_t w = pack2_bf16(v[c], v[c + 1]);
-            v[c] = bits2f(w << 16), v[c + 1] = bits2f(w & 0xFFFF0000u);
-        }
-    } else if constexpr (CDT == MX_FP16) {
-#pragma unroll
-        for (int c = 0; c < 8; c++) v[c] = (float)(_Float16)v[c];
-    }
-}
-
 // CDT: the type fp32 values are rounded to before they are quantized (MX_FP32: none).
 template <int DT, int U, bool FLAT, int CDT = MX_FP32>
 __global__ __launch_bounds__(256) void quant_rows_kernel(const void *__restrict__ x, uint32_t chunks_per_row,

@@ -101,3 +101,33 @@ def test_ring_gemm_short_and_long_products_in_one_launch(oracle):
     ops = [_operands(oracle, *s) for s in [(200, 512, 1536), (1536, 512, 256), (130, 60, 640), (264, 129, 384)]]
     for o, out in zip(ops, mxfp8_matmul_pq_batch([_dev(o, panels=i == 1) for i, o in enumerate(ops)], torch.bfloat16)):
         assert oracle.rel_error(out.cpu(), oracle.gemm_nt(*o)) < TOL[torch.bfloat16]
+
+
+@pytest.mark.parametrize("m,n,k", [(1, 1, 128), (3, 17, 640), (16, 4100, 4096), (17, 48, 1152), (32, 520, 2048)])
+@pytest.mark.parametrize("xt,ct", [(torch.bfloat16, torch.bfloat16), (torch.float16, torch.float16), (torch.float32, torch.bfloat16), (torch.float32, torch.float16)])
+def test_activations_quantized_inside_the_product(m, n, k, xt, ct):
+    """The bits of the row quantizer and the product behind it, for rows at any pitch; zeros, infinities and NaN among them."""
+    import ctypes
+
+    from kohakuwullm_amd import _lib
+    from kohakuwullm_amd.kernels.mxfp8 import mxfp8_matmul_pq, quantize_mx
+
+    g = torch.Generator(device=DEV).manual_seed(SEED + m)
+    x = torch.randn(m, k + 8, device=DEV, generator=g).to(xt)[:, :k]
+    x[0, :32] = 0
+    x[-1, 40], x[-1, 70] = float("inf"), float("nan")
+    ws = [quantize_mx(torch.randn(c, k, device=DEV, generator=g).bfloat16()) for c in (n, 50)]
+    outs = [torch.empty(m, w[0].shape[0], device=DEV, dtype=ct) for w in ws]
+
+    def call(rows=m, depth=k, out=ct, at=0):
+        records = _lib.words(_lib.GemmProblem, [(0, 0, q.data_ptr(), s.data_ptr(), o.data_ptr(), rows, q.shape[0], depth, 0, 0, k, k // 32, q.shape[0])
+                                                for (q, s), o in zip(ws, outs)])
+        return _lib.load().mx_activation_gemm_nt(x.data_ptr() + at, _lib.MX_DTYPE[xt], x.stride(0), ctypes.byref(records), 2, _lib.MX_DTYPE[out], _lib.stream_of(x))
+
+    assert call() == _lib.MX_OK
+    xq, xs = quantize_mx(x.to(ct))
+    for o, w in zip(outs, ws):
+        want = mxfp8_matmul_pq(xq, xs, *w, ct)
+        assert torch.equal(o.view(torch.int16), want.view(torch.int16)) or torch.equal(o.isnan(), want.isnan()) and torch.equal(o.nan_to_num(), want.nan_to_num())
+    refused = [call(rows=33), call(depth=k - 32), call(at=2), call(out=torch.float32)]
+    assert refused == [_lib.MX_EUNSUPPORTED] * 4
