@@ -24,9 +24,9 @@ struct DenseArgs {
     int tiles_m, tiles_n;
     int c_vec;
     int accumulate;  // fp32 atomic add into C (split-K)
-    int split_k;     // number of K slices; tile ids run over tiles_m * tiles_n * split_k
-    float *slice_ws;  // with split_k > 1 and no accumulate: slice s of tile i leaves its fp32 partial in slot
-                      // i * split_k + s of this buffer and slice_reduce_kernel adds the slices
+    int split_k;     // number of K slices of the tiles from dp_tiles on
+    float *slice_ws;  // with split_k > 1 and no accumulate: slice s of tile dp_tiles + i leaves its fp32 partial in slot
+                      // i * split_k + s of this buffer and slice_reduce adds the slices
     // Even K split of the last, partial round of tiles.  Tile ids [0, dp_tiles) are whole tiles
     // dealt round-robin; the K stages of the remaining sk_tiles tiles are laid end to end (each
     // tile padded to KT4 stages) and cut into gridDim.x equal ranges of sk_q stages, one per
@@ -88,17 +88,20 @@ struct DenseProblem {
         }
         t.sk = -1;
         if (p.sk_tiles && next_id >= p.dp_tiles) return false;
-        if (next_id >= per_slice * p.split_k) return false;
-        const int slice = next_id / per_slice;
-        const int index = next_id - slice * per_slice;
+        // whole tiles, then slice after slice of the others: units that run side by side read the same part of K
+        const int cut = per_slice - p.dp_tiles;
+        if (next_id >= p.dp_tiles + cut * p.split_k) return false;
+        const bool whole = next_id < p.dp_tiles;
+        const int slice = whole ? 0 : (next_id - p.dp_tiles) / cut;
+        const int index = next_id - slice * cut, split = whole ? 1 : p.split_k;
         int tm, tn;
         tile_of(index, p.tiles_m, p.tiles_n, tm, tn, stagger_columns(p.K), p.xcds);
-        t.slot = p.slice_ws ? index * p.split_k + slice : -1;
+        t.slot = p.slice_ws && !whole ? (index - p.dp_tiles) * p.split_k + slice : -1;
         t.m0 = tm * S::BM;
         t.n0 = tn * S::BN;
         const int KT = ((p.K + 127) >> 7);
         // K slices are multiples of 4 stages so every slice starts on a 16-byte scale boundary
-        const int per = (((KT + p.split_k - 1) / p.split_k) + 3) & ~3;
+        const int per = (((KT + split - 1) / split) + 3) & ~3;
         t.kt0 = slice * per < KT ? slice * per : KT;
         t.kt1 = t.kt0 + per < KT ? t.kt0 + per : KT;
         next_id += stride;
@@ -336,16 +339,16 @@ __global__ __launch_bounds__(S::NTHR) void split_reduce_kernel(DenseArgs p) {
     }
 }
 
-// Adds the split_k fp32 slices of every tile, in slice order, and stores C.  One block per (tile, i).
+// Adds the split_k fp32 slices of every tile that was cut, in slice order, and stores C.  One block per (tile, i).
 template <typename S, int CDT>
 __device__ __forceinline__ void slice_reduce(const DenseArgs &p, int block) {
-    const int index = block / S::MT, i = block % S::MT;
+    const int local = block / S::MT, index = p.dp_tiles + local, i = block % S::MT;
     const int tid = threadIdx.x;
     v4f sum[S::NT];
 #pragma unroll
     for (int j = 0; j < S::NT; j++) sum[j] = v4f{0.f, 0.f, 0.f, 0.f};
     for (int sl = 0; sl < p.split_k; sl++) {
-        const v4f *src = (const v4f *)p.slice_ws + (int64_t)(index * p.split_k + sl) * (S::BM * S::BN / 4);
+        const v4f *src = (const v4f *)p.slice_ws + (int64_t)(local * p.split_k + sl) * (S::BM * S::BN / 4);
 #pragma unroll
         for (int j = 0; j < S::NT; j++) sum[j] += src[(i * S::NT + j) * S::NTHR + tid];
     }
@@ -364,11 +367,6 @@ __device__ __forceinline__ void slice_reduce(const DenseArgs &p, int block) {
             store_run<CDT, S::NT>(p.c, (int64_t)m * p.ldc + n, run, p.N - n < S::NT ? p.N - n : S::NT, p.c_vec != 0);
         }
     }
-}
-
-template <typename S, int CDT>
-__global__ __launch_bounds__(S::NTHR) void slice_reduce_kernel(DenseArgs p) {
-    slice_reduce<S, CDT>(p, (int)blockIdx.x);
 }
 
 // Up to MX_BATCH_MAX products on the ring kernel's tiles behind one launch: workgroup `id` belongs to the problem whose
@@ -399,11 +397,11 @@ __global__ __launch_bounds__(SKINNY_WAVES * 64) void gemm_nt_skinny_kernel(RingA
 }
 
 // slice_reduce for every problem of such a launch that was cut along K (`end` counts blocks of those).
-template <int CDT>
-__global__ __launch_bounds__(RingShape::NTHR) void ring_reduce_kernel(RingArgs b) {
+template <typename S, int CDT>
+__global__ __launch_bounds__(S::NTHR) void reduce_slices_kernel(RingArgs b) {
     int j = 0;
     while (j + 1 < b.count && (int)blockIdx.x >= b.end[j]) j++;
-    slice_reduce<RingShape, CDT>(b.prob[j], (int)blockIdx.x - (j ? b.end[j - 1] : 0));
+    slice_reduce<S, CDT>(b.prob[j], (int)blockIdx.x - (j ? b.end[j - 1] : 0));
 }
 
 // Any K % 32 == 0, any alignment: one thread per output element.  The slow path.
@@ -600,6 +598,29 @@ static int launch_skinny(const DenseArgs *probs, int count, hipStream_t st) {
     else return launch_skinny_tiles<CDT, 8, 1, SRC>(b, blocks, st);
 }
 
+// K stages of each of the `wgs` equal ranges that the stages of `rest` tiles, laid end to end, are cut into: a multiple of 4 (scale
+// fetches are 16-byte aligned) and at least an eighth of a tile, so no tile is cut into more than 9 pieces.
+static int64_t deal_q(int64_t rest, int KT, int wgs) {
+    const int KT4 = (KT + 3) & ~3;
+    const int64_t q = (rest * KT4 + wgs - 1) / wgs;
+    return ((q < KT4 / 8 ? KT4 / 8 : q) + 3) & ~(int64_t)3;
+}
+
+// K slices for the `rest` tiles of a last, partial round on `wgs` workgroups that have two fp32 tile slots each: the count in
+// [1, 8] that ends the round soonest, priced in K stages into `t` (a slice is at least 8 stages; a cut round costs 8 stages for its
+// second launch and a tenth of one per fp32 partial tile).
+static int rest_slices(int64_t rest, int KT, int wgs, bool may_cut, int64_t &t) {
+    int best = 1;
+    t = rest ? KT + 4 : 0;
+    for (int c = 2; c <= 8 && rest && may_cut && c * rest <= 2 * wgs; c++) {
+        const int per = ((KT + c - 1) / c + 3) & ~3;
+        if (per < 8 || (c - 1) * per >= KT) break;
+        const int64_t cut = (c * rest + wgs - 1) / wgs * (per + 4) + 8 + c * rest / 10;
+        if (cut < t) t = cut, best = c;
+    }
+    return best;
+}
+
 template <typename S, int CDT>
 static int launch_tiled(DenseArgs a, float *ws, int ws_slots, hipStream_t st, bool phased = false) {
     a.tiles_m = (a.M + S::BM - 1) / S::BM;
@@ -609,13 +630,11 @@ static int launch_tiled(DenseArgs a, float *ws, int ws_slots, hipStream_t st, bo
     const int mode = scale_mode(a);
     const int64_t work = (int64_t)a.tiles_m * a.tiles_n * a.split_k;
     const int cus = num_cus();
-    a.dp_tiles = (int)work, a.sk_tiles = 0, a.sk_q = 0, a.sk_ws = nullptr;
+    a.dp_tiles = a.split_k > 1 ? 0 : (int)work, a.sk_tiles = 0, a.sk_q = 0, a.sk_ws = nullptr;
     // The last round of tiles occupies `rest` of the `cus` workgroups for a whole tile time.
     // Dealing the K stages of those tiles evenly over all workgroups instead saves
     // (cus - rest) / cus of a tile time and costs an fp32 round trip of every piece plus a
-    // second launch; in units of one K stage, measured: 4 + 0.15 per piece.  Ranges are sk_q
-    // stages, a multiple of 4 (scale fetches are 16-byte aligned) and at least an eighth of a
-    // tile, so no tile is cut into more than 9 pieces.
+    // second launch; in units of one K stage, measured: 4 + 0.15 per piece.
     const int rest = (int)(work % cus);
     const int KT = ((a.K + 127) >> 7), KT4 = (KT + 3) & ~3;
     bool deal = a.split_k == 1 && !a.accumulate && rest > 0 && KT4 >= 8;
@@ -623,9 +642,7 @@ static int launch_tiled(DenseArgs a, float *ws, int ws_slots, hipStream_t st, bo
     deal = deal && !ring_pays(a);  // an alternative kernel splits K where the default would, and there the default is the ring
 #endif
     if (deal) {
-        int64_t q = ((int64_t)rest * KT4 + cus - 1) / cus;
-        if (q < KT4 / 8) q = KT4 / 8;
-        q = (q + 3) & ~(int64_t)3;
+        const int64_t q = deal_q(rest, KT, cus);
         const double pieces = (double)rest * KT4 / q + rest;
         const double gain = (double)(KT4 - q), cost = 4.0 + 0.15 * pieces;
         float *slots = gain > 1.25 * cost && ws_slots >= 2 * cus ? ws : nullptr;  // two slots per workgroup
@@ -677,7 +694,7 @@ static int launch_pair(DenseArgs a, hipStream_t st) {
     a.c_vec = aligned(a.c, 16) && (a.ldc * (CDT == MX_FP32 ? 4 : 2)) % 16 == 0;
     const int mode = scale_mode(a);
     const int64_t work = (int64_t)a.tiles_m * a.tiles_n * a.split_k;
-    a.dp_tiles = (int)work, a.sk_tiles = 0, a.sk_q = 0, a.sk_ws = nullptr;
+    a.dp_tiles = a.split_k > 1 ? 0 : (int)work, a.sk_tiles = 0, a.sk_q = 0, a.sk_ws = nullptr;
     const int wgs = 2 * num_cus();
     dim3 grid((unsigned)(work < wgs ? work : wgs)), block(S::NTHR);
     const int rc = mode == SCALES_VEC16   ? launch_with_lds<gemm_nt_pair_kernel<S, CDT, SCALES_VEC16>>(grid, block, S::LDS_BYTES, st, a)
@@ -709,9 +726,10 @@ static int launch_ring(DenseArgs *probs, int count, float *ws, int ws_slots, hip
         a.tiles_n = (a.N + S::BN - 1) / S::BN;
         a.c_vec = aligned(a.c, 16) && (a.ldc * (CDT == MX_FP32 ? 4 : 2)) % 16 == 0;
         const int tiles = a.tiles_m * a.tiles_n;
-        a.dp_tiles = tiles, a.sk_tiles = 0, a.sk_q = 0, a.sk_ws = nullptr;
+        a.sk_tiles = 0, a.sk_q = 0, a.sk_ws = nullptr;
         a.xcds = 8, a.phased = 0;
         a.split_k = ring_slices(a, free_tiles);
+        a.dp_tiles = a.split_k > 1 ? 0 : tiles;
         a.slice_ws = nullptr;
         if (a.split_k > 1) {
             a.slice_ws = ws + slot * (S::BM * S::BN);
@@ -728,7 +746,7 @@ static int launch_ring(DenseArgs *probs, int count, float *ws, int ws_slots, hip
     const dim3 grid((unsigned)blocks), block(S::NTHR);
     const int rc = launch_with_lds<gemm_nt_ring_kernel<CDT>>(grid, block, RING_LDS_BYTES, st, b);
     if (rc != MX_OK) return rc;
-    if (red.count) ring_reduce_kernel<CDT><<<dim3((unsigned)rblocks), block, 0, st>>>(red);
+    if (red.count) reduce_slices_kernel<S, CDT><<<dim3((unsigned)rblocks), block, 0, st>>>(red);
     return hipGetLastError() == hipSuccess ? MX_OK : MX_ELAUNCH;
 }
 
@@ -755,14 +773,15 @@ static int gemm_dispatch(DenseArgs a, float *ws, int ws_slots, hipStream_t st, b
     return launch_tiled<DenseShape, CDT>(a, ws, ws_slots, st, phased);
 }
 
-// Several products behind one launch, the eight XCDs shared out among them whole.  Every problem
-// gets one XCD, the rest go, one at a time, to the problem that would otherwise finish last; cost
-// of a problem on n workgroups = rounds of tiles x (K stages + 4 for the tile's prologue and
-// epilogue).  A problem with few, long tiles (a weight gradient) may in addition be cut into 2 or
-// 4 K slices that run as independent tiles and leave fp32 partial sums for slice_reduce_kernel;
-// every combination of slice counts is priced (a partial tile costs about 0.1 stage of
-// everyone's time) and the cheapest plan wins, against running the products one after the other
-// as well.
+// Several products behind one launch, the eight XCDs shared out among them whole.  Every problem gets one XCD, the rest go, one
+// at a time, to the problem that would otherwise finish last; cost of a problem on n workgroups = rounds of tiles x (K stages + 4
+// for the tile's prologue and epilogue), with the tiles of its last, partial round whole or in K slices (rest_slices), whichever
+// ends sooner.  Taken where it beats the products one after the other, and, for products that would each go to the ring kernel
+// alone, where it beats the ring's tiles side by side.  us before (all tiles of a problem cut into 1, 2 or 4 slices, or the ring) / now:
+//   dX and both dW of a 1536 x 4096 feed-forward over 5003 / 6144 tokens, fp32 results   200 / 167   211 / 189
+//   ... of a 1024 x 2816 one over 4096 / 8192 tokens, bf16                               87.8 / 78.4   135 / 120
+//   dX and dW of a 2048 -> 3072 layer over 3001 / 4096                                   53.4 / 47.7   72.2 / 60.1
+//   ... of 1536 -> 1536 over 6144 / 11000 / 16384                                        59.2 / 53.3   92.7 / 77.7   116.6 / 96.4
 template <int CDT>
 static int batch_dispatch(DenseArgs *probs, int count, float *ws, int ws_slots, hipStream_t st) {
     typedef DenseShape S;
@@ -774,7 +793,6 @@ static int batch_dispatch(DenseArgs *probs, int count, float *ws, int ws_slots, 
     for (int j = 0; j < count; j++) skinny = skinny && tiled_ok(probs[j]) && skinny_pays(probs[j]);
     if (skinny && count) return launch_skinny<CDT>(probs, count, st);
     for (int j = 0; j < count; j++) ring = ring && tiled_ok(probs[j]) && ring_pays(probs[j]);
-    if (ring && count) return launch_ring<CDT>(probs, count, ws, ws_slots, st);
     bool fuse = count > 1 && count <= MX_BATCH_MAX;
     DenseBatchArgs b;
     int64_t tiles[MX_BATCH_MAX], alone = 0;
@@ -798,8 +816,7 @@ static int batch_dispatch(DenseArgs *probs, int count, float *ws, int ws_slots, 
         const int64_t rest = tiles[j] % cus, KT4 = (KT[j] + 3) & ~3;
         alone += tiles[j] / cus * (KT[j] + 4);
         if (rest) {
-            int64_t q = (rest * KT4 + cus - 1) / cus;
-            q = ((q < KT4 / 8 ? KT4 / 8 : q) + 3) & ~(int64_t)3;
+            const int64_t q = deal_q(rest, KT[j], cus);
             const double pieces = (double)rest * KT4 / q + rest, cost = 4.0 + 0.15 * pieces;
             alone += KT4 >= 8 && ws_slots >= 2 * cus && (double)(KT4 - q) > 1.25 * cost ? q + (int64_t)cost : KT[j] + 4;
         }
@@ -811,56 +828,48 @@ static int batch_dispatch(DenseArgs *probs, int count, float *ws, int ws_slots, 
         // products of the feed-forward block (1.5, 0.75 and 0.4 rounds) 482 against 536.
         if (tiles[j] >= 2 * (int64_t)cus) fuse = false;
     }
-    // Plan: a number of whole XCDs for every problem (they add up to 8) and a number of K slices,
-    // chosen together by pricing every combination.
-    int share[MX_BATCH_MAX], slices[MX_BATCH_MAX], best_share[MX_BATCH_MAX], best_slices[MX_BATCH_MAX];
-    int64_t best = -1;
-    fuse = fuse && cus % 8 == 0 && count <= 8;
+    // Plan: a number of whole XCDs for every problem (they add up to 8); the tiles of its last, partial round whole or in K slices.
+    int share[MX_BATCH_MAX], slices[MX_BATCH_MAX];
+    int64_t finish[MX_BATCH_MAX], load[MX_BATCH_MAX], longest = 0;
+    fuse = fuse && cus % 8 == 0;
+    const int per_xcd = cus / 8;
     if (fuse) {
-        const int per_xcd = cus / 8;
-        const int slots = ws_slots < 2 * cus ? ws_slots : 2 * cus;  // fp32 tile slots the caller's workspace offers
-        auto per_slice = [&](int j) { return (((KT[j] + slices[j] - 1) / slices[j]) + 3) & ~3; };
-        auto units = [&](int j) { return tiles[j] * slices[j]; };
-        auto finish = [&](int j) {
-            return (units(j) + per_xcd * share[j] - 1) / (per_xcd * share[j]) * (per_slice(j) + 4);
+        auto price = [&](int j) {
+            const int wgs = per_xcd * share[j];
+            int64_t last;
+            slices[j] = rest_slices(tiles[j] % wgs, KT[j], wgs, ws_slots >= 2 * cus, last);
+            finish[j] = tiles[j] / wgs * (KT[j] + 4) + last;
+            load[j] = finish[j] + tiles[j] * (KT[j] + 4) / (2 * wgs);
         };
-        int combos = 1;
-        for (int j = 0; j < count; j++) combos *= 3;
-        for (int code = 0; code < combos; code++) {
-            int64_t partial = 0;
-            bool ok = true;
-            for (int j = 0, c = code; j < count; j++, c /= 3) {
-                slices[j] = 1 << (c % 3);
-                // every slice must own K stages, and at least 16 of them to be worth a partial tile
-                if (slices[j] > 1 && (KT[j] < 16 * slices[j] || (slices[j] - 1) * per_slice(j) >= KT[j])) ok = false;
-                if (slices[j] > 1) partial += units(j);
-                share[j] = 1;
-            }
-            if (!ok || partial > slots) continue;
-            // the XCDs beyond one each go, one at a time, to the problem that would finish last
-            for (int left = 8 - count; left > 0; left--) {
-                int worst = 0;
-                for (int j = 1; j < count; j++)
-                    if (finish(j) > finish(worst)) worst = j;
-                share[worst]++;
-            }
-            int64_t together = partial ? 4 + partial / 10 : 0;
-            int64_t longest = 0;
-            for (int j = 0; j < count; j++) longest = finish(j) > longest ? finish(j) : longest;
-            together += longest;
-            if (best < 0 || together < best) {
-                best = together;
-                for (int j = 0; j < count; j++) best_share[j] = share[j], best_slices[j] = slices[j];
-            }
+        for (int j = 0; j < count; j++) share[j] = 1, price(j);
+        // The XCDs beyond one each go, one at a time, to the problem that would finish last; rounds being whole, one XCD more
+        // often changes nothing, so the work per workgroup counts half as much.
+        for (int left = 8 - count; left > 0; left--) {
+            int worst = 0;
+            for (int j = 1; j < count; j++)
+                if (load[j] > load[worst]) worst = j;
+            share[worst]++;
+            price(worst);
         }
-        fuse = best >= 0 && best < alone;
+        for (int j = 0; j < count; j++) longest = finish[j] > longest ? finish[j] : longest;
+        for (int j = 0; j < count; j++) {  // partial tiles are written for the problem that the others wait for, or not at all
+            const int wgs = per_xcd * share[j];
+            if ((tiles[j] + wgs - 1) / wgs * (KT[j] + 4) <= longest) slices[j] = 1;
+        }
+        fuse = longest < alone;
     }
-    float *scratch = nullptr;
-    if (fuse) {
-        bool any = false;
-        for (int j = 0; j < count; j++) any = any || best_slices[j] > 1;
-        if (any) scratch = ws;  // the plan fitted its partial tiles into the workspace's slots
+    // Ring tiles side by side against the plan, in us: 0.6 per stage and 2.5 per tile of a CU's share and 8, against 1.57 per stage
+    // of the plan and 6.  us ring / plan where the line lies: 2048 x 2048 x 3072 with its dW 42.7 / 46.4, 3001 x 2048 x 2048 36.3 / 47.0,
+    // 4096 x 2048 x 2048 48.4 / 59.0, 3001 x 2048 x 3072 52.8 / 47.0, 4096 x 1024 x 5632 with two dW 87.9 / 78.5.
+    if (ring && fuse) {
+        double stages = 0, blocks = 0;
+        for (int j = 0; j < count; j++) {
+            const int64_t small = tiles_of(probs[j], RingShape::BM);
+            blocks += small, stages += (double)small * KT[j];
+        }
+        ring = mode != SCALES_VEC16 || 0.6 * stages / cus + 2.5 * blocks / cus + 8 < 1.57 * longest + 6;
     }
+    if (ring && count) return launch_ring<CDT>(probs, count, ws, ws_slots, st);
     if (!fuse) {
         for (int j = 0; j < count; j++) {
             int rc = gemm_dispatch<CDT>(probs[j], ws, ws_slots, st);
@@ -868,17 +877,25 @@ static int batch_dispatch(DenseArgs *probs, int count, float *ws, int ws_slots, 
         }
         return MX_OK;
     }
+    RingArgs red;
+    red.count = 0;
     b.x_lo[0] = 0;
-    int64_t slot_base = 0;
+    int64_t slot = 0;
+    int rblocks = 0;
     for (int j = 0; j < count; j++) {
         DenseArgs &a = probs[j];
-        a.split_k = best_slices[j];
-        a.xcds = best_share[j];
-        if (a.split_k > 1) {
-            a.slice_ws = scratch + slot_base * (S::BM * S::BN);
-            slot_base += tiles[j] * a.split_k;
+        a.xcds = share[j];
+        const int rest = (int)(tiles[j] % (per_xcd * share[j]));
+        if (slices[j] > 1) {
+            a.split_k = slices[j];
+            a.dp_tiles -= rest;
+            a.slice_ws = ws + slot * (S::BM * S::BN);
+            slot += rest * slices[j];
+            red.prob[red.count] = a;
+            rblocks += rest * S::MT;
+            red.end[red.count++] = rblocks;
         }
-        b.x_lo[j + 1] = b.x_lo[j] + best_share[j];
+        b.x_lo[j + 1] = b.x_lo[j] + share[j];
         b.prob[j] = a;
     }
     b.count = count;
@@ -891,9 +908,7 @@ static int batch_dispatch(DenseArgs *probs, int count, float *ws, int ws_slots, 
                        ? launch_with_lds<gemm_nt_batch_kernel<S, CDT, SCALES_DWORD>>(grid, block, S::LDS_BYTES, st, b)
                        : launch_with_lds<gemm_nt_batch_kernel<S, CDT, SCALES_BYTES>>(grid, block, S::LDS_BYTES, st, b);
     if (rc != MX_OK) return rc;
-    for (int j = 0; j < count; j++)
-        if (probs[j].split_k > 1)
-            slice_reduce_kernel<S, CDT><<<dim3((unsigned)(tiles[j] * S::MT)), dim3(S::NTHR), 0, st>>>(probs[j]);
+    if (red.count) reduce_slices_kernel<S, CDT><<<dim3((unsigned)rblocks), block, 0, st>>>(red);
     return hipGetLastError() == hipSuccess ? MX_OK : MX_ELAUNCH;
 }
 

@@ -131,3 +131,25 @@ def test_activations_quantized_inside_the_product(m, n, k, xt, ct):
         assert torch.equal(o.view(torch.int16), want.view(torch.int16)) or torch.equal(o.isnan(), want.isnan()) and torch.equal(o.nan_to_num(), want.nan_to_num())
     refused = [call(rows=33), call(depth=k - 32), call(at=2), call(out=torch.float32)]
     assert refused == [_lib.MX_EUNSUPPORTED] * 4
+
+
+@pytest.mark.parametrize("k", [(8192, 8192), (8320, 8192), (8192 + 32, 9216)])  # 16 scale bytes, 4 and 1 at a time; slices of unequal length
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+def test_batch_cuts_the_tiles_of_its_last_round(k, dtype):
+    """130 tiles each on half of the chip: a round of whole tiles and two tiles in K slices, ragged rows and columns among them."""
+    from kohakuwullm_amd.kernels.mxfp8 import mxfp8_matmul_pq_batch
+
+    g = torch.Generator(DEV).manual_seed(SEED)
+
+    def codes(rows, cols):  # every finite code, scales over eight octaves
+        q = torch.randint(0, 254, (rows, cols), generator=g, device=DEV, dtype=torch.uint8)
+        q = q + (q >= 127).to(torch.uint8)
+        return q, torch.randint(115, 123, (rows, cols // 32), generator=g, device=DEV, dtype=torch.uint8)
+
+    def value(q, s):
+        return q.view(F8).double() * torch.exp2(s.double() - 127.0).repeat_interleave(32, dim=1)
+
+    problems = [(*codes(m, kk), *codes(n, kk)) for (m, n), kk in zip(((3300, 2500), (2490, 3310)), k)]
+    for (aq, a_s, bq, b_s), out in zip(problems, mxfp8_matmul_pq_batch([(a.view(F8), s, b.view(F8), t) for a, s, b, t in problems], dtype)):
+        ref = value(aq, a_s) @ value(bq, b_s).T
+        assert ((out.double() - ref).norm() / ref.norm()).item() < TOL[dtype]
