@@ -99,10 +99,10 @@ __device__ __forceinline__ void skinny_gemm(const Args &p, int tile, uint8_t *sm
                     E::unpack(x[u][q], v);
                     if constexpr (SRC == MX_FP32) round_values<CAST>(v);
                     const uint32_t byte = scale_byte(quad_max(amax8(v)));
-                    const float inv = inv_scale(byte);
+                    const float scale = block_scale(byte);
                     v2i codes;
-                    codes[0] = (int)pack4_e4m3(v[0] * inv, v[1] * inv, v[2] * inv, v[3] * inv);
-                    codes[1] = (int)pack4_e4m3(v[4] * inv, v[5] * inv, v[6] * inv, v[7] * inv);
+                    codes[0] = (int)pack4_e4m3(v[0], v[1], v[2], v[3], scale);
+                    codes[1] = (int)pack4_e4m3(v[4], v[5], v[6], v[7], scale);
                     const int row = 4 * q + g;
                     *(v2i *)(mine + u * skinny_stage_bytes(MT) + row * 128 + (((r16 >> 1) ^ swz_a(row)) << 4) + 8 * (r16 & 1)) = codes;
                     if ((r16 & 3) == 0) ((uint8_t *)(my_scales + u * 16 * MT + row))[r16 >> 2] = (uint8_t)byte;

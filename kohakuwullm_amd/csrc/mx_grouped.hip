@@ -454,9 +454,9 @@ struct GroupedProblem {
                     for (int e = 0; e < 4; e++) r[e] = gv[e] * sigmoid_f(gv[e]) * vv[e];
                     const float amax = oct_max(fmaxf(fmaxf(fabsf(r[0]), fabsf(r[1])), fmaxf(fabsf(r[2]), fabsf(r[3]))));
                     const uint32_t byte = scale_byte(amax);
-                    const float inv = inv_scale(byte);
+                    const float scale = block_scale(byte);
                     if (ok) {
-                        *(uint32_t *)(p.hq + (int64_t)m * p.ldhq + h) = pack4_e4m3(r[0] * inv, r[1] * inv, r[2] * inv, r[3] * inv);
+                        *(uint32_t *)(p.hq + (int64_t)m * p.ldhq + h) = pack4_e4m3(r[0], r[1], r[2], r[3], scale);
                         if ((L.r16 & 7) == 0) p.hs[(int64_t)m * p.ldhs + (hblock >> 5)] = (uint8_t)byte;
                     }
 #pragma unroll
@@ -475,12 +475,12 @@ struct GroupedProblem {
                 cm = fmaxf(cm, __shfl_xor(cm, 16, 64));
                 cm = fmaxf(cm, __shfl_xor(cm, 32, 64));
                 const uint32_t byte = scale_byte(cm);
-                const float inv = inv_scale(byte);
+                const float scale = block_scale(byte);
                 const int col = L.wn * (S::WTN / 2) + 4 * L.r16 + e;  // hidden unit inside the tile
 #pragma unroll
                 for (int ii = 0; ii < 2; ii++) {
                     const int row = L.wm * S::WTM + 16 * (2 * blk + ii) + 4 * L.g;  // 4 consecutive rows: one dword
-                    const uint32_t w = pack4_e4m3(a[ii][0][e] * inv, a[ii][1][e] * inv, a[ii][2][e] * inv, a[ii][3][e] * inv);
+                    const uint32_t w = pack4_e4m3(a[ii][0][e], a[ii][1][e], a[ii][2][e], a[ii][3][e], scale);
                     // column-major, BM bytes per hidden unit, 16-byte chunks XOR-swizzled by the lane's r16
                     *(uint32_t *)(lds.a + col * S::BM + ((((row >> 4) ^ (col >> 2)) & (CH - 1)) << 4) + (row & 15)) = w;
                 }
@@ -657,7 +657,7 @@ struct GroupedProblem {
                 const float amax_g = quad_max(amax8(dg));
                 const float amax_v = quad_max(amax8(dv));
                 const uint32_t bg = scale_byte(amax_g), bv = scale_byte(amax_v);
-                const float ig = inv_scale(bg), iv = inv_scale(bv);
+                const float gscale = block_scale(bg), vscale = block_scale(bv);
                 if (ok) {
                     uint32_t w[4], x[4];
                     float tg[8], tv[8];
@@ -676,10 +676,10 @@ struct GroupedProblem {
 #pragma unroll
                     for (int e = 0; e < 4; e++) keep[0][i][v][e] = w[e], keep[1][i][v][e] = x[e];
                     v2i cg, cv;
-                    cg[0] = (int)pack4_e4m3(dg[0] * ig, dg[1] * ig, dg[2] * ig, dg[3] * ig);
-                    cg[1] = (int)pack4_e4m3(dg[4] * ig, dg[5] * ig, dg[6] * ig, dg[7] * ig);
-                    cv[0] = (int)pack4_e4m3(dv[0] * iv, dv[1] * iv, dv[2] * iv, dv[3] * iv);
-                    cv[1] = (int)pack4_e4m3(dv[4] * iv, dv[5] * iv, dv[6] * iv, dv[7] * iv);
+                    cg[0] = (int)pack4_e4m3(dg[0], dg[1], dg[2], dg[3], gscale);
+                    cg[1] = (int)pack4_e4m3(dg[4], dg[5], dg[6], dg[7], gscale);
+                    cv[0] = (int)pack4_e4m3(dv[0], dv[1], dv[2], dv[3], vscale);
+                    cv[1] = (int)pack4_e4m3(dv[4], dv[5], dv[6], dv[7], vscale);
                     uint8_t *qp = p.dpq + (int64_t)m * p.lddpq + h;
                     *(v2i *)qp = cg;
                     *(v2i *)(qp + H) = cv;
@@ -737,12 +737,12 @@ struct GroupedProblem {
                     cm = fmaxf(cm, __shfl_xor(cm, 16, 64));
                     cm = fmaxf(cm, __shfl_xor(cm, 32, 64));
                     const uint32_t byte = scale_byte(cm);
-                    const float inv = inv_scale(byte);
+                    const float scale = block_scale(byte);
                     const int col = L.wn * (S::WTN / 2) + 4 * o_r16 + e;
 #pragma unroll
                     for (int ii = 0; ii < 2; ii++) {
                         const int row = L.wm * S::WTM + 16 * (2 * blk + ii) + 4 * o_g;  // 4 consecutive rows: one dword
-                        const uint32_t w = pack4_e4m3(val[ii][0] * inv, val[ii][1] * inv, val[ii][2] * inv, val[ii][3] * inv);
+                        const uint32_t w = pack4_e4m3(val[ii][0], val[ii][1], val[ii][2], val[ii][3], scale);
                         // column-major, BM bytes per column, 16-byte chunks XOR-swizzled by the lane's r16
                         *(uint32_t *)(codes + col * S::BM + ((((row >> 4) ^ (col >> 2)) & (CH - 1)) << 4) + (row & 15)) = w;
                     }

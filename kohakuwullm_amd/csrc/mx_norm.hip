@@ -82,12 +82,12 @@ __device__ __forceinline__ void norm_chunk(const NormArgs &a, int64_t row, int c
     if (!a.q) return;
     const float amax = quad_max(amax8(y));
     const uint32_t byte = scale_byte(amax);
-    const float inv = inv_scale(byte);
+    const float scale = block_scale(byte);
     const uint32_t packed = gather16(byte, lane);
     if (!ok) return;
     v2i codes;
-    codes[0] = (int)pack4_e4m3(y[0] * inv, y[1] * inv, y[2] * inv, y[3] * inv);
-    codes[1] = (int)pack4_e4m3(y[4] * inv, y[5] * inv, y[6] * inv, y[7] * inv);
+    codes[0] = (int)pack4_e4m3(y[0], y[1], y[2], y[3], scale);
+    codes[1] = (int)pack4_e4m3(y[4], y[5], y[6], y[7], scale);
     *(v2i *)(a.q + row * a.ldq + c * 8) = codes;
     // 16 lanes hold 4 consecutive blocks: one dword when all four exist and the scale row is
     // dword-aligned there, single bytes otherwise

@@ -61,12 +61,12 @@ __global__ __launch_bounds__(256) void quant_rows_kernel(const void *__restrict_
     for (int u = 0; u < U; u++) {
         float amax = quad_max(amax8(v[u]));
         uint32_t byte = scale_byte(amax);
-        float inv = inv_scale(byte);
+        const float scale = block_scale(byte);
         uint32_t packed = gather_row_scales(byte, lane);
         if (ok[u]) {
             v2i codes;
-            codes[0] = (int)pack4_e4m3(v[u][0] * inv, v[u][1] * inv, v[u][2] * inv, v[u][3] * inv);
-            codes[1] = (int)pack4_e4m3(v[u][4] * inv, v[u][5] * inv, v[u][6] * inv, v[u][7] * inv);
+            codes[0] = (int)pack4_e4m3(v[u][0], v[u][1], v[u][2], v[u][3], scale);
+            codes[1] = (int)pack4_e4m3(v[u][4], v[u][5], v[u][6], v[u][7], scale);
             *(v2i *)(q + qoff[u]) = codes;
             // The 16 lanes of a DPP row hold 4 consecutive blocks.  They are all valid or
             // the tail of the tensor cuts the group, in which case bytes are stored singly.
@@ -119,12 +119,12 @@ __global__ __launch_bounds__(256) void quant_heads_kernel(const void *__restrict
         const uint32_t chunk = base + u * 256;
         float amax = quad_max(amax8(v[u]));
         uint32_t byte = scale_byte(amax);
-        float inv = inv_scale(byte);
+        const float scale = block_scale(byte);
         uint32_t packed = gather_row_scales(byte, lane);
         if (ok[u]) {
             v2i codes;
-            codes[0] = (int)pack4_e4m3(v[u][0] * inv, v[u][1] * inv, v[u][2] * inv, v[u][3] * inv);
-            codes[1] = (int)pack4_e4m3(v[u][4] * inv, v[u][5] * inv, v[u][6] * inv, v[u][7] * inv);
+            codes[0] = (int)pack4_e4m3(v[u][0], v[u][1], v[u][2], v[u][3], scale);
+            codes[1] = (int)pack4_e4m3(v[u][4], v[u][5], v[u][6], v[u][7], scale);
             *(v2i *)(q + (int64_t)chunk * 8) = codes;
             bool group_full = (chunk | 15u) < total_chunks;
             if (pack_scales && group_full) {
@@ -155,11 +155,11 @@ __global__ __launch_bounds__(256) void quant_rows_generic_kernel(const void *__r
         amax = fmaxf(amax, fabsf(v[i]));
     }
     uint32_t byte = scale_byte(amax);
-    float inv = inv_scale(byte);
+    const float scale = block_scale(byte);
     uint8_t *qo = q + row * ldq + kb * MX_BLOCK;
 #pragma unroll
     for (int i = 0; i < MX_BLOCK; i += 4) {
-        uint32_t c = pack4_e4m3(v[i] * inv, v[i + 1] * inv, v[i + 2] * inv, v[i + 3] * inv);
+        uint32_t c = pack4_e4m3(v[i], v[i + 1], v[i + 2], v[i + 3], scale);
         qo[i] = (uint8_t)c;
         qo[i + 1] = (uint8_t)(c >> 8);
         qo[i + 2] = (uint8_t)(c >> 16);
@@ -242,7 +242,7 @@ __device__ __forceinline__ void quant_tile(float (&v)[R][8], const QuantTileOut 
         for (int i = 0; i < R; i++) {
             float amax = quad_max(amax8(v[i]));
             uint32_t byte = scale_byte(amax);
-            float inv = inv_scale(byte);
+            const float scale = block_scale(byte);
             // the scale bytes of a tile row in one word: four (R = 8, 16 lanes) or two (R = 4, 8 lanes)
             uint32_t packed;
             if (R == 8) {
@@ -255,8 +255,8 @@ __device__ __forceinline__ void quant_tile(float (&v)[R][8], const QuantTileOut 
             }
             if (col_ok && (whole || row0 + i < M)) {
                 v2i codes;
-                codes[0] = (int)pack4_e4m3(v[i][0] * inv, v[i][1] * inv, v[i][2] * inv, v[i][3] * inv);
-                codes[1] = (int)pack4_e4m3(v[i][4] * inv, v[i][5] * inv, v[i][6] * inv, v[i][7] * inv);
+                codes[0] = (int)pack4_e4m3(v[i][0], v[i][1], v[i][2], v[i][3], scale);
+                codes[1] = (int)pack4_e4m3(v[i][4], v[i][5], v[i][6], v[i][7], scale);
                 stream_store<NTS>((v2i *)(o.q + (o.q_ks ? (col >> 7) * o.q_ks + (row0 + i) * 128 + (col & 127) : (row0 + i) * o.ldq + col)), codes);
                 uint8_t *sp = o.s + (row0 + i) * o.lds + (col >> 5);
                 bool full = !EDGE || kc0 + G::TK <= K;
@@ -293,15 +293,15 @@ __device__ __forceinline__ void quant_tile(float (&v)[R][8], const QuantTileOut 
 #pragma unroll
     for (int c = 0; c < 8; c++) {
         uint32_t byte = scale_byte(cm[c]);
-        float inv = inv_scale(byte);
+        const float scale = block_scale(byte);
         uint8_t *dst = tile + (cg * 8 + c) * QC_PITCH + rg * R;
         if (R == 8) {
             v2i codes;
-            codes[0] = (int)pack4_e4m3(v[0][c] * inv, v[1][c] * inv, v[2][c] * inv, v[3][c] * inv);
-            codes[1] = (int)pack4_e4m3(v[R - 4][c] * inv, v[R - 3][c] * inv, v[R - 2][c] * inv, v[R - 1][c] * inv);
+            codes[0] = (int)pack4_e4m3(v[0][c], v[1][c], v[2][c], v[3][c], scale);
+            codes[1] = (int)pack4_e4m3(v[R - 4][c], v[R - 3][c], v[R - 2][c], v[R - 1][c], scale);
             *(v2i *)dst = codes;
         } else {
-            *(uint32_t *)dst = pack4_e4m3(v[0][c] * inv, v[1][c] * inv, v[2][c] * inv, v[3][c] * inv);
+            *(uint32_t *)dst = pack4_e4m3(v[0][c], v[1][c], v[2][c], v[3][c], scale);
         }
         if (rg % (32 / R) == 0) tscale[(cg * 8 + c) * 4 + wave] = (uint8_t)byte;
     }
@@ -361,12 +361,12 @@ __device__ __forceinline__ void quant_tile_raw(typename Elem<DT>::raw (&r)[8], c
             for (int c = 0; c < 8; c++) v[c] = E::elem(r[i], c);
             const float amax = quad_max(amax8(v));
             const uint32_t byte = scale_byte(amax);
-            const float inv = inv_scale(byte);
+            const float scale = block_scale(byte);
             const uint32_t packed = gather_row_scales(byte, lane);
             if (col_ok && (whole || row0 + i < M)) {
                 v2i codes;
-                codes[0] = (int)pack4_e4m3(v[0] * inv, v[1] * inv, v[2] * inv, v[3] * inv);
-                codes[1] = (int)pack4_e4m3(v[4] * inv, v[5] * inv, v[6] * inv, v[7] * inv);
+                codes[0] = (int)pack4_e4m3(v[0], v[1], v[2], v[3], scale);
+                codes[1] = (int)pack4_e4m3(v[4], v[5], v[6], v[7], scale);
                 stream_store<NTS>((v2i *)(o.q + (o.q_ks ? (col >> 7) * o.q_ks + (row0 + i) * 128 + (col & 127) : (row0 + i) * o.ldq + col)), codes);
                 uint8_t *sp = o.s + (row0 + i) * o.lds + (col >> 5);
                 const bool full = !EDGE || kc0 + G::TK <= K;
@@ -391,10 +391,10 @@ __device__ __forceinline__ void quant_tile_raw(typename Elem<DT>::raw (&r)[8], c
         cm = fmaxf(cm, __shfl_xor(cm, 16, 64));
         cm = fmaxf(cm, __shfl_xor(cm, 32, 64));
         const uint32_t byte = scale_byte(cm);
-        const float inv = inv_scale(byte);
+        const float scale = block_scale(byte);
         v2i codes;
-        codes[0] = (int)pack4_e4m3(v[0] * inv, v[1] * inv, v[2] * inv, v[3] * inv);
-        codes[1] = (int)pack4_e4m3(v[4] * inv, v[5] * inv, v[6] * inv, v[7] * inv);
+        codes[0] = (int)pack4_e4m3(v[0], v[1], v[2], v[3], scale);
+        codes[1] = (int)pack4_e4m3(v[4], v[5], v[6], v[7], scale);
         *(v2i *)(tile + (cg * 8 + c) * QC_PITCH + rg * 8) = codes;
         if ((rg & 3) == 0) tscale[(cg * 8 + c) * 4 + wave] = (uint8_t)byte;
     }
@@ -830,12 +830,12 @@ __global__ __launch_bounds__(256) void swiglu_quant_rows_kernel(const void *__re
         if constexpr (ROUNDED) round_values<DT>(v);
         float amax = quad_max(amax8(v));
         uint32_t byte = scale_byte(amax);
-        float inv = inv_scale(byte);
+        const float scale = block_scale(byte);
         uint32_t packed = gather_row_scales(byte, lane);
         if (ok[u]) {
             v2i codes;
-            codes[0] = (int)pack4_e4m3(v[0] * inv, v[1] * inv, v[2] * inv, v[3] * inv);
-            codes[1] = (int)pack4_e4m3(v[4] * inv, v[5] * inv, v[6] * inv, v[7] * inv);
+            codes[0] = (int)pack4_e4m3(v[0], v[1], v[2], v[3], scale);
+            codes[1] = (int)pack4_e4m3(v[4], v[5], v[6], v[7], scale);
             *(v2i *)(q + qoff[u]) = codes;
             bool group_full = ((base + u * 256) | 15u) < total_chunks;
             if (pack_scales && group_full) {
