@@ -5,9 +5,10 @@
 //
 // As a composition of library operators the same work is 15 launches forward and 20 backward over tensors of a few KB to
 // a few MB, with the hidden states widened to fp32 in memory first: 160 + 300 us of a 1.55 ms block at 16384 tokens of
-// 1024 and 64 experts, and nothing but launches at a few tokens.  Here it is two launches forward (28 us; one where the
-// tokens fit a workgroup, which then needs no histogram cleared in front of it) and three backward (47 us).
+// 1024 and 64 experts, and nothing but launches at a few tokens.  Here it is two launches forward (25 us; one where the
+// tokens fit a workgroup, which then needs no histogram cleared in front of it) and three backward (45 us).
 #include <atomic>
+#include <type_traits>
 
 #include "mx_common.h"
 
@@ -58,13 +59,14 @@ struct RouterArgs {
 
 constexpr int ROUTER_WAVES = 8, ROUTER_ROWS = 16;
 
-// Largest of the wave's 64 unsigned values, to every lane (DPP: a running maximum along the rows, then across them).
-__device__ __forceinline__ uint32_t wave_max_u32(uint32_t v) {
-    int x = (int)v;
-#define MX_DPP_MAX(ctrl, rows)                                                                     \
-    {                                                                                              \
-        const uint32_t o = (uint32_t)__builtin_amdgcn_update_dpp(0, x, ctrl, rows, 0xF, false);    \
-        x = (int)((uint32_t)x > o ? (uint32_t)x : o);                                              \
+// Largest of the wave's 64 unsigned values, to every lane (DPP: a running maximum along the rows, then across them), for several
+// values side by side.
+template <int N>
+__device__ __forceinline__ void wave_max_u32(uint32_t (&v)[N]) {
+#define MX_DPP_MAX(ctrl, rows)                                                                          \
+    _Pragma("unroll") for (int i = 0; i < N; i++) {                                                     \
+        const uint32_t o = (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v[i], ctrl, rows, 0xF, false); \
+        v[i] = v[i] > o ? v[i] : o;                                                                     \
     }
     MX_DPP_MAX(0x111, 0xF)  // row_shr:1
     MX_DPP_MAX(0x112, 0xF)
@@ -73,7 +75,8 @@ __device__ __forceinline__ uint32_t wave_max_u32(uint32_t v) {
     MX_DPP_MAX(0x142, 0xA)  // row_bcast:15 into rows 1 and 3
     MX_DPP_MAX(0x143, 0xC)  // row_bcast:31 into rows 2 and 3
 #undef MX_DPP_MAX
-    return (uint32_t)__builtin_amdgcn_readlane(x, 63);
+#pragma unroll
+    for (int i = 0; i < N; i++) v[i] = (uint32_t)__builtin_amdgcn_readlane((int)v[i], 63);
 }
 
 template <int DT>
@@ -90,25 +93,30 @@ __device__ __forceinline__ v4f mfma_16bit(v4i a, v4i b, v4f c) {
 // an operand of the 16-bit MFMA (16x16x32) as it stands; its products are exact and its sums fp32 (measured against fp64:
 // rms error of a logit 2.4e-7 at D = 1024, the fp32 library product 3.9e-7).  Operands of mixed or fp32 type run on the fp32
 // MFMA (16x16x4), step i taking element i of every lane.  The K axis is dealt to the eight waves 32 at a time, ROUTER_AHEAD
-// such steps are requested before the first is used, and the waves' partial logits meet in LDS, sixteen tokens at a time.
-// Then a wave selects for two tokens: top_k times the maximum of the experts' keys, one or more experts per lane; ties go to
-// the lower expert.
+// such steps are requested before the first is used, and the waves' partial logits meet in LDS.
+// Then a wave selects for two tokens, or for four at a time: top_k times the maximum of the experts' keys, one or more experts per
+// lane; ties go to the lower expert.
 // What bounds it: the loads of the operands at large token counts -- a lane group of 16 reads 16 rows, so a load instruction
 // takes the texture path 64 clocks instead of 16 -- which is why a workgroup reads w once for 64 tokens when there are enough
-// of them (16384 x 1024, 64 experts: 35 us with one tile of 16 tokens, 26 us with four, of which 10 us are the selection),
-// and the chain load - product - selection of one workgroup at small ones (10 us at 32 tokens).
+// of them (16384 x 1024, 64 experts: 35 us with one tile of 16 tokens, 23 us with four; 26 with half as many loads in flight and
+// one selection at a time), and the chain load - product - selection of one workgroup at small ones (9 us at 32 tokens).
 constexpr int ROUTER_AHEAD = 4;
 template <int XDT, int WDT, int NT, int MT>
 __global__ __launch_bounds__(ROUTER_WAVES * 64, MT > 1 ? 2 : NT <= 8 ? 4 : 2) void router_topk_kernel(RouterArgs p) {
     typedef typename Elem<XDT>::type X;
     typedef typename Elem<WDT>::type W;
     constexpr int PITCH = NT * 16 + 4;
-    constexpr int AHEAD = NT <= 4 && XDT != MX_FP32 && WDT != MX_FP32 ? (MT > 2 ? 2 : ROUTER_AHEAD) : 1;  // as registers allow
+    constexpr int AHEAD = NT <= 4 && XDT != MX_FP32 && WDT != MX_FP32 ? ROUTER_AHEAD : 1;  // as registers allow
     extern __shared__ float slices[];  // [wave][token][expert], then the histogram
-    int32_t *hist = (int32_t *)(slices + ROUTER_WAVES * ROUTER_ROWS * PITCH);
+    int32_t *hist = (int32_t *)(slices + ROUTER_WAVES * ROUTER_ROWS * MT * PITCH);
     const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6), r = lane & 15, g = lane >> 4;
     const int first = blockIdx.x * ROUTER_ROWS * MT;
     for (int e = tid; e < p.E; e += ROUTER_WAVES * 64) hist[e] = 0;
+
+    constexpr int Q = (NT * 16 + 63) / 64;  // experts per lane
+    float bias[Q];
+#pragma unroll
+    for (int q = 0; q < Q; q++) bias[q] = p.bias && lane + 64 * q < p.E ? load_float(p.bias, p.bias_dtype, lane + 64 * q) : 0.0f;
 
     const X *xr[MT];
     const W *wr[NT];
@@ -167,66 +175,78 @@ __global__ __launch_bounds__(ROUTER_WAVES * 64, MT > 1 ? 2 : NT <= 8 ? 4 : 2) vo
             }
         }
     }
+    float *mine = slices + wave * ROUTER_ROWS * MT * PITCH;
 #pragma unroll
-    for (int m = 0; m < MT; m++) {
-        const int t0 = first + 16 * m;
-        if (MT > 1 && t0 >= p.T) break;  // uniform in the workgroup
-        if (m) __syncthreads();  // the previous sixteen tokens' logits have been read
-        float *mine = slices + wave * ROUTER_ROWS * PITCH;
+    for (int m = 0; m < MT; m++)
 #pragma unroll
         for (int j = 0; j < NT; j++)
 #pragma unroll
-            for (int v = 0; v < 4; v++) mine[(4 * g + v) * PITCH + 16 * j + r] = acc[m][j][v];
-        __syncthreads();
+            for (int v = 0; v < 4; v++) mine[(16 * m + 4 * g + v) * PITCH + 16 * j + r] = acc[m][j][v];
+    __syncthreads();
 
-        constexpr int Q = (NT * 16 + 63) / 64;  // experts per lane
+    // A wave's tokens in groups of two or four side by side: every step of a selection waits for the one before it.  One barrier
+    // for all tiles of 16: behind the stores of a tile's results, each further one waited for those to reach memory.
+    constexpr int TOKENS = ROUTER_ROWS * MT / ROUTER_WAVES, U = TOKENS < 4 ? TOKENS : 4;
 #pragma unroll 1
-        for (int u = 0; u < ROUTER_ROWS / ROUTER_WAVES; u++) {
-            const int row = wave * (ROUTER_ROWS / ROUTER_WAVES) + u, t = t0 + row;
-            if (t >= p.T) break;  // uniform in the wave
-            float score[Q];
-            uint32_t key[Q];  // 0: no expert, or one already taken (no float has that key)
+    for (int row0 = wave * TOKENS; row0 < (wave + 1) * TOKENS && first + row0 < p.T; row0 += U) {
+        float score[U][Q];
+        uint32_t key[U][Q];  // 0: no expert, or one already taken (no float has that key)
 #pragma unroll
-            for (int q = 0; q < Q; q++) {
-                const int e = lane + 64 * q;
+        for (int q = 0; q < Q; q++) {
+            const int e = lane + 64 * q;
+            float part[U][ROUTER_WAVES];
+#pragma unroll
+            for (int u = 0; u < U; u++)
+#pragma unroll
+                for (int s = 0; s < ROUTER_WAVES; s++) part[u][s] = slices[(s * ROUTER_ROWS * MT + row0 + u) * PITCH + (e < p.E ? e : 0)];
+#pragma unroll
+            for (int u = 0; u < U; u++) {
                 float logit = 0.0f;
-                if (e < p.E) {
 #pragma unroll
-                    for (int s = 0; s < ROUTER_WAVES; s++) logit += slices[(s * ROUTER_ROWS + row) * PITCH + e];
-                }
-                score[q] = router_sigmoid(logit);
-                float by = score[q];
-                if (p.bias && e < p.E) by += load_float(p.bias, p.bias_dtype, e);
-                key[q] = e < p.E ? ordered_key(by) : 0u;
+                for (int s = 0; s < ROUTER_WAVES; s++) logit += part[u][s];
+                score[u][q] = router_sigmoid(logit);
+                key[u][q] = e < p.E ? ordered_key(p.bias ? score[u][q] + bias[q] : score[u][q]) : 0u;
             }
-            float total = 0.0f, mine_s = 0.0f;
-            int mine_e = 0;
-            for (int i = 0; i < p.top_k; i++) {
-                uint32_t best = key[0];
+        }
+        float total[U], mine_s[U];
+        int mine_e[U];
 #pragma unroll
-                for (int q = 1; q < Q; q++) best = key[q] > best ? key[q] : best;
-                best = wave_max_u32(best);
+        for (int u = 0; u < U; u++) total[u] = mine_s[u] = 0.0f, mine_e[u] = 0;
+        for (int i = 0; i < p.top_k; i++) {
+            uint32_t best[U];
+#pragma unroll
+            for (int u = 0; u < U; u++) {
+                best[u] = key[u][0];
+#pragma unroll
+                for (int q = 1; q < Q; q++) best[u] = key[u][q] > best[u] ? key[u][q] : best[u];
+            }
+            wave_max_u32(best);
+#pragma unroll
+            for (int u = 0; u < U; u++) {
                 bool open = true;
 #pragma unroll
                 for (int q = 0; q < Q; q++) {
-                    const uint64_t holders = __ballot(open && key[q] == best);
-                    if (holders == 0) continue;  // uniform; at q the first lane of the lowest experts wins
+                    const uint64_t holders = __ballot(open && key[u][q] == best[u]);
+                    if (Q > 1 && holders == 0) continue;  // uniform; at q the first lane of the lowest experts wins
                     const int at = __builtin_ctzll(holders);
-                    const float s = bits2f((uint32_t)__builtin_amdgcn_readlane((int)f2bits(score[q]), at));
-                    total += s;
-                    if (lane == i) mine_s = s, mine_e = at + 64 * q;
-                    if (lane == at) key[q] = 0u;
+                    const float s = bits2f((uint32_t)__builtin_amdgcn_readlane((int)f2bits(score[u][q]), at));
+                    total[u] += s;
+                    if (lane == i) mine_s[u] = s, mine_e[u] = at + 64 * q;
+                    if (lane == at) key[u][q] = 0u;
                     open = false;
                 }
             }
-            total = clamp_total(total);
-            if (lane < p.top_k) {
-                const int64_t at = (int64_t)t * p.top_k + lane;
-                p.idx[at] = mine_e;
-                store_float(p.weight, XDT, at, (p.norm ? mine_s / total : mine_s) * p.factor);
-                if (p.scores) p.scores[at] = mine_s;
-                atomicAdd(&hist[mine_e], 1);
-            }
+        }
+#pragma unroll
+        for (int u = 0; u < U; u++) {
+            const int t = first + row0 + u;
+            if (t >= p.T || lane >= p.top_k) continue;
+            const float sum = clamp_total(total[u]);
+            const int64_t at = (int64_t)t * p.top_k + lane;
+            p.idx[at] = mine_e[u];
+            store_float(p.weight, XDT, at, (p.norm ? mine_s[u] / sum : mine_s[u]) * p.factor);
+            if (p.scores) p.scores[at] = mine_s[u];
+            atomicAdd(&hist[mine_e[u]], 1);
         }
     }
     __syncthreads();
@@ -257,64 +277,77 @@ struct RouterBwdArgs {
     int chunks, chunk_tokens;
 };
 
-// d loss / d logit of the picks of tokens [lo, lo + n): through the factor, the optional normalisation and the sigmoid.
-// w_i = f s_i / S with S = sum s (or 1) gives ds_i = f (g_i - [S above the clamp] (sum_j g_j s_j) / S) / S.
-// One thread per pick, so the loads are contiguous; sink(pick, gradient, expert) takes each.
-template <typename F>
-__device__ __forceinline__ void form_picks(const RouterBwdArgs &p, int64_t lo, int n, v2f *gs, int threads, F &&sink) {
-    const int total = n * p.top_k;
-    const int64_t base = lo * p.top_k;
-    for (int i = threadIdx.x; i < total; i += threads) gs[i] = v2f{load_float(p.gw, p.gw_dtype, base + i) * p.factor, p.scores[base + i]};
-    __syncthreads();
-    for (int i = threadIdx.x; i < total; i += threads) {
-        const int e = (int)p.idx[base + i];
-        const float g = gs[i][0], s = gs[i][1];
-        float ds = g;
-        if (p.norm) {
-            const int first = i / p.top_k * p.top_k;
-            float sum = 0.0f, dot = 0.0f;
-            for (int j = 0; j < p.top_k; j++) {
-                const v2f other = gs[first + j];
-                sum += other[1];
-                dot += other[0] * other[1];
-            }
-            const float S = clamp_total(sum);
-            ds = (g - (sum < 1e-9f ? 0.0f : dot / S)) / S;
-        }
-        sink(i, ds * s * (1.0f - s), e);
+// d loss / d logit of a pick, through the factor (in g already), the optional normalisation and the sigmoid: w_i = f s_i / S with
+// S = sum s (or 1) gives ds_i = f (g_i - [S above the clamp] (sum_j g_j s_j) / S) / S.
+__device__ __forceinline__ float pick_gradient(const RouterBwdArgs &p, float g, float s, float sum, float dot) {
+    float ds = g;
+    if (p.norm) {
+        const float S = clamp_total(sum);
+        ds = (g - (sum < 1e-9f ? 0.0f : dot / S)) / S;
     }
-    __syncthreads();
+    return ds * s * (1.0f - s);
 }
 
 // dx[t] = sum over the picks of dlogit * w[expert], a wave per token.  top_k of E terms are not zero, so this is a gather of
-// top_k rows of the router matrix, not a matrix product.  16384 x 1024 bf16, 6 picks: 17 us for 201 MB of rows read through
-// L2, where the matrix's 128 KB stay, and 34 MB of dx written: 12 TB/s of the one, and 2 of the other, far from the 5.1 a
-// copy reaches -- the gather is what it waits for, not the store.
-constexpr int ROUTER_MAX_K = 16, ROUTER_DX_TOKENS = 16;
+// top_k rows of the router matrix, not a matrix product.  Lane i of a wave forms the gradient of the token's pick i, the sums over
+// the picks go lane by lane through scalar registers, and the next token's picks are requested ahead: a wave waits for nobody else.
+// us with sixteen tokens' picks formed by a workgroup in LDS, behind two round trips to memory and two barriers / now, bf16 and 6
+// picks: 2777 x 1024 12.7 / 8.1, 16384 x 1024 16.8 / 18.0 (201 MB of rows from L2 and 5 us of multiplications by the vector ALU;
+// with the matrix in LDS 22.4, its copy costs more than L2 does).
+constexpr int ROUTER_MAX_K = 16;
 template <int XDT, int WDT>
 __global__ __launch_bounds__(256) void router_dx_kernel(RouterBwdArgs p) {
     typedef typename Elem<XDT>::type X;
     typedef typename Elem<WDT>::type W;
-    __shared__ v2i picks[ROUTER_DX_TOKENS * ROUTER_MAX_K];
-    __shared__ v2f gs[ROUTER_DX_TOKENS * ROUTER_MAX_K];
-    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-    const int64_t lo = (int64_t)blockIdx.x * ROUTER_DX_TOKENS;
-    const int n = (int)(p.T - lo < ROUTER_DX_TOKENS ? p.T - lo : ROUTER_DX_TOKENS);
-    form_picks(p, lo, n, gs, 256, [&](int i, float dl, int e) { picks[i] = v2i{(int)f2bits(dl), e}; });
-    for (int u = wave; u < n; u += 4) {
-        for (int col = lane * 8; col < p.D; col += 512) {
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int64_t stride = (int64_t)gridDim.x * 4, mine = lane < p.top_k ? lane : 0;
+    int64_t t = (int64_t)blockIdx.x * 4 + wave;
+    if (t >= p.T) return;
+    struct Pick {
+        float g, s;
+        int e;
+    };
+    auto pick_of = [&](int64_t token) {
+        const int64_t at = token * p.top_k + mine;
+        return Pick{load_float(p.gw, p.gw_dtype, at) * p.factor, p.scores[at], (int)p.idx[at]};
+    };
+    Pick next = pick_of(t);
+    for (; t < p.T; t += stride) {
+        const float g = next.g, s = next.s;
+        const int e = next.e;
+        next = pick_of(t + stride < p.T ? t + stride : t);
+        float sum = 0.0f, dot = 0.0f;
+        if (p.norm) {
+            for (int j = 0; j < p.top_k; j++) {
+                const float sj = bits2f((uint32_t)__builtin_amdgcn_readlane((int)f2bits(s), j));
+                sum += sj;
+                dot += bits2f((uint32_t)__builtin_amdgcn_readlane((int)f2bits(g), j)) * sj;
+            }
+        }
+        const float dl = pick_gradient(p, g, s, sum, dot);
+        for (int first = 0; first < p.D; first += 512) {  // every lane of the wave goes along: the picks are read from them
+            const int col = first + lane * 8, from = col < p.D ? col : 0;
             float acc[8];
 #pragma unroll
             for (int c = 0; c < 8; c++) acc[c] = 0.0f;
-#pragma unroll 4
-            for (int i = 0; i < p.top_k; i++) {
-                const v2i pick = picks[u * p.top_k + i];
-                float wv[8];
-                Elem<WDT>::load8((const W *)p.w + (int64_t)pick[1] * p.D + col, wv);
+            for (int i0 = 0; i0 < p.top_k; i0 += 8) {
+                typename Elem<WDT>::raw row[8];
 #pragma unroll
-                for (int c = 0; c < 8; c++) acc[c] += bits2f((uint32_t)pick[0]) * wv[c];
+                for (int i = 0; i < 8; i++)  // all of them are requested before the first is waited for
+                    if (i0 + i < p.top_k)
+                        row[i] = Elem<WDT>::template load_raw<false>((const W *)p.w + (int64_t)__builtin_amdgcn_readlane(e, i0 + i) * p.D + from);
+#pragma unroll
+                for (int i = 0; i < 8; i++) {
+                    if (i0 + i >= p.top_k) break;  // uniform
+                    const float dli = bits2f((uint32_t)__builtin_amdgcn_readlane((int)f2bits(dl), i0 + i));
+                    float wv[8];
+                    Elem<WDT>::unpack(row[i], wv);
+#pragma unroll
+                    for (int c = 0; c < 8; c++) acc[c] += dli * wv[c];
+                }
             }
-            X *dst = (X *)p.dx + (lo + u) * p.lddx + col;
+            if (col >= p.D) continue;
+            X *dst = (X *)p.dx + t * p.lddx + col;
             if (XDT == MX_FP32) {
                 ((v4f *)dst)[0] = v4f{acc[0], acc[1], acc[2], acc[3]};
                 ((v4f *)dst)[1] = v4f{acc[4], acc[5], acc[6], acc[7]};
@@ -337,14 +370,25 @@ __global__ __launch_bounds__(256) void router_dx_kernel(RouterBwdArgs p) {
 // them.  A lane loads four columns of each of eight tokens, so column tile j of a wave holds columns c0 + 4 r + j.
 // bf16 hidden states run on the bf16 MFMA: the fp32 gradient is kept whole as the sum of three bf16 (8 bits each), the
 // products are exact and the sums fp32, and 48 MFMAs per 32 tokens take 768 clocks where the fp32 form needs 4096 (16384 x
-// 1024, 64 experts: 25 us, bound by the read of x and 17 MB of partial sums); other types take the fp32 MFMA.  The chunks' fp32 partial matrices are added in order by router_dw_kernel (deterministic).
-constexpr int ROUTER_CHUNK = 256, ROUTER_DW_COLS = 256;
+// 1024, 64 experts: 22 us, 25 with four waves, one step of x ahead and the picks fetched in turn; the read of x and 17 MB of
+// partial sums take 10 of them, the chain picks - gradients - products most of the others); other types take the fp32 MFMA.  The chunks' fp32 partial matrices are added in order by router_dw_kernel (deterministic).
+constexpr int ROUTER_CHUNK = 256, ROUTER_DW_COLS = 256, ROUTER_DW_THREADS = 512;
 __host__ __device__ constexpr int router_dw_pitch(int tokens, bool split) { return split ? tokens + 8 : tokens + 4; }
 __host__ __device__ constexpr int router_dw_lds(int tokens, int top_k, bool split) {
-    return (split ? 3 * 64 * router_dw_pitch(tokens, true) * 2 : 64 * router_dw_pitch(tokens, false) * 4) + tokens * top_k * 8;
+    const int used = (split ? 3 * 64 * router_dw_pitch(tokens, true) * 2 : 64 * router_dw_pitch(tokens, false) * 4) + tokens * top_k * 8;
+    return used < 65536 ? 65536 : used;  // at the end the odd steps' sums of 64 x 256 elements
 }
+// f(std::integral_constant<int, 0>{}), ..., f(std::integral_constant<int, N - 1>{})
+template <int N, int I = 0, typename F>
+__device__ __forceinline__ void static_for_steps(F &&f) {
+    if constexpr (I < N) {
+        f(std::integral_constant<int, I>{});
+        static_for_steps<N, I + 1>(f);
+    }
+}
+
 template <int XDT>
-__global__ __launch_bounds__(256) void router_dw_partial_kernel(RouterBwdArgs p) {
+__global__ __launch_bounds__(ROUTER_DW_THREADS) void router_dw_partial_kernel(RouterBwdArgs p) {
     typedef typename Elem<XDT>::type X;
     constexpr bool SPLIT = XDT == MX_BF16;
     typedef X x4 __attribute__((ext_vector_type(4)));
@@ -354,7 +398,8 @@ __global__ __launch_bounds__(256) void router_dw_partial_kernel(RouterBwdArgs p)
     const int dense_bytes = SPLIT ? 3 * plane * 2 : plane * 4;
     v2f *const gs = (v2f *)(dw_smem + dense_bytes);
     const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6), r = lane & 15, g = lane >> 4;
-    const int e0 = (int)blockIdx.y * 64, col = (int)blockIdx.x * ROUTER_DW_COLS + wave * 64 + 4 * r;
+    const int e0 = (int)blockIdx.y * 64, col = (int)blockIdx.x * ROUTER_DW_COLS + (wave & 3) * 64 + 4 * r;
+    const int half = wave >> 2;  // waves 0-3 take the even steps of 32 tokens, waves 4-7 the odd ones
     const int64_t lo = (int64_t)blockIdx.z * p.chunk_tokens;
     const int n = (int)(p.T - lo < p.chunk_tokens ? p.T - lo : p.chunk_tokens);
     const bool col_in = col < p.D;
@@ -366,12 +411,48 @@ __global__ __launch_bounds__(256) void router_dw_partial_kernel(RouterBwdArgs p)
             raw[i] = *(const x4 *)(base + (int64_t)(t < n ? t : n - 1) * p.ldx);
         }
     };
-    x4 cur[8], ahead[8];
-    if (n > 0) load(0, cur);
-    for (int i = tid * 16; i < dense_bytes; i += 256 * 16) *(v4i *)(dw_smem + i) = v4i{0, 0, 0, 0};
-    form_picks(p, lo, n, gs, 256, [&](int i, float v, int expert) {  // (the zeros are in place behind its first barrier)
-        const int e = expert - e0, at = e * pitch + i / p.top_k;
-        if (e < 0 || e >= 64) return;
+    // The chunk's picks, one thread per pick and all of them requested at once, in front of x: loads return in order.
+    constexpr int PICKS = ROUTER_CHUNK * ROUTER_MAX_K / ROUTER_DW_THREADS;
+    const int total = n * p.top_k;
+    float pg[PICKS], ps[PICKS];
+    int pe[PICKS];
+#pragma unroll
+    for (int k = 0; k < PICKS; k++) {
+        const int i = tid + k * ROUTER_DW_THREADS;
+        if (k * ROUTER_DW_THREADS >= total) break;  // uniform
+        const int64_t at = lo * p.top_k + (i < total ? i : 0);
+        pg[k] = load_float(p.gw, p.gw_dtype, at) * p.factor, ps[k] = p.scores[at], pe[k] = (int)p.idx[at];
+    }
+    constexpr int AHEAD = 4;  // of the wave's steps
+    const int steps = (n + 31) / 32;
+    x4 buf[AHEAD][8];
+    static_for_steps<AHEAD>([&](auto s) {
+        if (2 * s.value + half < steps) load(2 * s.value + half, buf[s.value]);
+    });
+    for (int i = tid * 16; i < dense_bytes; i += ROUTER_DW_THREADS * 16) *(v4i *)(dw_smem + i) = v4i{0, 0, 0, 0};
+#pragma unroll
+    for (int k = 0; k < PICKS; k++) {
+        const int i = tid + k * ROUTER_DW_THREADS;
+        if (i < total) gs[i] = v2f{pg[k], ps[k]};
+    }
+    __syncthreads();  // the zeros are in place as well
+#pragma unroll
+    for (int k = 0; k < PICKS; k++) {
+        const int i = tid + k * ROUTER_DW_THREADS;
+        if (k * ROUTER_DW_THREADS >= total) break;
+        if (i >= total) continue;
+        float sum = 0.0f, dot = 0.0f;
+        if (p.norm) {
+            const int token0 = i / p.top_k * p.top_k;
+            for (int j = 0; j < p.top_k; j++) {
+                const v2f other = gs[token0 + j];
+                sum += other[1];
+                dot += other[0] * other[1];
+            }
+        }
+        const float v = pick_gradient(p, pg[k], ps[k], sum, dot);
+        const int e = pe[k] - e0, at = e * pitch + i / p.top_k;
+        if (e < 0 || e >= 64) continue;
         if constexpr (SPLIT) {
             uint16_t *d = (uint16_t *)dw_smem;
             const uint32_t hi = f2bf16(v);
@@ -383,15 +464,14 @@ __global__ __launch_bounds__(256) void router_dw_partial_kernel(RouterBwdArgs p)
         } else {
             ((float *)dw_smem)[at] = v;
         }
-    });
+    }
+    __syncthreads();
     v4f acc[4][4];
 #pragma unroll
     for (int m = 0; m < 4; m++)
 #pragma unroll
         for (int j = 0; j < 4; j++) acc[m][j] = v4f{0.f, 0.f, 0.f, 0.f};
-    const int steps = (n + 31) / 32;
-    for (int step = 0; step < steps; step++) {
-        if (step + 1 < steps) load(step + 1, ahead);
+    auto use = [&](int step, const x4 (&cur)[8]) {
         const int tok = 32 * step + 8 * g;
         if constexpr (SPLIT) {
             v4i b[4];
@@ -421,9 +501,24 @@ __global__ __launch_bounds__(256) void router_dw_partial_kernel(RouterBwdArgs p)
                         acc[m][j] = __builtin_amdgcn_mfma_f32_16x16x4f32(i < 4 ? a0[i & 3] : a1[i & 3], to_float(cur[i][j]), acc[m][j], 0, 0, 0);
             }
         }
+    };
+    for (int first = half; first < steps; first += 2 * AHEAD)
+        static_for_steps<AHEAD>([&](auto s) {
+            const int step = first + 2 * s.value;
+            if (step >= steps) return;
+            use(step, buf[s.value]);
+            if (step + 2 * AHEAD < steps) load(step + 2 * AHEAD, buf[s.value]);
+        });
+    __syncthreads();  // the gradients have been read: their place takes the odd steps' sums
+    v4f *const odd = (v4f *)dw_smem + (wave & 3) * 16 * 64 + lane;
+    if (half) {
 #pragma unroll
-        for (int i = 0; i < 8; i++) cur[i] = ahead[i];
+        for (int i = 0; i < 16; i++) odd[i * 64] = acc[i >> 2][i & 3];
     }
+    __syncthreads();
+    if (half) return;
+#pragma unroll
+    for (int i = 0; i < 16; i++) acc[i >> 2][i & 3] += odd[i * 64];
     if (!col_in) return;
 #pragma unroll
     for (int m = 0; m < 4; m++)
@@ -474,7 +569,7 @@ static int router_chunk_tokens(int64_t T, int64_t D, int64_t E, int cus) {
 
 template <int XDT, int WDT, int NT, int MT>
 static int launch_router(const RouterArgs &a, hipStream_t st) {
-    const int lds = ROUTER_WAVES * ROUTER_ROWS * (NT * 16 + 4) * 4 + NT * 16 * 4;
+    const int lds = ROUTER_WAVES * ROUTER_ROWS * MT * (NT * 16 + 4) * 4 + NT * 16 * 4;
     if (lds > 65536) {
         static std::atomic<uint64_t> done;
         if (!allow_dynamic_lds((const void *)router_topk_kernel<XDT, WDT, NT, MT>, lds, done)) return MX_ELAUNCH;
@@ -512,7 +607,7 @@ static int launch_router_dw(const RouterBwdArgs &a, hipStream_t st) {
     static_assert(router_dw_lds(ROUTER_CHUNK, ROUTER_MAX_K, true) <= 160 * 1024, "gradients and picks of a chunk fit the LDS");
     if (!allow_dynamic_lds((const void *)router_dw_partial_kernel<XDT>, most < 65536 ? 65536 : most, done)) return MX_ELAUNCH;
     const dim3 grid((unsigned)((a.D + ROUTER_DW_COLS - 1) / ROUTER_DW_COLS), (unsigned)((a.E + 63) / 64), (unsigned)a.chunks);
-    router_dw_partial_kernel<XDT><<<grid, dim3(256), router_dw_lds(a.chunk_tokens, a.top_k, XDT == MX_BF16), st>>>(a);
+    router_dw_partial_kernel<XDT><<<grid, dim3(ROUTER_DW_THREADS), router_dw_lds(a.chunk_tokens, a.top_k, XDT == MX_BF16), st>>>(a);
     return MX_OK;
 }
 
@@ -562,7 +657,8 @@ extern "C" int mx_router_topk_backward(const void *grad_weight, int gw_dtype, co
     a.chunks = T ? (int)((T + a.chunk_tokens - 1) / a.chunk_tokens) : 1;
     if (a.chunks > 65535) return MX_EUNSUPPORTED;
     if (dx && T) {
-        const dim3 grid((unsigned)((T + ROUTER_DX_TOKENS - 1) / ROUTER_DX_TOKENS)), block(256);
+        const int64_t most = 8 * (int64_t)num_cus(), blocks = (T + 3) / 4;  // 32 waves per CU
+        const dim3 grid((unsigned)(blocks < most ? blocks : most)), block(256);
         if (x_dtype == MX_BF16 && w_dtype == MX_BF16) router_dx_kernel<MX_BF16, MX_BF16><<<grid, block, 0, st>>>(a);
         else if (x_dtype == MX_BF16) router_dx_kernel<MX_BF16, MX_FP32><<<grid, block, 0, st>>>(a);
         else if (x_dtype == MX_FP16 && w_dtype == MX_FP16) router_dx_kernel<MX_FP16, MX_FP16><<<grid, block, 0, st>>>(a);

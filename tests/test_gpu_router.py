@@ -21,6 +21,7 @@ BF, HF, F32 = torch.bfloat16, torch.float16, torch.float32
     (130, 136, 256, 5, HF, F32, True, True),
     (5003, 1024, 64, 6, BF, BF, True, True),
     (12301, 136, 48, 4, HF, HF, True, True),
+    (33001, 16, 17, 16, BF, BF, True, False),  # five tokens for a wave of the dx kernel, whole chunks of 256 tokens and 16 picks
 ])
 def test_route_topk(tokens, dim, experts, top_k, xdt, wdt, norm, biased):
     from kohakuwullm_amd.kernels.moe.router import can_route, route_topk
