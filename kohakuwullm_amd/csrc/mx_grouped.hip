@@ -90,7 +90,8 @@ __device__ __forceinline__ void unpack8(const v4i &w, float (&v)[8]) {
             v[2 * i + 1] = bits2f((uint32_t)w[i] & 0xFFFF0000u);
         } else {
             typedef _Float16 h2 __attribute__((ext_vector_type(2)));
-            h2 h = __builtin_bit_cast(h2, w[i]);
+            const int word = w[i];  // an element handed to __builtin_bit_cast in place is read as element 0, whatever i is
+            const h2 h = __builtin_bit_cast(h2, word);
             v[2 * i] = (float)h[0];
             v[2 * i + 1] = (float)h[1];
         }

@@ -939,3 +939,47 @@ def test_token_axis_operands_stage_major_are_the_same_bytes(counts, hid):
         want = grouped_mxfp8_wgrad(*rows[a], *rows[b], offsets, m)
         for la, lb in ((panels, panels), (panels, rows), (rows, panels)):
             assert torch.equal(grouped_mxfp8_wgrad(*la[a], *lb[b], offsets, m), want), (a, b)
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("tokens,dim,top_k,gated", [(1, 8, 1, True), (37, 264, 6, False), (130, 1024, 9, True)])
+def test_combine_in_both_types(tokens, dim, top_k, gated, dtype):
+    """Pairs without a position, more slots than are fetched at once."""
+    from kohakuwullm_amd.kernels.mxfp8.moe import combine_sorted_rows
+
+    g = torch.Generator().manual_seed(SEED)
+    pairs = tokens * top_k
+    positions = torch.randperm(pairs, generator=g).int()
+    positions[torch.rand(pairs, generator=g) < 0.2] = -1
+    y = torch.randn(pairs, dim, generator=g).to(dtype)
+    gate = torch.rand(pairs, generator=g).to(dtype) if gated else None
+    offsets = torch.tensor([0, pairs], dtype=torch.int32, device=DEV)
+    rows = torch.where(positions[:, None] >= 0, y.double()[positions.clamp_min(0).long()], 0.0)
+    terms = (rows * (1.0 if gate is None else gate.double()[:, None])).view(tokens, top_k, dim)
+    out = combine_sorted_rows(y.to(DEV), None, offsets, 1, None if gate is None else gate.to(DEV), tokens, top_k,
+                              positions=positions.to(DEV)).cpu().double()
+    ref, size = terms.sum(1), terms.abs().sum(1)
+    # one rounding to 16 bits (half a unit), and an fp32 sum of top_k terms
+    half_ulp = 2.0**-8 if dtype == torch.bfloat16 else 2.0**-11
+    assert ((out - ref).abs() <= ref.abs() * half_ulp + size * 2.0**-24 * (top_k + 1) + 2.0**-25).all()
+
+
+def test_expert_block_in_fp16_agrees_with_the_one_in_bf16():
+    """Forward and every gradient: the combine and the SwiGLU' of the GEMM2-dgrad epilogue unpack 16-bit values of both types."""
+    from kohakuwullm_amd.models.moe import MoEMLP
+    from kohakuwullm_amd.models.mxfp8_swap import swap_mxfp8
+
+    x0 = torch.randn(300, 256, generator=torch.Generator().manual_seed(SEED)).to(DEV)
+    results = {}
+    for dtype in (torch.bfloat16, torch.float16):
+        torch.manual_seed(SEED)
+        block = MoEMLP(256, hidden=128, num_experts=4, top_k=2, num_shared=0).to(DEV).to(torch.bfloat16).to(dtype)
+        swap_mxfp8(block)
+        x = x0.bfloat16().to(dtype).requires_grad_(True)
+        y = block(x)
+        y.backward(torch.ones_like(y) * 2.0**-6)
+        results[dtype] = [y.detach(), x.grad, block.w_in.grad, block.w_out.grad]
+    for a, b in zip(*results.values()):
+        # the same codes of the same weights and inputs; rounding of the intermediates to 8 bits moves a share of the e4m3 codes by a
+        # step of 2^-3, some percent of the norm
+        assert (a.float() - b.float()).norm() <= 0.06 * a.float().norm(), (a.float() - b.float()).norm() / a.float().norm()
