@@ -410,6 +410,14 @@ int mx_experts_combine(const void *y, int64_t ldy, const int32_t *order, const i
                        void *out, int dtype, int64_t ldo, int64_t M, int64_t N, void *stream);
 
 /*
+ * The same on top of base (T,N), rows ldb elements apart, in the type of out: out[t] = base[t] + the sum, rounded once.
+ * base may be NULL.
+ */
+int mx_experts_combine_onto(const void *base, int64_t ldb, const void *y, int64_t ldy, const int32_t *order, const int32_t *offsets,
+                            int64_t E, const void *gate, int gate_dtype, int32_t *inv, int64_t T, int64_t top_k,
+                            void *out, int dtype, int64_t ldo, int64_t M, int64_t N, void *stream);
+
+/*
  * DGRAD through GEMM2, the combine and SwiGLU at once: acc = dq[token_of[m]] . w_out_dgrad[e]^T
  * (M,H); dgate[order[m]] += <acc, dequant(hq,hs)[m]> (fp32 atomics, caller-zeroed);
  * dh = acc * gate[order[m]]; SwiGLU backward from the stored pre; dpre (M,2H) stored in

@@ -802,13 +802,15 @@ __global__ __launch_bounds__(256) void invert_order_kernel(const int32_t *__rest
 template <int CDT>
 __global__ __launch_bounds__(256) void combine_kernel(const uint16_t *__restrict__ y, int64_t ldy,
                                                        const int32_t *__restrict__ inv, const void *__restrict__ gate,
-                                                       int gate_f32, int top_k, uint16_t *__restrict__ out, int64_t ldo,
-                                                       int64_t T, int N8) {
+                                                       int gate_f32, int top_k, const uint16_t *__restrict__ base, int64_t ldb,
+                                                       uint16_t *__restrict__ out, int64_t ldo, int64_t T, int N8) {
     const int64_t idx = (int64_t)blockIdx.x * 256 + threadIdx.x;
     const int64_t t = idx / N8;
     const int c = (int)(idx - t * N8) * 8;
     if (t >= T) return;
     float acc[8];
+    v4i onto = {0, 0, 0, 0};
+    if (base) onto = *(const v4i *)(base + t * ldb + c);
 #pragma unroll
     for (int e = 0; e < 8; e++) acc[e] = 0.0f;
     // Eight slots at a time: their positions and gate factors first, then all their rows, then the sums in slot order.
@@ -836,6 +838,12 @@ __global__ __launch_bounds__(256) void combine_kernel(const uint16_t *__restrict
 #pragma unroll
             for (int e = 0; e < 8; e++) acc[e] += scale[k] * v[e];
         }
+    }
+    if (base) {
+        float v[8];
+        unpack8<CDT>(onto, v);
+#pragma unroll
+        for (int e = 0; e < 8; e++) acc[e] += v[e];
     }
     uint32_t w[4];
 #pragma unroll
@@ -1487,13 +1495,20 @@ extern "C" int mx_experts_gemm2_dgrad(const uint8_t *dq, const uint8_t *ds, int6
 extern "C" int mx_experts_combine(const void *y, int64_t ldy, const int32_t *order, const int32_t *offsets, int64_t E,
                                   const void *gate, int gate_dtype, int32_t *inv, int64_t T, int64_t top_k, void *out,
                                   int dtype, int64_t ldo, int64_t M, int64_t N, void *stream) {
+    return mx_experts_combine_onto(nullptr, 0, y, ldy, order, offsets, E, gate, gate_dtype, inv, T, top_k, out, dtype, ldo, M, N, stream);
+}
+
+extern "C" int mx_experts_combine_onto(const void *base, int64_t ldb, const void *y, int64_t ldy, const int32_t *order,
+                                       const int32_t *offsets, int64_t E, const void *gate, int gate_dtype, int32_t *inv, int64_t T,
+                                       int64_t top_k, void *out, int dtype, int64_t ldo, int64_t M, int64_t N, void *stream) {
+    if (base && ldb < N) return MX_EINVAL;
     if (E <= 0 || E >= (1 << 20) || T < 0 || top_k <= 0 || top_k > 0x7FFF || M < 0 || N < 0 || M >= 0x7FFFFFFF ||
         T * top_k >= 0x7FFFFFFF || ldy < N || ldo < N || (order && !offsets) || !inv)
         return MX_EINVAL;
     if (dtype != MX_BF16 && dtype != MX_FP16) return MX_EINVAL;
     if (gate && gate_dtype != MX_FP32 && gate_dtype != dtype) return MX_EINVAL;
     if (T == 0 || N == 0) return MX_OK;
-    if (N % 8 || !aligned(y, 16) || !aligned(out, 16) || ldy % 8 || ldo % 8) return MX_EUNSUPPORTED;
+    if (N % 8 || !aligned(y, 16) || !aligned(out, 16) || ldy % 8 || ldo % 8 || (base && (!aligned(base, 16) || ldb % 8))) return MX_EUNSUPPORTED;
     hipStream_t st = (hipStream_t)stream;
     if (mx::stream_is_capturing(st)) return MX_ECAPTURE;
     const int64_t pairs = T * top_k;
@@ -1507,11 +1522,11 @@ extern "C" int mx_experts_combine(const void *y, int64_t ldy, const int32_t *ord
     if (dtype == MX_BF16)
         combine_kernel<MX_BF16><<<dim3((unsigned)blocks), dim3(256), 0, st>>>((const uint16_t *)y, ldy, inv, gate,
                                                                              gate_dtype == MX_FP32, (int)top_k,
-                                                                             (uint16_t *)out, ldo, T, n8);
+                                                                             (const uint16_t *)base, ldb, (uint16_t *)out, ldo, T, n8);
     else
         combine_kernel<MX_FP16><<<dim3((unsigned)blocks), dim3(256), 0, st>>>((const uint16_t *)y, ldy, inv, gate,
                                                                              gate_dtype == MX_FP32, (int)top_k,
-                                                                             (uint16_t *)out, ldo, T, n8);
+                                                                             (const uint16_t *)base, ldb, (uint16_t *)out, ldo, T, n8);
     return hipGetLastError() == hipSuccess ? MX_OK : MX_ELAUNCH;
 }
 

@@ -43,7 +43,7 @@ namespace {
     F(mx_swiglu_quantize_tokens) F(mx_swiglu_bwd_quantize_tokens) F(mx_gemm_nt) F(mx_gemm_nt_batch) F(mx_activation_gemm_nt) F(mx_rmsnorm_quantize) \
     F(mx_rmsnorm_backward) F(mx_rmsnorm_weight_grad) F(mx_router_topk) F(mx_router_backward_workspace)                      \
     F(mx_router_topk_backward) F(mx_expert_sort_workspace) F(mx_expert_sort_positions) F(mx_experts_gemm1)                  \
-    F(mx_grouped_gemm_nt) F(mx_experts_combine) F(mx_experts_gemm2_dgrad) F(mx_quantize_cols_grouped) F(mx_grouped_wgrad_nt)
+    F(mx_grouped_gemm_nt) F(mx_experts_combine_onto) F(mx_experts_gemm2_dgrad) F(mx_quantize_cols_grouped) F(mx_grouped_wgrad_nt)
 
 struct Library {
 #define F(name) decltype(&::name) name = nullptr;
@@ -817,14 +817,15 @@ struct Routing {
     const int32_t *p(const Tensor &t) const { return (const int32_t *)t.const_data_ptr(); }
 };
 
-// y = a . w^T row by row, then out[t] = sum over t's pairs of gate * y.
-Tensor routed_product(const Quantized &a, const Stack &w, const Routing &r, const Tensor &gate, int64_t tokens, ScalarType type, bool made, Tensor &positions) {
+// y = a . w^T row by row, then out[t] = base[t], where given, + sum over t's pairs of gate * y.
+Tensor routed_product(const Quantized &a, const Stack &w, const Routing &r, const Tensor &gate, int64_t tokens, ScalarType type, bool made, Tensor &positions,
+                      const Tensor &base = Tensor()) {
     const Tensor y = empty({r.m, w.n}, type, a.q), out = empty({tokens, w.n}, type, a.q);
     const int code = code_of(type);
     MX_RUN(mx_grouped_gemm_nt, bytes(a.q), bytes(a.s), r.m, a.q.stride(0), a.s.stride(0), nullptr, MX_STACK(w), r.p(r.offsets), w.e, y.data_ptr(), code,
            w.n, r.m, w.n, w.k, stream_of(a.q));
     if (!made) positions = empty({tokens * r.top_k}, I32, a.q);
-    MX_RUN(mx_experts_combine, y.const_data_ptr(), w.n, made ? nullptr : r.p(r.order), r.p(r.offsets), w.e,
+    MX_RUN(mx_experts_combine_onto, base.defined() ? base.const_data_ptr() : nullptr, base.defined() ? base.stride(0) : 0, y.const_data_ptr(), w.n, made ? nullptr : r.p(r.order), r.p(r.offsets), w.e,
            gate.defined() ? gate.const_data_ptr() : nullptr, gate.defined() ? code_of(gate.scalar_type()) : 0, (int32_t *)positions.data_ptr(), tokens,
            r.top_k, out.data_ptr(), code, w.n, r.m, w.n, stream_of(a.q));
     return out;
@@ -848,7 +849,11 @@ PyObject *py_experts_forward(Args &a) {
     const Stack w_in = stack(a.quantized()), w_out = stack(a.quantized());
     const int64_t hidden = a.integer();
     const bool needs_grad = a.flag(), token_axis = a.flag();
+    const Tensor base = a.tensor();
     MX_NEED(plain(x) && x.dim() == 2 && x.stride(1) == 1 && half_type(x.scalar_type()) && hidden % BLOCK == 0 && w_out.n % 8 == 0);
+    if (base.defined())
+        MX_NEED(plain(base) && base.sizes() == x.sizes() && base.scalar_type() == x.scalar_type() && base.stride(1) == 1 && base.stride(0) >= base.size(1) &&
+                base.stride(0) % 8 == 0 && aligned(base, 16));
     const int64_t dim = x.size(1);
     MX_NEED(w_in.k == dim && w_in.n == 2 * hidden && w_out.n == dim && w_out.k == hidden && w_out.e == w_in.e && dim % BLOCK == 0);
     Routing r = routing(x, gate, token_of, order, offsets, positions, w_in.e);
@@ -862,7 +867,7 @@ PyObject *py_experts_forward(Args &a) {
            (uint8_t *)h.q.data_ptr(), hidden, (uint8_t *)h.s.data_ptr(), hidden / BLOCK, needs_grad ? pre.data_ptr() : nullptr, needs_grad ? 2 * hidden : 0,
            codes_out(ht), token_axis ? PANEL : 0, scales_out(ht), token_axis ? ht.s.stride(0) : 0, code_of(type), r.m, hidden, dim, stream_of(x));
     Tensor inverse = positions;
-    const Tensor out = routed_product(h, w_out, r, gate, x.size(0), type, positions.defined(), inverse);
+    const Tensor out = routed_product(h, w_out, r, gate, x.size(0), type, positions.defined(), inverse, base);
     return wrap_all({out, h.q, h.s, pre, ht.q, ht.s, inverse});
 }
 

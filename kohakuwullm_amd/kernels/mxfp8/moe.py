@@ -25,7 +25,7 @@ from kohakuwullm_amd.kernels.mxfp8.grouped import (
     token_axis_pitch,
     quantize_mx_cols_grouped,
 )
-from kohakuwullm_amd.kernels.mxfp8.quantize import BLOCK_SCALE, quantize_mx, quantize_mx_cols
+from kohakuwullm_amd.kernels.mxfp8.quantize import BLOCK_SCALE, aligned_rows, quantize_mx, quantize_mx_cols
 
 _FP8 = torch.float8_e4m3fn
 _ACT_DTYPES = (torch.bfloat16, torch.float16)
@@ -137,13 +137,13 @@ def launch_scatter_gemm(aq, a_s, wq, ws, out, token_of, order, gate, offsets, in
 
 
 def combine_sorted_rows(y, order, offsets, num_experts, gate, tokens: int, top_k: int, positions=None,
-                        return_positions: bool = False):
+                        return_positions: bool = False, base=None):
     """``out[t] = sum_k gate[t*top_k+k] * y[position of pair t*top_k+k]``: the scatter-add as a gather.
 
     ``order`` must be the pair index ``token * top_k + slot`` (what ``expert_sort`` produces).
     Deterministic; every row of the result is written.  ``positions``: the pair -> sorted position
     table an earlier call for the same routing returned (``return_positions=True``); with it the
-    call skips rebuilding the table from ``order``.
+    call skips rebuilding the table from ``order``.  ``base``: ``(tokens, N)`` in ``y``'s type, added before the one rounding.
     """
     m, n = y.shape
     out = torch.empty(tokens, n, device=y.device, dtype=y.dtype)
@@ -151,10 +151,12 @@ def combine_sorted_rows(y, order, offsets, num_experts, gate, tokens: int, top_k
     if reuse and (positions.numel() != tokens * top_k or positions.dtype != torch.int32 or positions.device != y.device
                   or not positions.is_contiguous()):
         raise ValueError(f"positions {tuple(positions.shape)} {positions.dtype} does not fit {tokens} tokens x top_k {top_k}")
+    base = None if base is None else aligned_rows(base)
     inv = positions if reuse else torch.empty(tokens * top_k, device=y.device, dtype=torch.int32)
+    onto = () if base is None else (base.data_ptr(), base.stride(0))
     _lib.invoke(
-        "mx_experts_combine", y.element_size() * n * (tokens * top_k + tokens), y,
-        y.data_ptr(), y.stride(0), 0 if reuse else order.data_ptr(), offsets.data_ptr(), num_experts,
+        "mx_experts_combine_onto" if onto else "mx_experts_combine", y.element_size() * n * (tokens * top_k + tokens), y,
+        *onto, y.data_ptr(), y.stride(0), 0 if reuse else order.data_ptr(), offsets.data_ptr(), num_experts,
         0 if gate is None else gate.data_ptr(), 0 if gate is None else _lib.MX_DTYPE[gate.dtype], inv.data_ptr(),
         tokens, top_k, out.data_ptr(), _lib.MX_DTYPE[out.dtype], out.stride(0), m, n,
     )
@@ -162,8 +164,8 @@ def combine_sorted_rows(y, order, offsets, num_experts, gate, tokens: int, top_k
 
 
 def _routed_product(aq, a_s, wq, ws, token_of, order, gate, offsets, tokens: int, top_k: int, dtype, positions=None,
-                    return_positions: bool = False):
-    """``out[token] += scale * (a[m] . w[e(m)]^T)`` over the sorted rows.
+                    return_positions: bool = False, base=None):
+    """``out[token] += scale * (a[m] . w[e(m)]^T)`` over the sorted rows, on top of ``base`` where given.
 
     When ``order`` is a pair index (``top_k`` > 0) the rows are written once by the grouped GEMM
     and gathered per token; otherwise the scatter GEMM adds them into a zeroed output with
@@ -172,8 +174,8 @@ def _routed_product(aq, a_s, wq, ws, token_of, order, gate, offsets, tokens: int
     n = wq.shape[1]
     if top_k > 0 and n % 8 == 0:
         y = grouped_mxfp8_gemm(aq, a_s, wq, ws, offsets, out_dtype=dtype, rows=token_of.numel())
-        return combine_sorted_rows(y, order, offsets, wq.shape[0], gate, tokens, top_k, positions, return_positions)
-    out = torch.zeros(tokens, n, device=aq.device, dtype=dtype)
+        return combine_sorted_rows(y, order, offsets, wq.shape[0], gate, tokens, top_k, positions, return_positions, base)
+    out = torch.zeros(tokens, n, device=aq.device, dtype=dtype) if base is None else base.clone(memory_format=torch.contiguous_format)
     launch_scatter_gemm(aq, a_s, wq, ws, out, token_of, order if gate is not None else None, gate, offsets)
     return (out, None) if return_positions else out
 
@@ -202,15 +204,15 @@ def launch_gemm2_dgrad(dq, ds, token_of, order, gate, wq, ws, hq, hs, pre, dpre,
 
 class _MXFP8Experts(torch.autograd.Function):
     @staticmethod
-    def forward(ctx, x, w_in, w_out, gate, token_of, order, offsets, packed, hidden, positions, differentiable):
+    def forward(ctx, x, w_in, w_out, gate, token_of, order, offsets, packed, hidden, positions, differentiable, base):
         del w_in, w_out  # present so autograd routes dW to the master parameters
         rows, dim = x.shape
         m = token_of.numel()
         # the grad mode comes from the caller: in here it is always off, and `needs_input_grad` does not know it
-        needs_grad = differentiable and any(ctx.needs_input_grad)
+        needs_grad = ctx.routed = differentiable and any(ctx.needs_input_grad[:4])
         if TOKEN_AXIS_STAGE_MAJOR:
             made = host.experts_forward(x, gate, token_of, order, offsets, positions, packed.in_fwd, packed.out_fwd, hidden, needs_grad,
-                                        differentiable and ctx.needs_input_grad[2])
+                                        differentiable and ctx.needs_input_grad[2], base)
             if made is not None:
                 out, hq, hs, pre, htq, hts, positions = made
                 if needs_grad:
@@ -233,7 +235,7 @@ class _MXFP8Experts(torch.autograd.Function):
         top_k = gate.numel() // rows if rows and gate.numel() % rows == 0 else 0
         # the pair -> sorted position table of the combine serves the backward's combine too
         out, positions = _routed_product(hq, hs, *packed.out_fwd, token_of, order, gate, offsets, rows, top_k, x.dtype,
-                                         positions, return_positions=True)
+                                         positions, return_positions=True, base=base)
         if needs_grad:
             ctx.positions = positions
             ctx.save_for_backward(x, hq, hs, pre, gate, token_of, order, offsets, htq, hts)
@@ -243,6 +245,9 @@ class _MXFP8Experts(torch.autograd.Function):
 
     @staticmethod
     def backward(ctx, dout):
+        dbase = dout if ctx.needs_input_grad[11] else None
+        if not ctx.routed:
+            return (None,) * 11 + (dbase,)
         x, hq, hs, pre, gate, token_of, order, offsets, htq, hts = ctx.saved_tensors
         packed = ctx.packed
         hidden, dim, m, rows, top_k = ctx.shapes
@@ -250,7 +255,7 @@ class _MXFP8Experts(torch.autograd.Function):
             made = host.experts_backward(dout, x, hq, hs, pre, gate, token_of, order, offsets, ctx.positions, htq, hts, packed.in_dgrad,
                                          packed.out_dgrad, hidden, *ctx.needs_input_grad[1:3])
             if made is not None:
-                return *made, None, None, None, None, None, None, None
+                return *made, None, None, None, None, None, None, None, dbase
         dev = dout.device
         dout = dout.contiguous()
         dq, ds = quantize_mx(dout)
@@ -279,7 +284,7 @@ class _MXFP8Experts(torch.autograd.Function):
             # dW_in[e] = dpre rows of e .T @ x rows of e
             xtq, xts = quantize_mx_cols_grouped(x, offsets, m, index=token_of, stage_major=TOKEN_AXIS_STAGE_MAJOR)
             dw_in = grouped_mxfp8_wgrad(ptq, pts, xtq, xts, offsets, m, dout.dtype)
-        return dx, dw_in, dw_out, dgate.to(gate.dtype), None, None, None, None, None, None, None
+        return dx, dw_in, dw_out, dgate.to(gate.dtype), None, None, None, None, None, None, None, dbase
 
 
 def _validate_expert_call(x, w_in, w_out, token_of, order) -> int:
@@ -310,7 +315,7 @@ def _validate_expert_call(x, w_in, w_out, token_of, order) -> int:
 
 
 def mxfp8_moe_experts(x, w_in, w_out, gate, token_of, order, offsets, packed: MXFP8ExpertWeights,
-                      positions: torch.Tensor | None = None) -> torch.Tensor:
+                      positions: torch.Tensor | None = None, base: torch.Tensor | None = None) -> torch.Tensor:
     """The whole routed-expert path in MXFP8: gather, SwiGLU MLP, gate, combine.
 
     Args:
@@ -325,13 +330,17 @@ def mxfp8_moe_experts(x, w_in, w_out, gate, token_of, order, offsets, packed: MX
         packed: the four quantized copies, refreshed after each optimizer step.
         positions: ``(T*top_k,)`` int32, the inverse of ``order`` (pair index -> sorted position, -1 for none below
             ``offsets[E]``); made from ``order`` when not given.
+        base: ``(T, dim)`` in ``x``'s type: what the tokens' sums are added to, before they are rounded.
     """
+    if base is not None and (base.shape != x.shape or base.dtype != x.dtype or base.device != x.device):
+        raise ValueError(f"base {tuple(base.shape)} {base.dtype} on {base.device} does not match x {tuple(x.shape)} {x.dtype}")
     hidden = _validate_expert_call(x, w_in, w_out, token_of, order)
-    if TOKEN_AXIS_STAGE_MAJOR and host.unrecorded(x, gate, w_in, w_out):
-        made = host.experts_forward(x, gate, token_of, order, offsets, positions, packed.in_fwd, packed.out_fwd, hidden, False, False)
+    if TOKEN_AXIS_STAGE_MAJOR and host.unrecorded(x, gate, w_in, w_out, base):
+        made = host.experts_forward(x, gate, token_of, order, offsets, positions, packed.in_fwd, packed.out_fwd, hidden, False, False, base)
         if made is not None:
             return made[0]
-    return _MXFP8Experts.apply(x, w_in, w_out, gate, token_of, order, offsets, packed, hidden, positions, torch.is_grad_enabled())
+    return _MXFP8Experts.apply(x, w_in, w_out, gate, token_of, order, offsets, packed, hidden, positions, torch.is_grad_enabled(),
+                                base)
 
 
 def mxfp8_moe_experts_reference(x, w_in, w_out, gate, token_of, order, offsets) -> torch.Tensor:

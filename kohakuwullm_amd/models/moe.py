@@ -25,7 +25,7 @@ import torch.nn as nn
 import torch.nn.functional as F
 
 from kohakuwullm_amd.kernels.moe.moe_dispatch import combine_routed, expert_counts, expert_sort, expert_sort_positions  # noqa: F401  (expert_sort: importable from here)
-from kohakuwullm_amd.kernels.moe.router import can_route, route_fitting, route_topk  # noqa: F401  (route_topk: importable from here)
+from kohakuwullm_amd.kernels.moe.router import can_route, plain_call, route_fitting, route_topk  # noqa: F401  (route_topk: importable from here)
 from kohakuwullm_amd.kernels.mxfp8.linear import compute_dtype
 from kohakuwullm_amd.kernels.mxfp8.moe import (
     MXFP8ExpertWeights,
@@ -271,12 +271,12 @@ class MoEMLP(nn.Module):
         scaled = out_sorted[:real] * weight.index_select(0, order[:real].long()).unsqueeze(-1)
         return x.new_zeros(flat.shape[0], self.dim).index_add_(0, token_of[:real].long(), scaled)
 
-    def _routed_mxfp8(self, flat, topk_weight, order, token_of, offsets, positions=None):
+    def _routed_mxfp8(self, flat, topk_weight, order, token_of, offsets, positions=None, base=None):
         if self._packed is None:
             self._refresh_mxfp8()
         x = flat.to(compute_dtype(flat))  # compute dtype follows autocast; the activation may arrive fp32
         return mxfp8_moe_experts(x, self.w_in, self.w_out, topk_weight.reshape(-1), token_of, order,
-                                 offsets[: self.num_experts + 1], self._packed, positions)
+                                 offsets[: self.num_experts + 1], self._packed, positions, base)
 
     def _routed_mxfp8_unfused(self, flat, topk_weight, order, token_of, offsets):
         if self._packed is None:
@@ -296,6 +296,12 @@ class MoEMLP(nn.Module):
         inverse = self._routed == self._routed_mxfp8 and not self._has_sentinel
         offsets, order, token_of, _, *positions = expert_sort_positions(topk_idx.reshape(-1), counts, topk_idx.shape[-1],
                                                                         self.num_buckets, inverse)
+        if inverse and self.shared is not None and type(self)._routed_mxfp8 is MoEMLP._routed_mxfp8:
+            # the combine adds the routed rows to the shared expert's output: a pass over both less, and a rounding
+            shared = self.shared(flat)
+            if plain_call(flat, shared) and shared.shape == flat.shape and shared.dtype == compute_dtype(flat) and shared.device == flat.device:
+                return self._routed(flat, topk_weight, order, token_of, offsets, *positions, shared).reshape(shape)
+            return (self._routed(flat, topk_weight, order, token_of, offsets, *positions) + shared).reshape(shape)
         out = self._routed(flat, topk_weight, order, token_of, offsets, *positions if inverse else ())
         if self.shared is not None:
             out = out + self.shared(flat)  # dtype by promotion, as the reference's forward (components/moe.py:395-449)

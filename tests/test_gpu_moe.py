@@ -943,8 +943,9 @@ def test_token_axis_operands_stage_major_are_the_same_bytes(counts, hid):
 
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
 @pytest.mark.parametrize("tokens,dim,top_k,gated", [(1, 8, 1, True), (37, 264, 6, False), (130, 1024, 9, True)])
-def test_combine_in_both_types(tokens, dim, top_k, gated, dtype):
-    """Pairs without a position, more slots than are fetched at once."""
+@pytest.mark.parametrize("margin", [None, 8, 1])  # none, and a base whose rows lie apart or have to be laid out anew
+def test_combine_in_both_types(tokens, dim, top_k, gated, margin, dtype):
+    """Pairs without a position, more slots than are fetched at once, on top of another matrix."""
     from kohakuwullm_amd.kernels.mxfp8.moe import combine_sorted_rows
 
     g = torch.Generator().manual_seed(SEED)
@@ -956,12 +957,16 @@ def test_combine_in_both_types(tokens, dim, top_k, gated, dtype):
     offsets = torch.tensor([0, pairs], dtype=torch.int32, device=DEV)
     rows = torch.where(positions[:, None] >= 0, y.double()[positions.clamp_min(0).long()], 0.0)
     terms = (rows * (1.0 if gate is None else gate.double()[:, None])).view(tokens, top_k, dim)
+    base = None
+    if margin is not None:
+        base = torch.randn(tokens, dim + 2 * margin, generator=g).to(dtype).to(DEV)[:, margin : margin + dim]
+        terms = torch.cat([base.cpu().double()[:, None], terms], dim=1)
     out = combine_sorted_rows(y.to(DEV), None, offsets, 1, None if gate is None else gate.to(DEV), tokens, top_k,
-                              positions=positions.to(DEV)).cpu().double()
+                              positions=positions.to(DEV), base=base).cpu().double()
     ref, size = terms.sum(1), terms.abs().sum(1)
-    # one rounding to 16 bits (half a unit), and an fp32 sum of top_k terms
+    # one rounding to 16 bits (half a unit), and an fp32 sum of top_k or top_k + 1 terms
     half_ulp = 2.0**-8 if dtype == torch.bfloat16 else 2.0**-11
-    assert ((out - ref).abs() <= ref.abs() * half_ulp + size * 2.0**-24 * (top_k + 1) + 2.0**-25).all()
+    assert ((out - ref).abs() <= ref.abs() * half_ulp + size * 2.0**-24 * (top_k + 2) + 2.0**-25).all()
 
 
 def test_expert_block_in_fp16_agrees_with_the_one_in_bf16():
@@ -983,3 +988,33 @@ def test_expert_block_in_fp16_agrees_with_the_one_in_bf16():
         # the same codes of the same weights and inputs; rounding of the intermediates to 8 bits moves a share of the e4m3 codes by a
         # step of 2^-3, some percent of the norm
         assert (a.float() - b.float()).norm() <= 0.06 * a.float().norm(), (a.float() - b.float()).norm() / a.float().norm()
+
+
+def test_shared_expert_gets_the_gradient_of_the_sum():
+    """The combine onto the shared expert's output: what it computes is the sum, and each side's gradients are the ones of its own."""
+    from kohakuwullm_amd.models.moe import MoEMLP
+    from kohakuwullm_amd.models.mxfp8_swap import swap_mxfp8
+
+    torch.manual_seed(SEED)
+    block = MoEMLP(256, hidden=128, num_experts=8, top_k=2, num_shared=1).to(DEV).to(torch.bfloat16)
+    swap_mxfp8(block)
+    x = torch.randn(70, 256, device=DEV, dtype=torch.bfloat16, requires_grad=True)
+    up = torch.randn(70, 256, device=DEV, dtype=torch.bfloat16) * 1e-2
+    block(x).backward(up)
+    got = [x.grad, *(p.grad.clone() for p in block.parameters())]
+    out = block(x.detach())
+    shared = block.shared
+    block.shared, x2 = None, x.detach().requires_grad_(True)
+    block.zero_grad(), shared.zero_grad()
+    routed, extra = block(x2), shared(x2)
+    assert ((out - (routed + extra)).float().abs() <= 2.0**-7 * (routed.abs() + extra.abs()).float() + 1e-6).all()
+    torch.autograd.backward([routed, extra], [up, up])
+    block.shared = shared
+    for a, b in zip(got, [x2.grad, *(p.grad for p in block.parameters())]):
+        assert (a.float() - b.float()).norm() <= 8e-3 * b.float().norm()  # the gate's gradient is added in any order
+    # nothing but the shared expert is trained: the routed side has no backward to run
+    for name, p in block.named_parameters():
+        p.requires_grad_(name.startswith("shared."))
+        p.grad = None
+    block(x.detach()).backward(up)
+    assert all((p.grad is not None) == name.startswith("shared.") for name, p in block.named_parameters())
