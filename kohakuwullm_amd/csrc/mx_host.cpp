@@ -76,7 +76,14 @@ void check(int status, const char *what) {
     if (done) PyErr_SetString(PyExc_RuntimeError, what);
     throw python_error();
 }
-#define MX_RUN(name, ...) check(lib.name(__VA_ARGS__), #name)
+// Other Python threads run while a launch waits for a place in its queue or an allocation for memory, as they do under ctypes and
+// in PyTorch's own operators.  Nothing in the guarded scope touches a Python object.
+struct Unlocked {
+    PyThreadState *state = PyEval_SaveThread();
+    ~Unlocked() noexcept(false) { PyEval_RestoreThread(state); }  // ends a daemon thread by unwinding it at interpreter exit
+};
+#define MX_CALL(name, ...) ([&] { Unlocked open; return lib.name(__VA_ARGS__); }())
+#define MX_RUN(name, ...) check(MX_CALL(name, __VA_ARGS__), #name)
 
 // ---- tensors ---------------------------------------------------------------------------------------------------------------
 
@@ -105,6 +112,7 @@ bool aligned(const Tensor &t, uintptr_t a) { return (uintptr_t)t.const_data_ptr(
 void *stream_of(const Tensor &t) { return (void *)c10::hip::getCurrentHIPStream(t.device().index()).stream(); }
 
 Tensor empty(at::IntArrayRef size, ScalarType type, const Tensor &like) {
+    Unlocked open;
     return Tensor(at::detail::empty_cuda(size, type, like.device(), std::nullopt));
 }
 
@@ -364,7 +372,7 @@ bool activation_products(const Tensor &x, const Tensor &x2d, ScalarType compute,
         outs.push_back(empty(with_last(x, q.size(0)), compute, x2d));
         d[j] = {nullptr, nullptr, bytes(q), bytes(s), outs.back().data_ptr(), x2d.size(0), q.size(0), q.size(1), 0, 0, q.stride(0), s.stride(0), q.size(0)};
     }
-    const int status = lib.mx_activation_gemm_nt(x2d.const_data_ptr(), code_of(x2d.scalar_type()), x2d.stride(0), d, (int)ws.size(), code_of(compute), stream_of(x2d));
+    const int status = MX_CALL(mx_activation_gemm_nt, x2d.const_data_ptr(), code_of(x2d.scalar_type()), x2d.stride(0), d, (int)ws.size(), code_of(compute), stream_of(x2d));
     if (status == MX_EUNSUPPORTED) {
         outs.clear();
         return false;
@@ -535,7 +543,7 @@ PyObject *py_quantize_dual_batch(Args &a) {
         PyList_SET_ITEM(out, (Py_ssize_t)j, wrap_all({q, s, qt, st}));
         at += n;
     }
-    const int status = lib.mx_quantize_dual_batch(problems.data(), (int)problems.size(), code, stream_of(xs[0]));
+    const int status = MX_CALL(mx_quantize_dual_batch, problems.data(), (int)problems.size(), code, stream_of(xs[0]));
     if (status != MX_OK) Py_DECREF(out);
     check(status, "mx_quantize_dual_batch");
     return out;

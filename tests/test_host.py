@@ -211,3 +211,42 @@ def test_refresh_and_pitched_products():
     _both(lambda: [t for four in quantize_mx_dual_batch(ws) for t in four])
     q, s = quantize_mx(ws[1])
     _both(lambda: [mxfp8_matmul_pq(q, s, q, s, F32, out_pad=24)])
+
+
+@pytest.mark.gpu
+def test_threads_on_their_own_streams():
+    """A launch and an allocation let other Python threads run: passes that overlap in time give what each gives alone."""
+    import threading
+
+    from kohakuwullm_amd.kernels.mxfp8.linear import MXFP8Linear
+
+    torch.manual_seed(SEED)
+    layers = [MXFP8Linear(512, 384 + 128 * i).to(DEV).to(BF) for i in range(4)]
+    inputs = [torch.randn(300 + i, 512, device=DEV).to(BF) for i in range(4)]
+
+    def run(lin, x0):
+        x = x0.clone().requires_grad_()
+        y = lin(x)
+        dx, dw = torch.autograd.grad(y, [x, lin.weight], torch.full_like(y, 1e-2))
+        return [y.detach(), dx, dw]
+
+    want = [run(lin, x) for lin, x in zip(layers, inputs)]
+    torch.cuda.synchronize()
+    got = [[] for _ in layers]
+
+    def work(i):
+        stream = torch.cuda.Stream()
+        with torch.cuda.stream(stream):
+            for _ in range(20):
+                got[i].append(run(layers[i], inputs[i]))
+        stream.synchronize()
+
+    threads = [threading.Thread(target=work, args=(i,)) for i in range(4)]
+    for t in threads:
+        t.start()
+    for t in threads:
+        t.join()
+    for i, passes in enumerate(got):
+        assert len(passes) == 20
+        for one in passes:
+            assert all(torch.equal(_bits(a), _bits(b)) for a, b in zip(one, want[i]))
