@@ -933,7 +933,7 @@ struct WgradArgs {
     // K split for few, long tiles (a handful of busy experts): `slots` fp32 tile slots; every
     // workgroup derives the same number of K slices per tile from the offsets (wgrad_slices),
     // slice s of the j-th tile of a non-empty expert leaves its partial sum in slot j * slices + s,
-    // and wgrad_reduce_kernel adds the slices in order.  slots == 0: whole tiles only.
+    // and wgrad_finish_kernel adds the slices in order.  slots == 0: whole tiles only.
     float *ws;
     int slots;
 };
@@ -943,7 +943,7 @@ struct WgradArgs {
 // tiles_per_expert workgroups, one per output tile, takes each range.  A range that covers an
 // expert's stages only in part leaves fp32 partial sums: at most two per workgroup (the end of
 // an expert an earlier group began, the beginning of one a later group ends), in slots 2 u and
-// 2 u + 1 of workgroup-unit u, and wgrad_reduce_kernel adds an expert's pieces in group order.
+// 2 u + 1 of workgroup-unit u, and wgrad_finish_kernel adds an expert's pieces in group order.
 // Every workgroup works one range of equal length, where whole K slices left a ragged second
 // round and one fp32 partial tile per slice (measured at six busy experts of 16384 rows:
 // 480 partial tiles and two rounds against 336 and one).
@@ -1002,7 +1002,7 @@ struct WgradProblem {
     const WgradArgs p;
     // Units are dealt round-robin over the workgroups: the (tile, K slice) units of the non-empty
     // experts, compactly numbered so they spread evenly wherever those experts sit among the E.
-    // (The dW of an expert without rows is zero-filled by wgrad_zero_kernel, launched first.)
+    // (The dW of an expert without rows is zero-filled by wgrad_finish_kernel, launched behind.)
     int next_unit, kb_end;
     int live, slices;
     // incremental scan: expert scan_e is the scan_live-th non-empty one and its first K stage
@@ -1164,27 +1164,21 @@ struct WgradProblem {
     }
 };
 
-// dW of the experts without rows: zeros.  A plain streaming fill, launched ahead of the GEMM.  (As
-// part of it, in one burst, the fills of 58 empty experts cost three times what they cost here: vector
-// memory operations retire in order, so the first stage's wait for its copies waits for every store
-// issued before them.  Spread over the K stages, a few stores per thread in front of each stage's
-// copies, they cost the GEMM exactly the 14 us the separate launch takes.)  One block per (expert, 64 rows).
-template <int CDT>
-__global__ __launch_bounds__(256) void wgrad_zero_kernel(WgradArgs p, int chunks) {
-    const int e = blockIdx.x / chunks, m0 = (blockIdx.x % chunks) * 64;
-    if (p.offsets[e + 1] > p.offsets[e]) return;
+// 64 rows, from row m0 on, of the dW of expert e, which has no rows: zeros, a plain streaming fill.
+template <int CDT, int THREADS>
+__device__ __forceinline__ void wgrad_zero_rows(const WgradArgs &p, int e, int m0) {
     const int esz = CDT == MX_FP32 ? 4 : 2;
     char *base = (char *)p.dw + ((int64_t)e * p.stride_dwe + (int64_t)m0 * p.lddw) * esz;
     const int rows = p.N - m0 < 64 ? p.N - m0 : 64;
     if (p.c_vec && (p.Kout * esz) % 16 == 0) {
         const int per_row = p.Kout * esz / 16;
-        for (int idx = threadIdx.x; idx < rows * per_row; idx += 256) {
+        for (int idx = threadIdx.x; idx < rows * per_row; idx += THREADS) {
             const int m = idx / per_row, c = idx - m * per_row;
             *(v4i *)(base + (int64_t)m * p.lddw * esz + c * 16) = v4i{0, 0, 0, 0};
         }
         return;
     }
-    for (int idx = threadIdx.x; idx < rows * p.Kout; idx += 256) {
+    for (int idx = threadIdx.x; idx < rows * p.Kout; idx += THREADS) {
         const int m = idx / p.Kout, n = idx - m * p.Kout;
         char *dst = base + ((int64_t)m * p.lddw + n) * esz;
         if (esz == 4) *(float *)dst = 0.0f;
@@ -1205,17 +1199,29 @@ __global__ __launch_bounds__(S::NTHR) void grouped_wgrad_kernel(WgradArgs args) 
     persistent_gemm<S, SCALES, WgradProblem<S, CDT, TB>, SCALES == SCALES_COPY>(prob, smem);
 }
 
-// Adds the K slices of every tile of every non-empty expert, in slice order, and stores dW.
-// One unit per (tile of a non-empty expert, i), numbered compactly as in the GEMM; the host does
-// not know how many experts have rows, so a fixed number of workgroups stride over the units
-// (none when the GEMM kept its tiles whole).
+// What is left behind the GEMM, for a fixed number of workgroups: the host does not know how many experts have rows, nor
+// whether the GEMM cut its tiles, and usually there is nothing to do.
+// First the dW of the experts without rows, in units of 64 rows.  (Inside the GEMM, in one burst, the fills of 58 empty experts cost
+// three times what they cost here: vector memory operations retire in order, so the first stage's wait for its copies waits for
+// every store issued before them.  Spread over the K stages, a few stores per thread in front of each stage's copies, they cost
+// the GEMM exactly the 14 us they take by themselves.  As a launch of their own, in front of the GEMM, they cost 2 us more per call
+// where there are none to do: a mixture of experts trained on 2777 tokens, two calls a pass, 499.3 / 495.8 us.)
+// Then the K slices of every tile of every non-empty expert, added in slice order: one unit per (tile of a non-empty expert,
+// i), numbered compactly as in the GEMM; none when it kept its tiles whole.
 template <typename S, int CDT>
-__global__ __launch_bounds__(S::NTHR) void wgrad_reduce_kernel(WgradArgs p, int workgroups) {
+__global__ __launch_bounds__(S::NTHR) void wgrad_finish_kernel(WgradArgs p, int workgroups) {
     __shared__ ExpertTable table;
     const bool tabled = p.E <= MX_TABLE_MAX;
     if (tabled) build_live_table(table, p.offsets, p.E);
     int live;
     const int slices = wgrad_slices(p, workgroups, live, tabled ? &table : nullptr);
+    if (live < p.E) {
+        const uint32_t chunks = (uint32_t)(p.N + 63) / 64;
+        for (uint32_t unit = blockIdx.x; unit < p.E * chunks; unit += gridDim.x) {
+            const int e = (int)(unit / chunks);
+            if (p.offsets[e + 1] <= p.offsets[e]) wgrad_zero_rows<CDT, S::NTHR>(p, e, (int)(unit % chunks) * 64);
+        }
+    }
     if (slices == 1) return;
     const int per_e = p.tiles_m * p.tiles_n;
     const int tid = threadIdx.x;
@@ -1555,14 +1561,14 @@ static int launch_wgrad(WgradArgs a, float *ws, int64_t ws_bytes, hipStream_t st
                         (int64_t)a.Kout * a.ldbs < ((int64_t)1 << 32);
     const int chunks = (a.N + 63) / 64;
     if ((int64_t)a.E * chunks >= 0x7FFFFFFF) return MX_EUNSUPPORTED;
-    wgrad_zero_kernel<CDT><<<dim3((unsigned)(a.E * chunks)), dim3(256), 0, st>>>(a, chunks);
     const int rc = staged ? launch_with_lds<grouped_wgrad_kernel<S, CDT, SCALES_COPY>>(grid, block, S::LDS_BYTES_AHEAD, st, a)
                    : quad ? launch_with_lds<grouped_wgrad_kernel<S, CDT, SCALES_QUAD>>(grid, block, S::LDS_BYTES, st, a)
                           : launch_with_lds<grouped_wgrad_kernel<S, CDT, SCALES_DWORD>>(grid, block, S::LDS_BYTES, st, a);
     if (rc != MX_OK) return rc;
     // tiles are only split while (tiles x slices) fit the 2 * cus slots, so 4 * cus workgroups cover every unit at once
-    const int64_t units = work * S::MT < 4 * (int64_t)cus ? work * S::MT : 4 * (int64_t)cus;
-    if (a.slots) wgrad_reduce_kernel<S, CDT><<<dim3((unsigned)units), block, 0, st>>>(a, (int)grid.x);
+    const int64_t fills = (int64_t)a.E * chunks, sums = a.slots ? work * S::MT : 0, units = fills > sums ? fills : sums;
+    const int64_t most = 4 * (int64_t)cus;
+    wgrad_finish_kernel<S, CDT><<<dim3((unsigned)(units < most ? units : most)), block, 0, st>>>(a, (int)grid.x);
     return hipGetLastError() == hipSuccess ? MX_OK : MX_ELAUNCH;
 }
 

@@ -288,6 +288,37 @@ def test_wgrad_even_k_split_ranges_straddle_experts(oracle, counts):
             assert oracle.rel_error(dw[i].cpu(), ref) < TOL, (i, cnt)
 
 
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16, torch.float32])
+@pytest.mark.parametrize("counts", [[0, 130, 0, 0, 1], [0] * 1200 + [40] + [0] * 30, [0] * 9 + [1], [64, 3]])
+@pytest.mark.parametrize("n,k", [(200, 128), (65, 100), (520, 264)])
+def test_wgrad_of_experts_without_rows_is_zero(counts, n, k, dtype):
+    """Whole and partial units of 64 rows, vector and element stores, more units than workgroups, with and without K slices:
+    zeros over whatever lay in the memory before, and the other experts' gradients as each has them alone."""
+    from kohakuwullm_amd.kernels.mxfp8.grouped import grouped_mxfp8_wgrad, quantize_mx_cols_grouped
+
+    g = torch.Generator(device=DEV).manual_seed(SEED)
+    m = sum(counts)
+    offsets = torch.zeros(len(counts) + 1, dtype=torch.int32)
+    offsets[1:] = torch.tensor(counts).cumsum(0)
+    pad = lambda w: -(-w // 32) * 32  # noqa: E731  (the quantizer's widths)
+    a, b = (torch.randn(max(m, 1), pad(w), device=DEV, generator=g).bfloat16() for w in (n, k))
+    (aq, as_), (bq, bs) = (quantize_mx_cols_grouped(t, offsets.to(DEV), m) for t in (a, b))
+    aq, as_, bq, bs = aq[:n], as_[:n], bq[:k], bs[:k]
+    torch.full((len(counts), n, k), float("nan"), device=DEV, dtype=dtype)  # the block the allocator hands out next
+    dw = grouped_mxfp8_wgrad(aq, as_, bq, bs, offsets.to(DEV), m, dtype)
+    for e, rows in enumerate(counts):
+        if not rows:
+            continue
+        lo = int(offsets[e])
+        one = torch.tensor([0, rows], dtype=torch.int32, device=DEV)
+        (oq, os_), (pq, ps) = (quantize_mx_cols_grouped(t[lo:lo + rows], one, rows) for t in (a, b))
+        want = grouped_mxfp8_wgrad(oq[:n], os_[:n], pq[:k], ps[:k], one, rows, torch.float32)[0]
+        # the same products of 128 rows or one, in fp32 sums of another order at most, and one rounding
+        assert (dw[e].float() - want).norm() <= (1e-5 if dtype == torch.float32 else 4e-3) * want.norm()
+    empty = torch.tensor([c == 0 for c in counts], device=DEV)
+    assert not dw[empty].count_nonzero()
+
+
 @pytest.mark.parametrize("counts,n,k", [([50] * 300, 256, 256), ([50, 300, 1, 129, 128, 5, 0, 257] * 45, 512, 256),
                                         ([128] * 130 + [4000] + [1] * 140, 256, 512)])
 def test_wgrad_runs_of_single_stage_tiles(oracle, counts, n, k):
