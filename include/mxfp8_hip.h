@@ -507,6 +507,15 @@ int mx_router_topk_backward(const void *grad_weight, int gw_dtype, const int64_t
                             int64_t top_k, int norm, float factor, void *dx, int64_t lddx, void *dw, float *workspace,
                             int64_t workspace_len, void *stream);
 
+/*
+ * The same on top of onto (T, D), rows ldonto elements apart, in x's type: dx = onto + the gradient, rounded once.  onto may be
+ * NULL, and has to be where dx is.
+ */
+int mx_router_topk_backward_onto(const void *onto, int64_t ldonto, const void *grad_weight, int gw_dtype, const int64_t *idx,
+                                 const float *scores, const void *x, int x_dtype, int64_t ldx, const void *w, int w_dtype, int64_t T,
+                                 int64_t D, int64_t E, int64_t top_k, int norm, float factor, void *dx, int64_t lddx, void *dw,
+                                 float *workspace, int64_t workspace_len, void *stream);
+
 /* ---- expert dispatch either side of the routed-expert GEMMs ------------------------------ */
 
 /*

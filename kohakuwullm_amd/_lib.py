@@ -72,6 +72,8 @@ SIGNATURES = {
     "mx_router_backward_workspace": (_i64, [_i64, _i64, _i64]),
     "mx_router_topk_backward": (
         _ci, [_p, _ci, _p, _p, _p, _ci, _i64, _p, _ci, _i64, _i64, _i64, _i64, _ci, _f, _p, _i64, _p, _p, _i64, _p]),
+    "mx_router_topk_backward_onto": (
+        _ci, [_p, _i64, _p, _ci, _p, _p, _p, _ci, _i64, _p, _ci, _i64, _i64, _i64, _i64, _ci, _f, _p, _i64, _p, _p, _i64, _p]),
     "mx_expert_counts": (_ci, [_p, _ci, _i64, _i64, _p, _p]),
     "mx_expert_sort_workspace": (_i64, [_i64, _i64]),
     "mx_expert_sort": (_ci, [_p, _ci, _i64, _p, _i64, _i64, _p, _p, _p, _p, _p, _i64, _p]),

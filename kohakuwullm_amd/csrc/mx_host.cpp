@@ -42,7 +42,7 @@ namespace {
     F(mx_quantize_rows) F(mx_quantize_tokens) F(mx_quantize_tokens_side) F(mx_join_codes) F(mx_quantize_dual_batch)         \
     F(mx_swiglu_quantize_tokens) F(mx_swiglu_bwd_quantize_tokens) F(mx_gemm_nt) F(mx_gemm_nt_batch) F(mx_activation_gemm_nt) F(mx_rmsnorm_quantize) \
     F(mx_rmsnorm_backward) F(mx_rmsnorm_weight_grad) F(mx_router_topk) F(mx_router_backward_workspace)                      \
-    F(mx_router_topk_backward) F(mx_expert_sort_workspace) F(mx_expert_sort_positions) F(mx_experts_gemm1)                  \
+    F(mx_router_topk_backward_onto) F(mx_expert_sort_workspace) F(mx_expert_sort_positions) F(mx_experts_gemm1)                  \
     F(mx_grouped_gemm_nt) F(mx_experts_combine_onto) F(mx_experts_gemm2_dgrad) F(mx_quantize_cols_grouped) F(mx_grouped_wgrad_nt)
 
 struct Library {
@@ -759,6 +759,10 @@ PyObject *py_route_backward(Args &a) {
     const bool norm = a.flag();
     const double factor = a.number();
     const bool need_dx = a.flag(), need_dw = a.flag();
+    const Tensor onto = a.tensor();  // what dx is added to, or nothing
+    if (onto.defined())
+        MX_NEED(need_dx && plain(x) && plain(onto) && onto.dim() == 2 && onto.sizes() == x.sizes() && onto.scalar_type() == x.scalar_type() && onto.stride(1) == 1 &&
+                onto.stride(0) >= onto.size(1) && onto.stride(0) * onto.element_size() % 16 == 0 && aligned(onto, 16));
     MX_NEED(plain(grad) && plain(x) && plain(w) && plain(idx) && plain(scores) && x.dim() == 2 && w.dim() == 2 && idx.dim() == 2 && x.numel() > 0 &&
             w.is_contiguous() && aligned(w, 16) && idx.is_contiguous() && scores.is_contiguous() && idx.scalar_type() == at::kLong &&
             scores.scalar_type() == at::kFloat && x.stride(1) == 1 && x.stride(0) >= x.size(1) && x.stride(0) * x.element_size() % 16 == 0 &&
@@ -775,7 +779,7 @@ PyObject *py_route_backward(Args &a) {
         MX_NEED(words >= 0);
         scratch = empty({words}, at::kFloat, x);
     }
-    MX_RUN(mx_router_topk_backward, g.const_data_ptr(), gc, (const int64_t *)idx.const_data_ptr(), (const float *)scores.const_data_ptr(),
+    MX_RUN(mx_router_topk_backward_onto, onto.defined() ? onto.const_data_ptr() : nullptr, onto.defined() ? onto.stride(0) : 0, g.const_data_ptr(), gc, (const int64_t *)idx.const_data_ptr(), (const float *)scores.const_data_ptr(),
            x.const_data_ptr(), xc, x.stride(0), w.const_data_ptr(), wc, t, d, e, idx.size(1), norm, (float)factor,
            need_dx ? dx.data_ptr() : nullptr, d, need_dw ? dw.data_ptr() : nullptr, words ? (float *)scratch.data_ptr() : nullptr, words, stream_of(x));
     return wrap_all({dx, dw});

@@ -60,7 +60,7 @@ def composed_gradients(grad, x, weight, idx, norm: bool, factor: float):
 
 class _RouteTopK(torch.autograd.Function):
     @staticmethod
-    def forward(ctx, x, weight, bias, top_k, norm, factor):
+    def forward(ctx, x, weight, bias, top_k, norm, factor, through=False):
         (t, d), e, dev = x.shape, weight.shape[0], x.device
         need = ctx.needs_input_grad[0] or ctx.needs_input_grad[1]
         made = host.route_forward(x, weight, bias, top_k, norm, factor, need)
@@ -82,19 +82,24 @@ class _RouteTopK(torch.autograd.Function):
             ctx.norm, ctx.factor = norm, factor
         ctx.mark_non_differentiable(idx, counts)
         ctx.set_materialize_grads(False)
-        return idx, gate, counts
+        return (idx, gate, counts, x) if through else (idx, gate, counts)
 
     @staticmethod
-    def backward(ctx, _idx, grad, _counts):
+    def backward(ctx, _idx, grad, _counts, onto=None):
+        rest = (None,) * 5
+        if not ctx.needs_input_grad[0]:
+            onto = None
         if grad is None:
-            return (None,) * 6
+            return onto, None, *rest
         x, weight, idx, scores = ctx.saved_tensors
-        if torch.is_grad_enabled() or not plain_call(grad):  # create_graph; a vmap over upstream gradients
+        if torch.is_grad_enabled() or not plain_call(grad, *(() if onto is None else (onto,))):
+            # create_graph; a vmap over upstream gradients
             dx, dw = composed_gradients(grad, x, weight, idx, ctx.norm, ctx.factor)
-            return dx if ctx.needs_input_grad[0] else None, dw if ctx.needs_input_grad[1] else None, None, None, None, None
-        made = host.route_backward(grad, x, weight, idx, scores, ctx.norm, ctx.factor, *ctx.needs_input_grad[:2])
+            dx = dx if onto is None else dx + onto
+            return dx if ctx.needs_input_grad[0] else None, dw if ctx.needs_input_grad[1] else None, *rest
+        made = host.route_backward(grad, x, weight, idx, scores, ctx.norm, ctx.factor, *ctx.needs_input_grad[:2], onto)
         if made is not None:
-            return *made, None, None, None, None
+            return *made, *rest
         # as they were saved, unless a saved-tensor hook laid them out anew
         x, weight, idx, scores = aligned_rows(x), aligned_rows(weight.contiguous()), idx.contiguous(), scores.contiguous()
         (t, d), e, lib = x.shape, weight.shape[0], _lib.load()
@@ -103,13 +108,15 @@ class _RouteTopK(torch.autograd.Function):
         dw = torch.empty_like(weight) if ctx.needs_input_grad[1] else None
         words = lib.mx_router_backward_workspace(t, d, e) if dw is not None else 0
         scratch = torch.empty(words, device=x.device, dtype=torch.float32)
+        onto = None if onto is None else aligned_rows(onto)
+        below = () if onto is None else (onto.data_ptr(), onto.stride(0))
         _lib.invoke(
-            "mx_router_topk_backward", 4.0 * t * d * e, x, grad.data_ptr(), _lib.MX_DTYPE[grad.dtype], idx.data_ptr(),
+            "mx_router_topk_backward_onto" if below else "mx_router_topk_backward", 4.0 * t * d * e, x, *below, grad.data_ptr(), _lib.MX_DTYPE[grad.dtype], idx.data_ptr(),
             scores.data_ptr(), x.data_ptr(), _lib.MX_DTYPE[x.dtype], x.stride(0), weight.data_ptr(), _lib.MX_DTYPE[weight.dtype],
             t, d, e, idx.shape[1], int(ctx.norm), float(ctx.factor), 0 if dx is None else dx.data_ptr(), d,
             0 if dw is None else dw.data_ptr(), scratch.data_ptr() if words else 0, words,
         )
-        return dx, dw, None, None, None, None
+        return dx, dw, *rest
 
 
 def route_topk(x: torch.Tensor, weight: torch.Tensor, bias: torch.Tensor | None, top_k: int, norm: bool, factor: float):
@@ -125,12 +132,15 @@ def route_topk(x: torch.Tensor, weight: torch.Tensor, bias: torch.Tensor | None,
     return route_fitting(x, weight, bias, top_k, norm, factor)
 
 
-def route_fitting(x, weight, bias, top_k: int, norm: bool, factor: float):
-    """:func:`route_topk` of operands that :func:`can_route` has just looked at (a second look takes 2.6 us)."""
+def route_fitting(x, weight, bias, top_k: int, norm: bool, factor: float, through: bool = False):
+    """:func:`route_topk` of operands that :func:`can_route` has just looked at (a second look takes 2.6 us).
+
+    ``through``: ``x`` is returned behind the results, for whoever computes on it next.  Its gradient then comes through the
+    router's node, whose kernel adds its own to it: one rounding, and no launch to add the two."""
     # a copied input is copied in front of the graph's node, which then keeps the tensor it differentiates
     x = aligned_rows(x)
     if host.unrecorded(x, weight):
         made = host.route_forward(x, weight, bias, top_k, norm, factor, False)
         if made is not None:
-            return made[0], made[1], made[3]
-    return _RouteTopK.apply(x, weight, bias, top_k, norm, factor)
+            return (made[0], made[1], made[3], x) if through else (made[0], made[1], made[3])
+    return _RouteTopK.apply(x, weight, bias, top_k, norm, factor, through)

@@ -99,6 +99,17 @@ class TopKRouter(nn.Module):
         return (self.score_func == "sigmoid" and self.n_groups == 1 and self.aux_loss_weight <= 0 and self.z_loss_weight <= 0
                 and can_route(x, self.weight, self.top_k, self.expert_bias))
 
+    def route_through(self, x: torch.Tensor):
+        """:meth:`route`, and ``x`` behind its results for the experts to compute on (``route_fitting``)."""
+        if not (torch.is_grad_enabled() and self._on_kernels(x)):
+            return *self.route(x), x
+        self.aux_loss = self.z_loss = None
+        topk_idx, topk_weight, counts, x = route_fitting(x, self.weight, self.expert_bias, self.top_k, self.norm_topk_prob and self.top_k > 1,
+                                                         self.routed_scaling_factor, True)
+        if self.training and self.load_accum is not None:
+            self.load_accum += counts
+        return topk_idx, topk_weight, counts, x
+
     def route(self, x: torch.Tensor):
         """``(topk_idx (T, k), topk_weight (T, k) in x.dtype, counts (E,) int32)``."""
         if self._on_kernels(x):
@@ -290,7 +301,10 @@ class MoEMLP(nn.Module):
         shape = x.shape
         flat = x.reshape(-1, shape[-1])
         seen_by_router = flat if route_on is None else route_on.reshape(-1, route_on.shape[-1])
-        topk_idx, topk_weight, counts = self.router.route(seen_by_router)
+        if flat.requires_grad and route_on is None and getattr(self.router.route, "__func__", None) is TopKRouter.route:
+            topk_idx, topk_weight, counts, flat = self.router.route_through(flat)
+        else:
+            topk_idx, topk_weight, counts = self.router.route(seen_by_router)
         # slot width from the tensor, not top_k: a router may pad it
         # the fused path gathers by the inverse order, which covers the real experts alone: with a sentinel bucket it makes its own
         inverse = self._routed == self._routed_mxfp8 and not self._has_sentinel

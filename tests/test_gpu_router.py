@@ -191,3 +191,37 @@ def test_router_of_another_width_raises():
     with pytest.raises(RuntimeError):
         block(x, route_on=x[:, :64])
     assert block(x, route_on=x[:, :128].contiguous()).shape == x.shape
+
+
+@pytest.mark.parametrize("dtype", [BF, HF, F32])
+@pytest.mark.parametrize("tokens,dim,top_k", [(1, 8, 1), (37, 520, 3), (9000, 256, 6)])
+@pytest.mark.parametrize("layout", ["plain", "pitched", "transposed", "broadcast", "none"])
+def test_gradient_that_comes_through_the_router(tokens, dim, top_k, dtype, layout):
+    """``through``: what x's further use gives is added to the router's gradient in its kernel, however it lies."""
+    from kohakuwullm_amd.kernels.moe.router import route_fitting
+
+    g = torch.Generator(device=DEV).manual_seed(7)
+    x = torch.randn(tokens, dim, device=DEV, generator=g).to(dtype).requires_grad_()
+    w = (torch.randn(16, dim, device=DEV, generator=g) * dim**-0.5).to(dtype).requires_grad_()
+    up = torch.randn(tokens, top_k, device=DEV, generator=g).to(dtype)
+    onto = torch.randn(tokens, dim, device=DEV, generator=g).to(dtype)
+    onto = {"plain": onto, "pitched": torch.empty(tokens, dim + 4, device=DEV, dtype=dtype)[:, :dim].copy_(onto),
+            "transposed": onto.t().contiguous().t(), "broadcast": onto[:1].expand(tokens, dim), "none": None}[layout]
+    plain = torch.autograd.grad(route_fitting(x, w, None, top_k, True, 1.5)[1], [x, w], up)
+    idx, gate, counts, same = route_fitting(x, w, None, top_k, True, 1.5, True)
+    assert same.data_ptr() == x.data_ptr() and torch.equal(same, x)
+    if onto is None:
+        dx, dw = torch.autograd.grad(gate, [x, w], up)
+        assert torch.equal(dx, plain[0]) and torch.equal(dw, plain[1])
+        return
+    dx, dw = torch.autograd.grad([gate, same], [x, w], [up, onto], retain_graph=True)
+    assert torch.equal(dw, plain[1])
+    # the gradient itself and the sum rounded once each on one side, the sum alone on the other
+    unit = {BF: 2.0**-8, HF: 2.0**-11, F32: 2.0**-23}[dtype]
+    want = plain[0].double() + onto.double()
+    # ... and fp32 sums of top_k terms of up to 3 max|up| max|w| (s / S <= 1) and `onto`, in another order
+    terms = top_k * 3.0 * up.abs().max().double() * w.detach().abs().max().double()
+    assert ((dx.double() - want).abs() <= unit * (plain[0].double().abs() + want.abs()) + 2.0**-21 * (terms + onto.double().abs())).all()
+    assert torch.equal(torch.autograd.grad(same, x, onto, retain_graph=True)[0], onto)  # the gate weights unused
+    again = torch.autograd.grad([gate, same], [x, w], [up, onto], create_graph=True)  # by operators
+    assert again[0].requires_grad and (again[0].double() - want).norm() <= 4 * unit * want.norm() + 1e-5 * want.norm()
