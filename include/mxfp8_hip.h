@@ -284,7 +284,8 @@ int mx_unswizzle_scales(const uint8_t *swizzled, int64_t rows, int64_t cols, uin
  * has the K stages of those tiles dealt over all workgroups (fp32 partial tiles go through the
  * workspace, a second kernel adds them in a fixed order).  With less, every tile is computed
  * whole: same product, fp32 sums in another order, slower on such shapes.  The workspace holds
- * nothing between calls; calls that may overlap in time need separate ones.
+ * nothing between calls; calls that may overlap in time on the device need separate ones.  Threads that
+ * issue on one stream may share one: the launches of a call that go through it are issued back to back.
  * epilogue: MX_EPI_NONE, or MX_EPI_ACCUMULATE optionally with MX_EPI_SPLIT_K(n); a negative value is
  * MX_EINVAL, any other bit of the low byte MX_EUNSUPPORTED.
  * Replaces mxfp8_matmul_pq / _mxfp8_matmul_pq

@@ -210,8 +210,9 @@ def gemm_workspace(t: torch.Tensor) -> torch.Tensor:
     """Scratch for the K splits of ``mx_gemm_nt`` / ``mx_gemm_nt_batch`` / ``mx_grouped_wgrad_nt`` on ``t``'s device.
 
     One tensor per (device, current stream), allocated the first time that stream asks and kept: calls on one
-    stream run in order and may share it, work on another stream gets its own, and the hot path never goes
-    back to the allocator for a 128 MiB block that smaller tensors may have carved up in the meantime.
+    stream, from whichever threads, run in order and may share it (the library issues the launches of a call that go
+    through it back to back), work on another stream gets its own, and the hot path never goes back to the allocator
+    for a 128 MiB block that smaller tensors may have carved up in the meantime.
     The library itself allocates nothing.
     """
     index = t.get_device()

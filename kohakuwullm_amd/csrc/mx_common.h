@@ -5,6 +5,7 @@
 #include <stdint.h>
 
 #include <atomic>
+#include <mutex>
 
 #include "mxfp8_hip.h"
 
@@ -18,6 +19,10 @@ bool stream_is_capturing(hipStream_t st);
 int num_cus();  // CUs of the current device (cached per device ordinal)
 // hipFuncSetAttribute(MaxDynamicSharedMemorySize) once per device; `done` has one bit per device ordinal.
 bool allow_dynamic_lds(const void *kernel, int bytes, std::atomic<uint64_t> &done);
+// The turn on a caller's scratch: held from the launch that leaves partial sums there to the launch that adds them, so that another
+// thread issuing on the same stream cannot put launches on the same scratch in between.  Null (nothing goes through scratch): no
+// turn is taken.
+std::unique_lock<std::mutex> scratch_turn(const void *scratch);
 
 typedef int v8i __attribute__((ext_vector_type(8)));
 typedef int v4i __attribute__((ext_vector_type(4)));

@@ -479,6 +479,12 @@ bool stream_is_capturing(hipStream_t st) {
     }
     return cap != hipStreamCaptureStatusNone;
 }
+
+std::unique_lock<std::mutex> scratch_turn(const void *scratch) {
+    static std::mutex turns[16];  // one per stream's scratch as far as their number goes; two that share one only wait for each other
+    if (!scratch) return {};
+    return std::unique_lock<std::mutex>(turns[(uintptr_t)scratch * 0x9E3779B97F4A7C15ull >> 60]);
+}
 }  // namespace mx
 
 // fp32 tile slots a caller's workspace holds for the K splits (dense and expert WGRAD): the kernels use at
@@ -654,6 +660,7 @@ static int launch_tiled(DenseArgs a, float *ws, int ws_slots, hipStream_t st, bo
         }
     }
     dim3 grid((unsigned)(work < cus && !a.sk_tiles ? work : cus)), block(S::NTHR);
+    const auto turn = scratch_turn(a.sk_ws);
     int rc;
     a.phased = phased ? 1 : 0;
 #ifdef MX_BENCH_VARIANTS
@@ -744,6 +751,7 @@ static int launch_ring(DenseArgs *probs, int count, float *ws, int ws_slots, hip
         b.end[j] = blocks;
     }
     const dim3 grid((unsigned)blocks), block(S::NTHR);
+    const auto turn = scratch_turn(red.count ? ws : nullptr);
     const int rc = launch_with_lds<gemm_nt_ring_kernel<CDT>>(grid, block, RING_LDS_BYTES, st, b);
     if (rc != MX_OK) return rc;
     if (red.count) reduce_slices_kernel<S, CDT><<<dim3((unsigned)rblocks), block, 0, st>>>(red);
@@ -902,6 +910,7 @@ static int batch_dispatch(DenseArgs *probs, int count, float *ws, int ws_slots, 
     const dim3 grid((unsigned)cus), block(S::NTHR);
     bool ahead = mode == SCALES_VEC16;
     for (int j = 0; j < count; j++) ahead = ahead && ahead_pays(probs[j]);
+    const auto turn = scratch_turn(red.count ? ws : nullptr);
     const int rc = ahead ? launch_with_lds<gemm_nt_batch_kernel<S, CDT, SCALES_COPY, true>>(grid, block, S::LDS_BYTES_AHEAD, st, b)
                    : mode == SCALES_VEC16 ? launch_with_lds<gemm_nt_batch_kernel<S, CDT, SCALES_VEC16>>(grid, block, S::LDS_BYTES, st, b)
                    : mode == SCALES_DWORD

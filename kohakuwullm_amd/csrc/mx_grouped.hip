@@ -1561,6 +1561,7 @@ static int launch_wgrad(WgradArgs a, float *ws, int64_t ws_bytes, hipStream_t st
                         (int64_t)a.Kout * a.ldbs < ((int64_t)1 << 32);
     const int chunks = (a.N + 63) / 64;
     if ((int64_t)a.E * chunks >= 0x7FFFFFFF) return MX_EUNSUPPORTED;
+    const auto turn = scratch_turn(a.ws);
     const int rc = staged ? launch_with_lds<grouped_wgrad_kernel<S, CDT, SCALES_COPY>>(grid, block, S::LDS_BYTES_AHEAD, st, a)
                    : quad ? launch_with_lds<grouped_wgrad_kernel<S, CDT, SCALES_QUAD>>(grid, block, S::LDS_BYTES, st, a)
                           : launch_with_lds<grouped_wgrad_kernel<S, CDT, SCALES_DWORD>>(grid, block, S::LDS_BYTES, st, a);

@@ -250,3 +250,48 @@ def test_threads_on_their_own_streams():
         assert len(passes) == 20
         for one in passes:
             assert all(torch.equal(_bits(a), _bits(b)) for a, b in zip(one, want[i]))
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("way", ["extension", "ctypes"])
+def test_threads_on_one_stream_share_the_scratch_of_k_splits(way):
+    """Products whose partial sums go through the stream's one scratch tensor, issued by several threads at once: what each gives
+    alone, bit for bit.  Ring slices, the dealt last round of large tiles, slices in a batch and the expert weight gradient."""
+    import threading
+
+    from kohakuwullm_amd.kernels.mxfp8 import mxfp8_matmul_pq, mxfp8_matmul_pq_batch
+    from kohakuwullm_amd.kernels.mxfp8.grouped import grouped_mxfp8_wgrad, quantize_mx_cols_grouped
+
+    g = torch.Generator(device=DEV).manual_seed(SEED)
+
+    def operands(rows, k):
+        codes = torch.randint(0, 120, (rows, k), device=DEV, generator=g, dtype=torch.uint8).view(torch.float8_e4m3fn)
+        return codes, torch.randint(118, 126, (rows, k // 32), device=DEV, generator=g, dtype=torch.uint8)
+
+    ring, dealt = ((*operands(m, k), *operands(n, k)) for m, n, k in ((300, 500, 8192), (1500, 4096, 16384)))
+    both = [(*operands(3300, 8192), *operands(2500, 8192)), (*operands(2490, 8192), *operands(3310, 8192))]
+    offsets = torch.tensor([0, 4000, 4000, 9000], dtype=torch.int32, device=DEV)
+    rows = torch.randn(9000, 256, device=DEV, generator=g).to(BF)
+    rq, rs = quantize_mx_cols_grouped(rows, offsets, 9000)
+    jobs = [lambda: [mxfp8_matmul_pq(*ring, F32)], lambda: [mxfp8_matmul_pq(*dealt, BF)], lambda: mxfp8_matmul_pq_batch(both, BF),
+            lambda: [grouped_mxfp8_wgrad(rq, rs, rq, rs, offsets, 9000)]]
+    with contextlib.nullcontext() if way == "extension" else _python():
+        want = [job() for job in jobs]
+        torch.cuda.synchronize()
+        got, start = [[] for _ in jobs], threading.Barrier(len(jobs))
+
+        def work(i):
+            start.wait()
+            for _ in range(25):
+                got[i].append(jobs[i]())
+
+        threads = [threading.Thread(target=work, args=(i,)) for i in range(len(jobs))]
+        for t in threads:
+            t.start()
+        for t in threads:
+            t.join()
+        torch.cuda.synchronize()
+    for i, passes in enumerate(got):
+        assert len(passes) == 25
+        for outs in passes:
+            assert all(torch.equal(a, b) for a, b in zip(outs, want[i])), i
