@@ -115,18 +115,19 @@ def words(record: type[ctypes.Structure], rows) -> ctypes.Array:
     return (_i64 * len(flat))(*flat)
 
 
-_lib: ctypes.CDLL | None = None
+_lib: ctypes.CDLL | None = None  # what calls go to
+_product: ctypes.CDLL | None = None
 
 
 class MXFP8LibraryError(RuntimeError):
     """The HIP library is missing, or one of its entry points returned an error."""
 
 
-def load() -> ctypes.CDLL:
-    """Load (once) and type the library.  Raises if it has not been built."""
-    global _lib
-    if _lib is not None:
-        return _lib
+def product() -> ctypes.CDLL:
+    """The product library, loaded once and typed, also while calls go to another one.  Raises if it has not been built."""
+    global _product
+    if _product is not None:
+        return _product
     if not os.path.exists(LIB_PATH):
         raise MXFP8LibraryError(
             f"{LIB_PATH} is missing: build it with `make -C {os.path.join(_HERE, 'csrc')}` "
@@ -137,8 +138,16 @@ def load() -> ctypes.CDLL:
         fn = getattr(lib, name)  # AttributeError here means the header and the build disagree
         fn.restype = restype
         fn.argtypes = argtypes
-    _lib = lib
+    _product = lib
     return lib
+
+
+def load() -> ctypes.CDLL:
+    """The library calls go to: the product library, unless :class:`variants_library` is in force."""
+    global _lib
+    if _lib is None:
+        _lib = product()
+    return _lib
 
 
 # Measured-slower alternative kernels live in a library of their own, built from the same sources with
@@ -250,3 +259,6 @@ def invoke(name: str, work: float, tensor: torch.Tensor, *args) -> None:
     end.record()
     check(status, name)
     TIMER.append((name, work, start, end))
+
+
+own_invoke = invoke  # what the extension stands for (host.py), whatever is installed in its place

@@ -944,11 +944,12 @@ PyObject *py_experts_backward(Args &a) {
     return wrap_all({dx, dw_in, dw_out, dgate.scalar_type() == gate.scalar_type() ? dgate : dgate.to(gate.scalar_type())});
 }
 
-// bind(path, cdll, module): take the entry points from the library at `path`, which `cdll` is; `module` is the ctypes binding.
+// bind(path, cdll, invoke, module): take the entry points from the library at `path`, which `cdll` is; `module` is the ctypes binding,
+// `invoke` its own call function.
 PyObject *bind(PyObject *, PyObject *args) {
     const char *path;
-    PyObject *cdll, *module;
-    if (!PyArg_ParseTuple(args, "sOO", &path, &cdll, &module)) return nullptr;
+    PyObject *cdll, *invoke, *module;
+    if (!PyArg_ParseTuple(args, "sOOO", &path, &cdll, &invoke, &module)) return nullptr;
     void *so = dlopen(path, RTLD_NOW | RTLD_LOCAL);
     if (!so) return PyErr_Format(PyExc_RuntimeError, "%s: %s", path, dlerror());
     Library found;
@@ -959,15 +960,17 @@ PyObject *bind(PyObject *, PyObject *args) {
 #undef F
     lib = found;
     PyObject *dict = PyModule_GetDict(module);
-    PyObject *invoke = PyDict_GetItem(dict, s_invoke);
-    Py_INCREF(dict), Py_INCREF(cdll), Py_XINCREF(invoke);
+    Py_INCREF(dict), Py_INCREF(cdll), Py_INCREF(invoke);
     bound_cdll = cdll, bound_invoke = invoke, binding = dict;
     Py_RETURN_NONE;
 }
 
+// Whether plain calls are made here at present.
+PyObject *py_engaged(PyObject *, PyObject *) { return PyBool_FromLong(engaged()); }
+
 #define ENTRY(name) {#name, (PyCFunction)(void (*)(void))entry<py_##name>, METH_FASTCALL, nullptr}
 PyMethodDef methods[] = {
-    {"bind", bind, METH_VARARGS, nullptr},
+    {"bind", bind, METH_VARARGS, nullptr}, {"engaged", py_engaged, METH_NOARGS, nullptr},
     ENTRY(quantize_rows), ENTRY(quantize_tokens), ENTRY(quantize_side), ENTRY(join_codes), ENTRY(quantize_dual_batch),
     ENTRY(swiglu_tokens), ENTRY(swiglu_bwd_tokens), ENTRY(matmul), ENTRY(matmul_batch),
     ENTRY(linear_forward), ENTRY(linear_backward), ENTRY(group_forward), ENTRY(swiglu_mlp_forward),

@@ -12,11 +12,12 @@ def __getattr__(name: str):
         raise AttributeError(name)
     from kohakuwullm_amd import _lib
 
-    library = _lib.load()
+    _lib.load()
+    library = _lib.product()
     try:
         from kohakuwullm_amd import _host
     except ImportError as error:
         raise _lib.MXFP8LibraryError(f"kohakuwullm_amd/_host.so cannot be loaded ({error}): `make -C kohakuwullm_amd/csrc` builds it") from error
-    _host.bind(_lib.LIB_PATH, library, _lib)
+    _host.bind(_lib.LIB_PATH, library, _lib.own_invoke, _lib)
     globals().update({n: getattr(_host, n) for n in dir(_host) if not n.startswith("_") and n != "bind"})
     return globals()[name]

@@ -45,6 +45,27 @@ def test_calls_that_are_not_plain_are_declined():
         assert calls[0](x) is None
 
 
+def test_first_use_with_another_library_or_binding_installed():
+    """Whatever stands in the binding when the extension is first used, it makes calls for the product library and the binding's own
+    ``invoke`` alone."""
+    import subprocess
+    import sys
+
+    code = """
+from kohakuwullm_amd import _lib, host
+own, _lib.invoke = _lib.invoke, lambda *a: None
+with _lib.variants_library():
+    inside = [host.engaged()]
+    _lib.invoke = own
+    inside.append(host.engaged())
+assert inside == [False, False], inside
+assert host.engaged()
+_lib.TIMER = []
+assert not host.engaged()
+"""
+    subprocess.run([sys.executable, "-c", code], check=True, timeout=300)
+
+
 @contextlib.contextmanager
 def _python():
     """Calls inside go the Python way: a timer is installed."""
