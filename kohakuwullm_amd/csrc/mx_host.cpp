@@ -28,6 +28,7 @@
 #include <torch/csrc/Exceptions.h>
 #include <torch/csrc/autograd/python_variable.h>
 #include <torch/csrc/jit/frontend/tracer.h>
+#include <torch/headeronly/version.h>
 
 #include "mxfp8_hip.h"
 
@@ -989,5 +990,7 @@ PyMODINIT_FUNC PyInit__host() {
     s_invoke = PyUnicode_InternFromString("invoke");
     s_check = PyUnicode_InternFromString("check");
     s_workspace = PyUnicode_InternFromString("gemm_workspace");
-    return PyModule_Create(&module_def);
+    PyObject *module = PyModule_Create(&module_def);
+    if (module) PyModule_AddStringConstant(module, "torch_version", TORCH_VERSION);
+    return module;
 }

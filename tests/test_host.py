@@ -66,6 +66,32 @@ assert not host.engaged()
     subprocess.run([sys.executable, "-c", code], check=True, timeout=300)
 
 
+@pytest.mark.parametrize("spoil", ["sys.modules['kohakuwullm_amd._host'] = None", "torch.__version__ = '1.0.0'"])
+def test_without_the_extension_every_call_takes_the_python_way(spoil):
+    """Not built, or built against another PyTorch: a warning, and the functions in front of it do what they do for any other call."""
+    import subprocess
+    import sys
+
+    code = f"""
+import sys, warnings, torch
+{spoil}
+from kohakuwullm_amd import _lib, host
+from kohakuwullm_amd.kernels.mxfp8 import quantize_mx
+x = torch.zeros(32, 128)
+with warnings.catch_warnings(record=True) as seen:
+    warnings.simplefilter('always')
+    assert host.quantize_rows(x) is None and host.quantize_rows(x) is None and not host.unrecorded(x) and not host.engaged()
+assert [w.category for w in seen] == [RuntimeWarning], seen
+try:
+    quantize_mx(x)
+except _lib.MXFP8LibraryError as error:
+    assert 'lives on cpu' in str(error)
+else:
+    raise AssertionError
+"""
+    subprocess.run([sys.executable, "-c", code], check=True, timeout=300)
+
+
 @contextlib.contextmanager
 def _python():
     """Calls inside go the Python way: a timer is installed."""
