@@ -12,8 +12,6 @@
 #include <Python.h>
 #include <dlfcn.h>
 
-#include <map>
-#include <mutex>
 #include <vector>
 
 #include <ATen/ATen.h>
@@ -55,7 +53,7 @@ struct Library {
 PyObject *binding = nullptr;         // the dict of kohakuwullm_amd._lib
 PyObject *bound_cdll = nullptr;      // what its `_lib` holds while these pointers are the right ones
 PyObject *bound_invoke = nullptr;    // its own `invoke`
-PyObject *s_timer, *s_cdll, *s_invoke, *s_check, *s_workspace;
+PyObject *s_timer, *s_cdll, *s_invoke, *s_check, *s_workspace, *s_workspaces;
 
 // Thrown where a call turns out not to be plain; nothing has been launched then.
 struct Declined {};
@@ -277,24 +275,21 @@ Tokens swiglu_bwd_tokens(const Tensor &dh, const Tensor &gu, bool rounded) {
 
 // ---- products --------------------------------------------------------------------------------------------------------------
 
-// The binding's scratch tensor of (device, stream), asked for once per stream: the binding keeps one for each as well.
+// The binding's scratch tensor of (device, stream).  The binding keeps it, and alone: whoever empties its cache has the memory back.
 Tensor workspace(const Tensor &like) {
-    static std::mutex lock;
-    static auto *kept = new std::map<std::pair<int, void *>, Tensor>;  // outlives the interpreter: no destructor order to mind
-    const std::pair<int, void *> key(like.device().index(), stream_of(like));
-    {
-        std::lock_guard<std::mutex> hold(lock);
-        auto at = kept->find(key);
-        if (at != kept->end()) return at->second;
-    }
+    PyObject *kept = PyDict_GetItem(binding, s_workspaces);
+    PyObject *key = Py_BuildValue("(iK)", (int)like.device().index(), (unsigned long long)(uintptr_t)stream_of(like));
+    if (!key) throw python_error();
+    PyObject *ws = kept && PyDict_Check(kept) ? PyDict_GetItem(kept, key) : nullptr;
+    Py_DECREF(key);
+    if (ws && THPVariable_Check(ws)) return THPVariable_Unpack(ws);
     PyObject *arg = THPVariable_Wrap(like);
-    PyObject *ws = PyObject_CallFunctionObjArgs(PyDict_GetItem(binding, s_workspace), arg, nullptr);
+    ws = PyObject_CallFunctionObjArgs(PyDict_GetItem(binding, s_workspace), arg, nullptr);
     Py_DECREF(arg);
     if (!ws) throw python_error();
-    Tensor t = THPVariable_Unpack(ws);
+    const Tensor t = THPVariable_Unpack(ws);
     Py_DECREF(ws);
-    std::lock_guard<std::mutex> hold(lock);
-    return kept->emplace(key, t).first->second;
+    return t;
 }
 
 // Rows and contraction length of a code matrix, (rows, K) or stage-major (K / 128, rows, 128).
@@ -990,6 +985,7 @@ PyMODINIT_FUNC PyInit__host() {
     s_invoke = PyUnicode_InternFromString("invoke");
     s_check = PyUnicode_InternFromString("check");
     s_workspace = PyUnicode_InternFromString("gemm_workspace");
+    s_workspaces = PyUnicode_InternFromString("_WORKSPACES");
     PyObject *module = PyModule_Create(&module_def);
     if (module) PyModule_AddStringConstant(module, "torch_version", TORCH_VERSION);
     return module;

@@ -342,3 +342,20 @@ def test_threads_on_one_stream_share_the_scratch_of_k_splits(way):
         assert len(passes) == 25
         for outs in passes:
             assert all(torch.equal(a, b) for a, b in zip(outs, want[i])), i
+
+
+@pytest.mark.gpu
+def test_scratch_belongs_to_the_binding():
+    """Emptying its cache gives the memory back; the next product gets a scratch tensor anew, the same one from then on."""
+    from kohakuwullm_amd import _lib
+    from kohakuwullm_amd.kernels.mxfp8 import mxfp8_matmul_pq, quantize_mx
+
+    q, s = quantize_mx(torch.randn(256, 8192, device=DEV).to(BF))
+    want = mxfp8_matmul_pq(q, s, q, s, F32)
+    size = int(_lib.load().mx_gemm_workspace_bytes())
+    held = torch.cuda.memory_allocated()
+    _lib._WORKSPACES.clear()
+    assert held - torch.cuda.memory_allocated() >= size
+    for _ in range(2):
+        assert torch.equal(mxfp8_matmul_pq(q, s, q, s, F32), want)
+        assert [t.numel() for t in _lib._WORKSPACES.values()] == [size]
