@@ -290,19 +290,74 @@ __device__ __forceinline__ float pick_gradient(const RouterBwdArgs &p, float g, 
     return ds * s * (1.0f - s);
 }
 
+template <int XDT>
+__device__ __forceinline__ void dx_store(const RouterBwdArgs &p, int64_t t, int col, const float (&acc)[8]) {
+    typename Elem<XDT>::type *dst = (typename Elem<XDT>::type *)p.dx + t * p.lddx + col;
+    if (XDT == MX_FP32) {
+        ((v4f *)dst)[0] = v4f{acc[0], acc[1], acc[2], acc[3]};
+        ((v4f *)dst)[1] = v4f{acc[4], acc[5], acc[6], acc[7]};
+    } else if (XDT == MX_BF16) {
+        *(v4i *)dst = v4i{(int)pack2_bf16(acc[0], acc[1]), (int)pack2_bf16(acc[2], acc[3]), (int)pack2_bf16(acc[4], acc[5]),
+                          (int)pack2_bf16(acc[6], acc[7])};
+    } else {
+        typedef _Float16 h8 __attribute__((ext_vector_type(8)));
+        h8 h;
+#pragma unroll
+        for (int c = 0; c < 8; c++) h[c] = (_Float16)acc[c];
+        *(h8 *)dst = h;
+    }
+}
+
 // dx[t] = sum over the picks of dlogit * w[expert], a wave per token.  top_k of E terms are not zero, so this is a gather of
-// top_k rows of the router matrix, not a matrix product.  Lane i of a wave forms the gradient of the token's pick i, the sums over
-// the picks go lane by lane through scalar registers, and the next token's picks are requested ahead: a wave waits for nobody else.
-// us with sixteen tokens' picks formed by a workgroup in LDS, behind two round trips to memory and two barriers / now, bf16 and 6
-// picks: 2777 x 1024 12.7 / 8.1, 16384 x 1024 16.8 / 18.0 (201 MB of rows from L2 and 5 us of multiplications by the vector ALU;
-// with the matrix in LDS 22.4, its copy costs more than L2 does).
-// Where the caller has a gradient of the same hidden states in hand (what the experts give), the sums start from it: a launch
-// and a pass over three matrices less.  A mixture of experts trained on 16384 tokens 1106.6 / 1100.3 us, on 2777 492.4 / 488.6.
-constexpr int ROUTER_MAX_K = 16;
-template <int XDT, int WDT>
-__global__ __launch_bounds__(256) void router_dx_kernel(RouterBwdArgs p) {
+// top_k rows of the router matrix, not a matrix product.  Where the caller has a gradient of the same hidden states in hand (what
+// the experts give), the sums start from it: a launch and a pass over three matrices less.
+// pick(i) gives the gradient and the expert of the token's pick i, the same ones to every lane.
+template <int XDT, int WDT, typename F>
+__device__ __forceinline__ void router_dx_row(const RouterBwdArgs &p, int64_t t, int lane, F &&pick) {
     typedef typename Elem<XDT>::type X;
     typedef typename Elem<WDT>::type W;
+    for (int first = 0; first < p.D; first += 512) {  // every lane of the wave goes along: the picks are read from them
+        const int col = first + lane * 8, from = col < p.D ? col : 0;
+        typename Elem<XDT>::raw below;
+        if (p.onto) below = Elem<XDT>::template load_raw<false>((const X *)p.onto + t * p.ldonto + from);
+        float acc[8];
+        for (int i0 = 0; i0 < p.top_k; i0 += 8) {
+            typename Elem<WDT>::raw row[8];
+            float dl[8];
+#pragma unroll
+            for (int i = 0; i < 8; i++)  // all of them are requested before the first is waited for
+                if (i0 + i < p.top_k) {
+                    int e;
+                    pick(i0 + i, dl[i], e);
+                    row[i] = Elem<WDT>::template load_raw<false>((const W *)p.w + (int64_t)e * p.D + from);
+                }
+            if (i0 == 0) {
+                if (p.onto) {
+                    Elem<XDT>::unpack(below, acc);
+                } else {
+#pragma unroll
+                    for (int c = 0; c < 8; c++) acc[c] = 0.0f;
+                }
+            }
+#pragma unroll
+            for (int i = 0; i < 8; i++) {
+                if (i0 + i >= p.top_k) break;  // uniform
+                float wv[8];
+                Elem<WDT>::unpack(row[i], wv);
+#pragma unroll
+                for (int c = 0; c < 8; c++) acc[c] += dl[i] * wv[c];
+            }
+        }
+        if (col < p.D) dx_store<XDT>(p, t, col, acc);
+    }
+}
+
+// The picks' gradients in two ways, with the same sums in the same order (launch_router_dx chooses).
+// Few tokens: lane i of a wave forms the gradient of the token's pick i, the sums over the picks go lane by lane through scalar
+// registers, and the next token's picks are requested ahead.  A wave waits for nobody else, but all its lanes form six gradients.
+constexpr int ROUTER_MAX_K = 16, ROUTER_DX_TOKENS = 16;
+template <int XDT, int WDT>
+__global__ __launch_bounds__(256) void router_dx_few_kernel(RouterBwdArgs p) {
     const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int64_t stride = (int64_t)gridDim.x * 4, mine = lane < p.top_k ? lane : 0;
     int64_t t = (int64_t)blockIdx.x * 4 + wave;
@@ -318,7 +373,7 @@ __global__ __launch_bounds__(256) void router_dx_kernel(RouterBwdArgs p) {
     Pick next = pick_of(t);
     for (; t < p.T; t += stride) {
         const float g = next.g, s = next.s;
-        const int e = next.e;
+        const int mine_e = next.e;
         next = pick_of(t + stride < p.T ? t + stride : t);
         float sum = 0.0f, dot = 0.0f;
         if (p.norm) {
@@ -328,46 +383,66 @@ __global__ __launch_bounds__(256) void router_dx_kernel(RouterBwdArgs p) {
                 dot += bits2f((uint32_t)__builtin_amdgcn_readlane((int)f2bits(g), j)) * sj;
             }
         }
-        const float dl = pick_gradient(p, g, s, sum, dot);
-        for (int first = 0; first < p.D; first += 512) {  // every lane of the wave goes along: the picks are read from them
-            const int col = first + lane * 8, from = col < p.D ? col : 0;
-            float acc[8];
-            if (p.onto) {
-                Elem<XDT>::unpack(Elem<XDT>::template load_raw<false>((const X *)p.onto + t * p.ldonto + from), acc);
-            } else {
+        const float mine_dl = pick_gradient(p, g, s, sum, dot);
+        router_dx_row<XDT, WDT>(p, t, lane, [&](int i, float &dl, int &e) {
+            dl = bits2f((uint32_t)__builtin_amdgcn_readlane((int)f2bits(mine_dl), i));
+            e = __builtin_amdgcn_readlane(mine_e, i);
+        });
+    }
+}
+
+// Many tokens: a workgroup forms the gradients of sixteen tokens' picks in LDS, a thread per pick, behind two round trips to memory
+// and two barriers, which other workgroups fill; its waves then gather four tokens each.
+template <int XDT, int WDT, bool ONTO>
+__global__ __launch_bounds__(256) void router_dx_kernel(RouterBwdArgs p) {
+    __shared__ v2i picks[ROUTER_DX_TOKENS * ROUTER_MAX_K];
+    __shared__ v2f gs[ROUTER_DX_TOKENS * ROUTER_MAX_K];
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int64_t lo = (int64_t)blockIdx.x * ROUTER_DX_TOKENS;
+    const int n = (int)(p.T - lo < ROUTER_DX_TOKENS ? p.T - lo : ROUTER_DX_TOKENS);
+    static_assert(ROUTER_DX_TOKENS * ROUTER_MAX_K <= 256, "a pick per thread");
+    const int mine = threadIdx.x, total = n * p.top_k;
+    float g = 0.0f, s = 0.0f;
+    int expert = 0;
+    if (mine < total) {
+        const int64_t at = lo * p.top_k + mine;
+        g = load_float(p.gw, p.gw_dtype, at) * p.factor, s = p.scores[at], expert = (int)p.idx[at];
+        gs[mine] = v2f{g, s};
+    }
+    __syncthreads();
+    if (mine < total) {
+        float sum = 0.0f, dot = 0.0f;
+        if (p.norm) {
+            const int first = mine / p.top_k * p.top_k;
+            for (int j = 0; j < p.top_k; j++) {
+                const v2f other = gs[first + j];
+                sum += other[1];
+                dot += other[0] * other[1];
+            }
+        }
+        picks[mine] = v2i{(int)f2bits(pick_gradient(p, g, s, sum, dot)), expert};
+    }
+    __syncthreads();
+    for (int u = wave; u < n; u += 4) {
+        if constexpr (ONTO) {  // requested together with the rows
+            router_dx_row<XDT, WDT>(p, lo + u, lane, [&](int i, float &dl, int &e) {
+                const v2i pick = picks[u * p.top_k + i];
+                dl = bits2f((uint32_t)pick[0]), e = pick[1];
+            });
+        } else {
+            for (int col = lane * 8; col < p.D; col += 512) {
+                float acc[8];
 #pragma unroll
                 for (int c = 0; c < 8; c++) acc[c] = 0.0f;
-            }
-            for (int i0 = 0; i0 < p.top_k; i0 += 8) {
-                typename Elem<WDT>::raw row[8];
-#pragma unroll
-                for (int i = 0; i < 8; i++)  // all of them are requested before the first is waited for
-                    if (i0 + i < p.top_k)
-                        row[i] = Elem<WDT>::template load_raw<false>((const W *)p.w + (int64_t)__builtin_amdgcn_readlane(e, i0 + i) * p.D + from);
-#pragma unroll
-                for (int i = 0; i < 8; i++) {
-                    if (i0 + i >= p.top_k) break;  // uniform
-                    const float dli = bits2f((uint32_t)__builtin_amdgcn_readlane((int)f2bits(dl), i0 + i));
+#pragma unroll 4
+                for (int i = 0; i < p.top_k; i++) {
+                    const v2i pick = picks[u * p.top_k + i];
                     float wv[8];
-                    Elem<WDT>::unpack(row[i], wv);
+                    Elem<WDT>::load8((const typename Elem<WDT>::type *)p.w + (int64_t)pick[1] * p.D + col, wv);
 #pragma unroll
-                    for (int c = 0; c < 8; c++) acc[c] += dli * wv[c];
+                    for (int c = 0; c < 8; c++) acc[c] += bits2f((uint32_t)pick[0]) * wv[c];
                 }
-            }
-            if (col >= p.D) continue;
-            X *dst = (X *)p.dx + t * p.lddx + col;
-            if (XDT == MX_FP32) {
-                ((v4f *)dst)[0] = v4f{acc[0], acc[1], acc[2], acc[3]};
-                ((v4f *)dst)[1] = v4f{acc[4], acc[5], acc[6], acc[7]};
-            } else if (XDT == MX_BF16) {
-                *(v4i *)dst = v4i{(int)pack2_bf16(acc[0], acc[1]), (int)pack2_bf16(acc[2], acc[3]), (int)pack2_bf16(acc[4], acc[5]),
-                                  (int)pack2_bf16(acc[6], acc[7])};
-            } else {
-                typedef _Float16 h8 __attribute__((ext_vector_type(8)));
-                h8 h;
-#pragma unroll
-                for (int c = 0; c < 8; c++) h[c] = (_Float16)acc[c];
-                *(h8 *)dst = h;
+                dx_store<XDT>(p, lo + u, col, acc);
             }
         }
     }
@@ -608,6 +683,25 @@ static int launch_router_nt(const RouterArgs &a, hipStream_t st) {
     return launch_router_mt<XDT, WDT, 16>(a, st);
 }
 
+// Which of the two kernels: what a wave waits for decides while the chip is not full, and the instructions per token afterwards.
+// us few / many, bf16:
+//   tokens   1024, 6 picks   2048, 6    1024, 16    4096, 8     512, 6     256, 4     1024, 6 onto a gradient
+//   2777       5.6 / 9.7    8.5 / 16.7  8.5 / 13.3   15 / 27   4.4 / 5.8  4.4 / 4.2     5.9 / 10.2
+//   8192      10.3 / 11.8  16.7 / 20.4 17.2 / 16.6   30 / 34   7.1 / 7.1  6.0 / 4.8    11.9 / 14.0
+//   12288     13.1 / 13.1  21.8 / 23.6 22.9 / 20.2   41 / 42   9.2 / 8.1  7.4 / 5.4    19.4 / 19.3
+//   16384     17.0 / 15.1  26.7 / 26.6 30.4 / 24.6   56 / 53  11.6 / 9.1  9.4 / 6.2    26.2 / 22.9
+//   65536     54.4 / 39.1                106 / 78             36.6 / 23   30 / 16      100 / 90
+static bool dx_few(const RouterBwdArgs &a) { return a.T <= (a.D <= 512 ? 32 : 48) * num_cus(); }
+
+template <int XDT, int WDT>
+static void launch_router_dx(const RouterBwdArgs &a, hipStream_t st) {
+    const int64_t tokens = dx_few(a) ? 4 : ROUTER_DX_TOKENS, blocks = (a.T + tokens - 1) / tokens, most = 8 * (int64_t)num_cus();
+    const dim3 grid((unsigned)(dx_few(a) && blocks > most ? most : blocks)), block(256);  // few: 32 waves per CU, in strides
+    if (dx_few(a)) router_dx_few_kernel<XDT, WDT><<<grid, block, 0, st>>>(a);
+    else if (a.onto) router_dx_kernel<XDT, WDT, true><<<grid, block, 0, st>>>(a);
+    else router_dx_kernel<XDT, WDT, false><<<grid, block, 0, st>>>(a);
+}
+
 template <int XDT>
 static int launch_router_dw(const RouterBwdArgs &a, hipStream_t st) {
     static std::atomic<uint64_t> done;
@@ -674,13 +768,11 @@ extern "C" int mx_router_topk_backward_onto(const void *onto, int64_t ldonto, co
     a.chunks = T ? (int)((T + a.chunk_tokens - 1) / a.chunk_tokens) : 1;
     if (a.chunks > 65535) return MX_EUNSUPPORTED;
     if (dx && T) {
-        const int64_t most = 8 * (int64_t)num_cus(), blocks = (T + 3) / 4;  // 32 waves per CU
-        const dim3 grid((unsigned)(blocks < most ? blocks : most)), block(256);
-        if (x_dtype == MX_BF16 && w_dtype == MX_BF16) router_dx_kernel<MX_BF16, MX_BF16><<<grid, block, 0, st>>>(a);
-        else if (x_dtype == MX_BF16) router_dx_kernel<MX_BF16, MX_FP32><<<grid, block, 0, st>>>(a);
-        else if (x_dtype == MX_FP16 && w_dtype == MX_FP16) router_dx_kernel<MX_FP16, MX_FP16><<<grid, block, 0, st>>>(a);
-        else if (x_dtype == MX_FP16) router_dx_kernel<MX_FP16, MX_FP32><<<grid, block, 0, st>>>(a);
-        else router_dx_kernel<MX_FP32, MX_FP32><<<grid, block, 0, st>>>(a);
+        if (x_dtype == MX_BF16 && w_dtype == MX_BF16) launch_router_dx<MX_BF16, MX_BF16>(a, st);
+        else if (x_dtype == MX_BF16) launch_router_dx<MX_BF16, MX_FP32>(a, st);
+        else if (x_dtype == MX_FP16 && w_dtype == MX_FP16) launch_router_dx<MX_FP16, MX_FP16>(a, st);
+        else if (x_dtype == MX_FP16) launch_router_dx<MX_FP16, MX_FP32>(a, st);
+        else launch_router_dx<MX_FP32, MX_FP32>(a, st);
     }
     if (dw) {
         const int rc = x_dtype == MX_BF16   ? launch_router_dw<MX_BF16>(a, st)

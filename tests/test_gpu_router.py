@@ -225,3 +225,28 @@ def test_gradient_that_comes_through_the_router(tokens, dim, top_k, dtype, layou
     assert torch.equal(torch.autograd.grad(same, x, onto, retain_graph=True)[0], onto)  # the gate weights unused
     again = torch.autograd.grad([gate, same], [x, w], [up, onto], create_graph=True)  # by operators
     assert again[0].requires_grad and (again[0].double() - want).norm() <= 4 * unit * want.norm() + 1e-5 * want.norm()
+
+
+@pytest.mark.parametrize("dim,top_k,xdt,wdt,norm", [(520, 16, BF, BF, True), (8, 1, HF, F32, False), (512, 9, F32, F32, True), (1032, 6, HF, HF, True)])
+def test_dx_of_many_tokens(dim, top_k, xdt, wdt, norm):
+    """Past the count from which sixteen tokens share a workgroup: bit for bit the dx that the same tokens get in short batches."""
+    from kohakuwullm_amd.kernels.moe.router import route_fitting
+
+    g = torch.Generator(device=DEV).manual_seed(SEED)
+    tokens = (32 if dim <= 512 else 48) * torch.cuda.get_device_properties(DEV).multi_processor_count + 5
+    x = torch.randn(tokens, dim, device=DEV, generator=g).to(xdt).requires_grad_()
+    w = (torch.randn(48, dim, device=DEV, generator=g) * dim**-0.5).to(wdt).requires_grad_()
+    up = torch.randn(tokens, top_k, device=DEV, generator=g).to(xdt)
+    onto = torch.randn(tokens, dim + 8, device=DEV, generator=g).to(xdt)[:, :dim]
+
+    def gradients(rows):
+        part = x[rows]
+        _, gate, _, same = route_fitting(part, w, None, top_k, norm, 1.5, True)
+        alone = torch.autograd.grad(gate, part, up[rows], retain_graph=True)[0]
+        return alone, torch.autograd.grad([gate, same], part, [up[rows], onto[rows]])[0]
+
+    whole = gradients(slice(None))
+    for lo in range(0, tokens, 5000):
+        rows = slice(lo, min(lo + 5000, tokens))
+        for a, b in zip(whole, gradients(rows)):
+            assert torch.equal(a[rows], b)
