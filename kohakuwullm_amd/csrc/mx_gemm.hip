@@ -596,8 +596,11 @@ static int launch_skinny(const DenseArgs *probs, int count, hipStream_t st) {
         const int stages = ((probs[j].K >> 7) + SKINNY_WAVES - 1) / SKINNY_WAVES;
         per = stages > per ? stages : per;
     }
-    const bool one = per == 1 || blocks > num_cus();  // a stage in flight per wave leaves LDS for a second workgroup per CU
-    if (rows <= 16) return per > 2 ? launch_skinny_tiles<CDT, 1, 4, SRC>(b, blocks, st) : launch_skinny_tiles<CDT, 1, 2, SRC>(b, blocks, st);
+    // K stages in flight per wave: one leaves LDS for a second workgroup per CU, which two do not from 17 rows on.  Up to 16 rows one /
+    // two / four, us: 1536 -> 131072 43.3 / 56.1 / 90.2, 4096 -> 16384 18.6 / 18.8 / 25.5, 8192 -> 16384 35.0 / 32.8 / 37.2, 16384 ->
+    // 1536 17.3 / 15.7 / 15.9; with activations 4096 -> 4096 8.6 / 8.7 / 10.1, 1536 -> 8192 6.4 / 7.0 / 11.9.
+    const bool one = per == 1 || SRC != SRC_CODES || (blocks > num_cus() && (rows > 16 || per <= 4));
+    if (rows <= 16) return one ? launch_skinny_tiles<CDT, 1, 1, SRC>(b, blocks, st) : launch_skinny_tiles<CDT, 1, 2, SRC>(b, blocks, st);
     if (rows <= 32) return one ? launch_skinny_tiles<CDT, 2, 1, SRC>(b, blocks, st) : launch_skinny_tiles<CDT, 2, 2, SRC>(b, blocks, st);
     if constexpr (SRC != SRC_CODES) return MX_EUNSUPPORTED;
     else if (rows <= 64) return one ? launch_skinny_tiles<CDT, 4, 1, SRC>(b, blocks, st) : launch_skinny_tiles<CDT, 4, 2, SRC>(b, blocks, st);

@@ -49,6 +49,7 @@ def test_ring_gemm(oracle, m, n, k, dtype):
 @pytest.mark.parametrize("m,n,k", [
     (1, 1, 128), (1, 17, 384), (15, 16, 640), (16, 4100, 1024), (17, 48, 1152), (32, 4112, 2048), (33, 200, 896), (64, 520, 4224), (64, 4128, 256),
     (65, 72, 1280), (128, 129, 2176),  # the last group of 16 rows and of 16 columns, one K stage per wave, none, several
+    (7, 4112, 4096), (16, 4112, 4352), (16, 300, 3200),  # up to 16 rows: one stage at a time on a full chip, two past four stages, two
 ])
 @pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16, torch.float16])
 def test_gemm_of_few_rows(oracle, m, n, k, dtype):
