@@ -529,14 +529,14 @@ static int64_t tiles_of(const DenseArgs &a, int edge) { return (int64_t)((a.M + 
 // K slices of a ring product: a long contraction (64 stages and more) of few tiles is cut so that the chip has a workgroup per
 // CU, into slices of at least 16 stages.  512 x 512 x 8192 (16 tiles): 27.2 us whole, 18.2 in four slices; 512 x 1536 x 16384:
 // 76.2 and 31.9 us; 1536 x 512 x 4096 (32 stages) 16.8 whole, 16.7 and 18.4 in two and four: not worth it.
-static int ring_slices(const DenseArgs &a, int free_tiles) {
+static int ring_slices(const DenseArgs &a, int free_tiles, int cus) {
     const int KT = a.K >> 7;
     const int64_t tiles = tiles_of(a, RingShape::BM);
     if (KT < 64) return 1;
     int best = 1;
     for (int s = 2; s <= 8; s *= 2) {
         const int per = ((KT + s - 1) / s + 3) & ~3;
-        if (tiles * s <= num_cus() && tiles * s <= free_tiles && per >= 16 && (s - 1) * per < KT) best = s;
+        if (tiles * s <= cus && tiles * s <= free_tiles && per >= 16 && (s - 1) * per < KT) best = s;
     }
     return best;
 }
@@ -550,31 +550,81 @@ static int ring_slices(const DenseArgs &a, int free_tiles) {
 // 30.6 / 30.3, 4096 x 3072 x 2048 32.0 / 32.4, 2048 x 2048 x 16384 82.4 / 79.4, 5003 x 8192 x 1536 73 / 85, 1536 x 4096 x 16384 105 / 140.
 // K needs no whole groups of four stages (the token axis of a batch of odd length): both gradients of 512 -> 1536 over 2304 tokens
 // 29.2 / 11.8, of 1536 -> 1536 over 640 22.2 / 10.2, 4352 x 1024 x 2816 36.5 / 26.8.
+// No range of dealt stages is shorter than an eighth of a tile: one tile of K = 65536 (64 x 64) takes 94 us that way, 29 in slices.
 // A caller without a workspace gets neither K slices nor dealt stages.  The choice holds there too where slices were priced:
 // such a product has at most one tile per CU, and one round of whole ring tiles (0.52 per stage) is under one of whole large
 // ones (1.4).
-static bool ring_pays(const DenseArgs &a) {
-    if (!ring_ok(a)) return false;
-    const int64_t small = tiles_of(a, 128), large = tiles_of(a, 256), cus = num_cus();
-    if (small > 4 * cus) return false;
+static double ring_us(const DenseArgs &a, bool may_cut, int cus) {
     const double KT = a.K >> 7;
-    const int slices = ring_slices(a, 0x7FFFFFFF);
-    const double ring = slices > 1 ? 0.52 * KT / slices + 13.5 : (double)((small + cus - 1) / cus) * (0.52 * KT + 1.5) + 6;
-    const double stage = 2 * large > cus ? 1.6 : 1.4;
-    const double whole = (double)((large + cus - 1) / cus) * (KT + 4) * stage + 3, dealt = (double)large * KT / cus * 1.65 + 35;
-    return ring < (whole < dealt ? whole : dealt);
+    const int slices = may_cut ? ring_slices(a, 0x7FFFFFFF, cus) : 1;
+    return slices > 1 ? 0.52 * KT / slices + 13.5 : (double)((tiles_of(a, 128) + cus - 1) / cus) * (0.52 * KT + 1.5) + 6;
+}
+static double tiled_us(const DenseArgs &a, bool may_cut, int cus) {
+    const int64_t large = tiles_of(a, 256);
+    const double KT = a.K >> 7, even = (double)large * KT / cus, share = even > KT / 8 ? even : KT / 8;  // a range is an eighth of a tile at least
+    const double whole = (double)((large + cus - 1) / cus) * (KT + 4) * (2 * large > cus ? 1.6 : 1.4) + 3, dealt = share * 1.65 + 35;
+    return may_cut && dealt < whole ? dealt : whole;
+}
+static bool ring_pays(const DenseArgs &a) {
+    const int cus = num_cus();
+    return ring_ok(a) && tiles_of(a, 128) <= 4 * cus && ring_us(a, true, cus) < tiled_us(a, true, cus);
 }
 
-// Whether a product goes to the kernel for few rows: up to 64, and up to 128 where a CU has no second 16 columns to do.  us on
-// ring tiles / there, weights from HBM:
+// us of the kernel for few rows on products that share a launch: the longer of a wave's walk over its eighth of K and of a CU's
+// share of all walks (a quarter of a stage more for each workgroup), at so much per stage, and for up to 16 rows no less than the
+// weights take at what they were seen to be read at.  From 65 rows on a CU holds one workgroup, and a second round never paid.
+static double skinny_us(const DenseArgs *probs, int count, int cus) {
+    int rows = 0, stages = 0;
+    double blocks = 0, share = 0, weights = 0;
+    for (int j = 0; j < count; j++) {
+        const int KT = probs[j].K >> 7, own = (probs[j].N + SKINNY_N - 1) / SKINNY_N;
+        rows = probs[j].M > rows ? probs[j].M : rows;
+        stages = KT > stages ? KT : stages;
+        blocks += own, share += own * (KT + 2), weights += (double)probs[j].N * probs[j].K;
+    }
+    share /= SKINNY_WAVES * cus;
+    const int walk = (stages + SKINNY_WAVES - 1) / SKINNY_WAVES;
+    const bool quiet = 4 * blocks <= cus;
+    if (rows > 64) return blocks > cus ? 1e9 : 3 + walk * (quiet ? 2.6 : 3.2);
+    const double per_walk = rows <= 16 ? 0.5 : rows <= 32 ? (quiet ? 0.85 : 1.2) : quiet ? 1.45 : 1.75;
+    const double per_share = rows <= 16 ? 0.6 : rows <= 32 ? 1.15 : 1.9;
+    double t = walk * per_walk > share * per_share ? walk * per_walk : share * per_share;
+    if (rows <= 16 && weights / ((6.2 - 0.1 * rows) * 1e6) > t) t = weights / ((6.2 - 0.1 * rows) * 1e6);
+    return 3 + t;
+}
+
+// Whether products go to the kernel for few rows (up to 128): where it is quicker than ring tiles, which for many columns read the
+// weights at 5 TB/s and cut a long K over more CUs, neither of which this kernel does.
+// us on the other kernels / here, weights from HBM:
 //            512 -> 1536   2048 -> 3072   4096 -> 1536   1536 -> 8192   1024 -> 5632   256 -> 1000
 //   M = 1     6.1 / 3.1     10.8 / 4.1     17.0 / 5.1      9.6 / 4.9      7.4 / 4.4     5.3 / 2.8
 //   16        6.0 / 3.3     11.0 / 4.5     17.8 / 5.9      9.7 / 5.2      7.5 / 4.7     5.3 / 2.9
 //   64        6.3 / 3.9     12.0 / 6.6     19.1 / 10.0    10.3 / 8.3      7.9 / 6.0     5.5 / 3.6
 //   128       6.1 / 4.7     13.1 / 9.1     22.0 / 16.1    10.8 / 13.2     7.6 / 10.0    5.5 / 4.2
-static bool skinny_pays(const DenseArgs &a) {
-    return a.K % 128 == 0 && a.split_k == 1 && !a.accumulate && aligned(a.as, 4) && aligned(a.bs, 4) && a.ldas % 4 == 0 && a.ldbs % 4 == 0 &&
-           (a.M <= 64 || (a.M <= 128 && a.N <= SKINNY_N * num_cus()));
+// and, launches issued back to back, where the line lies:
+//           16384 -> 64   16384 -> 2048   8192 -> 8192   28672 -> 8192   1536 -> 16384   1536 -> 131072   4096 -> 131072
+//   M = 1    14.5 / 9.7    19.4 / 11.8    23.4 / 14.8     51.0 / 46.5     10.5 / 7.3      46.4 / 35.2       121 / 90
+//   16       14.8 / 10.9   20.0 / 16.0    23.8 / 17.8     52.0 / 64.3     10.7 / 7.5      47.6 / 43.3       125 / 129
+//   32       14.9 / 15.1   20.2 / 22.2    24.1 / 24.4     52.8 / 92.8     11.0 / 10.2     48.9 / 60.3       127 / 165
+//   64       14.9 / 23.0   20.6 / 32.5    24.6 / 36.0     54.9 / 134      11.7 / 15.0     52.3 / 96.6       132 / 251
+//   128      15.2 / 40.6   22.1 / 58.7    27.0 / 60.1     61.3 / 220      12.3 / 24.5     56.8 / 182        145 / 439
+// Over 51 pairs of widths and 1 to 128 rows, and batches of two to four, what is chosen takes over a tenth longer than the better one
+// only for up to 16 rows of K from 32768 on (16 rows of 65536 -> 512: 53 against 41).
+static bool skinny_pays(const DenseArgs *probs, int count, int ws_slots) {
+    const int cus = num_cus();
+    const bool may_cut = ws_slots >= 2 * cus;
+    double other = 0, tiles = 0, weights = 0;
+    for (int j = 0; j < count; j++) {
+        const DenseArgs &a = probs[j];
+        if (!ring_ok(a) || a.M > 128) return false;
+        const double ring = ring_us(a, may_cut, cus), tiled = tiled_us(a, may_cut, cus), alone = tiles_of(a, 128) <= 4 * cus && ring < tiled ? ring : tiled;
+        other = alone > other ? alone : other;
+        tiles += (double)tiles_of(a, 128) * (0.52 * (a.K >> 7) + 1.5) / cus;
+        weights += (double)a.N * a.K;
+    }
+    if (count > 1 && tiles + 6 > other) other = tiles + 6;
+    if (weights / 4.9e6 + 6 > other) other = weights / 4.9e6 + 6;
+    return count > 0 && skinny_us(probs, count, cus) < other;
 }
 
 template <int CDT, int MT, int U, int SRC>
@@ -738,7 +788,7 @@ static int launch_ring(DenseArgs *probs, int count, float *ws, int ws_slots, hip
         const int tiles = a.tiles_m * a.tiles_n;
         a.sk_tiles = 0, a.sk_q = 0, a.sk_ws = nullptr;
         a.xcds = 8, a.phased = 0;
-        a.split_k = ring_slices(a, free_tiles);
+        a.split_k = ring_slices(a, free_tiles, num_cus());
         a.dp_tiles = a.split_k > 1 ? 0 : tiles;
         a.slice_ws = nullptr;
         if (a.split_k > 1) {
@@ -779,7 +829,7 @@ static int gemm_dispatch(DenseArgs a, float *ws, int ws_slots, hipStream_t st, b
                                                                                   a.lda, a.ldas, a.ldb, a.ldbs, a.ldc);
         return hipGetLastError() == hipSuccess ? MX_OK : MX_ELAUNCH;
     }
-    if (!phased && skinny_pays(a)) return launch_skinny<CDT>(&a, 1, st);
+    if (!phased && skinny_pays(&a, 1, ws_slots)) return launch_skinny<CDT>(&a, 1, st);
     if (!phased && ring_pays(a)) return launch_ring<CDT>(&a, 1, ws, ws_slots, st);
     return launch_tiled<DenseShape, CDT>(a, ws, ws_slots, st, phased);
 }
@@ -801,8 +851,8 @@ static int batch_dispatch(DenseArgs *probs, int count, float *ws, int ws_slots, 
     // 1536 x 512 x 4096: 39 -> 20 us; 3001 x 2048 x 2048 beside 2048 x 2048 x 3072: 45 -> 41).  A mixed batch shares the XCDs
     // below instead: one launch for each kind won 7 % on one such batch and lost up to 25 % on the others.
     bool ring = true, skinny = true;
-    for (int j = 0; j < count; j++) skinny = skinny && tiled_ok(probs[j]) && skinny_pays(probs[j]);
-    if (skinny && count) return launch_skinny<CDT>(probs, count, st);
+    for (int j = 0; j < count; j++) skinny = skinny && tiled_ok(probs[j]);
+    if (skinny && skinny_pays(probs, count, ws_slots)) return launch_skinny<CDT>(probs, count, st);
     for (int j = 0; j < count; j++) ring = ring && tiled_ok(probs[j]) && ring_pays(probs[j]);
     bool fuse = count > 1 && count <= MX_BATCH_MAX;
     DenseBatchArgs b;

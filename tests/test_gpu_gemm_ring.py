@@ -154,3 +154,52 @@ def test_batch_cuts_the_tiles_of_its_last_round(k, dtype):
     for (aq, a_s, bq, b_s), out in zip(problems, mxfp8_matmul_pq_batch([(a.view(F8), s, b.view(F8), t) for a, s, b, t in problems], dtype)):
         ref = value(aq, a_s) @ value(bq, b_s).T
         assert ((out.double() - ref).norm() / ref.norm()).item() < TOL[dtype]
+
+
+def _sums(m, n, k):
+    """Operands whose product shows in which order fp32 sums took its K stages: 2^24 from the first of them, in which later ones
+    are lost, and 1 from every other."""
+    a, b = torch.zeros(m, k, dtype=torch.uint8), torch.zeros(n, k, dtype=torch.uint8)
+    a[:, ::128], b[:, ::128] = 0x38, 0x38  # one 1.0 per stage
+    a_s, b_s = torch.full((m, k // 32), 127, dtype=torch.uint8), torch.full((n, k // 32), 127, dtype=torch.uint8)
+    b_s[:, 0] = 127 + 24
+    return a, a_s, b, b_s
+
+
+@pytest.mark.parametrize("m,n,k,order", [
+    # eighths of K and their sums in order: the kernel for few rows
+    (16, 4096, 28672, "eighths"), (16, 16384, 1536, "eighths"), (64, 2048, 4096, "eighths"), (128, 2048, 4096, "eighths"), (32, 4096, 4096, "eighths"),
+    # a long K, whose eighths are walks of many stages: ring tiles in four slices of whole groups
+    (64, 8192, 8192, "quarters"), (128, 512, 8192, "quarters"), (48, 5000, 12800, "quarters"),
+    # many columns, whose workgroups share the CUs: ring tiles, or 256 x 256 ones past four rounds of them
+    (64, 32768, 1536, "whole"), (32, 49152, 1536, "whole"), (128, 5120, 1536, "whole"), (64, 150000, 512, "whole"),
+])
+def test_few_rows_go_where_their_columns_and_depth_say(m, n, k, order):
+    from kohakuwullm_amd.kernels.mxfp8 import mxfp8_matmul_pq
+
+    ops = _dev(_sums(m, n, k))
+    out = mxfp8_matmul_pq(*ops, torch.float32)
+    stages = k // 128
+    per = {"eighths": -(-stages // 8), "quarters": (-(-stages // 4) + 3) // 4 * 4, "whole": stages}[order]
+    assert torch.equal(out, torch.full_like(out, 2.0**24 + stages - per))
+
+
+def test_few_rows_in_a_batch_share_the_choice():
+    """Columns of all products together: 8192 each are few enough alone, four times 8192 are not."""
+    from kohakuwullm_amd.kernels.mxfp8 import mxfp8_matmul_pq, mxfp8_matmul_pq_batch
+
+    ops = _dev(_sums(64, 8192, 1536))
+    assert (mxfp8_matmul_pq(*ops, torch.float32) == 2.0**24 + 10).all()
+    for out in mxfp8_matmul_pq_batch([ops] * 4, torch.float32):
+        assert (out == 2.0**24).all()
+
+
+def test_few_rows_without_scratch_keep_a_long_k():
+    """A caller without a workspace gets no K slices from the other kernels, so the few-row kernel's eighths are the quicker ones."""
+    from kohakuwullm_amd import _lib
+
+    aq, a_s, bq, b_s = _dev(_sums(64, 512, 8192))
+    out = torch.empty(64, 512, device=DEV)
+    call = lambda ws, n: _lib.load().mx_gemm_nt(aq.data_ptr(), a_s.data_ptr(), bq.data_ptr(), b_s.data_ptr(), out.data_ptr(), 2, 64, 512, 8192, 8192, 256,
+                                                8192, 256, 512, 0, ws, n, _lib.stream_of(aq))  # noqa: E731
+    assert call(0, 0) == _lib.MX_OK and (out == 2.0**24 + 56).all()
