@@ -331,12 +331,12 @@ int mx_gemm_nt_batch(const mx_gemm_problem *problems, int count, int c_dtype, vo
 /* C_j = Q(x) B_j^T for up to four products of the same few rows x (M, K), bf16 / fp16 of c_dtype or fp32 (rounded to c_dtype
  * first), pitch ldx elements: Q is mx_quantize_rows, done inside the product, the same codes and scale bytes.  Of every problem
  * aq, a_scale, lda and ldas are not looked at; M and K are those of x.  MX_EUNSUPPORTED, with nothing launched, for what is
- * left to mx_quantize_rows and mx_gemm_nt_batch: more rows than the launch it saves is worth (over 32, or over 16
- * with K > 2048), K % 128 != 0, x or codes not on 16 bytes, stage-major
- * codes, scale rows not on 4 bytes, an fp32 result. */
+ * left to mx_quantize_rows and mx_gemm_nt_batch: more rows than the launch it saves is worth (taken are up to 16 rows with K <=
+ * 4096, and 17 to 32 with K <= 2048 and no more than 16 columns per CU over all problems), K % 128 != 0, more than four problems,
+ * x or codes not on 16 bytes, stage-major codes, scale rows not on 4 bytes, x of another 16-bit type than the result, an fp32
+ * result. */
 int mx_activation_gemm_nt(const void *x, int x_dtype, int64_t ldx, const mx_gemm_problem *problems, int count, int c_dtype,
                           void *stream);
-
 
 /*
  * ---- routed experts -------------------------------------------------------------------

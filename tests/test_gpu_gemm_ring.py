@@ -134,6 +134,33 @@ def test_activations_quantized_inside_the_product(m, n, k, xt, ct):
     assert refused == [_lib.MX_EUNSUPPORTED] * 4
 
 
+@pytest.mark.parametrize("rows,depth,columns,count,taken", [
+    (16, 4096, 64, 1, True), (16, 4224, 64, 1, False), (17, 2048, 64, 1, True), (17, 2176, 64, 1, False), (32, 128, 64, 1, True), (33, 128, 64, 1, False),
+    (17, 256, 4096, 1, True), (17, 256, 4112, 1, False), (17, 256, 2048, 2, True), (17, 256, 2064, 2, False), (16, 256, 20000, 1, True),
+    (8, 256, 64, 4, True), (8, 256, 64, 5, False),
+])
+def test_which_activations_are_quantized_inside_the_product(rows, depth, columns, count, taken):
+    """The limits that the header states (256 CUs), and nothing written past them."""
+    import ctypes
+
+    from kohakuwullm_amd import _lib
+    from kohakuwullm_amd.kernels.mxfp8 import mxfp8_matmul_pq, quantize_mx
+
+    g = torch.Generator(device=DEV).manual_seed(SEED)
+    x = torch.randn(rows, depth, device=DEV, generator=g).bfloat16()
+    q, s = quantize_mx(torch.randn(columns, depth, device=DEV, generator=g).bfloat16())
+    out = torch.full((count, rows, columns), 3.0, device=DEV, dtype=torch.bfloat16)
+    records = _lib.words(_lib.GemmProblem, [(0, 0, q.data_ptr(), s.data_ptr(), o.data_ptr(), rows, columns, depth, 0, 0, depth, depth // 32, columns) for o in out])
+    status = _lib.load().mx_activation_gemm_nt(x.data_ptr(), 0, depth, ctypes.byref(records), count, 0, _lib.stream_of(x))
+    assert status == (_lib.MX_OK if taken else _lib.MX_EUNSUPPORTED)
+    want = mxfp8_matmul_pq(*quantize_mx(x), q, s, torch.bfloat16) if taken else torch.full_like(out[0], 3.0)
+    assert all(_close(o, want) for o in out)
+
+
+def _close(a, b):
+    return ((a.double() - b.double()).norm() <= 4e-3 * b.double().norm()).item()  # the products' sums may be cut differently
+
+
 @pytest.mark.parametrize("k", [(8192, 8192), (8320, 8192), (8192 + 32, 9216)])  # 16 scale bytes, 4 and 1 at a time; slices of unequal length
 @pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
 def test_batch_cuts_the_tiles_of_its_last_round(k, dtype):
