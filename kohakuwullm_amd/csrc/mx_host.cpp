@@ -357,9 +357,15 @@ std::vector<Tensor> matmul_batch(const std::vector<Product> &ps, ScalarType type
 }
 
 // The products of a few rows with several weights, the rows quantized on the way; false, with nothing launched, for more rows
-// or another layout than that kernel takes.  `outs` are allocated here, x's shape with the weights' widths.
+// or another layout than that kernel takes, and for more than 64 columns per CU: every workgroup of 16 columns quantizes the rows
+// again, which then costs what the launch saves (us in two launches / in one, 16 rows: 1536 -> 16384 9.8 / 9.5, 1536 -> 32768
+// 15.8 / 16.9, 512 -> 131072 23.6 / 25.0, 1536 -> 131072 45.9 / 54.7).  `outs` are allocated here, x's shape with the weights' widths.
+constexpr int64_t FEW_ROW_COLUMNS = 64 * 256;
 bool activation_products(const Tensor &x, const Tensor &x2d, ScalarType compute, const std::vector<Quantized> &ws, std::vector<Tensor> &outs) {
     if (x2d.size(0) > 32 || ws.size() > 4) return false;
+    int64_t columns = 0;
+    for (const Quantized &w : ws) columns += w.q.defined() && w.q.dim() ? w.q.size(0) : 0;
+    if (columns > FEW_ROW_COLUMNS) return false;
     mx_gemm_problem d[4];
     for (size_t j = 0; j < ws.size(); j++) {
         const Tensor &q = ws[j].q, &s = ws[j].s;

@@ -158,6 +158,20 @@ def test_linear(layout, dtype, master, autocast, tokens, inp, out):
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("out,tensors", [(16384, 1), (16400, 3)])  # the result; codes and scale bytes of the rows as well
+def test_rows_are_quantized_inside_the_product_up_to_64_columns_per_cu(out, tensors):
+    from kohakuwullm_amd.kernels.mxfp8.linear import MXFP8Linear
+
+    torch.manual_seed(SEED)
+    lin, x = MXFP8Linear(256, out).to(DEV).to(BF), torch.randn(16, 256, device=DEV).to(BF)
+    with torch.no_grad():
+        _both(lambda: [lin(x)])
+        before = torch.cuda.memory_stats()["allocation.all.allocated"]
+        lin(x)
+    assert torch.cuda.memory_stats()["allocation.all.allocated"] - before == tensors
+
+
+@pytest.mark.gpu
 @pytest.mark.parametrize("layout", ["flat", "batched", "pitched", "transposed"])
 @pytest.mark.parametrize("dtype", [BF, F16])
 def test_attention_and_norm(layout, dtype):
