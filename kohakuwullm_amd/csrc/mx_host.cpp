@@ -2,8 +2,8 @@
 // filling in arguments -- as a CPython extension over libmxfp8_hip.so.
 //
 // Every function here stands for the plain case of a Python function of the same name in kernels/, which describes the
-// operation and serves every other case.  A function returns None, before it has launched anything, for a call that is not
-// plain: a tensor that is not a strided one on the current GPU, a shape or layout that is refused or laid out anew there, a
+// operation and serves every other case.  A function returns None, before it has launched any of the library's kernels, for a call
+// that is not plain: a tensor that is not a strided one on the current GPU, a shape or layout that is refused or laid out anew there, a
 // call that is traced, transformed, intercepted by a mode or dispatched by a subclass, a timer or another library installed in
 // the binding.  The caller then takes the Python way, where such a call raises, copies or dispatches as it always did.
 //
@@ -75,14 +75,15 @@ void check(int status, const char *what) {
     if (done) PyErr_SetString(PyExc_RuntimeError, what);
     throw python_error();
 }
-// Other Python threads run while a launch waits for a place in its queue or an allocation for memory, as they do under ctypes and
-// in PyTorch's own operators.  Nothing in the guarded scope touches a Python object.
+// Other Python threads run while a launch waits for a place in its queue, or an allocation or copy for memory, as they do under
+// ctypes and in PyTorch's own operators.  Nothing in the guarded scope touches a Python object.
 struct Unlocked {
     PyThreadState *state = PyEval_SaveThread();
     ~Unlocked() noexcept(false) { PyEval_RestoreThread(state); }  // ends a daemon thread by unwinding it at interpreter exit
 };
 #define MX_CALL(name, ...) ([&] { Unlocked open; return lib.name(__VA_ARGS__); }())
 #define MX_RUN(name, ...) check(MX_CALL(name, __VA_ARGS__), #name)
+#define MX_COPY(expression) ([&]() -> Tensor { Unlocked open; return (expression); }())  // a PyTorch operator that may allocate and launch
 
 // ---- tensors ---------------------------------------------------------------------------------------------------------------
 
@@ -137,17 +138,24 @@ int64_t token_extent(int64_t tokens) {
     return 16 * (groups - panels) <= panels && groups <= TILE_ROWS ? groups : panels;
 }
 
+Tensor contiguous(const Tensor &t) { return t.is_contiguous() ? t : MX_COPY(t.contiguous()); }
+// All dimensions but the last one as rows.
+Tensor as_matrix(const Tensor &x) {
+    if (x.dim() == 2) return x;
+    return x.is_contiguous() ? x.view({-1, x.size(-1)}) : MX_COPY(x.reshape({-1, x.size(-1)}));
+}
+
 // A matrix the quantizers read as it lies: unit column stride, rows that start on 16 bytes.
 Tensor aligned_rows(const Tensor &x) {
     const int64_t pitch = x.stride(0);
-    if (x.stride(1) != 1 || pitch < x.size(1) || pitch * x.element_size() % 16 || !aligned(x, 16)) return x.clone(at::MemoryFormat::Contiguous);
+    if (x.stride(1) != 1 || pitch < x.size(1) || pitch * x.element_size() % 16 || !aligned(x, 16)) return MX_COPY(x.clone(at::MemoryFormat::Contiguous));
     return x;
 }
 
 Tensor activation_matrix(const Tensor &x, ScalarType compute) {
     MX_NEED(plain(x) && x.dim() >= 1 && x.numel() > 0 && half_type(compute));
-    Tensor m = x.dim() == 2 ? x : x.reshape({-1, x.size(-1)});
-    if (m.scalar_type() != compute && m.scalar_type() != at::kFloat) m = m.to(compute);
+    Tensor m = as_matrix(x);
+    if (m.scalar_type() != compute && m.scalar_type() != at::kFloat) m = MX_COPY(m.to(compute));
     code_of(m.scalar_type());
     return aligned_rows(m);
 }
@@ -301,6 +309,14 @@ void code_shape(const Tensor &q, int64_t &rows, int64_t &k) {
         MX_NEED(q.dim() == 2 && q.stride(1) == 1);
         rows = q.size(0), k = q.size(1);
     }
+}
+
+// A quantized weight or saved operand, looked at before the first launch of a call whose products `describe` looks at later.
+void check_operand(const Quantized &t) {
+    MX_NEED(plain(t.q) && plain(t.s) && t.s.dim() == 2 && t.s.stride(1) == 1 && t.q.element_size() == 1 && t.s.element_size() == 1);
+    int64_t rows, k;
+    code_shape(t.q, rows, k);
+    MX_NEED(rows > 0 && k > 0 && k % BLOCK == 0 && t.s.size(0) == rows && t.s.size(1) == k / BLOCK);
 }
 
 struct Product {
@@ -559,7 +575,8 @@ PyObject *py_linear_forward(Args &a) {
     const ScalarType compute = a.dtype();
     const Quantized w{a.tensor(), a.tensor()};
     const bool token_axis = a.flag();
-    MX_NEED(plain(w.q) && w.q.dim() == 2 && x.defined() && x.dim() >= 1 && x.size(-1) == w.q.size(1));
+    check_operand(w);
+    MX_NEED(w.q.dim() == 2 && x.defined() && x.dim() >= 1 && x.size(-1) == w.q.size(1));
     const Tensor x2d = activation_matrix(x, compute);
     std::vector<Tensor> few;
     if (!token_axis && activation_products(x, x2d, compute, {w}, few)) return wrap_all({few[0], Tensor(), Tensor()});
@@ -584,7 +601,8 @@ PyObject *py_unrecorded(Args &a) {
 PyObject *py_linear_eval(Args &a) {
     const Tensor x = a.tensor(), weight = a.tensor();
     const Quantized w{a.tensor(), a.tensor()};
-    MX_NEED(x.defined() && unrecorded(x) && unrecorded(weight) && plain(w.q) && w.q.dim() == 2 && x.dim() >= 1 && x.size(-1) == w.q.size(1));
+    check_operand(w);
+    MX_NEED(x.defined() && unrecorded(x) && unrecorded(weight) && w.q.dim() == 2 && x.dim() >= 1 && x.size(-1) == w.q.size(1));
     const ScalarType compute = at::autocast::is_autocast_enabled(at::kCUDA) ? at::autocast::get_autocast_dtype(at::kCUDA) : x.scalar_type();
     const Tensor x2d = activation_matrix(x, compute);
     std::vector<Tensor> out;
@@ -603,21 +621,17 @@ PyObject *py_linear_backward(Args &a) {
     MX_NEED(plain(w.q) && w.q.dim() == 2 && dout.defined() && dout.dim() >= 1 && dout.size(-1) == w.q.size(1) && (need_dx || need_dw));
     code_of(x_type), code_of(dw_type);
     if (need_dw) MX_NEED(plain(xt.q) && xt.q.dim() == 3 && xt.q.size(0) * PANEL == token_extent(dout.numel() / dout.size(-1)));
-    // everything the products will look at later is looked at here: nothing may be declined behind a launch
-    auto operand = [](const Quantized &t) {
-        MX_NEED(plain(t.q) && plain(t.s) && t.s.dim() == 2 && t.s.stride(1) == 1);
-        int64_t rows, k;
-        code_shape(t.q, rows, k);
-        MX_NEED(t.q.dim() == 3 || (t.q.stride(0) >= k && t.q.stride(0) % 16 == 0 && aligned(t.q, 16)));
-        MX_NEED(k % BLOCK == 0 && t.s.size(0) == rows && t.s.size(1) == k / BLOCK);
-    };
-    operand(w);
-    if (need_dw) operand(xt);
+    for (const Quantized *t : {&w, &xt}) {
+        if (t == &xt && !need_dw) continue;
+        check_operand(*t);
+        // beside an operand in panels the kernels take aligned rows alone
+        MX_NEED(t->q.dim() == 3 || (t->q.stride(0) >= t->q.size(1) && t->q.stride(0) % 16 == 0 && aligned(t->q, 16)));
+    }
     const Tensor d2d = activation_matrix(dout, compute);
     const std::vector<int64_t> dx_size = with_last(dout, w.q.size(0));
     Tensor dx, dw;
     if (!need_dw) {
-        const Quantized d = quantize_rows(d2d.to(compute));
+        const Quantized d = quantize_rows(d2d.scalar_type() == compute ? d2d : MX_COPY(d2d.to(compute)));
         return wrap_all({matmul({d.q, d.s, w.q, w.s}, x_type, dx_size, 0), dw});
     }
     const Tokens d = quantize_tokens(d2d, compute, 0, true);
@@ -641,8 +655,9 @@ PyObject *py_group_forward(Args &a) {
     std::vector<Quantized> ws;
     for (Py_ssize_t j = 0; j < PySequence_Fast_GET_SIZE(caches); j++) {
         const std::vector<Tensor> c = Args::as_tensors(PySequence_Fast_GET_ITEM(caches, j));
-        MX_NEED(c.size() == 4 && plain(c[0]) && plain(c[1]) && c[0].dim() == 2 && c[0].is_contiguous() && c[1].is_contiguous() && x.defined() &&
-                x.dim() >= 1 && c[0].size(1) == x.size(-1) && c[1].dim() == 2 && c[1].size(0) == c[0].size(0) && c[1].size(1) * BLOCK == c[0].size(1));
+        MX_NEED(c.size() == 4);
+        check_operand({c[0], c[1]});
+        MX_NEED(c[0].dim() == 2 && c[0].is_contiguous() && c[1].is_contiguous() && x.defined() && x.dim() >= 1 && c[0].size(1) == x.size(-1));
         ws.push_back({c[0], c[1]});
     }
     MX_NEED(!ws.empty() && ws.size() <= 8);
@@ -673,9 +688,10 @@ PyObject *py_swiglu_mlp_forward(Args &a) {
     const Quantized in = a.quantized(), out = a.quantized();
     const bool rounded = a.flag(), wgrad_in = a.flag(), wgrad_out = a.flag();
     const int64_t pad = a.integer();
-    for (const Quantized *w : {&in, &out})
-        MX_NEED(plain(w->q) && plain(w->s) && w->q.dim() == 2 && w->q.is_contiguous() && w->s.is_contiguous() && w->s.dim() == 2 &&
-                w->s.size(0) == w->q.size(0) && w->s.size(1) * BLOCK == w->q.size(1) && w->q.element_size() == 1);
+    for (const Quantized *w : {&in, &out}) {
+        check_operand(*w);
+        MX_NEED(w->q.dim() == 2 && w->q.is_contiguous() && w->s.is_contiguous());
+    }
     MX_NEED(x.defined() && x.dim() >= 1 && x.size(-1) == in.q.size(1) && in.q.size(0) == 2 * out.q.size(1) && out.q.size(1) % PANEL == 0);
     const Tensor x2d = activation_matrix(x, compute);
     MX_NEED(x2d.size(0) * out.q.size(1) / 8 < ROW_CHUNKS);
@@ -704,7 +720,7 @@ PyObject *py_rmsnorm_forward(Args &a) {
     const Tensor x = a.tensor(), w = a.tensor();
     const double eps = a.number();
     MX_NEED(plain(x) && x.dim() >= 1 && x.numel() > 0 && half_type(x.scalar_type()) && (!w.defined() || norm_weight_ok(w, x)));
-    const Tensor x2d = x.reshape({-1, x.size(-1)}).contiguous();
+    const Tensor x2d = contiguous(as_matrix(x));
     const int64_t m = x2d.size(0), k = x2d.size(1);
     const Tensor rstd = empty({m}, at::kFloat, x), out = empty(x.sizes(), x.scalar_type(), x);
     MX_RUN(mx_rmsnorm_quantize, x2d.const_data_ptr(), code_of(x.scalar_type()), m, k, k, w.defined() ? w.const_data_ptr() : nullptr,
@@ -720,7 +736,7 @@ PyObject *py_rmsnorm_backward(Args &a) {
     MX_NEED(plain(dout) && plain(x2d) && plain(rstd) && x2d.dim() == 2 && x2d.numel() > 0 && x2d.is_contiguous() && rstd.is_contiguous() &&
             rstd.scalar_type() == at::kFloat && rstd.numel() == x2d.size(0) && dout.dim() >= 1 && dout.numel() == x2d.numel() &&
             dout.size(-1) == x2d.size(1) && dout.scalar_type() == x2d.scalar_type() && half_type(x2d.scalar_type()) && (!w.defined() || norm_weight_ok(w, x2d)));
-    const Tensor d2d = dout.reshape({-1, dout.size(-1)}).contiguous();
+    const Tensor d2d = contiguous(as_matrix(dout));
     const int64_t m = x2d.size(0), k = x2d.size(1), parts = std::max<int64_t>(1, std::min((m + 3) / 4, most));
     const bool has_w = w.defined() && need_dw;
     const Tensor dx = empty(dout.sizes(), x2d.scalar_type(), x2d);
@@ -769,7 +785,7 @@ PyObject *py_route_backward(Args &a) {
             w.is_contiguous() && aligned(w, 16) && idx.is_contiguous() && scores.is_contiguous() && idx.scalar_type() == at::kLong &&
             scores.scalar_type() == at::kFloat && x.stride(1) == 1 && x.stride(0) >= x.size(1) && x.stride(0) * x.element_size() % 16 == 0 &&
             aligned(x, 16) && grad.numel() == idx.numel() && scores.numel() == idx.numel());
-    const Tensor g = grad.contiguous();
+    const Tensor g = contiguous(grad);
     const int64_t t = x.size(0), d = x.size(1), e = w.size(0);
     const int gc = code_of(g.scalar_type()), xc = code_of(x.scalar_type()), wc = code_of(w.scalar_type());
     Tensor dx, dw, scratch;
@@ -907,13 +923,14 @@ PyObject *py_experts_backward(Args &a) {
                 s.stride(0) == s.size(1) + SCALE_ROW_SLACK && aligned(s, 4));
     };
     if (need_wout) token_operand(htq, hts, hidden);
-    const Tensor dout = dout_any.contiguous();
+    const Tensor dout = contiguous(dout_any);
     const ScalarType type = x.scalar_type();
     const int code = code_of(type);
     void *const st = stream_of(x);
     const Quantized d = quantize_rows(dout);
     const Quantized dp{empty({r.m, 2 * hidden}, FP8, x), empty({r.m, 2 * hidden / BLOCK}, U8, x)};
-    const Tensor dgate = empty({gate.numel()}, at::kFloat, x).zero_();
+    const Tensor dgate = empty({gate.numel()}, at::kFloat, x);
+    MX_COPY(dgate.zero_());
     const Quantized pt = expert_token_buffers(2 * hidden, mpad, x);
     MX_RUN(mx_experts_gemm2_dgrad, bytes(d.q), bytes(d.s), x.size(0), dim, dim / BLOCK, r.p(token_of), r.p(order), gate.const_data_ptr(),
            code_of(gate.scalar_type()), MX_STACK(w_out), r.p(offsets), w_out.e, bytes(hq), hidden, bytes(hs), hidden / BLOCK, pre.const_data_ptr(), nullptr,
@@ -943,7 +960,7 @@ PyObject *py_experts_backward(Args &a) {
     }
     const Quantized xt = columns(x, false);
     dw_in = wgrad(pt.q, pt.s, xt.q, xt.s);
-    return wrap_all({dx, dw_in, dw_out, dgate.scalar_type() == gate.scalar_type() ? dgate : dgate.to(gate.scalar_type())});
+    return wrap_all({dx, dw_in, dw_out, dgate.scalar_type() == gate.scalar_type() ? dgate : MX_COPY(dgate.to(gate.scalar_type()))});
 }
 
 // bind(path, cdll, invoke, module): take the entry points from the library at `path`, which `cdll` is; `module` is the ctypes binding,

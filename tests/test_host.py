@@ -172,6 +172,27 @@ def test_rows_are_quantized_inside_the_product_up_to_64_columns_per_cu(out, tens
 
 
 @pytest.mark.gpu
+def test_calls_are_declined_in_front_of_the_first_launch():
+    """A weight that only the product would object to: nothing has been allocated for the quantizer in front of it."""
+    from kohakuwullm_amd import host
+    from kohakuwullm_amd.kernels.mxfp8 import quantize_mx
+
+    x = torch.randn(40, 256, device=DEV).to(BF)
+    q, s = quantize_mx(torch.randn(512, 256, device=DEV).to(BF))
+    q2, s2 = quantize_mx(torch.randn(256, 256, device=DEV).to(BF))
+    bad = s.t().contiguous().t(), s[:-1], s.float()
+    with torch.no_grad():
+        assert host.linear_eval(x, x, q, s) is not None
+        before = torch.cuda.memory_stats()["allocation.all.allocated"]
+        for scale in bad:
+            assert host.linear_forward(x, BF, q, scale, True) is None and host.linear_eval(x, x, q, scale) is None
+            assert host.group_forward(x, BF, [(q, scale, q, scale)], True) is None
+            assert host.swiglu_mlp_forward(x, BF, (q, scale), (q2, s2), False, False, False, 0) is None
+            assert host.linear_backward(x, BF, None, None, q[:, :256], scale, True, False, BF, BF) is None
+        assert torch.cuda.memory_stats()["allocation.all.allocated"] == before
+
+
+@pytest.mark.gpu
 @pytest.mark.parametrize("layout", ["flat", "batched", "pitched", "transposed"])
 @pytest.mark.parametrize("dtype", [BF, F16])
 def test_attention_and_norm(layout, dtype):
