@@ -984,12 +984,19 @@ PyObject *bind(PyObject *, PyObject *args) {
     Py_RETURN_NONE;
 }
 
+// (token_extent(tokens), padded_rows(rows, experts)): sizes that the Python functions compute as well.
+PyObject *py_extents(PyObject *, PyObject *args) {
+    long long tokens, rows, experts;
+    if (!PyArg_ParseTuple(args, "LLL", &tokens, &rows, &experts)) return nullptr;
+    return Py_BuildValue("(LL)", (long long)token_extent(tokens), (long long)padded_rows(rows, experts));
+}
+
 // Whether plain calls are made here at present.
 PyObject *py_engaged(PyObject *, PyObject *) { return PyBool_FromLong(engaged()); }
 
 #define ENTRY(name) {#name, (PyCFunction)(void (*)(void))entry<py_##name>, METH_FASTCALL, nullptr}
 PyMethodDef methods[] = {
-    {"bind", bind, METH_VARARGS, nullptr}, {"engaged", py_engaged, METH_NOARGS, nullptr},
+    {"bind", bind, METH_VARARGS, nullptr}, {"engaged", py_engaged, METH_NOARGS, nullptr}, {"extents", py_extents, METH_VARARGS, nullptr},
     ENTRY(quantize_rows), ENTRY(quantize_tokens), ENTRY(quantize_side), ENTRY(join_codes), ENTRY(quantize_dual_batch),
     ENTRY(swiglu_tokens), ENTRY(swiglu_bwd_tokens), ENTRY(matmul), ENTRY(matmul_batch),
     ENTRY(linear_forward), ENTRY(linear_backward), ENTRY(group_forward), ENTRY(swiglu_mlp_forward),
@@ -1010,6 +1017,9 @@ PyMODINIT_FUNC PyInit__host() {
     s_workspace = PyUnicode_InternFromString("gemm_workspace");
     s_workspaces = PyUnicode_InternFromString("_WORKSPACES");
     PyObject *module = PyModule_Create(&module_def);
-    if (module) PyModule_AddStringConstant(module, "torch_version", TORCH_VERSION);
+    if (!module || PyModule_AddStringConstant(module, "torch_version", TORCH_VERSION) ||
+        PyModule_AddObject(module, "constants", Py_BuildValue("{s:L,s:L,s:L,s:L,s:L}", "BLOCK_SCALE", (long long)BLOCK, "PANEL", (long long)PANEL, "TILE_ROWS",
+                                                              (long long)TILE_ROWS, "ROW_CHUNKS", (long long)ROW_CHUNKS, "SCALE_ROW_SLACK", (long long)SCALE_ROW_SLACK)))
+        return nullptr;
     return module;
 }

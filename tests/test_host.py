@@ -45,6 +45,17 @@ def test_calls_that_are_not_plain_are_declined():
         assert calls[0](x) is None
 
 
+def test_sizes_and_limits_are_those_of_the_python_functions():
+    from kohakuwullm_amd import _host
+    from kohakuwullm_amd.kernels.mxfp8 import grouped, quantize
+
+    assert _host.constants == {n: getattr(grouped if n == "SCALE_ROW_SLACK" else quantize, n) for n in _host.constants} and len(_host.constants) == 5
+    assert grouped.WGRAD_ROW_TILE == quantize.PANEL and grouped.TOKEN_PITCH_PAD == 0
+    for rows in (1, 31, 128, 129, 511, 513, 2048, 2049, 8065, 16384, 65535 * 128 - 1, 65535 * 128, 65535 * 128 + 1, 2**40 + 7):
+        for experts in (1, 64):
+            assert _host.extents(rows, rows, experts) == (quantize.token_extent(rows), grouped.padded_rows(rows, experts))
+
+
 def test_first_use_with_another_library_or_binding_installed():
     """Whatever stands in the binding when the extension is first used, it makes calls for the product library and the binding's own
     ``invoke`` alone."""
