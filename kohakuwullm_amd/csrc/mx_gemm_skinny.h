@@ -2,8 +2,8 @@
 //
 // Tiles of 128 columns leave most of the chip without a share of the weights (2048 -> 3072: 24 workgroups), and each walks all
 // of K alone.  Here a workgroup owns 16 columns -- one 16-column sub-tile of the MFMA -- and its eight waves take an eighth of
-// the K stages each.  A wave fetches several of its stages at once into LDS of its own, waits for its own copies only, and the
-// eight partial sums meet in LDS and are added in wave order: one memory round trip and one barrier for K up to 2048.
+// the K stages each.  A wave fetches U of its stages at once into LDS of its own and waits for its own copies only: one memory round
+// trip per 1024 U of K.  The eight partial sums meet in LDS, behind two barriers, and are added in wave order.
 // The copy engine brings the operands although no wave shares them: it fetches a row's 128 bytes with eight neighbouring lanes,
 // where loads straight into the MFMA's operand registers have 16 bytes of another row in every neighbouring lane, which the
 // texture path takes at about 12 B per clock (64 rows of A: 10 us of a 10 us launch).
