@@ -1,5 +1,6 @@
-"""The small-tile GEMM (csrc/mx_gemm_ring.h) against dequantize-then-matmul in fp64 at the edges of what it takes: single
-groups of four K stages, ragged and single rows, K slices, padded rows, stage-major operands, several products in a launch.
+"""The small-tile GEMM (csrc/mx_gemm_ring.h) and the one for few rows (csrc/mx_gemm_skinny.h) against dequantize-then-matmul in
+fp64 at the edges of what they take: single groups of four K stages, ragged and single rows, K slices, padded rows, stage-major
+operands, several products in a launch.
 
 Tolerances are those of the other GEMM tests: 1e-4 in fp32 (the block-scaled MFMA's own adder), 4e-3 in bf16 (its rounding)."""
 
@@ -32,6 +33,8 @@ def _dev(ops, panels=False):
     (1, 1, 512), (1, 3072, 2048), (127, 129, 512), (128, 128, 1024), (129, 257, 1536), (700, 260, 4096),
     (300, 520, 8192),  # 15 tiles, cut into eight K slices
     (16, 40, 16384), (130, 1000, 10240),  # slices of unequal length
+    # the shapes above with up to 128 rows go to the kernel for few rows; these of their kind do not
+    (129, 1, 512), (129, 3072, 2048), (255, 129, 512), (256, 128, 1024), (129, 40, 16384), (100, 1000, 10240), (128, 5000, 512),
 ])
 @pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16, torch.float16])
 def test_ring_gemm(oracle, m, n, k, dtype):
