@@ -73,6 +73,7 @@ def test_gemm_of_few_rows(oracle, m, n, k, dtype):
     (130, 300, 128), (257, 129, 256), (200, 264, 384),  # without a whole group
     (129, 1, 640), (129, 130, 768), (300, 40, 1408), (513, 260, 2176), (300, 257, 896), (256, 128, 1152),
     (129, 40, 8320), (130, 200, 16384 + 384),  # K slices whose last one ends inside a group
+    (130, 200, 14464), (130, 200, 14592), (130, 200, 14720),  # ... or is one to three stages alone
 ])
 @pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
 def test_ring_gemm_ends_inside_a_group(oracle, m, n, k, dtype):
