@@ -1062,10 +1062,10 @@ extern "C" int mx_gemm_nt_batch(const mx_gemm_problem *problems, int count, int 
 // Which activations are quantized inside the product: every workgroup does it again, which costs as much as the launch it saves
 // at 16 rows of a K of 4096 or at 32 of 2048.  us in two launches / in one, weights from HBM:
 //            512 -> 1536   2048 -> 3072   4096 -> 1536   1536 -> 8192
-//   M = 1     5.2 / 3.3      6.3 / 4.7      7.6 / 6.2      7.1 / 5.5
-//   8         5.4 / 3.8      6.6 / 5.1      7.7 / 6.7      7.3 / 6.0
-//   16        5.4 / 4.4      7.0 / 5.8      8.2 / 8.0      7.6 / 7.2
-//   32        5.6 / 4.4      7.8 / 7.7      9.5 / 11.0     8.9 / 10.2
+//   M = 1     5.2 / 3.3      6.3 / 4.2      7.6 / 5.4      7.1 / 5.4
+//   8         5.4 / 3.8      6.6 / 4.6      7.7 / 6.1      7.3 / 5.5
+//   16        5.4 / 4.3      7.0 / 5.1      8.2 / 6.9      7.6 / 6.4
+//   32        5.6 / 4.4      7.8 / 6.5      9.5 / 11.0     8.9 / 9.5
 static bool activation_rows_ok(int64_t M, int64_t K, int64_t columns) {
     return M <= 16 ? K <= 4096 : M <= 32 && K <= 2048 && columns <= SKINNY_N * num_cus();
 }
