@@ -1059,8 +1059,8 @@ extern "C" int mx_gemm_nt_batch(const mx_gemm_problem *problems, int count, int 
     return flush();
 }
 
-// Which activations are quantized inside the product: every workgroup does it again, which costs as much as the launch it saves
-// at 16 rows of a K of 4096 or at 32 of 2048.  us in two launches / in one, weights from HBM:
+// Which activations are quantized inside the product: every workgroup does it again, which with more rows or a longer K costs
+// more than the launch it saves.  us in two launches / in one, weights from HBM:
 //            512 -> 1536   2048 -> 3072   4096 -> 1536   1536 -> 8192
 //   M = 1     5.2 / 3.3      6.3 / 4.2      7.6 / 5.4      7.1 / 5.4
 //   8         5.4 / 3.8      6.6 / 4.6      7.7 / 6.1      7.3 / 5.5
