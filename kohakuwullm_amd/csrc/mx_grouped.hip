@@ -20,6 +20,7 @@
 #include <type_traits>
 
 #include "mx_gemm_core.h"
+#include "mx_gemm_stream.h"
 
 namespace mx {
 
@@ -884,6 +885,111 @@ __global__ __launch_bounds__(S::NTHR) __attribute__((amdgpu_waves_per_eu(2, 2)))
     grouped_body<S, MODE, CDT, K512>(args, smem);
 }
 
+// ---- PLAIN on the stream of K stages (mx_gemm_stream.h) -------------------------------------------
+#define MX_TABLE_MAX_STREAM 500  // experts its tables hold
+
+template <int CDT>
+struct GroupedStream {
+    typedef StreamShape S;
+    struct Tile {
+        int a, b, c, stages;  // first row, one past the expert's last row, first column, K stages
+        int expert;
+    };
+    const GroupedArgs p;
+    const int *tiles, *rows;  // row tiles of the experts before e, offsets[e], for e in [0, E] (LDS)
+    int next_id;
+
+    __device__ GroupedStream(const GroupedArgs &a, const int *tiles_, const int *rows_) : p(a), tiles(tiles_), rows(rows_), next_id(blockIdx.x) {}
+
+    __device__ __forceinline__ bool next(Tile &t) {
+        const int total = p.tiles_n * __builtin_amdgcn_readfirstlane(tiles[p.E]), per_xcd = total >> 3;
+        if (next_id >= total) return false;
+        int id = next_id;
+        next_id += gridDim.x;
+        if (id < (per_xcd << 3)) id = (id & 7) * per_xcd + (id >> 3);  // as in GroupedProblem::next
+        const int rt = id / p.tiles_n;
+        // the last expert whose first row tile is at or before rt, 64 experts at a time
+        int e = 0;
+        for (int e0 = 0; e0 < p.E; e0 += 64) {
+            const int lane = threadIdx.x & 63, first = e0 + lane < p.E ? tiles[e0 + lane] : 0x7FFFFFFF;
+            const uint64_t mask = __ballot(first <= rt);
+            e = e0 + __builtin_popcountll(mask) - 1;
+            if (~mask) break;
+        }
+        t.expert = __builtin_amdgcn_readfirstlane(e);
+        t.a = __builtin_amdgcn_readfirstlane(rows[t.expert] + (rt - tiles[t.expert]) * S::BM);
+        t.b = __builtin_amdgcn_readfirstlane(rows[t.expert + 1]);
+        t.c = (id - rt * p.tiles_n) * S::BN;
+        t.stages = p.K >> 7;
+        return true;
+    }
+
+    // Rows of A past the expert's last one are the next expert's (computed, never stored); none past the matrix is read.
+    __device__ __forceinline__ void feed(const Tile &t, int loader, int lane, StreamFeed &f) const {
+        f.a = uniform_ptr(p.xq + (int64_t)t.a * p.ldx - COPY_BIAS);
+        f.b = uniform_ptr(p.wq + (int64_t)t.expert * p.stride_we + (int64_t)t.c * p.ldw - COPY_BIAS);
+        const bool of_a = loader < S::BM / 64;
+        f.s = uniform_ptr(of_a ? p.xs + (int64_t)t.a * p.ldxs : p.ws + (int64_t)t.expert * p.stride_wse + (int64_t)t.c * p.ldws);
+        f.a_ks = f.b_ks = 128;
+        const int64_t a_rows = p.x_rows - t.a;
+        const int a_last = (int)(a_rows < S::BM ? a_rows : S::BM) - 1, b_last = (p.N - t.c < S::BN ? p.N - t.c : S::BN) - 1;
+        auto row = [](int r, int last) { return r < last ? r : last; };
+#pragma unroll
+        for (int q = 0; q < 4; q++) {
+            const int r = stream_row(loader, lane, q), chunk = ((lane & 7) ^ swz_a(r)) << 4;
+            f.a_voff[q] = (uint32_t)(row(r, a_last) * p.ldx) + chunk + copy_bias(q);
+            f.b_voff[q] = (uint32_t)(row(b_row_of_lds<S>(r), b_last) * p.ldw) + chunk + copy_bias(q);
+        }
+        const int r = (loader & 1) * 64 + lane;
+        f.s_voff = (uint32_t)(of_a ? row(r, a_last) * p.ldxs : row(b_row_of_lds<S>(r), b_last) * p.ldws);
+    }
+
+    // Neighbouring lanes swap half of every two rows, so that a lane stores 16 bytes of one row instead of 8 of two: a store costs the
+    // CU's one path to memory 12 clocks whatever it carries (32 KB in stores of 8 bytes a lane 760 clocks, of 16 bytes 415).  Without the
+    // hint the output displaces the operand panels in the L2 (16662 rows, K = 512 25.8 -> 23.3 us).
+    __device__ __forceinline__ void store(const Tile &t, const Lane &L0, v4f (&acc)[S::MT][S::NT]) const {
+        const Lane L = opaque(L0);
+        const bool odd = L.lane & 1;
+        const int row = t.a + L.wm * S::WTM + 4 * (L.lane >> 4) + (odd ? 1 : 0), n = t.c + L.wn * S::WTN + 8 * ((L.lane & 15) >> 1);
+        const int rows = n < p.N ? t.b - row : 0;  // N % 8 == 0: a lane's run is inside or outside
+        uint16_t *const at = (uint16_t *)p.out + (int64_t)row * p.ldo + n;
+#pragma unroll
+        for (int i = 0; i < S::MT; i++)
+#pragma unroll
+            for (int v = 0; v < 4; v += 2) {
+                uint32_t own[2][2];
+#pragma unroll
+                for (int r = 0; r < 2; r++)
+#pragma unroll
+                    for (int h = 0; h < 2; h++) {
+                        float lo = acc[i][2 * h][v + r], hi = acc[i][2 * h + 1][v + r];
+                        round_pair<CDT>(lo, hi, own[r][h]);
+                    }
+                v4i w;
+#pragma unroll
+                for (int h = 0; h < 2; h++) {
+                    const int other = __builtin_amdgcn_mov_dpp((int)(odd ? own[0][h] : own[1][h]), 0xB1, 0xF, 0xF, true);  // lane ^ 1
+                    w[h] = odd ? other : (int)own[0][h];
+                    w[2 + h] = odd ? (int)own[1][h] : other;
+                }
+                if (16 * i + v < rows) stream_store<true>((v4i *)(at + (int64_t)(16 * i + v) * p.ldo), w);
+            }
+    }
+};
+
+template <int CDT>
+__global__ __launch_bounds__(STREAM_THREADS) void grouped_stream_kernel(GroupedArgs args) {
+    extern __shared__ __attribute__((aligned(1024))) uint8_t smem[];
+    __shared__ int tiles[MX_TABLE_MAX_STREAM + 1], rows[MX_TABLE_MAX_STREAM + 1];
+    build_row_tile_table(tiles, rows, args.offsets, args.E, StreamShape::BM);
+    for (int e = threadIdx.x; e <= args.E; e += STREAM_THREADS) rows[e] = args.offsets[e];
+    __syncthreads();
+    GroupedStream<CDT> prob(args, tiles, rows);
+    const int loader = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6) - StreamShape::NW;
+    if (loader < 0) stream_multiply(prob, smem);
+    else stream_load(prob, smem, loader);
+}
+
 // Slow path for shapes the tiled kernel does not take (PLAIN only): one thread per output element.
 template <int CDT>
 __global__ __launch_bounds__(256) void grouped_generic_kernel(GroupedArgs p) {
@@ -1363,8 +1469,41 @@ static int launch_grouped_shape(GroupedArgs a, hipStream_t st) {
     return hipGetLastError() == hipSuccess ? MX_OK : MX_ELAUNCH;
 }
 
+template <int CDT>
+static int launch_grouped_stream(GroupedArgs a, hipStream_t st) {
+    typedef StreamShape S;
+    a.tiles_n = (a.N + S::BN - 1) / S::BN;
+    a.tbound = (a.M + S::BM - 1) / S::BM + a.E;
+    const int64_t work = (int64_t)a.tiles_n * a.tbound;
+    if (work >= 0x7FFFFFFF) return MX_EUNSUPPORTED;
+    const int rc = launch_with_lds<grouped_stream_kernel<CDT>>(dim3((unsigned)(work < num_cus() ? work : num_cus())), dim3(STREAM_THREADS),
+                                                               STREAM_LDS_BYTES, st, a);
+    if (rc != MX_OK) return rc;
+    return hipGetLastError() == hipSuccess ? MX_OK : MX_ELAUNCH;
+}
+
+// Whether the plain product runs as a stream of K stages on 128 x 128 tiles: rows that are not gathered, whole groups of four stages,
+// 16-byte output runs, and up to six tiles per CU.  Few rows per expert fill 256 x 256 tiles to a fraction, and a few rounds of
+// large tiles end in a partial one; from there on twice the operand bytes per flop cost more than the stores under the K loops save.
+// us on the other shapes / here, 64 experts of 1024 columns, operands from HBM, by rows in all:
+//              1000          3000         8000          16662         33000        50000        98304
+//   K = 512   11.8 / 11.4  13.6 / 12.7  18.9 / 17.1  29.0 / 23.3  39.3 / 38.2  50.7 / 55.1  85.6 / 102.4
+//   K = 1024  19.8 / 17.8  21.6 / 19.0  27.4 / 26.0  43.5 / 36.5  59.1 / 59.5  76.2 / 83.5   131 / 155
+// (on another box 19.8 / 21.3 and 21.6 / 21.7 where this says 17.8 and 19.0, the rest within 4 %);
+// of 8 experts 8.1 / 6.3 and 11.1 / 7.6 (1000 rows), 23.7 / 16.7 and 35.0 / 23.8 (16662); of 32 experts 16.7 / 11.2 and 23.9 / 21.9 (8000).
+static bool stream_pays(const GroupedArgs &a) {
+    const int64_t limit = (int64_t)1 << 31;
+    if (a.index || a.K % 512 || (int64_t)a.N * a.K > (2 << 20) || !a.out_vec || a.N % 8 || a.E > MX_TABLE_MAX_STREAM || a.x_rows < a.M || 128 * a.ldx >= limit ||
+        128 * a.ldw >= limit || 128 * a.ldxs >= limit || 128 * a.ldws >= limit)
+        return false;
+    const double live = a.E < a.M ? a.E : a.M, rows = (double)a.M / StreamShape::BM + 0.5 * live;
+    return (rows > live ? rows : live) * ((a.N + StreamShape::BN - 1) / StreamShape::BN) <= 6.0 * num_cus();
+}
+
 template <int MODE, int CDT>
 static int launch_grouped(const GroupedArgs &a, hipStream_t st) {
+    if constexpr (MODE == MODE_PLAIN && CDT != MX_FP32)
+        if (stream_pays(a) && !MX_EXPERT_OTHER) return launch_grouped_stream<CDT>(a, st);
     if constexpr (MODE != MODE_SCATTER)
         if (slim_pays<MODE>(a) != MX_EXPERT_OTHER) return launch_grouped_shape<Slim, MODE, CDT>(a, st);
     return launch_grouped_shape<Big, MODE, CDT>(a, st);

@@ -122,6 +122,35 @@ def test_grouped_gemm_look_ahead_schedule(oracle, k, use_index, counts, n):
     assert oracle.rel_error(got32.cpu(), ref) < 1e-4
 
 
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("k, n, counts", [
+    (512, 8, [1]),  # one tile, one group of stages
+    (512, 136, [0, 127, 128, 129, 0, 1]),  # ends of row and column tiles, experts without rows
+    (1536, 1000, [300, 0, 77, 256, 640]),  # three groups per tile
+    (1024, 1024, [1] * 70 + [0] * 30 + [200] * 12),  # several tiles per workgroup, more than 64 experts
+])
+def test_grouped_gemm_stream_of_stages(oracle, k, n, counts, dtype):
+    """Rows in expert order, K a multiple of 512: the kernel whose loader waves run through tile boundaries.  Against the
+    oracle; bit for bit against the same product with its rows gathered by an identity index, which the other kernels take;
+    and rows behind the last expert are neither read from past the matrix nor written."""
+    from kohakuwullm_amd.kernels.mxfp8.grouped import grouped_mxfp8_gemm
+    from kohakuwullm_amd.kernels.mxfp8.quantize import quantize_mx
+
+    g = torch.Generator().manual_seed(SEED + 31)
+    e, m, spare = len(counts), sum(counts), 5
+    xq, xs = quantize_mx(torch.randn(m + spare, k, generator=g).to(DEV, dtype))
+    wq, ws = quantize_mx((torch.randn(e * n, k, generator=g) * 0.05).to(DEV, dtype))
+    wq, ws = wq.view(e, n, k), ws.view(e, n, k // 32)
+    offsets = torch.zeros(e + 1, dtype=torch.int32)
+    offsets[1:] = torch.tensor(counts).cumsum(0)
+    got, other = (torch.full((m + spare, n), 7.0, device=DEV, dtype=dtype) for _ in range(2))
+    grouped_mxfp8_gemm(xq, xs, wq, ws, offsets.to(DEV), out=got, out_dtype=dtype)
+    grouped_mxfp8_gemm(xq, xs, wq, ws, offsets.to(DEV), torch.arange(m + spare, device=DEV, dtype=torch.int32), out=other, out_dtype=dtype)
+    assert torch.equal(got.view(torch.int16), other.view(torch.int16)) and bool((got[m:] == 7.0).all())
+    ref = oracle.grouped_gemm_nt(xq.view(torch.uint8).cpu(), xs.cpu(), wq.view(torch.uint8).cpu(), ws.cpu(), offsets)
+    assert oracle.rel_error(got[:m].cpu(), ref[:m]) < TOL
+
+
 def test_grouped_gemm_sentinel_rows_untouched_and_errors(oracle):
     from kohakuwullm_amd.kernels.mxfp8.grouped import grouped_mxfp8_gemm
 
