@@ -25,8 +25,9 @@ constexpr int STREAM_LOADERS = 4;
 constexpr int STREAM_THREADS = StreamShape::NTHR + 64 * STREAM_LOADERS;
 constexpr int STREAM_SLOTS = 4;
 constexpr int STREAM_SLOT_BYTES = StreamShape::DATA_A + StreamShape::DATA_B;
+constexpr int STREAM_SCALES = STREAM_SLOTS * STREAM_SLOT_BYTES;               // where four buffers of scale bytes begin
 constexpr int STREAM_SCALE_BYTES = 16 * (StreamShape::BM + StreamShape::BN);  // of a group of four stages
-constexpr int STREAM_TILES = STREAM_SLOTS * STREAM_SLOT_BYTES + 2 * STREAM_SCALE_BYTES;  // where the tiles under way are described
+constexpr int STREAM_TILES = STREAM_SCALES + 4 * STREAM_SCALE_BYTES;          // where the tiles under way are described
 constexpr int STREAM_LDS_BYTES = STREAM_TILES + 4 * 16;
 
 // What a loader wave's next copies read: wave-uniform bases (biased, see dma16_run2) and the lane's offsets from them, for the four
@@ -40,8 +41,13 @@ struct StreamFeed {
 // LDS row, in the tile image of A or of B, of this lane's 16-byte chunk of a loader's copy q.
 __device__ __forceinline__ int stream_row(int loader, int lane, int q) { return (loader * 4 + q) * 8 + (lane >> 3); }
 
-// The loader waves.  `P` provides Tile (four integers, the last one its stages, whole groups of four), next(Tile &) and
-// feed(Tile, loader, lane, StreamFeed &).
+// Both sides take a tile in an even number of steps, a step per stage and, behind an odd number of stages, an idle one, which
+// fetches the last stage again and multiplies nothing: the fragments of a step are read into the one of two register sets that its
+// parity names.  Step n uses slot n % 4.  Tiles have two steps at least, so the fetches of the next four steps reach into three
+// groups of scale bytes at most, beside the one being multiplied: four buffers.
+
+// The loader waves.  `P` provides Tile (four integers, the last one its stages), next(Tile &) and feed(Tile, loader, lane,
+// StreamFeed &).
 template <typename P>
 __device__ __forceinline__ void stream_load(P &prob, uint8_t *smem, int loader) {
     typedef StreamShape S;
@@ -50,78 +56,71 @@ __device__ __forceinline__ void stream_load(P &prob, uint8_t *smem, int loader) 
     typename P::Tile t;
     StreamFeed f;
     const uint32_t copy_to = __builtin_amdgcn_readfirstlane(lds_addr(smem) + loader * 4096);
-    const uint32_t s_to = __builtin_amdgcn_readfirstlane(lds_addr(smem) + STREAM_SLOTS * STREAM_SLOT_BYTES + loader * 1024);
-    int buf = 0, number = 0, left = 0;  // scale buffer, tiles so far, stages of the tile still to fetch
-    auto advance = [&]() -> bool {
-        if (left) return true;
-        const bool more = prob.next(t);
-        if (loader == 0 && lane == 0) *(v4i *)(smem + STREAM_TILES + 16 * (number & 3)) = v4i{t.a, t.b, t.c, more ? t.stages : 0};
-        number++;
-        if (!more) return false;
-        prob.feed(t, loader, lane, f);
-        left = t.stages;
-        return true;
-    };
-    auto fetch = [&](auto sc) {  // stage sc of a group
-        constexpr int s = sc.value;
-        if constexpr (s == 0) {
+    const uint32_t s_to = __builtin_amdgcn_readfirstlane(lds_addr(smem) + STREAM_SCALES + loader * 1024);
+    int slot = 0, buf = 0, number = 0;  // bytes: the next step's slot, the next group's scale buffer; tiles so far
+    int at = 0, steps = 0, total = 0;   // steps fetched and to fetch of the tile; of all tiles so far
+    bool more = true;
+    auto fetch = [&]() {  // the next step; with no tile left, what the last one fetched
+        if (at == steps && more) {
+            more = prob.next(t);
+            if (loader == 0 && lane == 0) *(v4i *)(smem + STREAM_TILES + 16 * (number & 3)) = v4i{t.a, t.b, t.c, more ? t.stages : 0};
+            number++;
+            if (more) {
+                prob.feed(t, loader, lane, f);
+                at = 0, steps = (t.stages + 1) & ~1;
+                total += steps;
+            }
+        }
+        if (!total) return;  // a workgroup without tiles has nothing to fetch from
+        if ((at & 3) == 0 && at < steps) {
             dma16(f.s, f.s_voff, s_to + buf);
             f.s += 16;
-            buf ^= STREAM_SCALE_BYTES;
-            left -= 4;
+            buf = (buf + STREAM_SCALE_BYTES) & (4 * STREAM_SCALE_BYTES - 1);
         }
-        dma16_run4(f.a, f.a_voff[0], f.a_voff[1], f.a_voff[2], f.a_voff[3], copy_to + s * STREAM_SLOT_BYTES);
-        dma16_run4(f.b, f.b_voff[0], f.b_voff[1], f.b_voff[2], f.b_voff[3], copy_to + s * STREAM_SLOT_BYTES + S::DATA_A);
-        f.a += f.a_ks, f.b += f.b_ks;
+        dma16_run4(f.a, f.a_voff[0], f.a_voff[1], f.a_voff[2], f.a_voff[3], copy_to + slot);
+        dma16_run4(f.b, f.b_voff[0], f.b_voff[1], f.b_voff[2], f.b_voff[3], copy_to + slot + S::DATA_A);
+        slot = (slot + STREAM_SLOT_BYTES) & (STREAM_SLOTS * STREAM_SLOT_BYTES - 1);
+        if (at < steps) at++;
+        if (at < t.stages) f.a += f.a_ks, f.b += f.b_ks;
     };
-    if (!advance()) return;
-    static_for<4>([&](auto s) { fetch(s); });
-    wait_vm_allow_c<3 * OPS>();
-    __syncthreads();
-    // Group after group, one behind the fetches: at stage s the next stage has landed, and stage s of the next group goes out into
-    // the slot of the stage that is being multiplied, whose fragments every wave has.
-    while (advance()) {
-        static_for<4>([&](auto s) {
-            wait_vm_allow_c<2 * OPS>();
-            __syncthreads();
-            fetch(s);
-        });
+#pragma unroll 1
+    for (int s = 0; s < STREAM_SLOTS; s++) {
+        fetch();
+        if (!total) return;  // the multiplying waves have no tile either and have left
     }
-    static_for<4>([&](auto s) {
-        wait_vm_allow_c<(s.value < 2 ? 2 - s.value : 0) * OPS>();
+    wait_vm_allow_c<(STREAM_SLOTS - 1) * OPS>();
+    __syncthreads();
+    // Four steps behind the fetches: at a step the next one has landed, and the one four on goes out into the slot of the one that
+    // is being multiplied, whose fragments every wave has.
+    for (int step = 0; more || step < total; step++) {
+        wait_vm_allow_c<(STREAM_SLOTS - 2) * OPS>();
         __syncthreads();
-    });
+        fetch();
+    }
+    wait_vm_allow_c<0>();  // copies that no step waited for must not land in the next workgroup's LDS
 }
 
-// The multiplying waves.  `P` provides store(Tile, Lane, acc).
+// The multiplying waves.  `P` provides store(Tile, Lane, acc) and WHOLE, whether every tile is in whole groups of four stages.
 template <typename P>
 __device__ __forceinline__ void stream_multiply(P &prob, uint8_t *smem) {
     typedef StreamShape S;
-    constexpr int SLOT_BYTES = STREAM_SLOT_BYTES, SCALES = STREAM_SLOTS * STREAM_SLOT_BYTES;
+    constexpr int SLOT_BYTES = STREAM_SLOT_BYTES;
     const Lane L = lane_of<S>();
     typename P::Tile t;
     if (!prob.next(t)) return;
-    // LDS read bases: slots 0 and 1 within the 16-bit offset of an LDS read, slots 2 and 3 from a second set 64 KB on
     const int a_row = L.wm * S::WTM + L.r16, b_row = L.wn * S::WTN + L.r16;
     const int a_at = a_row * 128 + ((L.g ^ swz_a(a_row)) << 4), b_at = S::DATA_A + b_row * 128 + ((L.g ^ swz_a(b_row)) << 4);
-    const uint8_t *a_rd[2][2], *b_rd[2][2];
-#pragma unroll
-    for (int half = 0; half < 2; half++) {
-        const uint8_t *const base = smem + half * 2 * SLOT_BYTES;
-        a_rd[half][0] = base + a_at, a_rd[half][1] = base + (a_at ^ 64);
-        b_rd[half][0] = base + b_at, b_rd[half][1] = base + (b_at ^ 64);
-    }
-    const uint8_t *const sa_rd = smem + SCALES + a_row * 16 + L.g, *const sb_rd = smem + SCALES + (S::BM + b_row) * 16 + L.g;
+    const uint8_t *const a_rd[2] = {smem + a_at, smem + (a_at ^ 64)}, *const b_rd[2] = {smem + b_at, smem + (b_at ^ 64)};
+    const uint8_t *const sa_rd = smem + STREAM_SCALES + a_row * 16 + L.g, *const sb_rd = smem + STREAM_SCALES + (S::BM + b_row) * 16 + L.g;
     struct Frags {
         v8i a[S::MT], b[S::NT];
         int sa[S::MT], sb[S::NT];
     } fr[2];
-    auto read_fragment = [&](auto slot, auto which, Frags &to) {  // A rows first, then B rows
-        constexpr int off = (slot.value & 1) * SLOT_BYTES, half = slot.value >> 1;
+    auto read_fragment = [&](int slot, auto which, Frags &to) {  // A rows first, then B rows
         constexpr bool A = which.value < S::MT;
         constexpr int i = A ? which.value : which.value - S::MT;
-        const uint8_t *const(&at)[2] = A ? a_rd[half] : b_rd[half];
-        const v4i lo = *(const v4i *)(at[0] + off + i * 2048), hi = *(const v4i *)(at[1] + off + i * 2048);
+        const uint8_t *const(&at)[2] = A ? a_rd : b_rd;
+        const v4i lo = *(const v4i *)(at[0] + slot + i * 2048), hi = *(const v4i *)(at[1] + slot + i * 2048);
         (A ? to.a[A ? i : 0] : to.b[A ? 0 : i]) = __builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7);
     };
     auto read_scales = [&](int at, Frags &to) {
@@ -132,26 +131,28 @@ __device__ __forceinline__ void stream_multiply(P &prob, uint8_t *smem) {
     };
 
     v4f acc[S::MT][S::NT];
-    int buf = 0, number = 0;  // where the scale bytes of the current group lie, tiles so far
+    int half = 0, scales = 0, number = 0;  // bytes: the even step's slot, the current group's scale bytes; tiles so far
+    auto next_group = [&]() { return (scales + STREAM_SCALE_BYTES) & (4 * STREAM_SCALE_BYTES - 1); };
     __syncthreads();
-    static_for<S::MT + S::NT>([&](auto w) { read_fragment(std::integral_constant<int, 0>{}, w, fr[0]); });
+    static_for<S::MT + S::NT>([&](auto w) { read_fragment(0, w, fr[0]); });
     read_scales(0, fr[0]);
 
-    // Stage s of a group: its fragments are in fr[s & 1], the next stage's are read into the other set.
-    auto stage = [&](auto sc) {
-        constexpr int s = sc.value;
-        typedef std::integral_constant<int, (s + 1) & 3> after;
-        Frags &now = fr[s & 1], &then = fr[(s + 1) & 1];
-        const int scales = (s == 3 ? buf ^ STREAM_SCALE_BYTES : buf) + 4 * after::value;
-        __syncthreads();  // this stage's fragments are in registers: its slot may be filled again, and the next stage has landed
-        static_for<S::MT * S::NT>([&](auto step) {
-            constexpr int i = step.value % S::MT, j = step.value / S::MT;
-            acc[i][j] = __builtin_amdgcn_mfma_scale_f32_16x16x128_f8f6f4(now.a[i], now.b[j], acc[i][j], 0, 0, 0, now.sa[i], 0, now.sb[j]);
-            if constexpr (step.value < S::MT + S::NT) read_fragment(after{}, step, then);
-            if constexpr (step.value == S::MT + S::NT) read_scales(scales, then);
-            __builtin_amdgcn_sched_barrier(0);
-        });
-        if constexpr (s == 3) buf ^= STREAM_SCALE_BYTES;
+    // One step, even or odd: its fragments are in fr[odd], the next step's are read into the other set.
+    auto step = [&](auto odd, int next_slot, int next_scales, bool live) {
+        Frags &now = fr[odd.value], &then = fr[odd.value ^ 1];
+        __syncthreads();  // this step's fragments are in registers: its slot may be filled again; the next step has landed
+        if (live) {
+            static_for<S::MT * S::NT>([&](auto at) {
+                constexpr int i = at.value % S::MT, j = at.value / S::MT;
+                acc[i][j] = __builtin_amdgcn_mfma_scale_f32_16x16x128_f8f6f4(now.a[i], now.b[j], acc[i][j], 0, 0, 0, now.sa[i], 0, now.sb[j]);
+                if constexpr (at.value < S::MT + S::NT) read_fragment(next_slot, at, then);
+                if constexpr (at.value == S::MT + S::NT) read_scales(next_scales, then);
+                __builtin_amdgcn_sched_barrier(0);
+            });
+        } else {
+            static_for<S::MT + S::NT>([&](auto w) { read_fragment(next_slot, w, then); });
+            read_scales(next_scales, then);
+        }
 #pragma unroll
         for (int i = 0; i < S::MT; i++)
 #pragma unroll
@@ -163,7 +164,27 @@ __device__ __forceinline__ void stream_multiply(P &prob, uint8_t *smem) {
         for (int i = 0; i < S::MT; i++)
 #pragma unroll
             for (int j = 0; j < S::NT; j++) acc[i][j] = v4f{0.f, 0.f, 0.f, 0.f};
-        for (int left = stages; left; left -= 4) static_for<4>([&](auto s) { stage(s); });
+        typedef std::integral_constant<int, 0> even;
+        typedef std::integral_constant<int, 1> odd;
+        if constexpr (P::WHOLE) {  // whole groups begin with slot 0: slots are constants
+            for (int k = 0; k < stages; k += 4) {
+                step(even{}, SLOT_BYTES, scales + 4, true);
+                step(odd{}, 2 * SLOT_BYTES, scales + 8, true);
+                step(even{}, 3 * SLOT_BYTES, scales + 12, true);
+                scales = next_group();
+                step(odd{}, 0, scales, true);
+            }
+        } else {
+            for (int k = 0; k < stages; k += 2) {
+                step(even{}, half + SLOT_BYTES, scales + 4 * (k & 3) + 4, true);
+                // behind the odd step comes the group's second half, the next group's first stage, or the next tile's
+                const bool ends = (k & 2) || k + 2 >= stages;
+                const int from = ends ? next_group() : scales;
+                half ^= 2 * SLOT_BYTES;
+                step(odd{}, half, ends ? from : scales + 8, k + 1 < stages);
+                scales = from;
+            }
+        }
         prob.store(t, L, acc);
         // the next tile, as the loaders described it when they began to fetch it
         number++;
@@ -171,6 +192,54 @@ __device__ __forceinline__ void stream_multiply(P &prob, uint8_t *smem) {
         t.a = __builtin_amdgcn_readfirstlane(d[0]), t.b = __builtin_amdgcn_readfirstlane(d[1]), t.c = __builtin_amdgcn_readfirstlane(d[2]);
         stages = t.stages = __builtin_amdgcn_readfirstlane(d[3]);
     } while (stages);
+}
+
+// Stores a tile's rows [row0, row_end) and columns [col0, col_end) of a matrix: 16-byte runs (col_end % 8 == 0, fp32: % 4; rows on
+// 16 bytes).  With 16-bit results neighbouring lanes swap half of every two rows, so that a lane stores 16 bytes of one row instead
+// of 8 of two: a store costs the CU's one path to memory 12 clocks whatever it carries (32 KB in stores of 8 bytes a lane 760 clocks,
+// of 16 bytes 415).  The hint: without it the output displaces the operand panels in the L2 (GEMM2 of 16662 rows 25.8 -> 23.3 us).
+template <int CDT>
+__device__ __forceinline__ void stream_store_tile(void *out, int64_t ld, int row0, int row_end, int col0, int col_end, const Lane &L0,
+                                                  v4f (&acc)[StreamShape::MT][StreamShape::NT]) {
+    typedef StreamShape S;
+    static_assert(S::NT == 4, "four consecutive columns per lane");
+    const Lane L = opaque(L0);
+    if constexpr (CDT == MX_FP32) {
+        const int row = row0 + L.wm * S::WTM + 4 * (L.lane >> 4), col = col0 + L.wn * S::WTN + 4 * (L.lane & 15);
+        const int rows = col < col_end ? row_end - row : 0;
+        float *const at = (float *)out + (int64_t)row * ld + col;
+#pragma unroll
+        for (int i = 0; i < S::MT; i++)
+#pragma unroll
+            for (int v = 0; v < 4; v++)
+                if (16 * i + v < rows)
+                    stream_store<true>((v4f *)(at + (int64_t)(16 * i + v) * ld), v4f{acc[i][0][v], acc[i][1][v], acc[i][2][v], acc[i][3][v]});
+    } else {
+        const bool odd = L.lane & 1;
+        const int row = row0 + L.wm * S::WTM + 4 * (L.lane >> 4) + (odd ? 1 : 0), col = col0 + L.wn * S::WTN + 8 * ((L.lane & 15) >> 1);
+        const int rows = col < col_end ? row_end - row : 0;
+        uint16_t *const at = (uint16_t *)out + (int64_t)row * ld + col;
+        auto pack = [](float lo, float hi) -> uint32_t {
+            if (CDT == MX_BF16) return pack2_bf16(lo, hi);
+            typedef _Float16 h2 __attribute__((ext_vector_type(2)));
+            const h2 h = {(_Float16)lo, (_Float16)hi};
+            return __builtin_bit_cast(uint32_t, h);
+        };
+#pragma unroll
+        for (int i = 0; i < S::MT; i++)
+#pragma unroll
+            for (int v = 0; v < 4; v += 2) {
+                v4i w;
+#pragma unroll
+                for (int h = 0; h < 2; h++) {
+                    const int first = (int)pack(acc[i][2 * h][v], acc[i][2 * h + 1][v]), second = (int)pack(acc[i][2 * h][v + 1], acc[i][2 * h + 1][v + 1]);
+                    const int other = __builtin_amdgcn_mov_dpp(odd ? first : second, 0xB1, 0xF, 0xF, true);  // lane ^ 1
+                    w[h] = odd ? other : first;
+                    w[2 + h] = odd ? second : other;
+                }
+                if (16 * i + v < rows) stream_store<true>((v4i *)(at + (int64_t)(16 * i + v) * ld), w);
+            }
+    }
 }
 
 }  // namespace mx

@@ -891,6 +891,7 @@ __global__ __launch_bounds__(S::NTHR) __attribute__((amdgpu_waves_per_eu(2, 2)))
 template <int CDT>
 struct GroupedStream {
     typedef StreamShape S;
+    static constexpr bool WHOLE = true;
     struct Tile {
         int a, b, c, stages;  // first row, one past the expert's last row, first column, K stages
         int expert;
@@ -944,36 +945,8 @@ struct GroupedStream {
         f.s_voff = (uint32_t)(of_a ? row(r, a_last) * p.ldxs : row(b_row_of_lds<S>(r), b_last) * p.ldws);
     }
 
-    // Neighbouring lanes swap half of every two rows, so that a lane stores 16 bytes of one row instead of 8 of two: a store costs the
-    // CU's one path to memory 12 clocks whatever it carries (32 KB in stores of 8 bytes a lane 760 clocks, of 16 bytes 415).  Without the
-    // hint the output displaces the operand panels in the L2 (16662 rows, K = 512 25.8 -> 23.3 us).
-    __device__ __forceinline__ void store(const Tile &t, const Lane &L0, v4f (&acc)[S::MT][S::NT]) const {
-        const Lane L = opaque(L0);
-        const bool odd = L.lane & 1;
-        const int row = t.a + L.wm * S::WTM + 4 * (L.lane >> 4) + (odd ? 1 : 0), n = t.c + L.wn * S::WTN + 8 * ((L.lane & 15) >> 1);
-        const int rows = n < p.N ? t.b - row : 0;  // N % 8 == 0: a lane's run is inside or outside
-        uint16_t *const at = (uint16_t *)p.out + (int64_t)row * p.ldo + n;
-#pragma unroll
-        for (int i = 0; i < S::MT; i++)
-#pragma unroll
-            for (int v = 0; v < 4; v += 2) {
-                uint32_t own[2][2];
-#pragma unroll
-                for (int r = 0; r < 2; r++)
-#pragma unroll
-                    for (int h = 0; h < 2; h++) {
-                        float lo = acc[i][2 * h][v + r], hi = acc[i][2 * h + 1][v + r];
-                        round_pair<CDT>(lo, hi, own[r][h]);
-                    }
-                v4i w;
-#pragma unroll
-                for (int h = 0; h < 2; h++) {
-                    const int other = __builtin_amdgcn_mov_dpp((int)(odd ? own[0][h] : own[1][h]), 0xB1, 0xF, 0xF, true);  // lane ^ 1
-                    w[h] = odd ? other : (int)own[0][h];
-                    w[2 + h] = odd ? (int)own[1][h] : other;
-                }
-                if (16 * i + v < rows) stream_store<true>((v4i *)(at + (int64_t)(16 * i + v) * p.ldo), w);
-            }
+    __device__ __forceinline__ void store(const Tile &t, const Lane &L, v4f (&acc)[S::MT][S::NT]) const {
+        stream_store_tile<CDT>(p.out, p.ldo, t.a, t.b, t.c, p.N, L, acc);
     }
 };
 
@@ -1270,6 +1243,75 @@ struct WgradProblem {
     }
 };
 
+// The same units on the stream of K stages (mx_gemm_stream.h), for experts of few stages: whole 16-byte runs, scale rows with 12
+// readable bytes behind their last stage.
+template <int CDT, typename TB>
+struct WgradStream {
+    typedef StreamShape S;
+    static constexpr bool WHOLE = false;
+    struct Tile {
+        int a, b, c, stages;  // first row and column; the expert, or ~slot of a K slice
+        int kt0;
+    };
+    WgradProblem<S, CDT, TB> units;
+    const WgradArgs &p;
+    bool clamped = true;  // the lane offsets are those of a tile that reaches past a matrix (or of none yet)
+
+    __device__ WgradStream(const WgradArgs &args, const TB *table) : units(args, table), p(args) {}
+
+    __device__ __forceinline__ bool next(Tile &t) {
+        typename WgradProblem<S, CDT, TB>::Tile u;
+        if (!__builtin_amdgcn_readfirstlane((int)units.next(u))) return false;
+        auto same = [](int v) { return __builtin_amdgcn_readfirstlane(v); };  // the table's entries reach every lane alike
+        t = {same(u.m0), same(u.n0), same(u.slot >= 0 ? ~u.slot : u.expert), same(u.kt1 - u.kt0), same(u.kt0)};
+        return true;
+    }
+
+    __device__ __forceinline__ void feed(const Tile &t, int loader, int lane, StreamFeed &f) {
+        f.a_ks = p.a_ks ? p.a_ks : 128, f.b_ks = p.b_ks ? p.b_ks : 128;
+        f.a = uniform_ptr(p.aq + (int64_t)t.a * p.lda + t.kt0 * f.a_ks - COPY_BIAS);
+        f.b = uniform_ptr(p.bq + (int64_t)t.b * p.ldb + t.kt0 * f.b_ks - COPY_BIAS);
+        const bool of_a = loader < S::BM / 64;
+        f.s = uniform_ptr((of_a ? p.as + (int64_t)t.a * p.ldas : p.bs + (int64_t)t.b * p.ldbs) + 4 * t.kt0);
+        const bool inside = t.a + S::BM <= p.N && t.b + S::BN <= p.Kout;
+        if (inside && !clamped) return;  // whole tiles have the same lane offsets
+        clamped = !inside;
+        const int a_last = (p.N - t.a < S::BM ? p.N - t.a : S::BM) - 1, b_last = (p.Kout - t.b < S::BN ? p.Kout - t.b : S::BN) - 1;
+        auto row = [](int r, int last) { return r < last ? r : last; };
+#pragma unroll
+        for (int q = 0; q < 4; q++) {
+            const int r = stream_row(loader, lane, q), chunk = ((lane & 7) ^ swz_a(r)) << 4;
+            f.a_voff[q] = (uint32_t)(row(r, a_last) * p.lda) + chunk + copy_bias(q);
+            f.b_voff[q] = (uint32_t)(row(b_row_of_lds<S>(r), b_last) * p.ldb) + chunk + copy_bias(q);
+        }
+        const int r = (loader & 1) * 64 + lane;
+        f.s_voff = (uint32_t)(of_a ? row(r, a_last) * p.ldas : row(b_row_of_lds<S>(r), b_last) * p.ldbs);
+    }
+
+    __device__ __forceinline__ void store(const Tile &t, const Lane &L, v4f (&acc)[S::MT][S::NT]) const {
+        if (t.c >= 0) {
+            stream_store_tile<CDT>((char *)p.dw + (int64_t)t.c * p.stride_dwe * (CDT == MX_FP32 ? 4 : 2), p.lddw, t.a, p.N, t.b, p.Kout, L, acc);
+            return;
+        }
+        v4f *const dst = (v4f *)p.ws + (int64_t)~t.c * (S::BM * S::BN / 4);  // one K slice: fp32 partial, laid out [sub-tile][thread]
+#pragma unroll
+        for (int i = 0; i < S::MT; i++)
+#pragma unroll
+            for (int j = 0; j < S::NT; j++) dst[(i * S::NT + j) * S::NTHR + L.tid] = acc[i][j];
+    }
+};
+
+template <int CDT>
+__global__ __launch_bounds__(STREAM_THREADS) void grouped_wgrad_stream_kernel(WgradArgs args) {
+    extern __shared__ __attribute__((aligned(1024))) uint8_t smem[];
+    __shared__ ExpertTable table;
+    build_live_table(table, args.offsets, args.E);
+    WgradStream<CDT, ExpertTable> prob(args, &table);
+    const int loader = __builtin_amdgcn_readfirstlane((int)threadIdx.x >> 6) - StreamShape::NW;
+    if (loader < 0) stream_multiply(prob, smem);
+    else stream_load(prob, smem, loader);
+}
+
 // 64 rows, from row m0 on, of the dW of expert e, which has no rows: zeros, a plain streaming fill.
 template <int CDT, int THREADS>
 __device__ __forceinline__ void wgrad_zero_rows(const WgradArgs &p, int e, int m0) {
@@ -1368,15 +1410,16 @@ __global__ __launch_bounds__(S::NTHR) void wgrad_finish_kernel(WgradArgs p, int 
                 for (int jj = 0; jj < S::NT; jj++) sum[jj] += src[(i * S::NT + jj) * S::NTHR + tid];
             }
         }
-        const int n = (rem % p.tiles_n) * S::BN + wn * S::WTN + 8 * (lane & 15);
+        const int n = (rem % p.tiles_n) * S::BN + wn * S::WTN + S::NT * (lane & 15);
 #pragma unroll
         for (int v = 0; v < 4; v++) {
             const int m = (rem / p.tiles_n) * S::BM + wm * S::WTM + 16 * i + 4 * (lane >> 4) + v;
             if (m < p.N && n < p.Kout) {
-                const v4f lo = {sum[0][v], sum[1][v], sum[2][v], sum[3][v]};
-                const v4f hi = {sum[4][v], sum[5][v], sum[6][v], sum[7][v]};
-                store8<CDT>(p.dw, (int64_t)e * p.stride_dwe + (int64_t)m * p.lddw + n, lo, hi, p.Kout - n < 8 ? p.Kout - n : 8,
-                            p.c_vec != 0);
+                float run[S::NT];
+#pragma unroll
+                for (int jj = 0; jj < S::NT; jj++) run[jj] = sum[jj][v];
+                store_run<CDT, S::NT>(p.dw, (int64_t)e * p.stride_dwe + (int64_t)m * p.lddw + n, run, p.Kout - n < S::NT ? p.Kout - n : S::NT,
+                                      p.c_vec != 0);
             }
         }
     }
@@ -1676,9 +1719,9 @@ extern "C" int mx_experts_combine_onto(const void *base, int64_t ldb, const void
     return hipGetLastError() == hipSuccess ? MX_OK : MX_ELAUNCH;
 }
 
-template <int CDT>
-static int launch_wgrad(WgradArgs a, float *ws, int64_t ws_bytes, hipStream_t st) {
-    typedef Big S;
+template <typename S, int CDT>
+static int launch_wgrad_shape(WgradArgs a, float *ws, int64_t ws_bytes, hipStream_t st) {
+    constexpr bool STREAM = std::is_same<S, StreamShape>::value;
     a.tiles_m = (a.N + S::BM - 1) / S::BM;
     a.tiles_n = (a.Kout + S::BN - 1) / S::BN;
     const int esz = CDT == MX_FP32 ? 4 : 2;
@@ -1702,7 +1745,10 @@ static int launch_wgrad(WgradArgs a, float *ws, int64_t ws_bytes, hipStream_t st
     const int chunks = (a.N + 63) / 64;
     if ((int64_t)a.E * chunks >= 0x7FFFFFFF) return MX_EUNSUPPORTED;
     const auto turn = scratch_turn(a.ws);
-    const int rc = staged ? launch_with_lds<grouped_wgrad_kernel<S, CDT, SCALES_COPY>>(grid, block, S::LDS_BYTES_AHEAD, st, a)
+    int rc;
+    if constexpr (STREAM) rc = launch_with_lds<grouped_wgrad_stream_kernel<CDT>>(grid, dim3(STREAM_THREADS), STREAM_LDS_BYTES, st, a);
+    else
+        rc = staged ? launch_with_lds<grouped_wgrad_kernel<S, CDT, SCALES_COPY>>(grid, block, S::LDS_BYTES_AHEAD, st, a)
                    : quad ? launch_with_lds<grouped_wgrad_kernel<S, CDT, SCALES_QUAD>>(grid, block, S::LDS_BYTES, st, a)
                           : launch_with_lds<grouped_wgrad_kernel<S, CDT, SCALES_DWORD>>(grid, block, S::LDS_BYTES, st, a);
     if (rc != MX_OK) return rc;
@@ -1711,6 +1757,31 @@ static int launch_wgrad(WgradArgs a, float *ws, int64_t ws_bytes, hipStream_t st
     const int64_t most = 4 * (int64_t)cus;
     wgrad_finish_kernel<S, CDT><<<dim3((unsigned)(units < most ? units : most)), block, 0, st>>>(a, (int)grid.x);
     return hipGetLastError() == hipSuccess ? MX_OK : MX_ELAUNCH;
+}
+
+// Whether an expert dW runs as a stream of K stages on 128 x 128 tiles: up to 56 stages per CU, from about a stage and a quarter per
+// expert on unless its tiles are few.  Large tiles of experts with one to four stages are mostly their stores, which nothing
+// overlaps, and of few experts they leave CUs idle; with more stages twice the operand bytes per flop cost more than that.
+// us on 256 x 256 / here, dW of 1024 x 1024 and of 512 x 1024, by rows in experts:
+//   12000 in 64   50.0 / 44.7   27.6 / 26.4        16662 on 6 of 64   73.4 / 58.3   49.9 / 32.2
+//   16662 in 64   57.2 / 51.2   33.9 / 29.6        22216 in 32        45.9 / 41.1   24.9 / 24.3
+//   24000 in 64   60.3 / 54.3   37.8 / 31.8         2777 in 4         33.6 / 11.3   32.1 / 21.1
+//   33000 in 64   69.0 / 71.0   41.5 / 38.0        72000 in 32        85.6 / 116    51.7 / 61.7
+//    4800 in 64   41.5 / 42.5   23.5 / 25.3        12000 in 16 of 256 x 256 and 128 x 256   29.1 / 20.9   28.6 / 19.4
+static bool wgrad_stream_pays(const WgradArgs &a, int64_t M, int esz) {
+    const int64_t limit = (int64_t)1 << 31;
+    if (a.E > MX_TABLE_MAX || !aligned(a.dw, 16) || (a.lddw * esz) % 16 || (a.stride_dwe * esz) % 16 || a.Kout % 8 || a.ldas < a.KB + 12 ||
+        a.ldbs < a.KB + 12 || 128 * a.ldas >= limit || 128 * a.ldbs >= limit)
+        return false;
+    const double live = a.E < M ? a.E : M, cus = num_cus();
+    const double tiles = (double)((a.N + StreamShape::BM - 1) / StreamShape::BM) * ((a.Kout + StreamShape::BN - 1) / StreamShape::BN);
+    return tiles * ((double)M / 128 + 0.5 * live) <= 56 * cus && (M >= 160 * live || tiles * live <= 4 * cus);
+}
+
+template <int CDT>
+static int launch_wgrad(const WgradArgs &a, int64_t M, float *ws, int64_t ws_bytes, hipStream_t st) {
+    if (wgrad_stream_pays(a, M, CDT == MX_FP32 ? 4 : 2)) return launch_wgrad_shape<StreamShape, CDT>(a, ws, ws_bytes, st);
+    return launch_wgrad_shape<Big, CDT>(a, ws, ws_bytes, st);
 }
 
 extern "C" int mx_grouped_wgrad_nt(const uint8_t *aq, const uint8_t *as, int64_t lda, int64_t ldas, const uint8_t *bq,
@@ -1737,9 +1808,9 @@ extern "C" int mx_grouped_wgrad_nt(const uint8_t *aq, const uint8_t *as, int64_t
     hipStream_t st = (hipStream_t)stream;
     if (mx::stream_is_capturing(st)) return MX_ECAPTURE;
     switch (dw_dtype) {
-    case MX_BF16: return launch_wgrad<MX_BF16>(a, (float *)workspace, workspace_bytes, st);
-    case MX_FP16: return launch_wgrad<MX_FP16>(a, (float *)workspace, workspace_bytes, st);
-    case MX_FP32: return launch_wgrad<MX_FP32>(a, (float *)workspace, workspace_bytes, st);
+    case MX_BF16: return launch_wgrad<MX_BF16>(a, M, (float *)workspace, workspace_bytes, st);
+    case MX_FP16: return launch_wgrad<MX_FP16>(a, M, (float *)workspace, workspace_bytes, st);
+    case MX_FP32: return launch_wgrad<MX_FP32>(a, M, (float *)workspace, workspace_bytes, st);
     default: return MX_EINVAL;
     }
 }

@@ -381,6 +381,39 @@ def test_wgrad_runs_of_single_stage_tiles(oracle, counts, n, k):
             assert oracle.rel_error(dw[i], ref) < TOL, (i, cnt)
 
 
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16, torch.float32])
+@pytest.mark.parametrize("counts,n,k", [
+    ([1, 128, 129, 0, 300, 513, 640], 200, 136),  # one to five stages, even and odd; edges of tiles both ways
+    ([200] * 40, 512, 256),  # several tiles per workgroup
+    ([2777], 256, 264),  # one long expert: K slices
+    ([0, 700, 0, 3000, 5], 128, 128),  # ranges of K slices that straddle experts; workgroups without any
+])
+def test_wgrad_stream_of_stages(oracle, counts, n, k, dtype):
+    """Few stages per CU: the kernel whose loader waves run through tile boundaries.  Every expert against fp64 on the same
+    codes, rounded once to the result's type.  fp32: the bound of the other fp32 products here; the matrix core aligns the 128
+    products of a step to the largest one, which leaves 1.6e-5 of a norm whichever kernel issues it."""
+    from kohakuwullm_amd.kernels.mxfp8.grouped import grouped_mxfp8_wgrad, quantize_mx_cols_grouped
+
+    g = torch.Generator().manual_seed(SEED + 32)
+    m = sum(counts)
+    offsets = torch.zeros(len(counts) + 1, dtype=torch.int32)
+    offsets[1:] = torch.tensor(counts).cumsum(0)
+    a = (torch.randn(m, n, generator=g) * 1e-2).bfloat16()
+    b = torch.randn(m, k, generator=g).bfloat16()
+    atq, ats = quantize_mx_cols_grouped(a.to(DEV), offsets.to(DEV), m, stage_major=True)
+    btq, bts = quantize_mx_cols_grouped(b.to(DEV), offsets.to(DEV), m)
+    dw = grouped_mxfp8_wgrad(atq, ats, btq, bts, offsets.to(DEV), m, dtype)
+    assert torch.equal(dw, grouped_mxfp8_wgrad(atq, ats, btq, bts, offsets.to(DEV), m, dtype))  # deterministic
+    ad, bd = (oracle.dequant(*_padded_cols_ref(oracle, t.float(), offsets)[:2]) for t in (a, b))
+    pos = 0
+    for i, cnt in enumerate(counts):
+        ref = ad[:, pos : pos + cnt].double() @ bd[:, pos : pos + cnt].double().T
+        pos += -(-cnt // 128) * 128
+        got = dw[i].cpu().double()
+        bound = {torch.bfloat16: 4e-3, torch.float16: 1e-3, torch.float32: 1e-4}[dtype]
+        assert (got - ref).norm() <= bound * ref.norm(), (i, cnt)
+
+
 def _expert_oracle(ora, x, w_in, w_out, gate, token_of, order, offsets, dout):
     """The fused path's arithmetic restated with oracle primitives, stage by stage."""
     e, two_h, dim = w_in.shape
