@@ -1759,15 +1759,16 @@ static int launch_wgrad_shape(WgradArgs a, float *ws, int64_t ws_bytes, hipStrea
     return hipGetLastError() == hipSuccess ? MX_OK : MX_ELAUNCH;
 }
 
-// Whether an expert dW runs as a stream of K stages on 128 x 128 tiles: up to 56 stages per CU, from about a stage and a quarter per
-// expert on unless its tiles are few.  Large tiles of experts with one to four stages are mostly their stores, which nothing
-// overlaps, and of few experts they leave CUs idle; with more stages twice the operand bytes per flop cost more than that.
-// us on 256 x 256 / here, dW of 1024 x 1024 and of 512 x 1024, by rows in experts:
-//   12000 in 64   50.0 / 44.7   27.6 / 26.4        16662 on 6 of 64   73.4 / 58.3   49.9 / 32.2
-//   16662 in 64   57.2 / 51.2   33.9 / 29.6        22216 in 32        45.9 / 41.1   24.9 / 24.3
-//   24000 in 64   60.3 / 54.3   37.8 / 31.8         2777 in 4         33.6 / 11.3   32.1 / 21.1
-//   33000 in 64   69.0 / 71.0   41.5 / 38.0        72000 in 32        85.6 / 116    51.7 / 61.7
-//    4800 in 64   41.5 / 42.5   23.5 / 25.3        12000 in 16 of 256 x 256 and 128 x 256   29.1 / 20.9   28.6 / 19.4
+// Whether an expert dW runs as a stream of K stages on 128 x 128 tiles: up to 56 stages per CU, where large tiles would fill no more
+// than the CUs, or than half a round on top with four stages per expert.  Few large tiles leave CUs idle or are cut along K; many, of
+// two or three stages, are mostly their stores either way, and those of 256 columns reach memory faster: the dW of a routing block over 2777
+// tokens (16662 in 64) 30.7 / 40.0 and 51.4 / 51.6.  us on 256 x 256 / here, dW of 1024 x 1024 and of 1024 x 512, by rows in experts:
+//    4000 in 12   19.6 / 17.3           -              4000 in 20        -          37.8 / 16.1
+//   16000 in 12   31.9 / 30.1           -             16000 in 20        -          50.0 / 22.6
+//   48000 in 20        -           69.2 / 54.5        24000 in 32        -          33.2 / 30.7
+//   22216 in 32   45.9 / 43.0      27.2 / 26.4        33000 in 64   71.0 / 70.4     41.9 / 38.6 (48.9 / 44.0 where experts differ ninefold)
+//   16662 in 64   42.4 / 52.3      32.0 / 30.2         2777 in 4    33.6 / 11.3     32.1 / 21.1 (512 x 1024)
+//   of 256 x 256: 1000 in 16   14.0 / 10.8        60000 in 16   34.8 / 22.3        72000 in 32 of 1024 x 1024   85.6 / 116
 static bool wgrad_stream_pays(const WgradArgs &a, int64_t M, int esz) {
     const int64_t limit = (int64_t)1 << 31;
     if (a.E > MX_TABLE_MAX || !aligned(a.dw, 16) || (a.lddw * esz) % 16 || (a.stride_dwe * esz) % 16 || a.Kout % 8 || a.ldas < a.KB + 12 ||
@@ -1775,7 +1776,7 @@ static bool wgrad_stream_pays(const WgradArgs &a, int64_t M, int esz) {
         return false;
     const double live = a.E < M ? a.E : M, cus = num_cus();
     const double tiles = (double)((a.N + StreamShape::BM - 1) / StreamShape::BM) * ((a.Kout + StreamShape::BN - 1) / StreamShape::BN);
-    return tiles * ((double)M / 128 + 0.5 * live) <= 56 * cus && (M >= 160 * live || tiles * live <= 4 * cus);
+    return tiles * ((double)M / 128 + 0.5 * live) <= 56 * cus && tiles * live <= (M >= 480 * live ? 8 : 4) * cus;
 }
 
 template <int CDT>
