@@ -945,8 +945,9 @@ struct GroupedStream {
         f.s_voff = (uint32_t)(of_a ? row(r, a_last) * p.ldxs : row(b_row_of_lds<S>(r), b_last) * p.ldws);
     }
 
-    __device__ __forceinline__ void store(const Tile &t, const Lane &L, v4f (&acc)[S::MT][S::NT]) const {
-        stream_store_tile<CDT>(p.out, p.ldo, t.a, t.b, t.c, p.N, L, acc);
+    __device__ __forceinline__ void pack(const Lane &L, v4f (&acc)[S::MT][S::NT], v4i (&parts)[STREAM_PARTS]) const { stream_pack<CDT>(L, acc, parts); }
+    __device__ __forceinline__ void store_part(const Tile &t, const Lane &L, int n, const v4i &part) const {
+        stream_store_part<false>(p.out, p.ldo, t.a, t.b, t.c, p.N, L, n, part);
     }
 };
 
@@ -1526,21 +1527,25 @@ static int launch_grouped_stream(GroupedArgs a, hipStream_t st) {
 }
 
 // Whether the plain product runs as a stream of K stages on 128 x 128 tiles: rows that are not gathered, whole groups of four stages,
-// 16-byte output runs, and up to six tiles per CU.  Few rows per expert fill 256 x 256 tiles to a fraction, and a few rounds of
-// large tiles end in a partial one; from there on twice the operand bytes per flop cost more than the stores under the K loops save.
+// 16-byte output runs, and up to six tiles per CU (four where K is beyond 1024).  Few rows per expert fill 256 x 256 tiles to a
+// fraction, and a few rounds of large tiles end in a partial one; from there on twice the operand bytes per flop cost more than the
+// stores under the K loops save.
 // us on the other shapes / here, 64 experts of 1024 columns, operands from HBM, by rows in all:
-//              1000          3000         8000          16662         33000        50000        98304
-//   K = 512   11.8 / 11.4  13.6 / 12.7  18.9 / 17.1  29.0 / 23.3  39.3 / 38.2  50.7 / 55.1  85.6 / 102.4
-//   K = 1024  19.8 / 17.8  21.6 / 19.0  27.4 / 26.0  43.5 / 36.5  59.1 / 59.5  76.2 / 83.5   131 / 155
-// (on another box 19.8 / 21.3 and 21.6 / 21.7 where this says 17.8 and 19.0, the rest within 4 %);
-// of 8 experts 8.1 / 6.3 and 11.1 / 7.6 (1000 rows), 23.7 / 16.7 and 35.0 / 23.8 (16662); of 32 experts 16.7 / 11.2 and 23.9 / 21.9 (8000).
+//              200           1000         8000         16662        33000        98304
+//   K = 512   11.5 / 11.6  11.7 / 11.7  18.0 / 16.6  27.6 / 24.2  38.0 / 40.4  82.7 / 107
+//   K = 1024       -            -            -       41.4 / 36.8  55.8 / 59.5       -        (40000 in 32   55.0 / 68.5)
+// of 8 experts 1000 rows x K = 1024 11.3 / 8.2, 16662 x 1024 32.5 / 26.7; of 16, 65536 rows of 256 columns 26.2 / 23.8; K = 1536 and
+// 2048, 20000 in 16 (5 tiles per CU) 49.0 / 50.4 and 59.9 / 62.7, 8000 in 8 of 512 columns 21.0 / 19.8.
+// The results are stored without the non-temporal hint: the pass that adds them up per token finds them in the cache (16662 rows: 13.8
+// -> 9.4 and 10.6 -> 8.3 us).  With it 98304 x 1024 x 512 alone takes 72 us, but 107 behind the product that makes its operand, and
+// that pass 60 for 45.
 static bool stream_pays(const GroupedArgs &a) {
     const int64_t limit = (int64_t)1 << 31;
     if (a.index || a.K % 512 || (int64_t)a.N * a.K > (2 << 20) || !a.out_vec || a.N % 8 || a.E > MX_TABLE_MAX_STREAM || a.x_rows < a.M || 128 * a.ldx >= limit ||
         128 * a.ldw >= limit || 128 * a.ldxs >= limit || 128 * a.ldws >= limit)
         return false;
     const double live = a.E < a.M ? a.E : a.M, rows = (double)a.M / StreamShape::BM + 0.5 * live;
-    return (rows > live ? rows : live) * ((a.N + StreamShape::BN - 1) / StreamShape::BN) <= 6.0 * num_cus();
+    return (rows > live ? rows : live) * ((a.N + StreamShape::BN - 1) / StreamShape::BN) <= (a.K <= 1024 ? 6.0 : 4.0) * num_cus();
 }
 
 template <int MODE, int CDT>
