@@ -413,7 +413,7 @@ TRAFFIC_SOURCE = ("a constant, not measured in this run: the rocprofv3 --pmc FET
                   "profiles/gemm_nt_kernel_dense_ffn_fwd_bwd.md")
 
 GEMM_ENTRIES = ("mx_gemm_nt", "mx_gemm_nt_batch", "mx_grouped_gemm_nt", "mx_experts_gemm1", "mx_experts_scatter_gemm",
-                "mx_experts_gemm2_dgrad", "mx_grouped_wgrad_nt")
+                "mx_experts_gemm2_dgrad", "mx_experts_gemm2_dgrad_parts", "mx_grouped_wgrad_nt")
 
 
 def build_workload(name: str, dev, routing: str = "draws"):

@@ -441,6 +441,27 @@ int mx_experts_gemm2_dgrad(const uint8_t *dq, const uint8_t *ds, int64_t T, int6
                            float *dgate, int act_dtype, int64_t M, int64_t H, int64_t K, void *stream);
 
 /*
+ * The same with dgate in parts, one per 128 hidden units, whose sum does not depend on the order workgroups end in:
+ * parts (ceil(H/128), ldparts), parts[s][order[m]] = the product over units [128 s, 128 s + 128), for every m below offsets[E];
+ * nothing else of it is written.  A pair has one row at most, and ldparts is past the highest pair.
+ */
+int mx_experts_gemm2_dgrad_parts(const uint8_t *dq, const uint8_t *ds, int64_t T, int64_t lddq, int64_t ldds,
+                                 const int32_t *token_of, const int32_t *order, const void *gate, int gate_dtype,
+                                 const uint8_t *wq, const uint8_t *ws, int64_t stride_we, int64_t ldw,
+                                 int64_t stride_wse, int64_t ldws, const int32_t *offsets, int64_t E,
+                                 const uint8_t *hq, int64_t ldhq, const uint8_t *hs, int64_t ldhs, const void *pre,
+                                 void *dpre, int64_t ldpre, uint8_t *dpq, int64_t lddpq, uint8_t *dps, int64_t lddps,
+                                 uint8_t *ptq, int64_t ldptq, uint8_t *pts, int64_t ldpts,
+                                 float *parts, int64_t ldparts, int act_dtype, int64_t M, int64_t H, int64_t K, void *stream);
+
+/*
+ * dgate (pairs,), in dtype: the parts of each pair added up in fp32 in the order of their hidden units, and 0 where positions[pair],
+ * the pair's sorted position (inv of mx_experts_combine), is negative.  ldparts >= pairs.
+ */
+int mx_experts_gate_grad(const float *parts, int64_t ldparts, int64_t H, const int32_t *positions, void *dgate, int dtype,
+                         int64_t pairs, void *stream);
+
+/*
  * Token-axis quantizer over expert-sorted rows, feeding the experts' MXFP8 WGRAD.  Each
  * expert's rows are laid out from a fresh multiple of 128 in a padded position space of
  * Mpad = (ceil(M/128) + E) * 128 positions (rows past an expert's end are zero), so no 32-row

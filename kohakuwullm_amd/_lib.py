@@ -54,6 +54,10 @@ SIGNATURES = {
     "mx_experts_gemm2_dgrad": (
         _ci, [_p, _p, _i64, _i64, _i64, _p, _p, _p, _ci, _p, _p, _i64, _i64, _i64, _i64, _p, _i64, _p, _i64, _p, _i64,
               _p, _p, _i64, _p, _i64, _p, _i64, _p, _i64, _p, _i64, _p, _ci, _i64, _i64, _i64, _p]),
+    "mx_experts_gemm2_dgrad_parts": (
+        _ci, [_p, _p, _i64, _i64, _i64, _p, _p, _p, _ci, _p, _p, _i64, _i64, _i64, _i64, _p, _i64, _p, _i64, _p, _i64,
+              _p, _p, _i64, _p, _i64, _p, _i64, _p, _i64, _p, _i64, _p, _i64, _ci, _i64, _i64, _i64, _p]),
+    "mx_experts_gate_grad": (_ci, [_p, _i64, _i64, _p, _p, _ci, _i64, _p]),
     "mx_experts_combine": (_ci, [_p, _i64, _p, _p, _i64, _p, _ci, _p, _i64, _i64, _p, _ci, _i64, _i64, _i64, _p]),
     "mx_experts_combine_onto": (_ci, [_p, _i64, _p, _i64, _p, _p, _i64, _p, _ci, _p, _i64, _i64, _p, _ci, _i64, _i64, _i64, _p]),
     "mx_quantize_cols_grouped": (

@@ -13,7 +13,7 @@
 //   SCATTER    out[token(m)] += scale(m) * (a[m] . w[e(m)]^T), packed 16-bit atomics;
 //              scale = gate[order[m]] (GEMM2, experts.py:138-222) or 1 (GEMM1 dgrad,
 //              experts_bwd.py:167-247)
-//   DGRAD2     acc = dq[token(m)] . w_out_dgrad[e]^T; dgate[pair] += <acc, h>; dh = acc * gate;
+//   DGRAD2     acc = dq[token(m)] . w_out_dgrad[e]^T; dgate[pair] = <acc, h>; dh = acc * gate;
 //              SwiGLU' from the stored pre; dpre (M,2H) stored and requantized
 //                                                                         experts_bwd.py:29-164
 // The row gather costs nothing: every lane of the copy engine supplies its own global address.
@@ -56,7 +56,10 @@ struct GroupedArgs {
     void *dpre;  // DGRAD2 out: (M,2H) 16-bit
     uint8_t *dpq, *dps;  // DGRAD2 out: (M,2H), (M,2H/32)
     int64_t lddpq, lddps;
-    float *dgate;  // DGRAD2 out: (pairs,) fp32, accumulated
+    // DGRAD2 out, fp32: <acc, h> of each 128 columns, ld_dgate apart, element (s, pair) for columns [128 s, 128 s + 128);
+    // ld_dgate == 0: (pairs,), to which every 128 columns are added as they come
+    float *dgate;
+    int64_t ld_dgate;
 };
 
 template <int CDT>
@@ -571,6 +574,9 @@ struct GroupedProblem {
         const int hblock = t.n0 + L.wn * S::WTN + 32 * (o_r16 >> 2);  // the 32 hidden units of a quad
         const int h = t.n0 + L.wn * S::WTN + 8 * o_r16;
         const bool col_ok = hblock < H;
+        const int wave_n = t.n0 + L.wn * S::WTN;
+        static_assert(S::WTN == 128, "a wave's columns are one part of dgate");
+        float *const gate_part = p.dgate + (int64_t)(wave_n / S::WTN) * p.ld_dgate;
         auto row_at = [&](int i, int v) { return t.row0 + L.wm * S::WTM + 16 * i + 4 * o_g + v; };
         // Row metadata once per tile: lane l of a wave fetches the pair index and the gate factor of the wave's row l
         // (two dependent loads per tile); a step takes its rows' values from those lanes.  Fetched per slab of rows by
@@ -694,9 +700,14 @@ struct GroupedProblem {
 #pragma unroll
                     for (int e = 0; e < 4; e++) keep[0][i][v][e] = keep[1][i][v][e] = 0u;  // padding rows and columns
                 }
-                // the dot product over the expert width is split across lanes, waves and N tiles
+                // The dot product over the expert width is split across lanes, waves and N tiles.  A wave's 128 columns have a
+                // place of their own, and gate_grad_kernel adds those in order: added here as they came (16662 rows x 512), 5000
+                // of the fp32 sums differed from one pass to the next, and about one of the gradients rounded to bf16.
                 dot = row16_sum(dot);
-                if (row_ok && o_r16 == 0) atomicAdd(p.dgate + pair, dot);
+                if (row_ok && o_r16 == 0) {
+                    if (!p.ld_dgate) atomicAdd(p.dgate + pair, dot);
+                    else if (wave_n < H) gate_part[pair] = dot;
+                }
             }
             asm volatile("" ::: "memory");
         }
@@ -853,6 +864,19 @@ __global__ __launch_bounds__(256) void combine_kernel(const uint16_t *__restrict
         round_pair<CDT>(a, b, w[e]);
     }
     *(v4i *)(out + t * ldo + c) = v4i{(int)w[0], (int)w[1], (int)w[2], (int)w[3]};
+}
+
+// dgate[p] = the parts of pair p, added in the order of the columns they stand for; zero for a pair no row belongs to (whose parts
+// nothing has written).
+template <typename T>
+__global__ __launch_bounds__(256) void gate_grad_kernel(const float *__restrict__ parts, int64_t ld, int slices,
+                                                        const int32_t *__restrict__ positions, T *__restrict__ dgate, int64_t pairs) {
+    const int64_t p = (int64_t)blockIdx.x * 256 + threadIdx.x;
+    if (p >= pairs) return;
+    float sum = 0.0f;
+    if (positions[p] >= 0)
+        for (int s = 0; s < slices; s++) sum += parts[s * ld + p];
+    dgate[p] = (T)sum;
 }
 
 // Experts the row-tile tables of a workgroup hold.  Two workgroups share a CU's 160 KB under the 128 x 128 shape: their
@@ -1654,14 +1678,13 @@ extern "C" int mx_experts_scatter_gemm(const uint8_t *aq, const uint8_t *as, int
     return launch_grouped_dt<MODE_SCATTER>(out_dtype, a, (hipStream_t)stream);
 }
 
-extern "C" int mx_experts_gemm2_dgrad(const uint8_t *dq, const uint8_t *ds, int64_t T, int64_t lddq, int64_t ldds,
-                                      const int32_t *token_of, const int32_t *order, const void *gate, int gate_dtype,
-                                      const uint8_t *wq, const uint8_t *ws, int64_t stride_we, int64_t ldw,
-                                      int64_t stride_wse, int64_t ldws, const int32_t *offsets, int64_t E,
-                                      const uint8_t *hq, int64_t ldhq, const uint8_t *hs, int64_t ldhs, const void *pre,
-                                      void *dpre, int64_t ldpre, uint8_t *dpq, int64_t lddpq, uint8_t *dps,
-                                      int64_t lddps, uint8_t *ptq, int64_t ldptq, uint8_t *pts, int64_t ldpts,
-                                      float *dgate, int act_dtype, int64_t M, int64_t H, int64_t K, void *stream) {
+static int gemm2_dgrad(const uint8_t *dq, const uint8_t *ds, int64_t T, int64_t lddq, int64_t ldds, const int32_t *token_of,
+                       const int32_t *order, const void *gate, int gate_dtype, const uint8_t *wq, const uint8_t *ws,
+                       int64_t stride_we, int64_t ldw, int64_t stride_wse, int64_t ldws, const int32_t *offsets, int64_t E,
+                       const uint8_t *hq, int64_t ldhq, const uint8_t *hs, int64_t ldhs, const void *pre, void *dpre,
+                       int64_t ldpre, uint8_t *dpq, int64_t lddpq, uint8_t *dps, int64_t lddps, uint8_t *ptq, int64_t ldptq,
+                       uint8_t *pts, int64_t ldpts, float *dgate, int64_t ld_dgate, int act_dtype, int64_t M, int64_t H, int64_t K,
+                       void *stream) {
     if (!sizes_ok(E, M, H, K) || H % MX_BLOCK || lddq < K || ldw < K || ldhq < H || ldpre < 2 * H || lddpq < 2 * H ||
         lddps < 2 * H / MX_BLOCK || !token_of || !order || !gate || !pre || !dgate || (!dpre && !ptq) ||
         (ptq != nullptr) != (pts != nullptr))
@@ -1676,7 +1699,7 @@ extern "C" int mx_experts_gemm2_dgrad(const uint8_t *dq, const uint8_t *ds, int6
     a.token_of = token_of, a.order = order, a.gate = gate, a.gate_f32 = gate_dtype == MX_FP32;
     a.hq = (uint8_t *)hq, a.ldhq = ldhq, a.hs = (uint8_t *)hs, a.ldhs = ldhs;
     a.pre = (void *)pre, a.dpre = dpre, a.ldpre = ldpre, a.dpq = dpq, a.lddpq = lddpq, a.dps = dps, a.lddps = lddps;
-    a.dgate = dgate;
+    a.dgate = dgate, a.ld_dgate = ld_dgate;
     a.htq = ptq, a.ldhtq = ldptq, a.hts = pts, a.ldhts = ldpts, a.htq_ks = t_panels ? 2 * H * 128 : 0;
     if (K == 0 || !tiled_ok(a, T) || !aligned(hq, 8) || ldhq % 8 || !aligned(pre, 16) || (dpre && !aligned(dpre, 16)) ||
         ldpre % 8 || H % 8 || !aligned(dpq, 8) || lddpq % 8 ||
@@ -1684,6 +1707,51 @@ extern "C" int mx_experts_gemm2_dgrad(const uint8_t *dq, const uint8_t *ds, int6
         return MX_EUNSUPPORTED;
     if (mx::stream_is_capturing((hipStream_t)stream)) return MX_ECAPTURE;
     return launch_grouped_dt<MODE_DGRAD2>(act_dtype, a, (hipStream_t)stream);
+}
+
+extern "C" int mx_experts_gemm2_dgrad(const uint8_t *dq, const uint8_t *ds, int64_t T, int64_t lddq, int64_t ldds,
+                                      const int32_t *token_of, const int32_t *order, const void *gate, int gate_dtype,
+                                      const uint8_t *wq, const uint8_t *ws, int64_t stride_we, int64_t ldw,
+                                      int64_t stride_wse, int64_t ldws, const int32_t *offsets, int64_t E,
+                                      const uint8_t *hq, int64_t ldhq, const uint8_t *hs, int64_t ldhs, const void *pre,
+                                      void *dpre, int64_t ldpre, uint8_t *dpq, int64_t lddpq, uint8_t *dps,
+                                      int64_t lddps, uint8_t *ptq, int64_t ldptq, uint8_t *pts, int64_t ldpts,
+                                      float *dgate, int act_dtype, int64_t M, int64_t H, int64_t K, void *stream) {
+    return gemm2_dgrad(dq, ds, T, lddq, ldds, token_of, order, gate, gate_dtype, wq, ws, stride_we, ldw, stride_wse, ldws, offsets, E, hq,
+                       ldhq, hs, ldhs, pre, dpre, ldpre, dpq, lddpq, dps, lddps, ptq, ldptq, pts, ldpts, dgate, 0, act_dtype, M, H, K, stream);
+}
+
+extern "C" int mx_experts_gemm2_dgrad_parts(const uint8_t *dq, const uint8_t *ds, int64_t T, int64_t lddq, int64_t ldds,
+                                            const int32_t *token_of, const int32_t *order, const void *gate, int gate_dtype,
+                                            const uint8_t *wq, const uint8_t *ws, int64_t stride_we, int64_t ldw,
+                                            int64_t stride_wse, int64_t ldws, const int32_t *offsets, int64_t E,
+                                            const uint8_t *hq, int64_t ldhq, const uint8_t *hs, int64_t ldhs, const void *pre,
+                                            void *dpre, int64_t ldpre, uint8_t *dpq, int64_t lddpq, uint8_t *dps,
+                                            int64_t lddps, uint8_t *ptq, int64_t ldptq, uint8_t *pts, int64_t ldpts,
+                                            float *parts, int64_t ldparts, int act_dtype, int64_t M, int64_t H, int64_t K,
+                                            void *stream) {
+    if (ldparts <= 0) return MX_EINVAL;
+    return gemm2_dgrad(dq, ds, T, lddq, ldds, token_of, order, gate, gate_dtype, wq, ws, stride_we, ldw, stride_wse, ldws, offsets, E, hq,
+                       ldhq, hs, ldhs, pre, dpre, ldpre, dpq, lddpq, dps, lddps, ptq, ldptq, pts, ldpts, parts, ldparts, act_dtype, M, H, K,
+                       stream);
+}
+
+extern "C" int mx_experts_gate_grad(const float *parts, int64_t ldparts, int64_t H, const int32_t *positions, void *dgate, int dtype,
+                                    int64_t pairs, void *stream) {
+    if (pairs < 0 || pairs >= 0x7FFFFFFF || H < 0 || H >= 0x7FFFFFFF || ldparts < pairs || (pairs && (!positions || !dgate || (H && !parts))))
+        return MX_EINVAL;
+    if (pairs == 0) return MX_OK;
+    hipStream_t st = (hipStream_t)stream;
+    if (mx::stream_is_capturing(st)) return MX_ECAPTURE;
+    const dim3 grid((unsigned)((pairs + 255) / 256)), block(256);
+    const int slices = (int)((H + 127) / 128);
+    switch (dtype) {
+    case MX_BF16: gate_grad_kernel<__bf16><<<grid, block, 0, st>>>(parts, ldparts, slices, positions, (__bf16 *)dgate, pairs); break;
+    case MX_FP16: gate_grad_kernel<_Float16><<<grid, block, 0, st>>>(parts, ldparts, slices, positions, (_Float16 *)dgate, pairs); break;
+    case MX_FP32: gate_grad_kernel<float><<<grid, block, 0, st>>>(parts, ldparts, slices, positions, (float *)dgate, pairs); break;
+    default: return MX_EINVAL;
+    }
+    return hipGetLastError() == hipSuccess ? MX_OK : MX_ELAUNCH;
 }
 
 extern "C" int mx_experts_combine(const void *y, int64_t ldy, const int32_t *order, const int32_t *offsets, int64_t E,

@@ -42,7 +42,7 @@ namespace {
     F(mx_swiglu_quantize_tokens) F(mx_swiglu_bwd_quantize_tokens) F(mx_gemm_nt) F(mx_gemm_nt_batch) F(mx_activation_gemm_nt) F(mx_rmsnorm_quantize) \
     F(mx_rmsnorm_backward) F(mx_rmsnorm_weight_grad) F(mx_router_topk) F(mx_router_backward_workspace)                      \
     F(mx_router_topk_backward_onto) F(mx_expert_sort_workspace) F(mx_expert_sort_positions) F(mx_experts_gemm1)                  \
-    F(mx_grouped_gemm_nt) F(mx_experts_combine_onto) F(mx_experts_gemm2_dgrad) F(mx_quantize_cols_grouped) F(mx_grouped_wgrad_nt)
+    F(mx_grouped_gemm_nt) F(mx_experts_combine_onto) F(mx_experts_gemm2_dgrad_parts) F(mx_experts_gate_grad) F(mx_quantize_cols_grouped) F(mx_grouped_wgrad_nt)
 
 struct Library {
 #define F(name) decltype(&::name) name = nullptr;
@@ -929,13 +929,14 @@ PyObject *py_experts_backward(Args &a) {
     void *const st = stream_of(x);
     const Quantized d = quantize_rows(dout);
     const Quantized dp{empty({r.m, 2 * hidden}, FP8, x), empty({r.m, 2 * hidden / BLOCK}, U8, x)};
-    const Tensor dgate = empty({gate.numel()}, at::kFloat, x);
-    MX_COPY(dgate.zero_());
+    const Tensor dgate = empty({gate.numel()}, gate.scalar_type(), x), parts = empty({(hidden + PANEL - 1) / PANEL, gate.numel()}, at::kFloat, x);
     const Quantized pt = expert_token_buffers(2 * hidden, mpad, x);
-    MX_RUN(mx_experts_gemm2_dgrad, bytes(d.q), bytes(d.s), x.size(0), dim, dim / BLOCK, r.p(token_of), r.p(order), gate.const_data_ptr(),
+    MX_RUN(mx_experts_gemm2_dgrad_parts, bytes(d.q), bytes(d.s), x.size(0), dim, dim / BLOCK, r.p(token_of), r.p(order), gate.const_data_ptr(),
            code_of(gate.scalar_type()), MX_STACK(w_out), r.p(offsets), w_out.e, bytes(hq), hidden, bytes(hs), hidden / BLOCK, pre.const_data_ptr(), nullptr,
            2 * hidden, (uint8_t *)dp.q.data_ptr(), 2 * hidden, (uint8_t *)dp.s.data_ptr(), 2 * hidden / BLOCK, codes_out(pt), PANEL, scales_out(pt),
-           pt.s.stride(0), (float *)dgate.data_ptr(), code, r.m, hidden, dim, st);
+           pt.s.stride(0), (float *)parts.data_ptr(), gate.numel(), code, r.m, hidden, dim, st);
+    MX_RUN(mx_experts_gate_grad, (const float *)parts.const_data_ptr(), gate.numel(), hidden, (const int32_t *)positions.const_data_ptr(), dgate.data_ptr(),
+           code_of(gate.scalar_type()), gate.numel(), st);
     Tensor inverse = positions;
     const Tensor dx = routed_product(dp, w_in, r, Tensor(), x.size(0), type, true, inverse);
     const Tensor ws = workspace(x);
@@ -960,7 +961,7 @@ PyObject *py_experts_backward(Args &a) {
     }
     const Quantized xt = columns(x, false);
     dw_in = wgrad(pt.q, pt.s, xt.q, xt.s);
-    return wrap_all({dx, dw_in, dw_out, dgate.scalar_type() == gate.scalar_type() ? dgate : MX_COPY(dgate.to(gate.scalar_type()))});
+    return wrap_all({dx, dw_in, dw_out, dgate});
 }
 
 // bind(path, cdll, invoke, module): take the entry points from the library at `path`, which `cdll` is; `module` is the ctypes binding,

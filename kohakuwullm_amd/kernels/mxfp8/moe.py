@@ -185,12 +185,16 @@ def launch_gemm2_dgrad(dq, ds, token_of, order, gate, wq, ws, hq, hs, pre, dpre,
     """DGRAD through GEMM2 with its epilogue.
 
     ``ptq``/``pts`` ``(2H, Mpad)``/``(2H, Mpad//32)``, when given, receive ``dpre`` quantized along the
-    tokens; ``dpre`` may then be ``None``.
+    tokens; ``dpre`` may then be ``None``.  ``dgate`` fp32: zeros ``(pairs,)`` that the products are added to, in the order
+    workgroups end in, or ``(ceil(H / 128), pairs)`` for the product of each 128 hidden units (:func:`sum_gate_grad`).
     """
     m = token_of.numel()
     hidden, dim = wq.shape[1], wq.shape[2]
+    in_parts = dgate.dim() == 2
+    if in_parts and (dgate.shape != (-(-hidden // 128), gate.numel()) or not dgate.is_contiguous()):
+        raise ValueError(f"dgate {tuple(dgate.shape)} does not hold a contiguous part of {gate.numel()} pairs for each 128 of {hidden} hidden units")
     _lib.invoke(
-        "mx_experts_gemm2_dgrad", 2.0 * m * hidden * dim, dq,
+        "mx_experts_gemm2_dgrad_parts" if in_parts else "mx_experts_gemm2_dgrad", 2.0 * m * hidden * dim, dq,
         dq.data_ptr(), ds.data_ptr(), dq.shape[0], dq.stride(0), ds.stride(0), token_of.data_ptr(), order.data_ptr(),
         gate.data_ptr(), _lib.MX_DTYPE[gate.dtype], *_w_args(wq, ws), offsets.data_ptr(), wq.shape[0],
         hq.data_ptr(), hq.stride(0), hs.data_ptr(), hs.stride(0), pre.data_ptr(),
@@ -198,8 +202,22 @@ def launch_gemm2_dgrad(dq, ds, token_of, order, gate, wq, ws, hq, hs, pre, dpre,
         dpq.data_ptr(), dpq.stride(0), dps.data_ptr(), dps.stride(0),
         0 if ptq is None else ptq.data_ptr(), 0 if ptq is None else token_axis_pitch(ptq),
         0 if pts is None else pts.data_ptr(), 0 if pts is None else pts.stride(0),
-        dgate.data_ptr(), _lib.MX_DTYPE[pre.dtype], m, hidden, dim,
+        dgate.data_ptr(), *((dgate.stride(0),) if in_parts else ()), _lib.MX_DTYPE[pre.dtype], m, hidden, dim,
     )
+
+
+def sum_gate_grad(parts, positions, dtype) -> torch.Tensor:
+    """The gate gradient ``(pairs,)`` in ``dtype``: each pair's ``parts`` added in fp32 in the order of their hidden units.
+
+    ``positions``: the pair -> sorted position table (:func:`combine_sorted_rows`); a pair below 0 has no row and gets zero.
+    """
+    slices, pairs = parts.shape
+    dgate = torch.empty(pairs, device=parts.device, dtype=dtype)
+    _lib.invoke(
+        "mx_experts_gate_grad", parts.element_size() * parts.numel(), parts,
+        parts.data_ptr(), parts.stride(0), 128 * slices, positions.data_ptr(), dgate.data_ptr(), _lib.MX_DTYPE[dtype], pairs,
+    )
+    return dgate
 
 
 class _MXFP8Experts(torch.autograd.Function):
@@ -261,8 +279,12 @@ class _MXFP8Experts(torch.autograd.Function):
         dq, ds = quantize_mx(dout)
         dpq = torch.empty(m, 2 * hidden, device=dev, dtype=_FP8)
         dps = torch.empty(m, 2 * hidden // BLOCK_SCALE, device=dev, dtype=torch.uint8)
-        # fp32 and zeroed: this reduction crosses workgroups through an atomic
-        dgate = torch.zeros(gate.numel(), device=dev, dtype=torch.float32)
+        # The reduction over the hidden units crosses workgroups: a part per 128 of them, added in order behind.  Where a pair
+        # may have several rows (no table of positions), zeros that the atomics of all of them add to.
+        if ctx.positions is None:
+            dgate = torch.zeros(gate.numel(), device=dev, dtype=torch.float32)
+        else:
+            dgate = torch.empty(-(-hidden // 128), gate.numel(), device=dev, dtype=torch.float32)
         ptq = pts = None
         if ctx.needs_input_grad[1]:
             # dpre along the tokens, for dW_in: written by the epilogue; dpre itself never reaches memory
@@ -271,6 +293,7 @@ class _MXFP8Experts(torch.autograd.Function):
         dpre = None if ptq is not None else torch.empty(m, 2 * hidden, device=dev, dtype=dout.dtype)
         launch_gemm2_dgrad(dq, ds, token_of, order, gate, *packed.out_dgrad, hq, hs, pre, dpre, dpq, dps, dgate, offsets,
                            ptq, pts)
+        dgate = dgate.to(gate.dtype) if ctx.positions is None else sum_gate_grad(dgate, ctx.positions, gate.dtype)
         dx = _routed_product(dpq, dps, *packed.in_dgrad, token_of, order, None, offsets, rows, top_k, dout.dtype,
                              positions=ctx.positions)
 
@@ -284,7 +307,7 @@ class _MXFP8Experts(torch.autograd.Function):
             # dW_in[e] = dpre rows of e .T @ x rows of e
             xtq, xts = quantize_mx_cols_grouped(x, offsets, m, index=token_of, stage_major=TOKEN_AXIS_STAGE_MAJOR)
             dw_in = grouped_mxfp8_wgrad(ptq, pts, xtq, xts, offsets, m, dout.dtype)
-        return dx, dw_in, dw_out, dgate.to(gate.dtype), None, None, None, None, None, None, None, dbase
+        return dx, dw_in, dw_out, dgate, None, None, None, None, None, None, None, dbase
 
 
 def _validate_expert_call(x, w_in, w_out, token_of, order) -> int:

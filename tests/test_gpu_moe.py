@@ -1111,3 +1111,68 @@ def test_shared_expert_gets_the_gradient_of_the_sum():
         p.grad = None
     block(x.detach()).backward(up)
     assert all((p.grad is not None) == name.startswith("shared.") for name, p in block.named_parameters())
+
+
+@pytest.mark.parametrize("counts, hid, dtype", [
+    ([300, 0, 1, 257, 130], 96, torch.float32),  # one part, narrower than 128
+    ([200, 0, 56, 300], 160, torch.bfloat16),  # a whole part and a quarter of one
+    ([1, 700], 544, torch.float16),  # five parts: 256-column tiles end in a half without columns
+    ([250] * 64, 512, torch.float32),  # thousands of rows: workgroups end in another order each time
+])
+def test_gate_gradient_does_not_depend_on_the_order_of_workgroups(counts, hid, dtype):
+    """Each pair's products over 128 hidden units, added in their order: the same bits in every pass, on either tile shape and as
+    torch adds those parts up, zero for a pair whose row lies behind the last expert, and the sum of atomics up to rounding."""
+    from kohakuwullm_amd import _lib
+    from kohakuwullm_amd.kernels.mxfp8.moe import MXFP8ExpertWeights, launch_gemm1, launch_gemm2_dgrad, mxfp8_moe_experts, sum_gate_grad
+    from kohakuwullm_amd.kernels.mxfp8.quantize import quantize_mx
+
+    g = torch.Generator().manual_seed(SEED + 41)
+    act = torch.bfloat16 if dtype == torch.float32 else dtype
+    e, dim, top_k = len(counts), 256, 2
+    tokens = sum(counts) // 2 + max(counts) + 40
+    offsets, order, token_of = _routing(counts + [40], top_k, tokens)  # the last 40 rows belong to no expert
+    offsets, order, token_of = offsets[:-1].contiguous().to(DEV), order.to(DEV), token_of.to(DEV)
+    m, valid = token_of.numel(), sum(counts)
+    x, dout = (torch.randn(tokens, dim, generator=g).to(DEV, act) for _ in range(2))
+    gate = (torch.rand(tokens * top_k, generator=g) * 0.5 + 0.5).to(DEV, dtype)
+    w_in = (torch.randn(e, 2 * hid, dim, generator=g) * 0.06).to(DEV, act).requires_grad_()
+    w_out = (torch.randn(e, dim, hid, generator=g) * 0.06).to(DEV, act).requires_grad_()
+    packed = MXFP8ExpertWeights(w_in.detach(), w_out.detach())
+
+    def trained(timer):
+        _lib.TIMER = timer  # a timer sends calls the Python way, without one they go through the extension
+        leaf = gate.clone().requires_grad_()
+        mxfp8_moe_experts(x, w_in, w_out, leaf, token_of, order, offsets, packed).backward(dout)
+        _lib.TIMER = None
+        return leaf.grad
+
+    first = trained(None)
+    for timer in (None, [], None, []):
+        assert torch.equal(trained(timer), first)
+    routed = torch.zeros(gate.numel(), dtype=torch.bool, device=DEV)
+    routed[order[:valid].long()] = True
+    assert not first[~routed].any() and bool((~routed).any())
+
+    (xq, xs), (dq, ds) = quantize_mx(x), quantize_mx(dout)
+    empty = lambda *shape, dtype=torch.uint8: torch.empty(*shape, device=DEV, dtype=dtype)  # noqa: E731
+    hq, hs, pre = empty(m, hid, dtype=F8), empty(m, hid // 32), empty(m, 2 * hid, dtype=act)
+    launch_gemm1(xq, xs, token_of, *packed.in_fwd, hq, hs, pre, offsets, hid, dim, act)
+    parts_of = lambda: torch.full((-(-hid // 128), gate.numel()), 7.0, device=DEV)  # noqa: E731
+    sums = [parts_of(), parts_of(), torch.zeros(gate.numel(), device=DEV)]
+    for dgate in sums:
+        dpre, dpq, dps = empty(m, 2 * hid, dtype=act), empty(m, 2 * hid, dtype=F8), empty(m, 2 * hid // 32)
+        launch = lambda: launch_gemm2_dgrad(dq, ds, token_of, order, gate, *packed.out_dgrad, hq, hs, pre, dpre, dpq, dps,  # noqa: E731
+                                            dgate, offsets)  # noqa: B023
+        if dgate is sums[1]:
+            with _lib.variants_library():  # the other tile shape
+                launch()
+        else:
+            launch()
+    assert torch.equal(sums[0], sums[1]) and bool((sums[0][:, ~routed] == 7.0).all())
+    want = torch.zeros(gate.numel(), device=DEV)
+    for part in sums[0]:
+        want += torch.where(routed, part, 0.0)
+    positions = torch.full((gate.numel(),), -1, device=DEV, dtype=torch.int32)
+    positions[order[:valid].long()] = torch.arange(valid, device=DEV, dtype=torch.int32)
+    assert torch.equal(sum_gate_grad(sums[0], positions, dtype), want.to(dtype)) and torch.equal(first, want.to(dtype))
+    assert float((want - sums[2]).norm() / want.norm()) < 1e-6
