@@ -847,8 +847,8 @@ def main() -> None:
                     help="milliseconds of untimed steps between a first timed region (reported as ms_per_step_from_cold_start) "
                          "and the one the line's value comes from; 0: one timed region, straight after the warmup")
     ap.add_argument("--variants-library", action="store_true",
-                    help="run the workload on libmxfp8_hip_variants.so instead of the product library: for moe, the two fused "
-                         "expert kernels on 128 x 128 tiles with two workgroups per CU (measured slower; kept as evidence)")
+                    help="run the workload on libmxfp8_hip_variants.so instead of the product library: for moe, the expert "
+                         "kernels on the tiles that the shipped rules pass over (measured slower; kept as evidence)")
     ap.add_argument("--no-cpu-baseline", action="store_true")
     ap.add_argument("--breakdown", action="store_true",
                     help="also print the per-entry-point launch times of a step (the line's launch_breakdown) on stderr")

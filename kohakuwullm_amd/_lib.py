@@ -156,11 +156,13 @@ def load() -> ctypes.CDLL:
 
 # Measured-slower alternative kernels live in a library of their own, built from the same sources with
 # -DMX_BENCH_VARIANTS: the dense GEMM's three other tilings / schedules behind flags of `epilogue`
-# (csrc/mx_gemm_variants.h; the product library answers MX_EUNSUPPORTED to each), and the two fused expert kernels on
-# 128 x 128 tiles with two workgroups per CU in place of the shipped 256 x 256 ones (csrc/mx_grouped.hip).  Only the
-# benchmark (--variants-library) and the bit-equality tests of the kernels load it.
+# (csrc/mx_gemm_variants.h; the product library answers MX_EUNSUPPORTED to each), and the expert kernels on the tiles that
+# the shipped rules pass over (csrc/mx_grouped.hip), or, for the plain product and the dW, on the kernel that one of the
+# MX_ON_* flags names beside the output type (the product library answers MX_EINVAL).  Only the benchmark
+# (--variants-library) and the bit-equality tests of the kernels load it.
 VARIANTS_PATH = os.path.join(_HERE, "libmxfp8_hip_variants.so")
 MX_EPI_TILE_128, MX_EPI_PHASED, MX_EPI_WIDE_WAVES = 0x10, 0x20, 0x40
+MX_ON_256, MX_ON_128, MX_ON_STREAM = 0x10, 0x20, 0x30  # MX_ON_128: the plain product alone
 _variants: ctypes.CDLL | None = None
 
 

@@ -1495,11 +1495,21 @@ static bool slim_pays(const GroupedArgs &a) {
     const double big = rounds(Big::BM, Big::BN / half, cus), small = rounds(Slim::BM, Slim::BN / half, 2 * cus);
     return small < 1e6 && (MODE == MODE_PLAIN ? small <= big : 2 * small <= 3 * big);
 }
-// The variants library turns the rule round, so that the other shape can be compared with the shipped one at any size.
+
+// The variants library takes the kernel that the rules here pass over -- where the stream of K stages is chosen, the better one of the
+// two others -- and of the plain product and the dW the one that bits 4 and 5 of the output type name, so that each can be compared
+// with the others at any size it takes.  The product library answers such a type MX_EINVAL.
+enum { ON_RULE = 0, ON_BIG, ON_SLIM, ON_STREAM };
 #ifdef MX_BENCH_VARIANTS
 #define MX_EXPERT_OTHER true
+static int named_kernel(int &dtype) {
+    const int which = dtype < 0 ? ON_RULE : dtype >> 4;
+    if (which <= ON_STREAM) dtype -= which << 4;
+    return which;
+}
 #else
 #define MX_EXPERT_OTHER false
+static int named_kernel(int &) { return ON_RULE; }
 #endif
 
 template <typename S, int MODE, int CDT>
@@ -1550,10 +1560,16 @@ static int launch_grouped_stream(GroupedArgs a, hipStream_t st) {
     return hipGetLastError() == hipSuccess ? MX_OK : MX_ELAUNCH;
 }
 
-// Whether the plain product runs as a stream of K stages on 128 x 128 tiles: rows that are not gathered, whole groups of four stages,
-// 16-byte output runs, and up to six tiles per CU (four where K is beyond 1024).  Few rows per expert fill 256 x 256 tiles to a
-// fraction, and a few rounds of large tiles end in a partial one; from there on twice the operand bytes per flop cost more than the
-// stores under the K loops save.
+// What the stream takes of the plain product: rows that are not gathered, whole groups of four stages, 16-byte output runs, 32-bit offsets.
+static bool stream_takes(const GroupedArgs &a) {
+    const int64_t limit = (int64_t)1 << 31;
+    return !a.index && a.K % 512 == 0 && a.out_vec && a.N % 8 == 0 && a.E <= MX_TABLE_MAX_STREAM && a.x_rows >= a.M && 128 * a.ldx < limit &&
+           128 * a.ldw < limit && 128 * a.ldxs < limit && 128 * a.ldws < limit;
+}
+
+// Whether the plain product runs as a stream of K stages on 128 x 128 tiles: up to six tiles per CU (four where K is beyond 1024).
+// Few rows per expert fill 256 x 256 tiles to a fraction, and a few rounds of large tiles end in a partial one; from there on twice the
+// operand bytes per flop cost more than the stores under the K loops save.
 // us on the other shapes / here, 64 experts of 1024 columns, operands from HBM, by rows in all:
 //              200           1000         8000         16662        33000        98304
 //   K = 512   11.5 / 11.6  11.7 / 11.7  18.0 / 16.6  27.6 / 24.2  38.0 / 40.4  82.7 / 107
@@ -1564,20 +1580,22 @@ static int launch_grouped_stream(GroupedArgs a, hipStream_t st) {
 // -> 9.4 and 10.6 -> 8.3 us).  With it 98304 x 1024 x 512 alone takes 72 us, but 107 behind the product that makes its operand, and
 // that pass 60 for 45.
 static bool stream_pays(const GroupedArgs &a) {
-    const int64_t limit = (int64_t)1 << 31;
-    if (a.index || a.K % 512 || (int64_t)a.N * a.K > (2 << 20) || !a.out_vec || a.N % 8 || a.E > MX_TABLE_MAX_STREAM || a.x_rows < a.M || 128 * a.ldx >= limit ||
-        128 * a.ldw >= limit || 128 * a.ldxs >= limit || 128 * a.ldws >= limit)
-        return false;
+    if ((int64_t)a.N * a.K > (2 << 20)) return false;
     const double live = a.E < a.M ? a.E : a.M, rows = (double)a.M / StreamShape::BM + 0.5 * live;
     return (rows > live ? rows : live) * ((a.N + StreamShape::BN - 1) / StreamShape::BN) <= (a.K <= 1024 ? 6.0 : 4.0) * num_cus();
 }
 
 template <int MODE, int CDT>
-static int launch_grouped(const GroupedArgs &a, hipStream_t st) {
-    if constexpr (MODE == MODE_PLAIN && CDT != MX_FP32)
-        if (stream_pays(a) && !MX_EXPERT_OTHER) return launch_grouped_stream<CDT>(a, st);
+static int launch_grouped(const GroupedArgs &a, hipStream_t st, int which = ON_RULE) {
+    bool other = MX_EXPERT_OTHER;
+    if constexpr (MODE == MODE_PLAIN && CDT != MX_FP32) {
+        const bool pays = stream_takes(a) && (which == ON_STREAM || stream_pays(a));
+        if (pays && (which ? which == ON_STREAM : !other)) return launch_grouped_stream<CDT>(a, st);
+        if (pays) other = false;  // of the two that are left, the better one
+    }
+    if (which == ON_STREAM) return MX_EUNSUPPORTED;
     if constexpr (MODE != MODE_SCATTER)
-        if (slim_pays<MODE>(a) != MX_EXPERT_OTHER) return launch_grouped_shape<Slim, MODE, CDT>(a, st);
+        if (which ? which == ON_SLIM : slim_pays<MODE>(a) != other) return launch_grouped_shape<Slim, MODE, CDT>(a, st);
     return launch_grouped_shape<Big, MODE, CDT>(a, st);
 }
 
@@ -1615,7 +1633,7 @@ extern "C" int mx_grouped_gemm_nt(const uint8_t *xq, const uint8_t *xs, int64_t 
     if (mx::stream_is_capturing(st)) return MX_ECAPTURE;
     GroupedArgs a = base_args(xq, xs, ldx, ldxs, index, wq, ws, stride_we, ldw, stride_wse, ldws, offsets, E, M, N, K);
     a.out = out, a.ldo = ldo, a.x_rows = a_rows;
-    const int esz = out_dtype == MX_FP32 ? 4 : 2;
+    const int which = named_kernel(out_dtype), esz = out_dtype == MX_FP32 ? 4 : 2;
     a.out_vec = aligned(out, 16) && (ldo * esz) % 16 == 0;
     if (K == 0 || !tiled_ok(a, a_rows)) {
         if (K == 0) return MX_EUNSUPPORTED;
@@ -1630,9 +1648,9 @@ extern "C" int mx_grouped_gemm_nt(const uint8_t *xq, const uint8_t *xs, int64_t 
         return hipGetLastError() == hipSuccess ? MX_OK : MX_ELAUNCH;
     }
     switch (out_dtype) {
-    case MX_BF16: return launch_grouped<MODE_PLAIN, MX_BF16>(a, st);
-    case MX_FP16: return launch_grouped<MODE_PLAIN, MX_FP16>(a, st);
-    case MX_FP32: return launch_grouped<MODE_PLAIN, MX_FP32>(a, st);
+    case MX_BF16: return launch_grouped<MODE_PLAIN, MX_BF16>(a, st, which);
+    case MX_FP16: return launch_grouped<MODE_PLAIN, MX_FP16>(a, st, which);
+    case MX_FP32: return launch_grouped<MODE_PLAIN, MX_FP32>(a, st, which);
     default: return MX_EINVAL;
     }
 }
@@ -1832,6 +1850,13 @@ static int launch_wgrad_shape(WgradArgs a, float *ws, int64_t ws_bytes, hipStrea
     return hipGetLastError() == hipSuccess ? MX_OK : MX_ELAUNCH;
 }
 
+// What the stream takes of the expert dW: 16-byte output runs, scale rows with 12 readable bytes behind their last stage, 32-bit offsets.
+static bool wgrad_stream_takes(const WgradArgs &a, int esz) {
+    const int64_t limit = (int64_t)1 << 31;
+    return a.E <= MX_TABLE_MAX && aligned(a.dw, 16) && (a.lddw * esz) % 16 == 0 && (a.stride_dwe * esz) % 16 == 0 && a.Kout % 8 == 0 &&
+           a.ldas >= a.KB + 12 && a.ldbs >= a.KB + 12 && 128 * a.ldas < limit && 128 * a.ldbs < limit;
+}
+
 // Whether an expert dW runs as a stream of K stages on 128 x 128 tiles: up to 56 stages per CU, where large tiles would fill no more
 // than the CUs, or than half a round on top with four stages per expert.  Few large tiles leave CUs idle or are cut along K; many, of
 // two or three stages, are mostly their stores either way, and those of 256 columns reach memory faster: the dW of a routing block over 2777
@@ -1842,19 +1867,18 @@ static int launch_wgrad_shape(WgradArgs a, float *ws, int64_t ws_bytes, hipStrea
 //   22216 in 32   45.9 / 43.0      27.2 / 26.4        33000 in 64   71.0 / 70.4     41.9 / 38.6 (48.9 / 44.0 where experts differ ninefold)
 //   16662 in 64   42.4 / 52.3      32.0 / 30.2         2777 in 4    33.6 / 11.3     32.1 / 21.1 (512 x 1024)
 //   of 256 x 256: 1000 in 16   14.0 / 10.8        60000 in 16   34.8 / 22.3        72000 in 32 of 1024 x 1024   85.6 / 116
-static bool wgrad_stream_pays(const WgradArgs &a, int64_t M, int esz) {
-    const int64_t limit = (int64_t)1 << 31;
-    if (a.E > MX_TABLE_MAX || !aligned(a.dw, 16) || (a.lddw * esz) % 16 || (a.stride_dwe * esz) % 16 || a.Kout % 8 || a.ldas < a.KB + 12 ||
-        a.ldbs < a.KB + 12 || 128 * a.ldas >= limit || 128 * a.ldbs >= limit)
-        return false;
+static bool wgrad_stream_pays(const WgradArgs &a, int64_t M) {
     const double live = a.E < M ? a.E : M, cus = num_cus();
     const double tiles = (double)((a.N + StreamShape::BM - 1) / StreamShape::BM) * ((a.Kout + StreamShape::BN - 1) / StreamShape::BN);
     return tiles * ((double)M / 128 + 0.5 * live) <= 56 * cus && tiles * live <= (M >= 480 * live ? 8 : 4) * cus;
 }
 
 template <int CDT>
-static int launch_wgrad(const WgradArgs &a, int64_t M, float *ws, int64_t ws_bytes, hipStream_t st) {
-    if (wgrad_stream_pays(a, M, CDT == MX_FP32 ? 4 : 2)) return launch_wgrad_shape<StreamShape, CDT>(a, ws, ws_bytes, st);
+static int launch_wgrad(const WgradArgs &a, int64_t M, float *ws, int64_t ws_bytes, hipStream_t st, int which) {
+    const bool takes = wgrad_stream_takes(a, CDT == MX_FP32 ? 4 : 2);
+    if (which == ON_SLIM || (which == ON_STREAM && !takes)) return MX_EUNSUPPORTED;
+    if (takes && (which ? which == ON_STREAM : wgrad_stream_pays(a, M) != MX_EXPERT_OTHER))
+        return launch_wgrad_shape<StreamShape, CDT>(a, ws, ws_bytes, st);
     return launch_wgrad_shape<Big, CDT>(a, ws, ws_bytes, st);
 }
 
@@ -1881,10 +1905,11 @@ extern "C" int mx_grouped_wgrad_nt(const uint8_t *aq, const uint8_t *as, int64_t
     a.a_ks = a_panels ? N * 128 : 0, a.b_ks = b_panels ? Kout * 128 : 0;
     hipStream_t st = (hipStream_t)stream;
     if (mx::stream_is_capturing(st)) return MX_ECAPTURE;
+    const int which = named_kernel(dw_dtype);
     switch (dw_dtype) {
-    case MX_BF16: return launch_wgrad<MX_BF16>(a, M, (float *)workspace, workspace_bytes, st);
-    case MX_FP16: return launch_wgrad<MX_FP16>(a, M, (float *)workspace, workspace_bytes, st);
-    case MX_FP32: return launch_wgrad<MX_FP32>(a, M, (float *)workspace, workspace_bytes, st);
+    case MX_BF16: return launch_wgrad<MX_BF16>(a, M, (float *)workspace, workspace_bytes, st, which);
+    case MX_FP16: return launch_wgrad<MX_FP16>(a, M, (float *)workspace, workspace_bytes, st, which);
+    case MX_FP32: return launch_wgrad<MX_FP32>(a, M, (float *)workspace, workspace_bytes, st, which);
     default: return MX_EINVAL;
     }
 }

@@ -2,8 +2,11 @@
 
 Oracle = per-expert loop over the offset table of dequantize-then-matmul in fp64 on operands
 quantized by the oracle; 1e-2 relative Frobenius for 16-bit outputs.  Outputs accumulated with
-atomics (out, dx, dgate) are compared by norm, never bitwise: their summation order is free.
+atomics (out and dx of the scatter route, dgate of the entry that adds it up itself) are compared by norm, never
+bitwise: their summation order is free.
 """
+
+import contextlib
 
 import pytest
 import torch
@@ -809,6 +812,57 @@ def test_expert_kernels_on_small_tiles_agree(counts, hid):
     for name, a, b in zip("hq hs pre htq hts dpre dpq dps ptq pts".split(), shipped, small):
         assert torch.equal(a, b), name
     assert float((dgate - dgate_small).norm() / dgate.norm()) < 1e-5
+
+
+@contextlib.contextmanager
+def _on(flag: str):
+    """Plain expert products and dW inside run on the kernel that this flag of the variants library names."""
+    from kohakuwullm_amd import _lib
+
+    codes = _lib.MX_DTYPE
+    with _lib.variants_library():
+        _lib.MX_DTYPE = {dtype: code | getattr(_lib, flag) for dtype, code in codes.items()}
+        try:
+            yield
+        finally:
+            _lib.MX_DTYPE = codes
+
+
+@pytest.mark.parametrize("counts", [[1], [127, 128, 129], [0, 256, 0, 257, 1], [40] * 70])
+@pytest.mark.parametrize("n,k", [(1000, 512), (136, 1024)])
+def test_named_kernels_agree(counts, n, k):
+    """The plain product and the dW on each kernel that the variants library names: the same bits of the one, the dW within the
+    rounding of its result (K slices are added in another order), and no name in the product library."""
+    from kohakuwullm_amd import _lib
+    from kohakuwullm_amd.kernels.mxfp8.grouped import grouped_mxfp8_gemm, grouped_mxfp8_wgrad, quantize_mx_cols_grouped
+    from kohakuwullm_amd.kernels.mxfp8.quantize import quantize_mx
+
+    g = torch.Generator().manual_seed(SEED + k)
+    e, m = len(counts), sum(counts)
+    offsets = torch.tensor([0] + counts).cumsum(0).int().to(DEV)
+    x, dy = (torch.randn(m, width, generator=g).bfloat16().to(DEV) for width in (k, -(-n // 32) * 32))
+    xq, xs = quantize_mx(x)
+    wq, ws = quantize_mx((torch.randn(e * n, k, generator=g) * 0.1).bfloat16().to(DEV))
+    wq, ws = wq.view(e, n, k), ws.view(e, n, k // 32)
+    a, b = quantize_mx_cols_grouped(dy, offsets, m), quantize_mx_cols_grouped(x, offsets, m)
+    product = lambda: grouped_mxfp8_gemm(xq, xs, wq, ws, offsets)  # noqa: E731
+    dw = lambda: grouped_mxfp8_wgrad(a[0][:n], a[1][:n], *b, offsets, m)  # noqa: E731
+    y, grad = product(), dw()
+    for flag in ("MX_ON_256", "MX_ON_128", "MX_ON_STREAM"):
+        with _on(flag):
+            assert torch.equal(product(), y), flag
+            if flag == "MX_ON_128":
+                with pytest.raises(_lib.MXFP8LibraryError):
+                    dw()
+            else:
+                assert (dw().double() - grad.double()).norm() <= 4e-3 * grad.double().norm(), flag
+    _lib.MX_DTYPE, codes = {torch.bfloat16: _lib.MX_DTYPE[torch.bfloat16] | _lib.MX_ON_256}, _lib.MX_DTYPE
+    try:
+        for call in (product, dw):
+            with pytest.raises(ValueError):
+                call()
+    finally:
+        _lib.MX_DTYPE = codes
 
 
 @pytest.mark.parametrize("counts", [[1], [127, 128, 129], [0, 256, 0, 257, 1], [3] * 40, [700, 2, 0]])
