@@ -1857,20 +1857,30 @@ static bool wgrad_stream_takes(const WgradArgs &a, int esz) {
            a.ldas >= a.KB + 12 && a.ldbs >= a.KB + 12 && 128 * a.ldas < limit && 128 * a.ldbs < limit;
 }
 
-// Whether an expert dW runs as a stream of K stages on 128 x 128 tiles: up to 56 stages per CU, where large tiles would fill no more
-// than the CUs, or than half a round on top with four stages per expert.  Few large tiles leave CUs idle or are cut along K; many, of
-// two or three stages, are mostly their stores either way, and those of 256 columns reach memory faster: the dW of a routing block over 2777
-// tokens (16662 in 64) 30.7 / 40.0 and 51.4 / 51.6.  us on 256 x 256 / here, dW of 1024 x 1024 and of 1024 x 512, by rows in experts:
-//    4000 in 12   19.6 / 17.3           -              4000 in 20        -          37.8 / 16.1
-//   16000 in 12   31.9 / 30.1           -             16000 in 20        -          50.0 / 22.6
-//   48000 in 20        -           69.2 / 54.5        24000 in 32        -          33.2 / 30.7
-//   22216 in 32   45.9 / 43.0      27.2 / 26.4        33000 in 64   71.0 / 70.4     41.9 / 38.6 (48.9 / 44.0 where experts differ ninefold)
-//   16662 in 64   42.4 / 52.3      32.0 / 30.2         2777 in 4    33.6 / 11.3     32.1 / 21.1 (512 x 1024)
-//   of 256 x 256: 1000 in 16   14.0 / 10.8        60000 in 16   34.8 / 22.3        72000 in 32 of 1024 x 1024   85.6 / 116
+// Whether an expert dW runs as a stream of K stages on 128 x 128 tiles.  A large tile per CU is a round of four small ones, so large
+// tiles are the faster ones (half the operand bytes, wider stores) where their rounds are full, and lose what their last round leaves
+// idle: small ones are taken up to three quarters of that, from where on the two are within 8 % of each other or large ones ahead.
+// The operand bytes end it, at 60 stages per CU, or at 100 where small tiles are five eighths or less, or the large ones fewer than
+// three quarters of the CUs and so cut along K.  Each expert is taken to have rows, and as many as the others.
+// us on 256 x 256 / here, dW of 1024 x 512, in a stream of work behind the quantizers that make its operands, by rows per expert:
+//   experts   rounds  small     130          450          900          2400
+//     16       0.50    2/4   17.6 / 9.9   28.1 / 11.3  43.9 / 18.9  56.2 / 29.1   (cut)
+//     24       0.75    3/4   12.3 / 11.2  19.3 / 16.8  27.4 / 24.4  48.5 / 45.5
+//     32       1.00    4/4   11.3 / 10.7  21.1 / 20.5  29.0 / 30.9  54.5 / 63.3
+//     40       1.25    5/8   17.5 / 14.1  31.9 / 26.0  42.2 / 35.4  86.5 / 84.8   (96 stages per CU; again 75.1 / 64.6 of 1024 x 1024)
+//     48       1.50    6/8   19.9 / 19.5  32.5 / 28.1  44.1 / 38.0  87.7 / 100    (115)
+//     56       1.75    7/8   22.6 / 25.4  34.5 / 31.8  44.8 / 46.3  87.7 / 116
+//     64       2.00    8/8   23.8 / 28.0  32.7 / 34.9  50.3 / 56.9  97.7 / 130
+//     72       2.25    9/12  29.4 / 28.6  44.7 / 38.9  67.9 / 69.9   131 / 140    (71, 174)
+// of 1024 x 1024: 9000 in 6 40.0 / 20.2, 48000 in 8 (95, cut) 89.6 / 63.4, 14400 in 16 (4/4) 27.0 / 29.4, 48000 in 20 (5/8, 96) 80.9 / 69.0,
+// 36000 in 24 (6/8, 75) 60.3 / 51.6, 28800 in 32 (8/8) 43.5 / 51.6; 98304 in 6 (193, cut), operands from HBM, 130 / 171.
+// Where experts differ (lognormal, 0.7) large tiles may be cut in any case: 44800 in 64 78.4 / 50.0, but nothing here knows.
 static bool wgrad_stream_pays(const WgradArgs &a, int64_t M) {
     const double live = a.E < M ? a.E : M, cus = num_cus();
-    const double tiles = (double)((a.N + StreamShape::BM - 1) / StreamShape::BM) * ((a.Kout + StreamShape::BN - 1) / StreamShape::BN);
-    return tiles * ((double)M / 128 + 0.5 * live) <= 56 * cus && tiles * live <= (M >= 480 * live ? 8 : 4) * cus;
+    auto tiles = [&](int bm, int bn) { return (double)((a.N + bm - 1) / bm) * ((a.Kout + bn - 1) / bn); };
+    const double large = tiles(Big::BM, Big::BN) * live / cus, small = tiles(StreamShape::BM, StreamShape::BN);
+    const double stages = small * ((double)M / 128 + 0.5 * live) / cus;
+    return small * live <= 3 * ceil(large) * cus && stages <= (large < 0.75 || small * live <= 2.5 * ceil(large) * cus ? 100 : 60);
 }
 
 template <int CDT>

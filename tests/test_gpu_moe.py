@@ -24,6 +24,20 @@ def _dev(q, s):
     return q.to(DEV).view(F8), s.to(DEV)
 
 
+@contextlib.contextmanager
+def _on(flag: str):
+    """Plain expert products and dW inside run on the kernel that this flag of the variants library names."""
+    from kohakuwullm_amd import _lib
+
+    codes = _lib.MX_DTYPE
+    with _lib.variants_library():
+        _lib.MX_DTYPE = {dtype: code | getattr(_lib, flag) for dtype, code in codes.items()}
+        try:
+            yield
+        finally:
+            _lib.MX_DTYPE = codes
+
+
 def _routing(counts, top_k, tokens, seed=SEED):
     """offsets/order/token_of for given per-expert counts: position m of expert e takes distinct tokens."""
     g = torch.Generator().manual_seed(seed)
@@ -415,6 +429,33 @@ def test_wgrad_stream_of_stages(oracle, counts, n, k, dtype):
         got = dw[i].cpu().double()
         bound = {torch.bfloat16: 4e-3, torch.float16: 1e-3, torch.float32: 1e-4}[dtype]
         assert (got - ref).norm() <= bound * ref.norm(), (i, cnt)
+
+
+@pytest.mark.parametrize("experts,rows,n,k,flag", [
+    (23, 900, 1024, 512, "MX_ON_STREAM"), (8, 6000, 1024, 1024, "MX_ON_STREAM"), (8, 6600, 1024, 1024, "MX_ON_256"),  # large tiles cut along K
+    (24, 640, 1024, 512, None), (32, 130, 1024, 512, None), (32, 700, 1024, 1024, None),  # three of four small rounds, four of four, eight of eight
+    (40, 1000, 1024, 512, None), (48, 1000, 1024, 512, None), (48, 1400, 1024, 512, None),  # five of eight, six of eight, and with too many stages
+])
+def test_wgrad_on_either_side_of_the_rule(experts, rows, n, k, flag):
+    """The dW that ships against both kernels it is chosen from.  Whole tiles are the same bits on either; where large tiles would be
+    cut along K the sums come in another order, and the bits are those of the kernel named here."""
+    from kohakuwullm_amd.kernels.mxfp8.grouped import grouped_mxfp8_wgrad, quantize_mx_cols_grouped
+
+    g = torch.Generator(DEV).manual_seed(SEED + experts)
+    m = experts * rows
+    offsets = torch.arange(experts + 1, device=DEV, dtype=torch.int32) * rows
+    spread = torch.exp2(4 * torch.randn(m, 1, device=DEV, generator=g))  # block scales differ: with one for all, sums in any order are exact
+    a, b = ((torch.randn(m, width, device=DEV, generator=g) * spread).bfloat16() for width in (n, k))
+    operands = [t for x in (a, b) for t in quantize_mx_cols_grouped(x, offsets, m, stage_major=True)]
+    dw = grouped_mxfp8_wgrad(*operands, offsets, m)
+    for other in ("MX_ON_256", "MX_ON_STREAM"):
+        with _on(other):
+            got = grouped_mxfp8_wgrad(*operands, offsets, m)
+        if flag in (None, other):
+            assert torch.equal(got, dw), other
+        else:
+            assert not torch.equal(got, dw)
+            assert float((got.double() - dw.double()).norm()) <= 4e-3 * float(dw.double().norm())
 
 
 def _expert_oracle(ora, x, w_in, w_out, gate, token_of, order, offsets, dout):
@@ -812,20 +853,6 @@ def test_expert_kernels_on_small_tiles_agree(counts, hid):
     for name, a, b in zip("hq hs pre htq hts dpre dpq dps ptq pts".split(), shipped, small):
         assert torch.equal(a, b), name
     assert float((dgate - dgate_small).norm() / dgate.norm()) < 1e-5
-
-
-@contextlib.contextmanager
-def _on(flag: str):
-    """Plain expert products and dW inside run on the kernel that this flag of the variants library names."""
-    from kohakuwullm_amd import _lib
-
-    codes = _lib.MX_DTYPE
-    with _lib.variants_library():
-        _lib.MX_DTYPE = {dtype: code | getattr(_lib, flag) for dtype, code in codes.items()}
-        try:
-            yield
-        finally:
-            _lib.MX_DTYPE = codes
 
 
 @pytest.mark.parametrize("counts", [[1], [127, 128, 129], [0, 256, 0, 257, 1], [40] * 70])
