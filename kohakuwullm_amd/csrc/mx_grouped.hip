@@ -867,7 +867,7 @@ __global__ __launch_bounds__(256) void combine_kernel(const uint16_t *__restrict
 }
 
 // dgate[p] = the parts of pair p, added in the order of the columns they stand for; zero for a pair no row belongs to (whose parts
-// nothing has written).
+// nothing has written).  4.7 us for 19200 pairs of four parts, latency; the fill and the conversion that it replaces took 5.6.
 template <typename T>
 __global__ __launch_bounds__(256) void gate_grad_kernel(const float *__restrict__ parts, int64_t ld, int slices,
                                                         const int32_t *__restrict__ positions, T *__restrict__ dgate, int64_t pairs) {
@@ -1476,13 +1476,14 @@ typedef GemmShape<128, 128, 4, 1> Slim;
 // K loops, goes to Slim wherever that needs no more of them.  The fused kernels' rounds are epilogues, and in those half
 // the values are half the time less what the two workgroups share: 14 us against 22 (GEMM1), 24 against 44 (GEMM2-dgrad),
 // so three Slim rounds are taken in place of two.  Few rows per expert fill a Big tile to a fraction, and few tiles leave
-// CUs idle; from about 300 rows in 64 experts on, Big is ahead again (1536 rows: GEMM1 189 / 199 us, plain 135 / 189).
+// CUs idle; from about 300 rows in 64 experts on, Big is ahead again (1536 rows: GEMM1 189 / 199 us, plain 130 / 164).
 // us Big / Slim, 64 experts of 1024 x 512, top 6, by rows per expert:
 //                       3             48            188           260           384
 //   GEMM1          25.3 / 19.0   25.9 / 20.6   47.1 / 33.2   50.7 / 46.9   49.2 / 55.3
 //   GEMM2-dgrad    33.5 / 22.4   40.8 / 25.6   46.6 / 31.1   48.5 / 47.2   48.0 / 53.7
-//   plain, K 512   12.6 /  9.4   13.5 / 10.9   22.7 / 16.9   23.6 / 21.9   23.8 / 24.8
-//   plain, K 1024  19.0 / 14.8   19.6 / 16.3   32.6 / 24.9   33.5 / 32.8   34.8 / 39.7
+//   plain, K 512   15.3 / 12.4   16.4 / 13.7   28.6 / 24.6   29.2 / 29.0   30.6 / 38.1
+//   plain, K 1024  23.1 / 20.3   24.7 / 22.1   43.3 / 36.7   43.0 / 43.1   44.4 / 57.1
+// (plain: gathered rows, which the stream of K stages does not take; at 188 rows 20.5 / 22.3 and 29.6 / 34.1 if no expert has over 256)
 template <int MODE>
 static bool slim_pays(const GroupedArgs &a) {
     if (a.E > row_table_max<Slim, false>()) return false;  // its table of row tiles, half of Big's, keeps the lookup cheap
@@ -1567,31 +1568,51 @@ static bool stream_takes(const GroupedArgs &a) {
            128 * a.ldw < limit && 128 * a.ldxs < limit && 128 * a.ldws < limit;
 }
 
-// Whether the plain product runs as a stream of K stages on 128 x 128 tiles: up to six tiles per CU (four where K is beyond 1024).
-// Few rows per expert fill 256 x 256 tiles to a fraction, and a few rounds of large tiles end in a partial one; from there on twice the
-// operand bytes per flop cost more than the stores under the K loops save.
-// us on the other shapes / here, 64 experts of 1024 columns, operands from HBM, by rows in all:
-//              200           1000         8000         16662        33000        98304
-//   K = 512   11.5 / 11.6  11.7 / 11.7  18.0 / 16.6  27.6 / 24.2  38.0 / 40.4  82.7 / 107
-//   K = 1024       -            -            -       41.4 / 36.8  55.8 / 59.5       -        (40000 in 32   55.0 / 68.5)
-// of 8 experts 1000 rows x K = 1024 11.3 / 8.2, 16662 x 1024 32.5 / 26.7; of 16, 65536 rows of 256 columns 26.2 / 23.8; K = 1536 and
-// 2048, 20000 in 16 (5 tiles per CU) 49.0 / 50.4 and 59.9 / 62.7, 8000 in 8 of 512 columns 21.0 / 19.8.
+// How many tiles of `bm` rows `live` experts with M rows have, if they differ evenly by up to a fifth from the mean.
+static double expected_row_tiles(double M, double live, int bm) {
+    const double lo = 0.8 * M / live, hi = 1.2 * M / live;
+    auto upto = [bm](double x) {  // the integral of ceil(rows / bm)
+        const double whole = floor(x / bm);
+        return bm * whole * (whole + 1) / 2 + (whole + 1) * (x - whole * bm);
+    };
+    return live * (upto(hi) - upto(lo)) / (hi - lo);
+}
+
+// Whether the plain product runs as a stream of K stages on 128 x 128 tiles.  As for the dW (wgrad_stream_pays), a 256 x 256 tile per CU
+// is a round of four small ones: full rounds of those are faster, and rounds that few rows per expert or the last tiles leave partly
+// empty are not.  A stream's last round is short where it is not full, so its tiles are not counted in rounds; it is taken up to 0.68 of
+// the large ones.  Depth ends it, at 128 stages per CU.
+// us on the better one of the other shapes / here, behind the quantizer of the rows and in front of the pass that adds them up:
+//   64 experts of 1024 columns, by rows per expert (small tiles, of four times the rounds of large ones):
+//                16 (.50)     60 (.50)    130 (.77)    260 (.63)    400 (.90)    520 (.76)   1536 (.89)
+//     K = 512    8.8 / 9.6   9.9 / 9.7  13.5 / 14.6  26.5 / 24.9  26.3 / 33.4  35.7 / 38.5  61.0 / 80.4
+//     K = 1024  13.4 / 12.5 17.1 / 16.7 25.1 / 27.3  39.9 / 36.3  40.2 / 52.5  52.8 / 59.7   111 / 151
+//   K = 1024, 180 rows (1.0) 27.2 / 31.5, 215 (.57) 37.1 / 35.0; 32 experts, 400 rows (.90) 23.2 / 31.1, 700 (.75) 40.8 / 39.0,
+//   1400 (.95) 53.6 / 67.1; of 2048 columns in 8, 2000 rows (.67) 49.6 / 45.6
+//   8 experts, by width and depth, 130 rows (.10 to .38), 600 (.33 to .65) and 2000 (.50 to .83):
+//     1024 x 1536  10.2 / 8.8  15.7 / 13.6  41.8 / 35.4      2048 x 1536  12.0 / 8.4  25.2 / 24.4  63.2 / 59.0
+//     1024 x 2560  20.6 / 13.0 28.1 / 26.7  64.1 / 56.9      2048 x 2048  16.0 / 10.5 32.6 / 30.9  77.7 / 76.7 (144 stages per CU)
+//      512 x 4096  31.3 / 18.0 37.7 / 24.7  55.9 / 55.6      4096 x 4096  51.1 / 51.7  108 / 121    260 / 386  (49, 192, 544)
 // The results are stored without the non-temporal hint: the pass that adds them up per token finds them in the cache (16662 rows: 13.8
-// -> 9.4 and 10.6 -> 8.3 us).  With it 98304 x 1024 x 512 alone takes 72 us, but 107 behind the product that makes its operand, and
-// that pass 60 for 45.
+// and 10.6 us with it, 9.4 and 8.3 without, and 9.3 and 8.5 behind the other shapes).  With it 98304 x 1024 x 512 alone takes 72 us, but
+// 107 behind the product that makes its operand, and that pass 60 for 45.
 static bool stream_pays(const GroupedArgs &a) {
-    if ((int64_t)a.N * a.K > (2 << 20)) return false;
-    const double live = a.E < a.M ? a.E : a.M, rows = (double)a.M / StreamShape::BM + 0.5 * live;
-    return (rows > live ? rows : live) * ((a.N + StreamShape::BN - 1) / StreamShape::BN) <= (a.K <= 1024 ? 6.0 : 4.0) * num_cus();
+    const double live = a.E < a.M ? a.E : a.M, cus = num_cus();
+    const double small = expected_row_tiles(a.M, live, StreamShape::BM) * ((a.N + StreamShape::BN - 1) / StreamShape::BN) / cus;
+    const double large = expected_row_tiles(a.M, live, Big::BM) * ((a.N + Big::BN - 1) / Big::BN) / cus;
+    return small <= 0.68 * 4 * ceil(large - 0.02) && small * (a.K >> 7) <= 128;
 }
 
 template <int MODE, int CDT>
 static int launch_grouped(const GroupedArgs &a, hipStream_t st, int which = ON_RULE) {
     bool other = MX_EXPERT_OTHER;
     if constexpr (MODE == MODE_PLAIN && CDT != MX_FP32) {
-        const bool pays = stream_takes(a) && (which == ON_STREAM || stream_pays(a));
-        if (pays && (which ? which == ON_STREAM : !other)) return launch_grouped_stream<CDT>(a, st);
-        if (pays) other = false;  // of the two that are left, the better one
+        if (stream_takes(a)) {
+            const bool pays = stream_pays(a);
+            if (which ? which == ON_STREAM : pays != other) return launch_grouped_stream<CDT>(a, st);
+            if (!which && !other) return launch_grouped_shape<Big, MODE, CDT>(a, st);  // Slim is nowhere ahead of both
+            other = false;  // of the two that are left, the better one
+        }
     }
     if (which == ON_STREAM) return MX_EUNSUPPORTED;
     if constexpr (MODE != MODE_SCATTER)
@@ -1874,6 +1895,9 @@ static bool wgrad_stream_takes(const WgradArgs &a, int esz) {
 //     72       2.25    9/12  29.4 / 28.6  44.7 / 38.9  67.9 / 69.9   131 / 140    (71, 174)
 // of 1024 x 1024: 9000 in 6 40.0 / 20.2, 48000 in 8 (95, cut) 89.6 / 63.4, 14400 in 16 (4/4) 27.0 / 29.4, 48000 in 20 (5/8, 96) 80.9 / 69.0,
 // 36000 in 24 (6/8, 75) 60.3 / 51.6, 28800 in 32 (8/8) 43.5 / 51.6; 98304 in 6 (193, cut), operands from HBM, 130 / 171.
+// A routing block of 32 experts, both of its dW full rounds, takes with 600 rows per expert 343 us a pass on large tiles, 336 on small
+// ones and 348 with one of each; from 800 rows on large ones are ahead (382 / 390; 1300 rows 520 / 550).  One of 64 experts, of which
+// dW_in stays on large tiles in any case, 521 / 537 with 487 rows and 597 / 629 with 656.
 // Where experts differ (lognormal, 0.7) large tiles may be cut in any case: 44800 in 64 78.4 / 50.0, but nothing here knows.
 static bool wgrad_stream_pays(const WgradArgs &a, int64_t M) {
     const double live = a.E < M ? a.E : M, cus = num_cus();

@@ -892,6 +892,29 @@ def test_named_kernels_agree(counts, n, k):
         _lib.MX_DTYPE = codes
 
 
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("experts,rows,n,k", [
+    (64, 100, 1024, 512), (64, 180, 1024, 512), (64, 215, 1024, 512), (64, 300, 1024, 512),  # two, four, and more small tiles per CU
+    (8, 130, 2048, 2048), (8, 600, 512, 4096), (8, 2000, 2048, 1024), (8, 2000, 2048, 2560),  # wide and deep experts, up to and past 128 stages per CU
+    (8, 1, 4096, 512), (300, 3, 1000, 1536),
+])
+def test_plain_product_on_either_side_of_the_rule(experts, rows, n, k, dtype):
+    """The product that ships, on whichever kernel, has the bits of each of the three; experts differ in load, and one has no rows."""
+    from kohakuwullm_amd.kernels.mxfp8.grouped import grouped_mxfp8_gemm
+
+    g = torch.Generator(DEV).manual_seed(SEED + rows)
+    counts = [max(1, rows + (i * 37) % 61 * rows // 200 - rows // 7) for i in range(experts - 1)] + [0]
+    m, offsets = sum(counts), torch.tensor([0] + counts).cumsum(0).int().to(DEV)
+    codes = lambda *shape: torch.randint(-128, 127, shape, device=DEV, generator=g, dtype=torch.int8).view(torch.uint8) & 0xBF  # noqa: E731  (up to 1.875)
+    scales = lambda *shape: torch.randint(118, 126, shape, device=DEV, generator=g, dtype=torch.uint8)  # noqa: E731
+    operands = codes(m, k).view(F8), scales(m, k // 32), codes(experts, n, k).view(F8), scales(experts, n, k // 32)
+    y = grouped_mxfp8_gemm(*operands, offsets, out_dtype=dtype)
+    assert bool(y.isfinite().all()) and bool(y.any(dim=1).all())
+    for flag in ("MX_ON_256", "MX_ON_128", "MX_ON_STREAM"):
+        with _on(flag):
+            assert torch.equal(grouped_mxfp8_gemm(*operands, offsets, out_dtype=dtype), y), flag
+
+
 @pytest.mark.parametrize("counts", [[1], [127, 128, 129], [0, 256, 0, 257, 1], [3] * 40, [700, 2, 0]])
 @pytest.mark.parametrize("n,k,dtype", [(1000, 512, torch.bfloat16), (136, 384, torch.float16), (257, 1024, torch.float32)])
 def test_grouped_product_on_either_tile_shape(counts, n, k, dtype):
