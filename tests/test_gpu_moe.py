@@ -66,8 +66,8 @@ COUNT_CASES = [
     # many experts, most of them empty, the busy ones behind long runs of empties: the owner of a
     # tile is found through the per-workgroup expert tables (more than one 64-expert chunk)
     [0] * 70 + [200] + [0] * 130 + [129, 1] + [0] * 50,
-    # more experts than the expert dW kernel's smaller table beside its scale staging area holds (760), fewer than
-    # the full table (1024): the dW kernel with scale bytes in registers
+    # more experts than the 256 x 256 dW kernel's smaller table beside its scale staging area holds (760), fewer than
+    # the full table (1024)
     [0] * 780 + [150, 40] + [0] * 20,
     # more experts than the tables hold: the kernels fall back to walking `offsets`
     [0] * 1040 + [90, 0, 33] + [0] * 20,
@@ -110,10 +110,11 @@ def test_grouped_gemm(oracle, counts, use_index):
 @pytest.mark.parametrize("counts,n", [([3000, 0, 2500, 1, 4100, 700], 1792), ([5, 0, 130], 264), ([0, 0, 1], 8), ([257] * 9, 512)])
 def test_grouped_gemm_look_ahead_schedule(oracle, k, use_index, counts, n):
     """K a multiple of 512 with 16-byte aligned scale rows takes the schedule that fetches the A operand two K stages
-    ahead and its scale bytes through the copy engine.  More tiles than workgroups, so every workgroup crosses tile
-    boundaries (ragged last tiles, an empty and a one-row expert among them), and launches of one or a few tiles; with
-    and without gathered rows.  Against
-    the fp64 oracle, and bit for bit against the one-stage schedule, which scale rows of another pitch select."""
+    ahead and its scale bytes through the copy engine: on 256 x 256 tiles without gathered rows.  More tiles than workgroups,
+    so every workgroup crosses tile boundaries (ragged last tiles, an empty and a one-row expert among them), and launches of
+    one or a few tiles; with and without gathered rows.  16-bit results of rows in place may come from the stream of K stages,
+    so that schedule is also named.  Against the fp64 oracle, and bit for bit against the one-stage schedule, which scale rows
+    of another pitch select."""
     from kohakuwullm_amd.kernels.mxfp8.grouped import grouped_mxfp8_gemm
     from kohakuwullm_amd.kernels.mxfp8.quantize import quantize_mx
 
@@ -135,6 +136,9 @@ def test_grouped_gemm_look_ahead_schedule(oracle, k, use_index, counts, n):
     xs_other = torch.empty(tokens, k // 32 + 4, device=DEV, dtype=torch.uint8)[:, : k // 32]  # pitch not a multiple of 16
     xs_other.copy_(xs)
     assert torch.equal(got, grouped_mxfp8_gemm(xq, xs_other, wq, ws, offsets.to(DEV), index, rows=m))
+    with _on("MX_ON_256"):
+        for scales in (xs, xs_other):
+            assert torch.equal(got, grouped_mxfp8_gemm(xq, scales, wq, ws, offsets.to(DEV), index, rows=m))
     got32 = grouped_mxfp8_gemm(xq, xs, wq, ws, offsets.to(DEV), index, out_dtype=torch.float32, rows=m)
     assert oracle.rel_error(got32.cpu(), ref) < 1e-4
 
@@ -306,12 +310,12 @@ def test_grouped_token_axis_quantizer_many_rows(oracle, with_scale):
 def test_wgrad_even_k_split_ranges_straddle_experts(oracle, counts):
     """Few busy experts with several output tiles each: the K stages of all experts are cut into equal
     ranges, one per group of workgroups, and ranges end inside an expert and straddle two of them
-    (19 + 6 + 23 stages in ranges of 2, for the first case).  Every expert against the fp64 oracle."""
+    (19 + 6 + 23 stages in ranges of 3, for the first case).  Every expert against the fp64 oracle."""
     from kohakuwullm_amd.kernels.mxfp8.grouped import grouped_mxfp8_wgrad, quantize_mx_cols_grouped
 
     g = torch.Generator().manual_seed(SEED + 7)
     e, m = len(counts), sum(counts)
-    n, k = 512, 384  # 2 x 2 output tiles per expert
+    n, k = 512, 384  # 4 x 3 output tiles per expert
     offsets = torch.zeros(e + 1, dtype=torch.int32)
     offsets[1:] = torch.tensor(counts).cumsum(0)
     a = (torch.randn(m, n, generator=g) * 1e-2).bfloat16()
@@ -369,8 +373,9 @@ def test_wgrad_of_experts_without_rows_is_zero(counts, n, k, dtype):
                                         ([128] * 130 + [4000] + [1] * 140, 256, 512)])
 def test_wgrad_runs_of_single_stage_tiles(oracle, counts, n, k):
     """More (expert, tile) units than workgroups, most of them a single K stage (experts of up to 128 rows), in runs and
-    mixed with longer ones: the expert dW kernel fetches its A operand two stages ahead, and a stage that lies two tiles
-    on is fetched one stage ahead instead.  Every expert against the fp64 oracle."""
+    mixed with longer ones.  The kernel on 256 x 256 tiles, which the second case takes, fetches its A operand two stages ahead,
+    and a stage that lies two tiles on one stage ahead instead; the others take the stream of K stages, the third one cut into
+    ranges.  Every expert against the fp64 oracle."""
     from kohakuwullm_amd.kernels.mxfp8.grouped import grouped_mxfp8_wgrad, quantize_mx_cols_grouped
 
     g = torch.Generator().manual_seed(SEED + 8)
@@ -400,10 +405,10 @@ def test_wgrad_runs_of_single_stage_tiles(oracle, counts, n, k):
 
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16, torch.float32])
 @pytest.mark.parametrize("counts,n,k", [
-    ([1, 128, 129, 0, 300, 513, 640], 200, 136),  # one to five stages, even and odd; edges of tiles both ways
-    ([200] * 40, 512, 256),  # several tiles per workgroup
-    ([2777], 256, 264),  # one long expert: K slices
-    ([0, 700, 0, 3000, 5], 128, 128),  # ranges of K slices that straddle experts; workgroups without any
+    ([1, 128, 129, 0, 300, 513, 640], 200, 136),  # K cut into single stages; edges of tiles both ways
+    ([200] * 40, 512, 256),  # whole tiles of two stages, two of them on some workgroups
+    ([2777], 256, 264),  # one long expert, in ranges of three stages
+    ([0, 700, 0, 3000, 5], 128, 128),  # single stages; workgroups without any
 ])
 def test_wgrad_stream_of_stages(oracle, counts, n, k, dtype):
     """Few stages per CU: the kernel whose loader waves run through tile boundaries.  Every expert against fp64 on the same
@@ -456,6 +461,49 @@ def test_wgrad_on_either_side_of_the_rule(experts, rows, n, k, flag):
         else:
             assert not torch.equal(got, dw)
             assert float((got.double() - dw.double()).norm()) <= 4e-3 * float(dw.double().norm())
+
+
+MIXED = [385 + i * 137 % 716 for i in range(32)]  # four to nine stages, odd and even
+
+
+@pytest.mark.parametrize("counts,n,k", [
+    (MIXED, 500, 520),  # whole tiles of four to nine stages, two or three of differing length on a workgroup; edges of tiles both ways
+    (MIXED, 512, 256),  # one such tile on a workgroup
+    ([6000, 0, 3500, 200], 640, 512),  # on the stream, ranges of seven stages that end inside an expert and straddle two
+    ([2400, 0, 700, 2900], 512, 384), ([5000, 1], 512, 384), ([130, 0, 0, 4000, 0, 1500], 512, 384),  # 2 x 2 large tiles, ranges of one stage
+    ([128] * 130 + [4000] + [1] * 140, 256, 512),  # runs of single stages and a long expert; large tiles cut though they fill the CUs
+    ([50] * 300, 256, 256),  # whole tiles of a single stage
+    ([0] * 780 + [150, 40] + [0] * 20, 256, 192),  # experts that only the larger table holds: the large kernel's scale bytes in registers
+])
+def test_wgrad_on_each_kernel(oracle, counts, n, k):
+    """Each of the two dW kernels, named, and the one that ships, at tiles and ranges of every length: in each type against fp64 on
+    the same codes (bounds: test_wgrad_stream_of_stages), and the same bits again."""
+    from kohakuwullm_amd.kernels.mxfp8.grouped import grouped_mxfp8_wgrad, quantize_mx_cols_grouped
+
+    g = torch.Generator().manual_seed(SEED + 33)
+    m, panels = sum(counts), n % 32 == 0 and k % 32 == 0
+    offsets = torch.zeros(len(counts) + 1, dtype=torch.int32)
+    offsets[1:] = torch.tensor(counts).cumsum(0)
+    # Block scales differ from stage to stage.  A sum of 6000 products has a deviation of 1e-2 sqrt(6000 E[spread^4]) = 5, and its
+    # largest one is 1e-2 times 4.5^2 times 2^9 = 100: far below fp16's 65504.
+    spread = torch.exp2(torch.randn(m, 1, generator=g))
+    a, b = ((torch.randn(m, -(-w // 32) * 32, generator=g) * spread * std).bfloat16() for w, std in ((n, 1e-2), (k, 1.0)))
+    operands = []
+    for x, w in ((a, n), (b, k)):
+        q, s = quantize_mx_cols_grouped(x.to(DEV), offsets.to(DEV), m, stage_major=panels)
+        operands += [q if panels else q[:w], s[:w]]
+    ad, bd = (oracle.dequant(*_padded_cols_ref(oracle, t.float(), offsets)[:2]) for t in (a[:, :n], b[:, :k]))
+    want, pos = [], 0
+    for cnt in counts:
+        want.append(ad[:, pos : pos + cnt].double() @ bd[:, pos : pos + cnt].double().T)
+        pos += -(-cnt // 128) * 128
+    for dtype, bound in ((torch.bfloat16, 4e-3), (torch.float16, 1e-3), (torch.float32, 1e-4)):
+        for kernel in (contextlib.nullcontext(), _on("MX_ON_256"), _on("MX_ON_STREAM")):
+            with kernel:
+                dw, again = (grouped_mxfp8_wgrad(*operands, offsets.to(DEV), m, dtype) for _ in range(2))
+            assert torch.equal(dw, again)
+            for i, (got, ref) in enumerate(zip(dw.cpu(), want)):
+                assert float((got.double() - ref).norm()) <= bound * float(ref.norm()), (dtype, i, counts[i])
 
 
 def _expert_oracle(ora, x, w_in, w_out, gate, token_of, order, offsets, dout):
