@@ -15,7 +15,9 @@
 // spills at that.  0.43 us a stage with a tile on every CU (2.4 PFLOP/s), bound by the operand bytes between L2 and LDS; with the
 // loads and stores in the same eight waves 98304 x 1024 x 512 in 64 experts took 109 us, without its stores 58; with loaders of their
 // own 102 and 54, with the stores spread over the next tile's steps 72 (non-temporal; 107 if not).
-// Operand layout, swizzle, the output run of a lane and the order of the sums are those of mx_gemm_core.h: the same bits.
+// Operand layout, swizzle, the output run of a lane and the order in which a tile adds its K stages are those of mx_gemm_core.h: a tile
+// that is not cut along K has the same bits.  Where the expert dW is cut, the ranges of stages follow from the tiles per expert, and the
+// fp32 sums of the ranges are added in another order than 256 x 256 tiles have them in.
 #pragma once
 
 #include "mx_gemm_core.h"
